@@ -5,10 +5,10 @@
 // loops).  No counterpart in the reference.
 //
 // scratch holds the packed bodies (n_pad float4, then the pack kernel's
-// SF_BODY_STATE words) and, from the next 256-byte boundary, the slice
-// partials (one double4 per particle and block slice).  It is sized for N up
-// to SF_NOALLOC_MAX_N, where n_pad = N and the fast kernel writes 16 block
-// slices: 256 KiB + 256 B of bodies and 8 MiB of partials.  Each device
+// SF_BODY_STATE words) and, from the next 256-byte boundary, the force
+// kernel's partial sums.  It is sized for every N up to SF_NOALLOC_MAX_N:
+// 256 KiB + 256 B of bodies and 16.3 MiB of partials (65 planes of one float4
+// per body at the largest n_pad).  Each device
 // holds its own copy; its address comes from hipGetSymbolAddress, once per
 // device, on the first call with that device current.
 #include <hip/hip_runtime.h>
@@ -16,6 +16,7 @@
 #include <mutex>
 
 #include "../sf_internal.h"
+#include "pp_sym.h"
 
 extern "C" {
 size_t sf_pp_part_bytes(unsigned int n_pad);
@@ -27,11 +28,20 @@ int sfd_fill0(float* y, unsigned int n, hipStream_t s);
 namespace {
 
 constexpr unsigned kMaxN = SF_NOALLOC_MAX_N;
-constexpr unsigned kMaxBlockSlices = 16;   // of k_pp_fast at n_pad = kMaxN
 constexpr size_t kAlign = 256;
 constexpr size_t align_up(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 constexpr size_t kBodyBytes = align_up(SF_BODY_BYTES(kMaxN));
-constexpr size_t kPartBytes = (size_t)kMaxBlockSlices * kMaxN * 32u;
+// the largest partial sums over the sizes: sym_part_bytes from kSymMin
+// bodies; below, k_pp_fast's block slices (at most one double4 plane per 1024 bodies)
+constexpr size_t max_part_bytes() {
+	size_t most = 0;
+	for (unsigned n = 1024u; n <= kMaxN; n += 1024u) {
+		const size_t b = n >= kSymMin ? sym_part_bytes(n, sym_pp_wide(n)) : (size_t)(n / 1024u) * n * 32u;
+		if (b > most) most = b;
+	}
+	return most;
+}
+constexpr size_t kPartBytes = max_part_bytes();
 
 static __device__ __align__(256) unsigned char scratch[kBodyBytes + kPartBytes];
 

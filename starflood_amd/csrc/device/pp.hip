@@ -14,24 +14,25 @@
 // CPU path.  One lane owns one i; the j stream is wavefront-uniform, so the
 // compiler fetches it with scalar loads into SGPRs.
 //
-// k_pp_fast is the throughput kernel: 13 VALU operations plus one v_rsq_f32
-// per interaction, one i per lane, j fetched with scalar loads, partial sums
-// per tile of SF_TJ interactions folded into a Kahan-compensated running
-// sum, and the j range split into slices so the grid fills all 256 CUs.
+// k_pp_fast is the throughput kernel below 10240 bodies (from there
+// pp_sym.hip evaluates each pair once): 13 VALU operations plus one
+// v_rsq_f32 per interaction, one i per lane, j fetched with scalar loads,
+// partial sums per tile of SF_TJ interactions folded into a
+// Kahan-compensated running sum, and the j range split into slices so the
+// grid fills the CUs.
 // When every particle has the same mass m (k_pack_bodies checks the bits of
 // each mass on the device), the whole tiles of real particles drop the
 // per-pair mass product: they sum 1/s^3 (r_j - r_i) and 1/s with 12 VALU
 // operations plus the rsqrt, and the tile partial is scaled by m before the
 // fold.  A block's four wavefronts hold the same 64 particles and split its
 // slice into four sub-slices; their sums meet in LDS in FP64, in wavefront
-// order, so a block writes one double4 per particle.  Slice s is processed
-// by blocks with blockIdx % slices == s, which the dispatcher places on XCD
-// (s mod 8), so each XCD's L2 holds only its own part of the body array.
+// order, so a block writes one double4 per particle.
 // A second kernel adds the slice partials per i in fixed order in FP64,
 // which keeps the result deterministic.
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "pp_sym.h"
 
 namespace {
 
@@ -393,8 +394,13 @@ static PPGeometry pp_geometry(unsigned n_pad, unsigned slices) {
 }
 
 extern "C" size_t sfd_pp_part_bytes(unsigned n_pad, unsigned slices) {
+	if (n_pad >= kSymMin) return sym_part_bytes(n_pad, sym_pp_wide(n_pad));
 	return n_pad ? (size_t)pp_geometry(n_pad, slices).bslices * n_pad * sizeof(double4) : 0u;
 }
+
+// device/pp_sym.hip
+extern "C" int sfd_pp_sym(const float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys,
+                          float* part, float* acc, float* pot, hipStream_t s);
 
 extern "C" int sfd_pp_fast(const float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys,
                            float* part, unsigned slices, float* acc, float* pot, hipStream_t s) {
@@ -403,7 +409,9 @@ extern "C" int sfd_pp_fast(const float* body, unsigned N, unsigned n_pad, float 
 		sf_error("sfd_pp_fast", "n_pad %u is not a multiple of %u", n_pad, SF_TJ);
 		return -1;
 	}
-	// part holds sfd_pp_part_bytes(n_pad, slices): one double4 plane per block slice
+	// part holds sfd_pp_part_bytes(n_pad, slices)
+	if (n_pad >= kSymMin) return sfd_pp_sym(body, N, n_pad, eps2, G, acc_phys, part, acc, pot, s);
+	// one double4 plane per block slice
 	const PPGeometry g = pp_geometry(n_pad, slices);
 	const unsigned grid = (n_pad / 64u) * g.bslices;
 	double4* p4 = reinterpret_cast<double4*>(part);

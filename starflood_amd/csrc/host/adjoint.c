@@ -36,7 +36,8 @@ typedef struct {
 	unsigned int N, n_pad, slices;
 	float* body;   /* n_pad float4 */
 	float* nu;     /* n_pad float4 */
-	float* part;   /* slices x 2 x n_pad float4 */
+	float* part;   /* slices x 2 x n_pad float4, or the PP force's partial sums */
+	size_t part_bytes;
 } sf_pp_scratch;
 
 static void scratch_free(sf_pp_scratch* w) {
@@ -50,10 +51,12 @@ static int scratch_alloc(sf_pp_scratch* w, unsigned int N, const char* func) {
 	w->N = N;
 	w->n_pad = ((N ? N : 1u) + 1023u) / 1024u * 1024u;
 	w->slices = sf_pp_slice_count(w->n_pad);
-	const size_t plane = (size_t)w->n_pad * 4u * sizeof(float);
+	const size_t plane = (size_t)w->n_pad * 4u * sizeof(float), pp_bytes = sf_pp_part_bytes(w->n_pad);
+	w->part_bytes = plane * 2u * w->slices;
+	if (w->part_bytes < pp_bytes) w->part_bytes = pp_bytes;
 	if (hipMalloc((void**)&w->body, SF_BODY_BYTES(w->n_pad)) != hipSuccess ||
 	    hipMalloc((void**)&w->nu, plane) != hipSuccess ||
-	    hipMalloc((void**)&w->part, plane * 2u * w->slices) != hipSuccess) {
+	    hipMalloc((void**)&w->part, w->part_bytes) != hipSuccess) {
 		sf_error(func, "device allocation for N = %u failed", N);
 		scratch_free(w);
 		return -1;
@@ -71,8 +74,7 @@ static float eps2_of(const sf_params_t* p) { return (float)(p->epsilon * p->epsi
 
 static int force(const sf_params_t* p, sf_pp_scratch* w, const float* x, const float* m, float* acc, float* pot,
                  hipStream_t s) {
-	return sf_pp_force_arrays(p, w->N, w->n_pad, x, m, w->body, w->part,
-	                          (size_t)w->slices * 2u * w->n_pad * 4u * sizeof(float), acc, pot, s);
+	return sf_pp_force_arrays(p, w->N, w->n_pad, x, m, w->body, w->part, w->part_bytes, acc, pot, s);
 }
 
 /* g (=, or += when accumulate) J(x)^T (coef mu) */

@@ -101,16 +101,15 @@ void sf_ctx_destroy(sf_ctx* c) {
 	free(c);
 }
 
-int sf_ctx_reserve_part(sf_ctx* c, unsigned int slices) {
-	if (c->d_part && c->part_slices >= slices) return 0;
+int sf_ctx_reserve_part(sf_ctx* c, size_t bytes) {
+	if (c->d_part && c->part_bytes >= bytes) return 0;
 	if (c->d_part) {
 		hipStreamSynchronize(c->stream);
 		hipFree(c->d_part);
 		c->d_part = NULL;
 	}
-	const size_t bytes = (size_t)slices * 2u * 4u * c->n_pad * sizeof(float);
 	SF_HIP(hipMalloc((void**)&c->d_part, bytes), "sf_ctx_reserve_part");
-	c->part_slices = slices;
+	c->part_bytes = bytes;
 	return 0;
 }
 

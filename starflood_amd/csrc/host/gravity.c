@@ -8,10 +8,11 @@
 
 #include "sf_host.h"
 
-/* j slices of the fast kernel: enough blocks to give every CU several waves */
+/* j slices of the one-sided kernels (PP below 10240 bodies, the SPH all-pairs
+   passes): enough blocks to give every CU several waves */
 static unsigned int pp_slices(unsigned int n_pad) {
-	/* one j range per wavefront of 64 i; about 128k wavefronts (measured best
-	   at N = 262144: 32 ranges) while each range keeps at least 256 j */
+	/* one j range per wavefront of 64 i; about 128k wavefronts, while each
+	   range keeps at least 256 j */
 	const unsigned int iblocks = n_pad / 256u;
 	unsigned int s = iblocks ? (32768u + iblocks - 1u) / iblocks : 1u;
 	const unsigned int smax = n_pad / 256u;
@@ -25,22 +26,16 @@ static unsigned int pp_slices(unsigned int n_pad) {
 static float eps2_f32(double eps) { return (float)(eps * eps); }
 
 static int pp_on(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
-                 float* body, float** part, unsigned int* part_slices, sf_ctx* c, float* acc, float* pot,
-                 hipStream_t s) {
+                 float* body, sf_ctx* c, float* acc, float* pot, hipStream_t s) {
 	const int phys = p->acc_mode == SF_ACC_PHYSICAL;
 	if (p->precision == SF_PRECISION_EXACT) {
 		return sfd_pp_exact(pos, mas, N, eps2_f32(p->epsilon), (float)(-p->G), phys, p->kahan_solver,
 		                    p->kahan_energy, acc, pot, s);
 	}
 	const unsigned int slices = pp_slices(n_pad);
-	if (c) {
-		if (sf_ctx_reserve_part(c, slices)) return -1;
-		*part = c->d_part;
-	} else if (*part_slices < slices) {
-		return -1;
-	}
+	if (sf_ctx_reserve_part(c, sf_pp_part_bytes(n_pad))) return -1;
 	if (sfd_pack_bodies(pos, mas, N, n_pad, body, s)) return -1;
-	return sfd_pp_fast(body, N, n_pad, eps2_f32(p->epsilon), p->G, phys, *part, slices, acc, pot, s);
+	return sfd_pp_fast(body, N, n_pad, eps2_f32(p->epsilon), p->G, phys, c->d_part, slices, acc, pot, s);
 }
 
 unsigned int sf_pp_slice_count(unsigned int n_pad) { return pp_slices(n_pad); }
@@ -61,10 +56,8 @@ int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad,
 int sf_solve_gravity_pp(sf_ctx* c) {
 	const sf_params_t* p = sf_params();
 	const unsigned int N = c->N;
-	float* part = NULL;
-	unsigned int ps = 0;
-	return pp_on(p, N, c->n_pad, sf_blk(c->d_mem, N, SF_E_POS), sf_blk(c->d_mem, N, SF_E_MAS), c->d_body, &part, &ps,
-	             c, sf_blk(c->d_mem, N, SF_E_ACC), sf_blk(c->d_mem, N, SF_E_POT), c->stream);
+	return pp_on(p, N, c->n_pad, sf_blk(c->d_mem, N, SF_E_POS), sf_blk(c->d_mem, N, SF_E_MAS), c->d_body, c,
+	             sf_blk(c->d_mem, N, SF_E_ACC), sf_blk(c->d_mem, N, SF_E_POT), c->stream);
 }
 
 /* reference src/gravity.c:667-819: reads pos, mas; writes acc (assigned, not

@@ -60,7 +60,7 @@ int sf_solve_sph(sf_ctx* c) {
 	if (p->sph_model == SF_SPH_CUBIC_IDEAL) {
 		/* slice partials reuse the PP kernel's scratch (same stream, after it) */
 		const unsigned int slices = sf_pp_slice_count(c->n_pad);
-		if (sf_ctx_ensure_u(c) || sf_ctx_reserve_part(c, slices)) return -1;
+		if (sf_ctx_ensure_u(c) || sf_ctx_reserve_part(c, (size_t)slices * c->n_pad * 4u * sizeof(float))) return -1;
 		return sfd_sph_cubic(N, c->n_pad, (float)p->sph_gamma, p->acc_mode == SF_ACC_PHYSICAL, rho, prs, acc,
 		                     c->d_dudt, c->d_sph_tmp, c->d_part, slices, c->stream);
 	}

@@ -42,8 +42,8 @@ typedef struct sf_ctx {
 	float* d_mem;            /* device copy of sim.mem, same layout */
 	float* d_body;           /* SF_BODY_BYTES(n_pad): x, y, z, m (pad: m = 0), then SF_BODY_STATE words */
 	double* d_x64;           /* 3N FP64 positions for the FAST drift */
-	float* d_part;           /* PP partial sums, 8 * slices * n_pad floats */
-	unsigned int part_slices;
+	float* d_part;           /* partial sums of the PP and the SPH all-pairs passes */
+	size_t part_bytes;
 	double* d_red;           /* reduction scratch (blocks * SF_RED_VALUES) */
 	double* h_red;           /* pinned host mirror of the reduction result */
 	float* d_u;              /* SPH specific internal energy (N) */
@@ -58,8 +58,8 @@ typedef struct sf_ctx {
 sf_ctx* sf_ctx_lookup(const void* host_mem, const char* func);
 sf_ctx* sf_ctx_create(void* host_mem, unsigned int N, unsigned int dof);
 void sf_ctx_destroy(sf_ctx* c);
-/* Ensure the PP partial-sum scratch holds `slices` slices. */
-int sf_ctx_reserve_part(sf_ctx* c, unsigned int slices);
+/* Ensure the partial-sum scratch holds `bytes` bytes. */
+int sf_ctx_reserve_part(sf_ctx* c, size_t bytes);
 /* allocates (zeroed) d_u and d_dudt on first use */
 int sf_ctx_ensure_u(sf_ctx* c);
 /* The library's stream for work not tied to a simulation (lazy). */
@@ -106,9 +106,10 @@ int sfd_pack_bodies(const float* pos, const float* mas, unsigned int N, unsigned
 int sfd_pp_exact(const float* pos, const float* mas, unsigned int N, float eps2, float negG,
                  int acc_phys, int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s);
 
-/* Fast PP gravity: j-sliced partial sums into part (sfd_pp_part_bytes of
-   n_pad and slices), then a fixed-order FP64 combine into acc (AoS) and pot.
-   pot may be NULL (skip). */
+/* Fast PP gravity: partial sums into part (sfd_pp_part_bytes of n_pad and
+   slices), then a fixed-order FP64 combine into acc (AoS) and pot.  From
+   10240 bodies each pair is evaluated once (device/pp_sym.hip); below, every
+   i against `slices` ranges of j.  pot may be NULL (skip). */
 int sfd_pp_fast(const float* body, unsigned int N, unsigned int n_pad, float eps2, double G,
                 int acc_phys, float* part, unsigned int slices, float* acc, float* pot, hipStream_t s);
 size_t sfd_pp_part_bytes(unsigned int n_pad, unsigned int slices);
