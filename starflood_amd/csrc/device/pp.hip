@@ -9,10 +9,10 @@
 // -G m_i / eps), as the reference does.
 //
 // k_pp_exact keeps the reference's FP32 operation order (no contraction: the
-// file is compiled with -ffp-contract=off; IEEE divide and square root;
-// per-pair Kahan; j in index order), so its output is bit-identical to the
-// CPU path.  One lane owns one i; the j stream is wavefront-uniform, so the
-// compiler fetches it with scalar loads into SGPRs.
+// file is compiled with -ffp-contract=off; the IEEE quotients' and square
+// root's bits; per-pair Kahan; j in index order), so its output is
+// bit-identical to the CPU path.  The terms of a tile of j are made by some of
+// a block's wavefronts while others run the chains of sums.
 //
 // k_pp_fast is the throughput kernel below 10240 bodies (from there
 // pp_sym.hip evaluates each pair once): 13 VALU operations plus one
@@ -51,56 +51,164 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	s = t;
 }
 
+// 1 / s and 1 / sqrt(s) with the IEEE quotient's and square root's bits (each
+// rounded to nearest, the second from the rounded root), in 11 operations and
+// one v_rsq_f32 instead of two divisions and a square root of about 45:
+// Newton steps whose last operation is an FMA (Markstein's scheme).
+// Compared with 1.0f / s and 1.0f / sqrtf(s) on the device for every float
+// in [2^-96, 2^97): they differ only where the significand of s is all ones
+// or within one of it (1/s or 1/root then lies next to a rounding boundary).
+// kRootBits tells those, and kTopBits the values above the range.
+__device__ __forceinline__ void exact_inverses(float s, float& inv_s, float& inv_root) {
+	const float r = __builtin_amdgcn_rsqf(s);
+	const float g = s * r, h = 0.5f * r;
+	const float root = __builtin_fmaf(__builtin_fmaf(-g, g, s), h, g);
+	inv_root = __builtin_fmaf(r, __builtin_fmaf(-root, r, 1.0f), r);
+	const float q = r * r;
+	const float e = __builtin_fmaf(-s, q, 1.0f);
+	inv_s = __builtin_fmaf(q, __builtin_fmaf(e, e, e), q);
+}
+constexpr unsigned kRootBits = 0xFFFFFFFEu;   // bits(s) | 0xFF800000 at or above this: IEEE operations
+constexpr unsigned kTopBits = 0x6F800000u;    // bits(s) at or above this (2^96, inf, NaN): IEEE operations
+constexpr float kExactMinEps2 = 0x1p-96f;     // s >= eps2: below this, IEEE operations throughout
+
+// The exact kernel's block: 64 particles i, one per lane.  Each sum is a
+// chain over j in index order, four dependent additions a term, so a lane
+// per particle and every term in line left most of the card idle (64 blocks
+// at N = 16384) and waiting for one division after another.  Here kMakers
+// wavefronts make the terms of a tile of kExJ bodies, kExJ / kMakers each,
+// into LDS, while four wavefronts run the chains of the tile before, one
+// component each.
+//
+// Bound by issue: a chain takes four dependent operations of 2.5 ns (one
+// wavefront's issue interval) a body, and the three wavefronts of a SIMD issue
+// 12.3 instructions a body, about 14 ns; it takes 17.5 (N = 6000).  Two tiles
+// of 64 bodies fill 128 KiB of LDS, one block per CU.  Tiles of 48 with 12
+// makers took the same; tiles of 32 and two blocks per CU 375 us at N = 16384
+// against 320 (and 4.2 ms against 4.5 at N = 65536).  Before, with one lane
+// per particle: N = 1000 239 -> 20 us, N = 6000 1430 -> 105, N = 16384 3918 ->
+// 320, N = 65536 15.7 -> 4.5 ms.
+constexpr unsigned kExI = 64, kExJ = 64, kMakers = 8, kChains = 4;
+constexpr unsigned kExBlock = 64u * (kChains + kMakers);
+constexpr unsigned kExRun = kExJ / kMakers;   // consecutive j per maker and tile
+constexpr unsigned kExAhead = 16;             // terms a chain has read ahead
+
+// The terms of the reference's pair (src/gravity.c:709-769), FAST with
+// exact_inverses; returns what the caller's checks of s need.
+template <bool FAST>
+__device__ __forceinline__ float exact_terms(float xi, float yi, float zi, float xj, float yj, float zj, float mj,
+                                             float eps2, float* __restrict__ out) {
+	const float rx = xi - xj, ry = yi - yj, rz = zi - zj;
+	const float r2 = (rx * rx + ry * ry) + rz * rz;
+	const float s = r2 + eps2;
+	float inv_r2, inv_r1;
+	if (FAST) {
+		exact_inverses(s, inv_r2, inv_r1);
+	} else {
+		inv_r2 = 1.0f / s;
+		inv_r1 = 1.0f / sqrtf(s);
+	}
+	const float pj = mj * inv_r1;
+	const float w = pj * inv_r2;
+	out[0u * kExJ * kExI] = w * rx;
+	out[1u * kExJ * kExI] = w * ry;
+	out[2u * kExJ * kExI] = w * rz;
+	out[3u * kExJ * kExI] = pj;
+	return s;
+}
+
 template <bool KAHAN_ACC, bool KAHAN_POT, bool PHYS>
-__global__ __launch_bounds__(kBlock) void k_pp_exact(const float* __restrict__ pos, const float* __restrict__ mas,
-                                                     unsigned N, float eps2, float negG,
-                                                     float* __restrict__ acc, float* __restrict__ pot) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	const bool live = i < N;
-	const unsigned ii = live ? i : N - 1u;
-	const float xi = pos[3u * ii + 0u];
-	const float yi = pos[3u * ii + 1u];
-	const float zi = pos[3u * ii + 2u];
-	const float mi = mas[ii];
-
-	float sx = 0.0f, sy = 0.0f, sz = 0.0f, sp = 0.0f;
-	float cx = 0.0f, cy = 0.0f, cz = 0.0f, cp = 0.0f;
-
-	for (unsigned j = 0; j < N; ++j) {
-		const float mj = mas[j];
-		const float rx = xi - pos[3u * j + 0u];
-		const float ry = yi - pos[3u * j + 1u];
-		const float rz = zi - pos[3u * j + 2u];
-		const float r2 = (rx * rx + ry * ry) + rz * rz;
-		const float inv_r2 = 1.0f / (r2 + eps2);
-		const float inv_r1 = 1.0f / sqrtf(r2 + eps2);
-		const float pj = mj * inv_r1;
-		const float fx = pj * inv_r2 * rx;
-		const float fy = pj * inv_r2 * ry;
-		const float fz = pj * inv_r2 * rz;
-		if (KAHAN_ACC) {
-			kahan_add(sx, cx, fx);
-			kahan_add(sy, cy, fy);
-			kahan_add(sz, cz, fz);
-		} else {
-			sx += fx;
-			sy += fy;
-			sz += fz;
+__global__ __launch_bounds__(kExBlock) void k_pp_exact(const float* __restrict__ pos, const float* __restrict__ mas,
+                                                       unsigned N, float eps2, float negG, float* __restrict__ acc,
+                                                       float* __restrict__ pot) {
+	__shared__ float s_term[2][4][kExJ][kExI];
+	const unsigned lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const unsigned i = blockIdx.x * kExI + lane;
+	const unsigned tiles = (N + kExJ - 1u) / kExJ;
+	if (wv >= kChains) {
+		const unsigned ii = min(i, N - 1u);
+		const float xi = pos[3u * ii], yi = pos[3u * ii + 1u], zi = pos[3u * ii + 2u];
+		const unsigned first = (wv - kChains) * kExRun;
+		const bool fast = eps2 >= kExactMinEps2 && N >= kExRun;
+		// the run's bodies, in SGPRs and read one tile ahead: consecutive, from
+		// a clamped address (the run that reaches past N takes the slow loop)
+		float x[kExRun], y[kExRun], z[kExRun], m[kExRun];
+		auto read = [&](unsigned j0) {
+			const unsigned jc = min(j0, N - kExRun);
+			const float* __restrict__ p = pos + 3u * jc;
+			const float* __restrict__ q = mas + jc;
+#pragma unroll
+			for (unsigned u = 0; u < kExRun; ++u) {
+				x[u] = p[3u * u];
+				y[u] = p[3u * u + 1u];
+				z[u] = p[3u * u + 2u];
+				m[u] = q[u];
+			}
+		};
+		if (fast) read(first);
+		for (unsigned t = 0; t < tiles; ++t) {
+			float* out = &s_term[t & 1u][0][first][lane];
+			const unsigned j0 = t * kExJ + first;
+			bool slow = true;
+			if (fast) {
+				unsigned top = 0u, edge = 0u;
+#pragma unroll
+				for (unsigned u = 0; u < kExRun; ++u) {
+					const unsigned b = __float_as_uint(
+					    exact_terms<true>(xi, yi, zi, x[u], y[u], z[u], m[u], eps2, out + u * kExI));
+					top = max(top, b);
+					edge = max(edge, b | 0xFF800000u);
+				}
+				read(j0 + kExJ);
+				slow = __ballot(top >= kTopBits || edge >= kRootBits) != 0ull || j0 + kExRun > N;
+			}
+			if (slow) {
+#pragma unroll 1
+				for (unsigned u = 0; u < kExRun; ++u) {
+					const unsigned j = j0 + u;
+					if (j >= N) break;
+					exact_terms<false>(xi, yi, zi, pos[3u * j], pos[3u * j + 1u], pos[3u * j + 2u], mas[j], eps2,
+					                   out + u * kExI);
+				}
+			}
+			__syncthreads();
 		}
-		if (KAHAN_POT) {
-			kahan_add(sp, cp, pj);
+		__syncthreads();
+		return;
+	}
+	// chains: component wv of the block's 64 particles
+	const bool kahan = wv < 3u ? KAHAN_ACC : KAHAN_POT;
+	float s = 0.0f, c = 0.0f;
+	__syncthreads();
+	for (unsigned t = 0; t < tiles; ++t) {
+		const float* in = &s_term[t & 1u][wv][0][lane];
+		const unsigned n = min(N - t * kExJ, kExJ);
+		if (n == kExJ && kahan) {
+			float v[kExAhead], w[kExAhead];
+#pragma unroll
+			for (unsigned u = 0; u < kExAhead; ++u) v[u] = in[u * kExI];
+#pragma unroll
+			for (unsigned k = 0; k < kExJ; k += kExAhead) {
+				if (k + kExAhead < kExJ) {
+#pragma unroll
+					for (unsigned u = 0; u < kExAhead; ++u) w[u] = in[(k + kExAhead + u) * kExI];
+				}
+#pragma unroll
+				for (unsigned u = 0; u < kExAhead; ++u) kahan_add(s, c, v[u]);
+#pragma unroll
+				for (unsigned u = 0; u < kExAhead; ++u) v[u] = w[u];
+			}
+		} else if (kahan) {
+			for (unsigned k = 0; k < n; ++k) kahan_add(s, c, in[k * kExI]);
 		} else {
-			sp += pj;
+			for (unsigned k = 0; k < n; ++k) s += in[k * kExI];
 		}
+		__syncthreads();
 	}
-	if (live) {
-		// reference src/gravity.c:808-811: ((-G) * m_i) * acc_sum, (-G) * pot_sum
-		const float f = PHYS ? negG : negG * mi;
-		acc[3u * i + 0u] = f * sx;
-		acc[3u * i + 1u] = f * sy;
-		acc[3u * i + 2u] = f * sz;
-		pot[i] = negG * sp;
-	}
+	if (i >= N) return;
+	// reference src/gravity.c:808-811: ((-G) * m_i) * acc_sum, (-G) * pot_sum
+	if (wv == 3u) pot[i] = negG * s;
+	else acc[3u * i + wv] = (PHYS ? negG : negG * mas[i]) * s;
 }
 
 // One tile of SF_TJ interactions, j from jt.  nb holds the tile's first
@@ -355,7 +463,7 @@ extern "C" int sfd_pack_bodies(const float* pos, const float* mas, unsigned N, u
 extern "C" int sfd_pp_exact(const float* pos, const float* mas, unsigned N, float eps2, float negG, int acc_phys,
                             int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s) {
 	if (N == 0) return 0;
-	const dim3 grid((N + kBlock - 1) / kBlock), block(kBlock);
+	const dim3 grid((N + kExI - 1) / kExI), block(kExBlock);
 	const int sel = (kahan_acc ? 4 : 0) | (kahan_pot ? 2 : 0) | (acc_phys ? 1 : 0);
 	const int tok = sf_prof_begin("pp_exact", s);
 	switch (sel) {

@@ -102,7 +102,7 @@ void sf_prof_end(int token, hipStream_t s);
 int sfd_pack_bodies(const float* pos, const float* mas, unsigned int N, unsigned int n_pad,
                     float* body, hipStream_t s);
 
-/* Reference-order PP gravity (src/gravity.c:693-812), one lane per i. */
+/* Reference-order PP gravity (src/gravity.c:693-812). */
 int sfd_pp_exact(const float* pos, const float* mas, unsigned int N, float eps2, float negG,
                  int acc_phys, int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s);
 
