@@ -2,8 +2,7 @@
 // reductions of the state (reference src/simulation.c:381-504).
 //
 // Exact policy: FP32 elementwise updates in the reference's operation order
-// (file compiled with -ffp-contract=off) and a sequential FP64 Kahan sum in
-// index order, so T and V are bit-identical to the reference's.
+// (file compiled with -ffp-contract=off); T and V are exact_sum.hip's.
 // Fast policy: kick and FP64 drift fused in one pass over the state, and
 // tree-shaped FP64 block reductions with a fixed grid, which are
 // deterministic and more accurate than a sequential sum.
@@ -43,21 +42,6 @@ __global__ __launch_bounds__(kBlock) void k_energy_terms(const float* __restrict
 	const float v2 = (vx * vx + vy * vy) + vz * vz;
 	ken[i] = 0.5f * m * v2;
 	pen[i] = m * pot[i];
-}
-
-// Sequential FP64 Kahan in index order; a single lane, for bit parity with
-// src/simulation.c:455-497.
-__global__ void k_energy_sum_sequential(const float* __restrict__ x, unsigned N, double* __restrict__ out) {
-	if (blockIdx.x != 0 || threadIdx.x != 0) return;
-	double S = 0.0, C = 0.0;
-	for (unsigned i = 0; i < N; ++i) {
-		const double y = (double)x[i] - C;
-		const double t = S + y;
-		const double z = t - S;
-		C = z - y;
-		S = t;
-	}
-	*out = S;
 }
 
 // x64 follows pos unless it rounds to it: a host-side change of pos (or a
@@ -213,13 +197,6 @@ extern "C" int sfd_energy_terms(const float* vel, const float* mas, const float*
 	hipLaunchKernelGGL(k_energy_terms, dim3(grid_for(N)), dim3(kBlock), 0, s, vel, mas, pot, N, ken, pen);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_energy_terms", "launch");
-}
-
-extern "C" int sfd_energy_sum_sequential(const float* x, unsigned N, double* out, hipStream_t s) {
-	const int tok = sf_prof_begin("energy_sum_seq", s);
-	hipLaunchKernelGGL(k_energy_sum_sequential, dim3(1), dim3(64), 0, s, x, N, out);
-	sf_prof_end(tok, s);
-	return sf_hip_check(hipGetLastError(), "sfd_energy_sum_sequential", "launch");
 }
 
 extern "C" int sfd_x64_refresh(const float* pos, double* x64, unsigned n3, hipStream_t s) {

@@ -22,10 +22,15 @@ typedef struct {
 } sf_node;
 
 /* --- reference octree (tree_ref.hip) --- */
-/* the reference's FP64 Kahan mean radius into avg[0] (r1: N doubles of scratch) */
-int sfd_mean_radius(const float* pos, unsigned int N, double* r1, double* avg, hipStream_t s);
-/* r1: N doubles of scratch */
-int sfd_tree_bounds_ref(const float* pos, unsigned int N, const double jitter[3], double* r1, float* bounds,
+/* exact_sum.hip.  The reference's FP64 Kahan mean radius: an interval that
+   holds it into avg[0], avg[1] (avg[0] NaN when a radius is not finite), or,
+   by the sequence itself, its value into both.  part: 2 SF_RADIUS_PARTIALS
+   doubles of scratch. */
+#define SF_RADIUS_PARTIALS 512u
+int sfd_mean_radius_interval(const float* pos, unsigned int N, double* part, double* avg, hipStream_t s);
+int sfd_mean_radius_sequence(const float* pos, unsigned int N, double* avg, hipStream_t s);
+/* the jittered cube bounds around that mean radius; part as above */
+int sfd_tree_bounds_ref(const float* pos, unsigned int N, const double jitter[3], double* part, float* bounds,
                         hipStream_t s);
 /* meta[0] = num_nodes, meta[1] = status (0 ok, 1 out of nodes, 2 too deep) */
 int sfd_tree_build_ref(const float* pos, const float* mas, unsigned int N, const float* bounds, unsigned int max_nodes,

@@ -267,10 +267,12 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 
 	double* red_out = c->d_red + (size_t)(sfd_reduce_scratch_doubles(N) - SF_RED_VALUES);
 	if (exact) {
-		if (sfd_energy_sum_sequential(ken, N, red_out + 12, s)) return STARFLOOD_FAILURE;   /* ken_sum */
-		if (timing) tev_record(5, s);
-		if (sfd_energy_sum_sequential(pen, N, red_out + 13, s)) return STARFLOOD_FAILURE;   /* pen_sum */
-		if (timing) tev_record(6, s);
+		/* ken_sum and pen_sum in one pass (its time is logged as ken_sum's) */
+		if (sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
+		if (timing) {
+			tev_record(5, s);
+			tev_record(6, s);
+		}
 	}
 	/* FP64 W, P, L (and T, V in the fast policy) */
 	if (sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, c->have_u ? c->d_u : NULL, N, p->G,
@@ -344,10 +346,7 @@ int sf_get_stats(const sim_t* sim_ptr, sf_stats_t* out) {
 	                     sf_blk(c->d_mem, N, SF_E_MAS), sf_blk(c->d_mem, N, SF_E_POT), ken, pen,
 	                     c->have_u ? c->d_u : NULL, N, p->G, p->epsilon, c->d_red, s))
 		return STARFLOOD_FAILURE;
-	if (exact) {
-		if (sfd_energy_sum_sequential(ken, N, red_out + 12, s)) return STARFLOOD_FAILURE;
-		if (sfd_energy_sum_sequential(pen, N, red_out + 13, s)) return STARFLOOD_FAILURE;
-	}
+	if (exact && sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
 	SF_HIP(hipMemcpyAsync(c->h_red, red_out, SF_RED_VALUES * sizeof(double), hipMemcpyDeviceToHost, s),
 	       "sf_get_stats");
 	if (sf_finish(c, "sf_get_stats")) return STARFLOOD_FAILURE;

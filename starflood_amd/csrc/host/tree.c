@@ -32,8 +32,7 @@ struct sf_tree_dev {
 	hipStream_t stream;      /* for tree_build called directly */
 	sf_tree_par_ctx par;     /* level-synchronous reference build: scratch, */
 	size_t par_bytes;        /* pinned state, side stream and events */
-	double* d_r1;            /* radii for the reference bounds */
-	unsigned int r1_n;
+	double* d_radius;        /* partial sums of the reference bounds' mean radius */
 	unsigned int* d_order;   /* walk order of the last parallel build (N entries) */
 	unsigned int order_n;    /* its N, 0 when the last build was serial */
 	void* d_link;            /* threaded links of the last complete parallel build (max_nodes x 2 u32) */
@@ -68,7 +67,7 @@ static void tree_dev_destroy(sf_tree_dev* d) {
 	for (int k = 0; k < 2; ++k)
 		if (d->par.ev[k]) hipEventDestroy(d->par.ev[k]);
 	if (d->par.side) hipStreamDestroy(d->par.side);
-	if (d->d_r1) hipFree(d->d_r1);
+	if (d->d_radius) hipFree(d->d_radius);
 	if (d->d_order) hipFree(d->d_order);
 	if (d->d_link) hipFree(d->d_link);
 	if (d->stream) hipStreamDestroy(d->stream);
@@ -284,15 +283,9 @@ int sf_solve_gravity_tree(sf_ctx* c, tree_t* tree, unsigned int step_number, int
 	if (p->tree_mode == SF_TREE_REFERENCE) {
 		double jit[4];
 		bounds_jitter(step_number, jit);
-		if (d->r1_n < N) {
-			SF_HIP(hipStreamSynchronize(s), "solve_gravity_part_tree");
-			if (d->d_r1) hipFree(d->d_r1);
-			d->d_r1 = NULL;
-			d->r1_n = 0;
-			SF_HIP(hipMalloc((void**)&d->d_r1, (size_t)N * sizeof(double)), "solve_gravity_part_tree");
-			d->r1_n = N;
-		}
-		if (N && sfd_tree_bounds_ref(pos, N, jit, d->d_r1, d->d_bounds, s)) return -1;
+		if (!d->d_radius)
+			SF_HIP(hipMalloc((void**)&d->d_radius, 2u * SF_RADIUS_PARTIALS * sizeof(double)), "solve_gravity_part_tree");
+		if (N && sfd_tree_bounds_ref(pos, N, jit, d->d_radius, d->d_bounds, s)) return -1;
 		const int rc = build_ref(d, tree, N, pos, mas, s);
 		SF_HIP(hipMemcpyAsync(tree->bounds, d->d_bounds, 6u * sizeof(float), hipMemcpyDeviceToHost, s),
 		       "solve_gravity_part_tree");

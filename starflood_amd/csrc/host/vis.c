@@ -38,9 +38,7 @@ typedef struct {
 	unsigned int sizex, sizey;
 	int* d_atomic;
 	float* d_render;
-	double* d_r1;         /* radii for the mean radius */
-	unsigned int r1_n;
-	double* d_avg;
+	double* d_avg;        /* the mean radius (2 doubles), then its partial sums */
 	double* h_avg;        /* pinned */
 } sf_vis_dev;
 
@@ -60,7 +58,6 @@ static void vis_dev_destroy(sf_vis_dev* d) {
 		if (g_vis[k] == d) g_vis[k] = NULL;
 	if (d->d_atomic) hipFree(d->d_atomic);
 	if (d->d_render) hipFree(d->d_render);
-	if (d->d_r1) hipFree(d->d_r1);
 	if (d->d_avg) hipFree(d->d_avg);
 	if (d->h_avg) hipHostFree(d->h_avg);
 	free(d);
@@ -86,8 +83,8 @@ static sf_vis_dev* vis_dev_get(const vis_t* v) {
 	const size_t n = 4u * (size_t)v->sizex * v->sizey;
 	if (hipMalloc((void**)&d->d_atomic, (n ? n : 1u) * sizeof(int)) != hipSuccess ||
 	    hipMalloc((void**)&d->d_render, (n ? n : 1u) * sizeof(float)) != hipSuccess ||
-	    hipMalloc((void**)&d->d_avg, sizeof(double)) != hipSuccess ||
-	    hipHostMalloc((void**)&d->h_avg, sizeof(double), hipHostMallocDefault) != hipSuccess) {
+	    hipMalloc((void**)&d->d_avg, (2u + 2u * SF_RADIUS_PARTIALS) * sizeof(double)) != hipSuccess ||
+	    hipHostMalloc((void**)&d->h_avg, 2u * sizeof(double), hipHostMallocDefault) != hipSuccess) {
 		sf_error("vis_draw", "device allocation for %u x %u pixels failed", v->sizex, v->sizey);
 		vis_dev_destroy(d);
 		return NULL;
@@ -211,18 +208,18 @@ int vis_draw(const vis_t* SF_RESTRICT vis_ptr, const sim_t* SF_RESTRICT sim_ptr)
 	const float* pos = sf_blk(c->d_mem, N, SF_E_POS);
 	double average_radius = 1.0;
 	if (N) {
-		if (d->r1_n < N) {
-			SF_HIP(hipStreamSynchronize(s), "vis_draw");
-			if (d->d_r1) hipFree(d->d_r1);
-			d->d_r1 = NULL;
-			d->r1_n = 0;
-			SF_HIP(hipMalloc((void**)&d->d_r1, (size_t)N * sizeof(double)), "vis_draw");
-			d->r1_n = N;
-		}
-		if (sfd_mean_radius(pos, N, d->d_r1, d->d_avg, s)) return STARFLOOD_FAILURE;
-		SF_HIP(hipMemcpyAsync(d->h_avg, d->d_avg, sizeof(double), hipMemcpyDeviceToHost, s), "vis_draw");
+		/* the frame uses (float)(1 / radius) alone: the sequence is summed only
+		   where the interval around its result leaves that open, or where the
+		   radius itself is printed */
+		if (sfd_mean_radius_interval(pos, N, d->d_avg + 2, d->d_avg, s)) return STARFLOOD_FAILURE;
+		SF_HIP(hipMemcpyAsync(d->h_avg, d->d_avg, 2u * sizeof(double), hipMemcpyDeviceToHost, s), "vis_draw");
 		SF_HIP(hipStreamSynchronize(s), "vis_draw");
-		average_radius = *d->h_avg;
+		if (p->verbose || !((float)(1.0 / d->h_avg[0]) == (float)(1.0 / d->h_avg[1]))) {
+			if (sfd_mean_radius_sequence(pos, N, d->d_avg, s)) return STARFLOOD_FAILURE;
+			SF_HIP(hipMemcpyAsync(d->h_avg, d->d_avg, 2u * sizeof(double), hipMemcpyDeviceToHost, s), "vis_draw");
+			SF_HIP(hipStreamSynchronize(s), "vis_draw");
+		}
+		average_radius = d->h_avg[0];
 	} else {
 		average_radius = 0.0 / 0.0;   /* the reference divides 0 by 0 */
 	}

@@ -44,7 +44,7 @@ typedef struct sf_ctx {
 	double* d_x64;           /* 3N FP64 positions for the FAST drift */
 	float* d_part;           /* partial sums of the PP and the SPH all-pairs passes */
 	size_t part_bytes;
-	double* d_red;           /* reduction scratch (blocks * SF_RED_VALUES) */
+	double* d_red;           /* reduction scratch (blocks * SF_RED_VALUES), then the exact energy sums' */
 	double* h_red;           /* pinned host mirror of the reduction result */
 	float* d_u;              /* SPH specific internal energy (N) */
 	float* d_dudt;           /* its derivative (N) */
@@ -124,9 +124,11 @@ int sfd_drift_exact(float* pos, const float* vel, unsigned int n3, float dt, hip
 /* ken_i = (0.5 m_i) |v_i|^2, pen_i = m_i pot_i */
 int sfd_energy_terms(const float* vel, const float* mas, const float* pot, unsigned int N,
                      float* ken, float* pen, hipStream_t s);
-/* Sequential FP64 Kahan of x[0..N) in index order (src/simulation.c:455-497),
-   written to *out.  One lane; for bit parity. */
-int sfd_energy_sum_sequential(const float* x, unsigned int N, double* out, hipStream_t s);
+/* exact_sum.hip: the sequential FP64 Kahan sums of ken and pen in index order
+   (src/simulation.c:455-497), bit for bit, into out[0] and out[1]; part is
+   scratch of sfd_energy_scratch_bytes(N). */
+size_t sfd_energy_scratch_bytes(unsigned int N);
+int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned int N, void* part, double* out, hipStream_t s);
 
 /* FAST KDK: kick + FP64 drift fused; x64 refreshed from pos where they
    disagree (sfd_x64_refresh, or inside the drift with refresh = 1). */
