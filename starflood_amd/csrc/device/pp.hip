@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "order_chain.h"
 #include "pp_sym.h"
 
 namespace {
@@ -72,143 +73,100 @@ constexpr unsigned kRootBits = 0xFFFFFFFEu;   // bits(s) | 0xFF800000 at or abov
 constexpr unsigned kTopBits = 0x6F800000u;    // bits(s) at or above this (2^96, inf, NaN): IEEE operations
 constexpr float kExactMinEps2 = 0x1p-96f;     // s >= eps2: below this, IEEE operations throughout
 
-// The exact kernel's block: 64 particles i, one per lane.  Each sum is a
-// chain over j in index order, four dependent additions a term, so a lane
-// per particle and every term in line left most of the card idle (64 blocks
-// at N = 16384) and waiting for one division after another.  Here kMakers
-// wavefronts make the terms of a tile of kExJ bodies, kExJ / kMakers each,
-// into LDS, while four wavefronts run the chains of the tile before, one
-// component each.
-//
-// Bound by issue: a chain takes four dependent operations of 2.5 ns (one
-// wavefront's issue interval) a body, and the three wavefronts of a SIMD issue
-// 12.3 instructions a body, about 14 ns; it takes 17.5 (N = 6000).  Two tiles
-// of 64 bodies fill 128 KiB of LDS, one block per CU.  Tiles of 48 with 12
-// makers took the same; tiles of 32 and two blocks per CU 375 us at N = 16384
-// against 320 (and 4.2 ms against 4.5 at N = 65536).  Before, with one lane
-// per particle: N = 1000 239 -> 20 us, N = 6000 1430 -> 105, N = 16384 3918 ->
-// 320, N = 65536 15.7 -> 4.5 ms.
-constexpr unsigned kExI = 64, kExJ = 64, kMakers = 8, kChains = 4;
-constexpr unsigned kExBlock = 64u * (kChains + kMakers);
-constexpr unsigned kExRun = kExJ / kMakers;   // consecutive j per maker and tile
-constexpr unsigned kExAhead = 16;             // terms a chain has read ahead
+// The terms of the reference's pair (src/gravity.c:709-769) and its sums:
+// the model that order_chain.h runs, components x, y, z and the potential.
+// Makers: 26 VALU operations, the rsq and 2 LDS writes a pair.  One lane per
+// particle with IEEE divisions took 239 us at N = 1000, 1430 at 6000, 3918 at
+// 16384 and 15.7 ms at 65536; this takes 14, 74, 323 and 4.5 ms.
+template <bool KAHAN_ACC, bool KAHAN_POT, bool PHYS>
+struct ExactPP {
+	static constexpr unsigned kComps = 4;
+	const float* __restrict__ pos;
+	const float* __restrict__ mas;
+	float eps2, negG;
+	float* __restrict__ acc;
+	float* __restrict__ pot;
 
-// The terms of the reference's pair (src/gravity.c:709-769), FAST with
-// exact_inverses; returns what the caller's checks of s need.
-template <bool FAST>
-__device__ __forceinline__ float exact_terms(float xi, float yi, float zi, float xj, float yj, float zj, float mj,
-                                             float eps2, float* __restrict__ out) {
-	const float rx = xi - xj, ry = yi - yj, rz = zi - zj;
-	const float r2 = (rx * rx + ry * ry) + rz * rz;
-	const float s = r2 + eps2;
-	float inv_r2, inv_r1;
-	if (FAST) {
-		exact_inverses(s, inv_r2, inv_r1);
-	} else {
-		inv_r2 = 1.0f / s;
-		inv_r1 = 1.0f / sqrtf(s);
+	struct Self {
+		float x, y, z;
+	};
+	struct Body {
+		float x, y, z, m;
+	};
+	struct Check {
+		unsigned top = 0u, edge = 0u;
+		__device__ bool bad() const { return top >= kTopBits || edge >= kRootBits; }
+	};
+	__device__ bool fast() const { return eps2 >= kExactMinEps2; }
+	__device__ Self self(unsigned i) const { return {pos[3u * i], pos[3u * i + 1u], pos[3u * i + 2u]}; }
+	__device__ __forceinline__ Body body(unsigned j, unsigned off) const {
+		const float* p = pos + 3u * (size_t)j;
+		return {p[3u * off], p[3u * off + 1u], p[3u * off + 2u], (mas + j)[off]};
 	}
-	const float pj = mj * inv_r1;
-	const float w = pj * inv_r2;
-	out[0u * kExJ * kExI] = w * rx;
-	out[1u * kExJ * kExI] = w * ry;
-	out[2u * kExJ * kExI] = w * rz;
-	out[3u * kExJ * kExI] = pj;
-	return s;
+
+	template <bool FAST>
+	__device__ __forceinline__ void terms(const Self& a, const Body& b, float (&out)[4], Check& chk) const {
+		const float rx = a.x - b.x, ry = a.y - b.y, rz = a.z - b.z;
+		const float r2 = (rx * rx + ry * ry) + rz * rz;
+		const float s = r2 + eps2;
+		float inv_r2, inv_r1;
+		if (FAST) {
+			exact_inverses(s, inv_r2, inv_r1);
+			const unsigned bits = __float_as_uint(s);
+			chk.top = max(chk.top, bits);
+			chk.edge = max(chk.edge, bits | 0xFF800000u);
+		} else {
+			inv_r2 = 1.0f / s;
+			inv_r1 = 1.0f / sqrtf(s);
+		}
+		const float pj = b.m * inv_r1;
+		const float w = pj * inv_r2;
+		out[0] = w * rx;
+		out[1] = w * ry;
+		out[2] = w * rz;
+		out[3] = pj;
+	}
+	__device__ __forceinline__ void step(unsigned comp, float& s, float& c, float x) const {
+		if (KAHAN_ACC || KAHAN_POT) {
+			chain::kahan(s, c, x);
+			// no compensation carried: the plain sum
+			if (KAHAN_ACC != KAHAN_POT) c = (comp < 3u ? KAHAN_ACC : KAHAN_POT) ? c : 0.0f;
+		} else {
+			s += x;
+		}
+	}
+	// reference src/gravity.c:808-811: ((-G) * m_i) * acc_sum, (-G) * pot_sum
+	__device__ void store(unsigned i, unsigned comp, float s) const {
+		if (comp == 3u) pot[i] = negG * s;
+		else acc[3u * i + comp] = (PHYS ? negG : negG * mas[i]) * s;
+	}
+};
+
+template <unsigned I, bool KAHAN_ACC, bool KAHAN_POT, bool PHYS>
+__global__ __launch_bounds__((chain::block_size<I, 4>())) void k_pp_exact(const float* __restrict__ pos,
+                                                                        const float* __restrict__ mas, unsigned N,
+                                                                        float eps2, float negG,
+                                                                        float* __restrict__ acc,
+                                                                        float* __restrict__ pot) {
+	chain::run<I>(ExactPP<KAHAN_ACC, KAHAN_POT, PHYS>{pos, mas, eps2, negG, acc, pot}, N);
 }
 
-template <bool KAHAN_ACC, bool KAHAN_POT, bool PHYS>
-__global__ __launch_bounds__(kExBlock) void k_pp_exact(const float* __restrict__ pos, const float* __restrict__ mas,
-                                                       unsigned N, float eps2, float negG, float* __restrict__ acc,
-                                                       float* __restrict__ pot) {
-	__shared__ float s_term[2][4][kExJ][kExI];
-	const unsigned lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const unsigned i = blockIdx.x * kExI + lane;
-	const unsigned tiles = (N + kExJ - 1u) / kExJ;
-	if (wv >= kChains) {
-		const unsigned ii = min(i, N - 1u);
-		const float xi = pos[3u * ii], yi = pos[3u * ii + 1u], zi = pos[3u * ii + 2u];
-		const unsigned first = (wv - kChains) * kExRun;
-		const bool fast = eps2 >= kExactMinEps2 && N >= kExRun;
-		// the run's bodies, in SGPRs and read one tile ahead: consecutive, from
-		// a clamped address (the run that reaches past N takes the slow loop)
-		float x[kExRun], y[kExRun], z[kExRun], m[kExRun];
-		auto read = [&](unsigned j0) {
-			const unsigned jc = min(j0, N - kExRun);
-			const float* __restrict__ p = pos + 3u * jc;
-			const float* __restrict__ q = mas + jc;
-#pragma unroll
-			for (unsigned u = 0; u < kExRun; ++u) {
-				x[u] = p[3u * u];
-				y[u] = p[3u * u + 1u];
-				z[u] = p[3u * u + 2u];
-				m[u] = q[u];
-			}
-		};
-		if (fast) read(first);
-		for (unsigned t = 0; t < tiles; ++t) {
-			float* out = &s_term[t & 1u][0][first][lane];
-			const unsigned j0 = t * kExJ + first;
-			bool slow = true;
-			if (fast) {
-				unsigned top = 0u, edge = 0u;
-#pragma unroll
-				for (unsigned u = 0; u < kExRun; ++u) {
-					const unsigned b = __float_as_uint(
-					    exact_terms<true>(xi, yi, zi, x[u], y[u], z[u], m[u], eps2, out + u * kExI));
-					top = max(top, b);
-					edge = max(edge, b | 0xFF800000u);
-				}
-				read(j0 + kExJ);
-				slow = __ballot(top >= kTopBits || edge >= kRootBits) != 0ull || j0 + kExRun > N;
-			}
-			if (slow) {
-#pragma unroll 1
-				for (unsigned u = 0; u < kExRun; ++u) {
-					const unsigned j = j0 + u;
-					if (j >= N) break;
-					exact_terms<false>(xi, yi, zi, pos[3u * j], pos[3u * j + 1u], pos[3u * j + 2u], mas[j], eps2,
-					                   out + u * kExI);
-				}
-			}
-			__syncthreads();
-		}
-		__syncthreads();
-		return;
+template <unsigned I>
+void launch_exact(int sel, const float* pos, const float* mas, unsigned N, float eps2, float negG, float* acc,
+                  float* pot, hipStream_t s) {
+	auto k = k_pp_exact<I, true, true, true>;
+	switch (sel) {
+	case 0: k = k_pp_exact<I, false, false, false>; break;
+	case 1: k = k_pp_exact<I, false, false, true>; break;
+	case 2: k = k_pp_exact<I, false, true, false>; break;
+	case 3: k = k_pp_exact<I, false, true, true>; break;
+	case 4: k = k_pp_exact<I, true, false, false>; break;
+	case 5: k = k_pp_exact<I, true, false, true>; break;
+	case 6: k = k_pp_exact<I, true, true, false>; break;
+	default: break;
 	}
-	// chains: component wv of the block's 64 particles
-	const bool kahan = wv < 3u ? KAHAN_ACC : KAHAN_POT;
-	float s = 0.0f, c = 0.0f;
-	__syncthreads();
-	for (unsigned t = 0; t < tiles; ++t) {
-		const float* in = &s_term[t & 1u][wv][0][lane];
-		const unsigned n = min(N - t * kExJ, kExJ);
-		if (n == kExJ && kahan) {
-			float v[kExAhead], w[kExAhead];
-#pragma unroll
-			for (unsigned u = 0; u < kExAhead; ++u) v[u] = in[u * kExI];
-#pragma unroll
-			for (unsigned k = 0; k < kExJ; k += kExAhead) {
-				if (k + kExAhead < kExJ) {
-#pragma unroll
-					for (unsigned u = 0; u < kExAhead; ++u) w[u] = in[(k + kExAhead + u) * kExI];
-				}
-#pragma unroll
-				for (unsigned u = 0; u < kExAhead; ++u) kahan_add(s, c, v[u]);
-#pragma unroll
-				for (unsigned u = 0; u < kExAhead; ++u) v[u] = w[u];
-			}
-		} else if (kahan) {
-			for (unsigned k = 0; k < n; ++k) kahan_add(s, c, in[k * kExI]);
-		} else {
-			for (unsigned k = 0; k < n; ++k) s += in[k * kExI];
-		}
-		__syncthreads();
-	}
-	if (i >= N) return;
-	// reference src/gravity.c:808-811: ((-G) * m_i) * acc_sum, (-G) * pot_sum
-	if (wv == 3u) pot[i] = negG * s;
-	else acc[3u * i + wv] = (PHYS ? negG : negG * mas[i]) * s;
+	hipLaunchKernelGGL(k, dim3((N + I - 1) / I), dim3(chain::block_size<I, 4>()), 0, s, pos, mas, N, eps2, negG, acc,
+	                   pot);
 }
 
 // One tile of SF_TJ interactions, j from jt.  nb holds the tile's first
@@ -463,19 +421,10 @@ extern "C" int sfd_pack_bodies(const float* pos, const float* mas, unsigned N, u
 extern "C" int sfd_pp_exact(const float* pos, const float* mas, unsigned N, float eps2, float negG, int acc_phys,
                             int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s) {
 	if (N == 0) return 0;
-	const dim3 grid((N + kExI - 1) / kExI), block(kExBlock);
 	const int sel = (kahan_acc ? 4 : 0) | (kahan_pot ? 2 : 0) | (acc_phys ? 1 : 0);
 	const int tok = sf_prof_begin("pp_exact", s);
-	switch (sel) {
-	case 0: hipLaunchKernelGGL((k_pp_exact<false, false, false>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	case 1: hipLaunchKernelGGL((k_pp_exact<false, false, true>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	case 2: hipLaunchKernelGGL((k_pp_exact<false, true, false>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	case 3: hipLaunchKernelGGL((k_pp_exact<false, true, true>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	case 4: hipLaunchKernelGGL((k_pp_exact<true, false, false>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	case 5: hipLaunchKernelGGL((k_pp_exact<true, false, true>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	case 6: hipLaunchKernelGGL((k_pp_exact<true, true, false>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	default: hipLaunchKernelGGL((k_pp_exact<true, true, true>), grid, block, 0, s, pos, mas, N, eps2, negG, acc, pot); break;
-	}
+	if (N <= chain::kFewN) launch_exact<32>(sel, pos, mas, N, eps2, negG, acc, pot, s);
+	else launch_exact<64>(sel, pos, mas, N, eps2, negG, acc, pot, s);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_pp_exact", "k_pp_exact launch");
 }

@@ -5,11 +5,10 @@
 // rho_i = sum_j 0.5 (W_i + W_j) m_j over every j, polytrope P = (0.1 rho)^2,
 // and acc_i += -m_i sum_{r^2 <= 1} (P_i/rho_i^2 + P_j/rho_j^2) 0.5 (n_i + n_j) r_ij
 // with n = -2 exp(-r^2/h^2) / (pi^{3/2} h^5).  The file is compiled with
-// -ffp-contract=off and IEEE division and square root, so every product,
-// quotient and Kahan step rounds as the reference's does; the per-particle
-// factors that do not depend on the pair ((a^2) a, h h, pi^{3/2} h^5 and
-// P/rho^2) are computed once per particle with the same operations, which
-// gives the same bits.  exp() is the device library's (faithfully rounded,
+// -ffp-contract=off, and every product, quotient and Kahan step rounds as the
+// reference's does; the per-particle factors that do not depend on the pair
+// ((a^2) a, h h, pi^{3/2} h^5 and P/rho^2) are computed once per particle with
+// the same operations, which gives the same bits.  exp() is the device library's (faithfully rounded,
 // like glibc's expf, but not always the same float) and (0.1 rho)^2 is the
 // correctly rounded product where glibc's powf is off by one ulp in about
 // 0.07% of cases: results agree with the reference to a few ulp, not bit
@@ -27,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "order_chain.h"
 
 namespace {
 
@@ -40,101 +40,185 @@ constexpr float kInvSqrtPi = (float)0.564189583547756286948079451560772585844050
 constexpr float kPiPow32 = (float)5.5683279968317078452848179821188357020136243902832;
 constexpr float kPi = 3.14159265358979323846f;
 
-__device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
-	const float y = x - c;
-	const float t = s + y;
-	const float z = t - s;
-	c = z - y;
-	s = t;
-}
-
 // ------------------------------------------------------------ reference model
-// a3 = (a a) a with a = INV_SQRT_PI / h (src/sph.c:116-119); hh = h h;
-// den = INV_POW_PI_3_2 h h h h h evaluated left to right (src/sph.c:239-240)
-__global__ __launch_bounds__(kBlock) void k_tables_ref(const float* __restrict__ rad, unsigned N,
-                                                       float* __restrict__ a3, float* __restrict__ hh,
-                                                       float* __restrict__ den) {
+// The density and force sums run on order_chain.h: terms made in parallel,
+// added in index order.  N = 6000 (us): density 1524 and force 2246 with one
+// lane per particle and IEEE divisions in line, now 94 and 132.  Bound by the
+// chains (12 ns a body for the density, 17 for the force, whose chains also
+// test for skipped pairs) while the particles fit 32 to a CU, then by the
+// makers.
+
+// RN(a / b) from inv = RN(1 / b): the quotient's estimate corrected once by
+// its residual (Markstein 1990), for normal b and quotients that neither
+// overflow nor vanish.  Compared with a / b on 1.7e10 operand pairs.
+__device__ __forceinline__ float divide_by(float a, float b, float inv) {
+	const float q = a * inv;
+	return __builtin_fmaf(__builtin_fmaf(-q, b, a), inv, q);
+}
+// the divisors for which that holds with room for every numerator here; the
+// others' inverse is set to NaN, which sends their pairs to IEEE divisions
+__device__ __forceinline__ bool divisor_ok(float b) { return b >= 0x1p-60f && b <= 0x1p60f; }
+constexpr unsigned kQuotTop = 0x71800000u;    // 2^100: larger quotients, inf and NaN take IEEE divisions
+constexpr unsigned kSkipBits = 0x7FBADBADu;   // a term that is not added (a NaN no operation returns)
+
+// Records: a = (x, y, z, m), h = (h h, 1 / (h h), a3, -), d = (h h, 1 / (h h),
+// den, 1 / den) with a3 = (a a) a, a = INV_SQRT_PI / h (src/sph.c:116-119) and
+// den = INV_POW_PI_3_2 h h h h h evaluated left to right (src/sph.c:239-240).
+__global__ __launch_bounds__(kBlock) void k_tables_ref(const float* __restrict__ pos, const float* __restrict__ mas,
+                                                       const float* __restrict__ rad, unsigned N,
+                                                       float4* __restrict__ ra, float4* __restrict__ rh,
+                                                       float4* __restrict__ rd) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
 	if (i >= N) return;
 	const float h = rad[i];
 	const float a = kInvSqrtPi / h;
-	a3[i] = a * a * a;
-	hh[i] = h * h;
-	den[i] = kPiPow32 * h * h * h * h * h;
+	const float hh = h * h, den = kPiPow32 * h * h * h * h * h;
+	const bool ok = divisor_ok(hh) && divisor_ok(den);
+	const float ihh = ok ? 1.0f / hh : __builtin_nanf("");
+	ra[i] = make_float4(pos[3u * i], pos[3u * i + 1u], pos[3u * i + 2u], mas[i]);
+	rh[i] = make_float4(hh, ihh, a * a * a, 0.0f);
+	rd[i] = make_float4(hh, ihh, den, 1.0f / den);
+}
+
+struct QuotCheck {
+	unsigned top = 0u;
+	__device__ bool bad() const { return top >= kQuotTop; }
+};
+
+// exp(-r2 / h h) for both smoothing lengths of a pair
+template <bool FAST>
+__device__ __forceinline__ void gauss_pair(float r2, float hi, float ihi, float hj, float ihj, float& ei, float& ej,
+                                           QuotCheck& chk) {
+	float qi, qj;
+	if (FAST) {
+		qi = divide_by(r2, hi, ihi);
+		qj = divide_by(r2, hj, ihj);
+		chk.top = max(chk.top, max(__float_as_uint(qi), __float_as_uint(qj)));   // r2 >= 0
+	} else {
+		qi = r2 / hi;
+		qj = r2 / hj;
+	}
+	ei = expf(-qi);
+	ej = expf(-qj);
 }
 
 // src/sph.c:35-145
 template <bool KAHAN>
-__global__ __launch_bounds__(kBlock) void k_rho_ref(const float* __restrict__ pos, const float* __restrict__ mas,
-                                                    const float* __restrict__ a3, const float* __restrict__ hh,
-                                                    unsigned N, float* __restrict__ rho) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	const unsigned ii = i < N ? i : N - 1u;
-	const float xi = pos[3u * ii], yi = pos[3u * ii + 1u], zi = pos[3u * ii + 2u];
-	const float a3i = a3[ii], hhi = hh[ii];
-	float s = 0.0f, c = 0.0f;
-	for (unsigned j = 0u; j < N; ++j) {
-		const float mj = mas[j];
-		const float rx = xi - pos[3u * j], ry = yi - pos[3u * j + 1u], rz = zi - pos[3u * j + 2u];
+struct RhoRef {
+	static constexpr unsigned kComps = 1;
+	const float4* __restrict__ ra;
+	const float4* __restrict__ rh;
+	float* __restrict__ rho;
+	struct Body {
+		float4 a, h;
+	};
+	using Self = Body;
+	using Check = QuotCheck;
+	__device__ bool fast() const { return true; }
+	__device__ Self self(unsigned i) const { return {ra[i], rh[i]}; }
+	__device__ __forceinline__ Body body(unsigned j, unsigned off) const { return {(ra + j)[off], (rh + j)[off]}; }
+	template <bool FAST>
+	__device__ __forceinline__ void terms(const Self& i, const Body& j, float (&out)[1], Check& chk) const {
+		const float rx = i.a.x - j.a.x, ry = i.a.y - j.a.y, rz = i.a.z - j.a.z;
 		const float r2 = (rx * rx) + (ry * ry) + (rz * rz);
-		const float wi = a3i * expf(-r2 / hhi);
-		const float wj = a3[j] * expf(-r2 / hh[j]);
-		const float t = 0.5f * (wi + wj) * mj;
-		if (KAHAN) kahan_add(s, c, t);
-		else s += t;
+		float ei, ej;
+		gauss_pair<FAST>(r2, i.h.x, i.h.y, j.h.x, j.h.y, ei, ej, chk);
+		const float wi = i.h.z * ei, wj = j.h.z * ej;
+		out[0] = 0.5f * (wi + wj) * j.a.w;
 	}
-	if (i < N) rho[i] = s;
+	__device__ __forceinline__ void step(unsigned, float& s, float& c, float x) const {
+		if (KAHAN) chain::kahan(s, c, x);
+		else s += x;
+	}
+	__device__ void store(unsigned i, unsigned, float s) const { rho[i] = s; }
+};
+
+template <unsigned I, bool KAHAN>
+__global__ __launch_bounds__((chain::block_size<I, 1>())) void k_rho_ref(const float4* __restrict__ ra,
+                                                                       const float4* __restrict__ rh, unsigned N,
+                                                                       float* __restrict__ rho) {
+	chain::run<I>(RhoRef<KAHAN>{ra, rh, rho}, N);
 }
 
 // P = (K rho)^(1/n + 1) with K = 0.1, n = 1 (src/sph.c:147-157), and the
-// momentum-equation factor P / rho^2 (src/sph.c:189-192, :225-226)
+// momentum-equation factor P / rho^2 (src/sph.c:189-192, :225-226), which
+// takes the mass's place in the record
 __global__ __launch_bounds__(kBlock) void k_eos_ref(const float* __restrict__ rho, unsigned N,
-                                                    float* __restrict__ prs, float* __restrict__ con) {
+                                                    float* __restrict__ prs, float4* __restrict__ ra) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
 	if (i >= N) return;
 	const float x = 0.100f * rho[i];
 	const float p = x * x;
 	prs[i] = p;
 	const float r2 = rho[i] * rho[i];
-	con[i] = 0.0f < r2 ? p / r2 : 0.0f;
+	ra[i].w = 0.0f < r2 ? p / r2 : 0.0f;
 }
 
-// src/sph.c:163-276
+// src/sph.c:163-276.  Pairs with r2 > 1 are not added; their chains see
+// kSkipBits.  2 exp / den: the numerator is scaled by 2^64 so that the
+// residual of a tiny quotient does not vanish.
 template <bool KAHAN>
-__global__ __launch_bounds__(kBlock) void k_force_ref(const float* __restrict__ pos, const float* __restrict__ mas,
-                                                      const float* __restrict__ hh, const float* __restrict__ den,
-                                                      const float* __restrict__ con, unsigned N,
-                                                      float* __restrict__ acc) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	const unsigned ii = i < N ? i : N - 1u;
-	const float xi = pos[3u * ii], yi = pos[3u * ii + 1u], zi = pos[3u * ii + 2u];
-	const float hhi = hh[ii], deni = den[ii], coni = con[ii];
-	float sx = 0.0f, sy = 0.0f, sz = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
-	for (unsigned j = 0u; j < N; ++j) {
-		const float rx = xi - pos[3u * j], ry = yi - pos[3u * j + 1u], rz = zi - pos[3u * j + 2u];
+struct ForceRef {
+	static constexpr unsigned kComps = 3;
+	const float4* __restrict__ ra;
+	const float4* __restrict__ rd;
+	const float* __restrict__ mas;
+	float* __restrict__ acc;
+	struct Body {
+		float4 a, d;
+	};
+	using Self = Body;
+	using Check = QuotCheck;
+	__device__ bool fast() const { return true; }
+	__device__ Self self(unsigned i) const { return {ra[i], rd[i]}; }
+	__device__ __forceinline__ Body body(unsigned j, unsigned off) const { return {(ra + j)[off], (rd + j)[off]}; }
+	template <bool FAST>
+	__device__ __forceinline__ void terms(const Self& i, const Body& j, float (&out)[3], Check& chk) const {
+		const float rx = i.a.x - j.a.x, ry = i.a.y - j.a.y, rz = i.a.z - j.a.z;
 		const float r2 = (rx * rx) + (ry * ry) + (rz * rz);
-		if (r2 > 1.0f) continue;
-		const float ni = -2.0f * expf(-r2 / hhi) / deni;
-		const float nj = -2.0f * expf(-r2 / hh[j]) / den[j];
-		const float g = 0.5f * (ni + nj);
-		const float cc = coni + con[j];
-		const float X = cc * (g * rx), Y = cc * (g * ry), Z = cc * (g * rz);
-		if (KAHAN) {
-			kahan_add(sx, cx, X);
-			kahan_add(sy, cy, Y);
-			kahan_add(sz, cz, Z);
+		float ei, ej, ni, nj;
+		gauss_pair<FAST>(r2, i.d.x, i.d.y, j.d.x, j.d.y, ei, ej, chk);
+		if (FAST) {
+			ni = divide_by(-0x1p65f * ei, i.d.z, i.d.w) * 0x1p-64f;
+			nj = divide_by(-0x1p65f * ej, j.d.z, j.d.w) * 0x1p-64f;
 		} else {
-			sx += X;
-			sy += Y;
-			sz += Z;
+			ni = -2.0f * ei / i.d.z;
+			nj = -2.0f * ej / j.d.z;
 		}
+		const float g = 0.5f * (ni + nj);
+		const float cc = i.a.w + j.a.w;
+		const float skip = __uint_as_float(kSkipBits);
+		const bool far = r2 > 1.0f;
+		out[0] = far ? skip : cc * (g * rx);
+		out[1] = far ? skip : cc * (g * ry);
+		out[2] = far ? skip : cc * (g * rz);
 	}
-	if (i < N) {
-		const float nm = -mas[i];
-		acc[3u * i + 0u] += nm * sx;
-		acc[3u * i + 1u] += nm * sy;
-		acc[3u * i + 2u] += nm * sz;
+	__device__ __forceinline__ void step(unsigned, float& s, float& c, float x) const {
+		const bool add = __float_as_uint(x) != kSkipBits;
+		float s1 = s, c1 = c;
+		if (KAHAN) chain::kahan(s1, c1, x);
+		else s1 += x;
+		s = add ? s1 : s;
+		c = add ? c1 : c;
 	}
+	__device__ void store(unsigned i, unsigned comp, float s) const { acc[3u * i + comp] += -mas[i] * s; }
+};
+
+template <unsigned I, bool KAHAN>
+__global__ __launch_bounds__((chain::block_size<I, 3>())) void k_force_ref(const float4* __restrict__ ra,
+                                                                         const float4* __restrict__ rd,
+                                                                         const float* __restrict__ mas, unsigned N,
+                                                                         float* __restrict__ acc) {
+	chain::run<I>(ForceRef<KAHAN>{ra, rd, mas, acc}, N);
+}
+
+template <unsigned I, bool KAHAN>
+void launch_ref(const float4* ra, const float4* rh, const float4* rd, const float* mas, unsigned N, float* rho,
+                float* prs, float4* ra_con, float* acc, hipStream_t s) {
+	const dim3 g((N + I - 1u) / I);
+	hipLaunchKernelGGL((k_rho_ref<I, KAHAN>), g, dim3(chain::block_size<I, 1>()), 0, s, ra, rh, N, rho);
+	hipLaunchKernelGGL(k_eos_ref, dim3((N + kBlock - 1u) / kBlock), dim3(kBlock), 0, s, rho, N, prs, ra_con);
+	hipLaunchKernelGGL((k_force_ref<I, KAHAN>), g, dim3(chain::block_size<I, 3>()), 0, s, ra, rd, mas, N, acc);
 }
 
 // ---------------------------------------------------------------- cubic model
@@ -305,16 +389,13 @@ size_t sfd_sph_tmp_floats(unsigned n_pad) { return 12u * (size_t)n_pad + 16u; }
 int sfd_sph_ref(const float* pos, const float* mas, const float* rad, unsigned N, int kahan, float* rho, float* prs,
                 float* acc, float* tmp, hipStream_t s) {
 	if (N == 0) return 0;
-	float* a3 = tmp;
-	float* hh = tmp + N;
-	float* den = tmp + 2u * (size_t)N;
-	float* con = tmp + 3u * (size_t)N;
-	hipLaunchKernelGGL(k_tables_ref, grid(N), dim3(kBlock), 0, s, rad, N, a3, hh, den);
-	if (kahan) hipLaunchKernelGGL(k_rho_ref<true>, grid(N), dim3(kBlock), 0, s, pos, mas, a3, hh, N, rho);
-	else hipLaunchKernelGGL(k_rho_ref<false>, grid(N), dim3(kBlock), 0, s, pos, mas, a3, hh, N, rho);
-	hipLaunchKernelGGL(k_eos_ref, grid(N), dim3(kBlock), 0, s, rho, N, prs, con);
-	if (kahan) hipLaunchKernelGGL(k_force_ref<true>, grid(N), dim3(kBlock), 0, s, pos, mas, hh, den, con, N, acc);
-	else hipLaunchKernelGGL(k_force_ref<false>, grid(N), dim3(kBlock), 0, s, pos, mas, hh, den, con, N, acc);
+	float4* ra = reinterpret_cast<float4*>(tmp);
+	float4* rh = ra + N;
+	float4* rd = ra + 2u * (size_t)N;
+	hipLaunchKernelGGL(k_tables_ref, grid(N), dim3(kBlock), 0, s, pos, mas, rad, N, ra, rh, rd);
+	auto go = N <= chain::kFewN ? (kahan ? launch_ref<32, true> : launch_ref<32, false>)
+	                            : (kahan ? launch_ref<64, true> : launch_ref<64, false>);
+	go(ra, rh, rd, mas, N, rho, prs, ra, acc, s);
 	return sf_hip_check(hipGetLastError(), "solve_sph", "launch");
 }
 
