@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "pp_sym.h"
 
 namespace {
 
@@ -134,6 +135,144 @@ __global__ __launch_bounds__(kBlock) void k_vjp(const float4* __restrict__ body,
 	part[(size_t)(2u * sl + 1u) * n_pad + k] = make_float4(Cx, Cy, Cz, 0.0f);
 }
 
+// ------------------------------------------------- each pair once (pp_sym.h)
+// From kSymMin bodies: w = m_k nu_j - m_j nu_k changes sign with the pair's
+// order and K does not, so a pair's term goes to k as it is and to j negated:
+// 29 VALU operations and one rsq with equal masses (35 with general ones) for
+// both, where the one-sided kernel takes 46 and two (52).  The layout is
+// pp_sym.hip's narrow one: 256 k per block, four per lane, the same in its
+// four wavefronts, a 64-body tile each, the j sums passed from lane to lane
+// through LDS.  VJP_FIGURES
+constexpr int kPer = 4;
+constexpr unsigned kWaves = kBlock / 64;
+
+struct KSet {
+	float x[kPer], y[kPer], z[kPer], m[kPer], nx[kPer], ny[kPer], nz[kPer];
+	float tx[kPer], ty[kPer], tz[kPer];
+};
+
+// At step s lane l meets body (l + s) mod 64; sb, sn and acc hold the tile
+// twice over, as in pp_sym.hip.  SYM false: pairs inside the set.
+template <bool UNIFORM, bool SYM>
+__device__ __forceinline__ void vjp_sym_tile(const float4* __restrict__ sb, const float4* __restrict__ sn,
+                                             float4* __restrict__ acc, unsigned lane, float eps2, KSet& a) {
+	const float4* bl = sb + lane;
+	const float4* nl = sn + lane;
+	float4* al = acc + lane;
+	float4 nb = bl[0], nn = nl[0];
+#pragma unroll 2
+	for (unsigned s = 0; s < kSymTile; ++s) {
+		float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+		if (SYM) o = al[s];
+		const float4 b = nb, n = nn;
+		nb = bl[s + 1u];   // s = 63: lane + 64, in the second copy
+		nn = nl[s + 1u];
+		float px = 0.0f, py = 0.0f, pz = 0.0f;
+#pragma unroll
+		for (int k = 0; k < kPer; ++k) {
+			const float dx = a.x[k] - b.x, dy = a.y[k] - b.y, dz = a.z[k] - b.z;
+			float r2 = __builtin_fmaf(dx, dx, eps2);
+			r2 = __builtin_fmaf(dy, dy, r2);
+			r2 = __builtin_fmaf(dz, dz, r2);
+			const float inv = __builtin_amdgcn_rsqf(r2);
+			const float inv2 = inv * inv;
+			const float inv3 = inv2 * inv;
+			const float i5_3 = inv3 * (-3.0f * inv2);   // -3 / s^5: every product below accumulates in place
+			// exactly zero when j == k, as in vjp_tile
+			const float wx = UNIFORM ? n.x - a.nx[k] : a.m[k] * n.x - b.w * a.nx[k];
+			const float wy = UNIFORM ? n.y - a.ny[k] : a.m[k] * n.y - b.w * a.ny[k];
+			const float wz = UNIFORM ? n.z - a.nz[k] : a.m[k] * n.z - b.w * a.nz[k];
+			const float dw = __builtin_fmaf(dz, wz, __builtin_fmaf(dy, wy, dx * wx));
+			const float q = i5_3 * dw;
+			a.tx[k] = __builtin_fmaf(q, dx, __builtin_fmaf(inv3, wx, a.tx[k]));
+			a.ty[k] = __builtin_fmaf(q, dy, __builtin_fmaf(inv3, wy, a.ty[k]));
+			a.tz[k] = __builtin_fmaf(q, dz, __builtin_fmaf(inv3, wz, a.tz[k]));
+			if (SYM) {   // k's sign; the tile's sums are negated at the end
+				px = __builtin_fmaf(q, dx, k ? __builtin_fmaf(inv3, wx, px) : inv3 * wx);
+				py = __builtin_fmaf(q, dy, k ? __builtin_fmaf(inv3, wy, py) : inv3 * wy);
+				pz = __builtin_fmaf(q, dz, k ? __builtin_fmaf(inv3, wz, pz) : inv3 * wz);
+			}
+		}
+		if (SYM) {
+			al[s] = make_float4(o.x + px, o.y + py, o.z + pz, 0.0f);
+			__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+		}
+	}
+}
+
+__global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict__ body, const float4* __restrict__ nu,
+                                                       unsigned n_pad, unsigned S, unsigned d0, unsigned chunks,
+                                                       unsigned dchunks, float eps2, float4* __restrict__ part_i,
+                                                       float4* __restrict__ part_j) {
+	__shared__ float4 s_mem[kWaves][6u * kSymTile];   // a wavefront's bodies, nu and j sums, then its k sums
+	const unsigned t = threadIdx.x, lane = t & 63u;
+	const unsigned wv = __builtin_amdgcn_readfirstlane(t >> 6);
+	const unsigned per = chunks + dchunks;
+	const unsigned ib = blockIdx.x / per, c = blockIdx.x % per;
+	const bool sym = c < chunks;
+	const unsigned nd = S / 2u - (((S & 1u) || ib < S / 2u) ? 0u : 1u);
+	const size_t out = (size_t)c * n_pad + ib * kSymNarrow + t;
+	const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	if (sym && d0 + c >= nd) {
+		part_i[out] = zero;
+		return;
+	}
+	unsigned jb = sym ? ib + 1u + d0 + c : ib;
+	if (jb >= S) jb -= S;
+	const unsigned j = jb * kSymNarrow + wv * kSymTile;
+	KSet a;
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) {
+		const float4 b = body[ib * kSymNarrow + 64u * k + lane], n = nu[ib * kSymNarrow + 64u * k + lane];
+		a.x[k] = b.x;
+		a.y[k] = b.y;
+		a.z[k] = b.z;
+		a.m[k] = b.w;
+		a.nx[k] = n.x;
+		a.ny[k] = n.y;
+		a.nz[k] = n.z;
+		a.tx[k] = a.ty[k] = a.tz[k] = 0.0f;
+	}
+	const float4 vb = body[j + lane], vn = nu[j + lane];
+	const unsigned n_uni = *reinterpret_cast<const unsigned*>(body + n_pad);
+	const bool uni = (ib + 1u) * kSymNarrow <= n_uni && j + kSymTile <= n_uni;
+	const float mu = body[0].w;
+	float4* sb = s_mem[wv];
+	float4* sn = sb + 2u * kSymTile;
+	float4* acc = sn + 2u * kSymTile;
+	sb[lane] = sb[lane + kSymTile] = vb;
+	sn[lane] = sn[lane + kSymTile] = vn;
+	acc[lane] = acc[lane + kSymTile] = zero;
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+	if (sym) {
+		if (uni) vjp_sym_tile<true, true>(sb, sn, acc, lane, eps2, a);
+		else vjp_sym_tile<false, true>(sb, sn, acc, lane, eps2, a);
+		const float4 p = acc[lane], q = acc[lane + kSymTile];
+		const double sc = uni ? -(double)mu : -1.0;
+		part_j[(size_t)c * n_pad + j + lane] =
+		    make_float4((float)(sc * ((double)p.x + (double)q.x)), (float)(sc * ((double)p.y + (double)q.y)),
+		                (float)(sc * ((double)p.z + (double)q.z)), 0.0f);
+	} else {
+		if (uni) vjp_sym_tile<true, false>(sb, sn, acc, lane, eps2, a);
+		else vjp_sym_tile<false, false>(sb, sn, acc, lane, eps2, a);
+	}
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+	const float sc = uni ? mu : 1.0f;
+#pragma unroll
+	for (int k = 0; k < kPer; ++k)
+		s_mem[wv][64u * k + lane] = make_float4(sc * a.tx[k], sc * a.ty[k], sc * a.tz[k], 0.0f);
+	__syncthreads();
+	double sx = 0.0, sy = 0.0, sz = 0.0;
+#pragma unroll
+	for (unsigned w = 0; w < kWaves; ++w) {
+		const float4 p = s_mem[w][t];
+		sx += (double)p.x;
+		sy += (double)p.y;
+		sz += (double)p.z;
+	}
+	part_i[out] = make_float4((float)sx, (float)sy, (float)sz, 0.0f);
+}
+
 // g_k (= or +=) G * sum over slices of (sum - compensation), in FP64
 // A block takes kCombI particles; its wavefronts take the slices s = w,
 // w + kCombG, ... (w = wavefront) and wavefront 0 adds their sums in order
@@ -163,6 +302,57 @@ __global__ __launch_bounds__(kBlock) void k_vjp_combine(const float4* __restrict
 		sx += red[q][0][kl];
 		sy += red[q][1][kl];
 		sz += red[q][2][kl];
+	}
+	float gx = (float)(G * sx), gy = (float)(G * sy), gz = (float)(G * sz);
+	if (accumulate) {
+		gx += g[3u * k + 0u];
+		gy += g[3u * k + 1u];
+		gz += g[3u * k + 2u];
+	}
+	g[3u * k + 0u] = gx;
+	g[3u * k + 1u] = gy;
+	g[3u * k + 2u] = gz;
+}
+
+// The same for a launch's planes of k_vjp_sym (one float4 per body and plane,
+// the k planes, then the j planes), added to the sums of the launches before
+// it (run, when !first), which all but the last keep there.
+__global__ __launch_bounds__(kBlock) void k_vjp_sym_combine(const float4* __restrict__ part, unsigned n_pad,
+                                                            unsigned planes, int first, int last,
+                                                            double4* __restrict__ run, unsigned N, double G,
+                                                            int accumulate, float* __restrict__ g) {
+	__shared__ double red[kCombG][3][kCombI];
+	const unsigned kl = threadIdx.x % kCombI, w = threadIdx.x / kCombI;
+	const unsigned k = blockIdx.x * kCombI + kl;   // < n_pad: the grid covers N in kCombI steps
+	// the number of sets is even: the last offset's plane reaches the upper half only
+	if (last && k < n_pad / 2u) --planes;
+	double sx = 0.0, sy = 0.0, sz = 0.0;
+#pragma unroll 4
+	for (unsigned s = w; s < planes; s += kCombG) {
+		const float4 a = part[(size_t)s * n_pad + k];
+		sx += (double)a.x;
+		sy += (double)a.y;
+		sz += (double)a.z;
+	}
+	red[w][0][kl] = sx;
+	red[w][1][kl] = sy;
+	red[w][2][kl] = sz;
+	__syncthreads();
+	if (w != 0 || k >= N) return;
+	for (unsigned q = 1; q < kCombG; ++q) {
+		sx += red[q][0][kl];
+		sy += red[q][1][kl];
+		sz += red[q][2][kl];
+	}
+	if (!first) {
+		const double4 r = run[k];
+		sx += r.x;
+		sy += r.y;
+		sz += r.z;
+	}
+	if (!last) {
+		run[k] = make_double4(sx, sy, sz, 0.0);
+		return;
 	}
 	float gx = (float)(G * sx), gy = (float)(G * sy), gz = (float)(G * sz);
 	if (accumulate) {
@@ -219,10 +409,16 @@ inline dim3 grid(unsigned n) { return dim3((n + kBlock - 1u) / kBlock); }
 
 extern "C" {
 
+// bytes of part for sfd_force_vjp: k_vjp_sym's planes, or below kSymMin
+// bodies slices x 2 x n_pad float4
+size_t sfd_vjp_part_bytes(unsigned n_pad, unsigned slices) {
+	return n_pad >= kSymMin ? sym_part_bytes(n_pad, false) : (size_t)slices * 2u * n_pad * 16u;
+}
+
 // g (=, or += when accumulate) G sum_j K(d_kj) (m_k nu_j - m_j nu_k) with
 // nu = coef mu (coef m mu): body is the packed (x, m) array of the force
 // kernel (n_pad entries), nu and part are scratch (n_pad float4 and
-// slices x 2 x n_pad float4).
+// sfd_vjp_part_bytes).
 int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned N, unsigned n_pad, float eps2,
                   double G, int acc_phys, float coef, float* nu, float* part, unsigned slices, int accumulate,
                   float* g, hipStream_t s) {
@@ -230,6 +426,24 @@ int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned
 	if (n_pad % kBlock != 0 || slices == 0) return -1;
 	float4* nu4 = reinterpret_cast<float4*>(nu);
 	hipLaunchKernelGGL(k_pack_nu, grid(n_pad), dim3(kBlock), 0, s, mu, mas, N, n_pad, coef, acc_phys, nu4);
+	if (n_pad >= kSymMin) {
+		const SymGeometry q = sym_geometry(n_pad, false);
+		const float4* b4 = reinterpret_cast<const float4*>(body);
+		float4* p4 = reinterpret_cast<float4*>(part);
+		double4* run = reinterpret_cast<double4*>(p4 + ((size_t)q.chunks + q.dchunks + q.per_launch) * n_pad);
+		for (unsigned d0 = 0; d0 < q.offsets; d0 += q.per_launch) {
+			const unsigned ch = d0 + q.per_launch < q.offsets ? q.per_launch : q.offsets - d0;
+			const int first = d0 == 0u, last = d0 + ch == q.offsets;
+			const unsigned pi = ch + (first ? q.dchunks : 0u);
+			const int tok = sf_prof_begin("force_vjp", s);
+			hipLaunchKernelGGL(k_vjp_sym, dim3(q.blocks * pi), dim3(kBlock), 0, s, b4, nu4, n_pad, q.blocks, d0, ch,
+			                   pi - ch, eps2, p4, p4 + (size_t)pi * n_pad);
+			sf_prof_end(tok, s);
+			hipLaunchKernelGGL(k_vjp_sym_combine, dim3((N + kCombI - 1) / kCombI), dim3(kBlock), 0, s, p4, n_pad,
+			                   pi + ch, first, last, run, N, G, accumulate, g);
+		}
+		return sf_hip_check(hipGetLastError(), "sfd_force_vjp", "launch");
+	}
 	// whole tiles per slice, every slice non-empty (at most the requested count)
 	const unsigned tiles = n_pad / kTile;
 	if (slices > tiles) slices = tiles;

@@ -26,6 +26,7 @@
 int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned int N, unsigned int n_pad,
                   float eps2, double G, int acc_phys, float coef, float* nu, float* part, unsigned int slices,
                   int accumulate, float* g, hipStream_t s);
+size_t sfd_vjp_part_bytes(unsigned int n_pad, unsigned int slices);
 int sfd_axpy(float* y, const float* x, unsigned int n, float a, hipStream_t s);
 int sfd_f32_to_f64(const float* x, unsigned int n, double* y, hipStream_t s);
 int sfd_f64_to_f32(const double* x, unsigned int n, float* y, hipStream_t s);
@@ -36,7 +37,7 @@ typedef struct {
 	unsigned int N, n_pad, slices;
 	float* body;   /* n_pad float4 */
 	float* nu;     /* n_pad float4 */
-	float* part;   /* slices x 2 x n_pad float4, or the PP force's partial sums */
+	float* part;   /* the partial sums of the force and of its VJP */
 	size_t part_bytes;
 } sf_pp_scratch;
 
@@ -52,7 +53,7 @@ static int scratch_alloc(sf_pp_scratch* w, unsigned int N, const char* func) {
 	w->n_pad = ((N ? N : 1u) + 1023u) / 1024u * 1024u;
 	w->slices = sf_pp_slice_count(w->n_pad);
 	const size_t plane = (size_t)w->n_pad * 4u * sizeof(float), pp_bytes = sf_pp_part_bytes(w->n_pad);
-	w->part_bytes = plane * 2u * w->slices;
+	w->part_bytes = sfd_vjp_part_bytes(w->n_pad, w->slices);
 	if (w->part_bytes < pp_bytes) w->part_bytes = pp_bytes;
 	if (hipMalloc((void**)&w->body, SF_BODY_BYTES(w->n_pad)) != hipSuccess ||
 	    hipMalloc((void**)&w->nu, plane) != hipSuccess ||
