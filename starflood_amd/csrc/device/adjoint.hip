@@ -142,7 +142,11 @@ __global__ __launch_bounds__(kBlock) void k_vjp(const float4* __restrict__ body,
 // both, where the one-sided kernel takes 46 and two (52).  The layout is
 // pp_sym.hip's narrow one: 256 k per block, four per lane, the same in its
 // four wavefronts, a 64-body tile each, the j sums passed from lane to lane
-// through LDS.  VJP_FIGURES
+// through LDS.  Bound by issue: 32 operations and the rsq a pair and
+// wavefront, 43 ns at N = 65536 (the model of pp_sym.hip says 38).  One-sided
+// -> this, with the combine, us: N = 10007 75 -> 57, 16384 137 -> 110 (general
+// masses 160 -> 125), 65536 1884 -> 1422; at 8192 the one-sided kernel's 49 is
+// not beaten.
 constexpr int kPer = 4;
 constexpr unsigned kWaves = kBlock / 64;
 

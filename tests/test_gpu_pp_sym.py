@@ -87,3 +87,36 @@ def test_force_without_potential_has_the_same_acc(N):
         assert lib.sf_force_dev(N, x.data_ptr(), m.data_ptr(), acc.data_ptr(), p, stream) == 0
     assert torch.equal(out[0], out[1])
     L.set_params()
+
+
+def vjp_rows(x, m, mu, rows):
+    """FP64 g_k and, per k, the size of its terms."""
+    for k in rows:
+        d = x[k] - x
+        s2 = (d * d).sum(1) + EPS * EPS
+        w = m[k] * mu - m[:, None] * mu[k]
+        size = m[k] * np.linalg.norm(mu, axis=1) + m * np.linalg.norm(mu[k])
+        g = (w * s2[:, None] ** -1.5 - 3.0 * d * ((d * w).sum(1) * s2 ** -2.5)[:, None]).sum(0)
+        yield k, g, (size * (s2 ** -1.5 + 3.0 * (d * d).sum(1) * s2 ** -2.5)).sum()
+
+
+@pytest.mark.parametrize("N,masses", [(9217, "equal"), (10240, "general"), (12289, "one_differs"), (26000, "equal"),
+                                      (140001, "general")])
+def test_vjp_pairs_once_close_to_fp64(N, masses):
+    """k_vjp_sym, over the same edges (140001 needs two launches): a term is a
+    product of six rounded factors, 20 u, and the walk of 64-term sums adds
+    less; 2e-6 of the terms' sizes is allowed."""
+    print(f"vjp_sym N={N} masses={masses}", flush=True)
+    lib = L.load()
+    L.set_params(epsilon=EPS, acc_mode=L.SF_ACC_PHYSICAL)
+    pos, mas = state(N, masses)
+    mu = np.random.default_rng(N + 1).normal(size=(N, 3)).astype(np.float32)
+    x, m, u = (torch.from_numpy(a).cuda() for a in (pos, mas, mu))
+    g = torch.empty_like(x)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.sf_force_vjp_dev(N, x.data_ptr(), m.data_ptr(), u.data_ptr(), g.data_ptr(), stream) == 0
+    got = g.cpu().numpy().astype(np.float64)
+    rows = np.unique(np.r_[0, 255, 256, N // 2, N - 1, np.linspace(0, N - 1, 27).astype(int)])
+    for k, want, size in vjp_rows(pos.astype(np.float64), mas.astype(np.float64), mu.astype(np.float64), rows):
+        assert np.abs(got[k] - want).max() <= 2e-6 * size, k
+    L.set_params()
