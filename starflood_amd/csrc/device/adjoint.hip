@@ -238,9 +238,11 @@ __global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict_
 		a.tx[k] = a.ty[k] = a.tz[k] = 0.0f;
 	}
 	const float4 vb = body[j + lane], vn = nu[j + lane];
-	const unsigned n_uni = *reinterpret_cast<const unsigned*>(body + n_pad);
-	const bool uni = (ib + 1u) * kSymNarrow <= n_uni && j + kSymTile <= n_uni;
 	const float mu = body[0].w;
+	bool differs = __float_as_uint(vb.w) != __float_as_uint(mu);
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) differs |= __float_as_uint(a.m[k]) != __float_as_uint(mu);
+	const bool uni = __ballot(differs) == 0ull;
 	float4* sb = s_mem[wv];
 	float4* sn = sb + 2u * kSymTile;
 	float4* acc = sn + 2u * kSymTile;
@@ -277,15 +279,65 @@ __global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict_
 	part_i[out] = make_float4((float)sx, (float)sy, (float)sz, 0.0f);
 }
 
-// g_k (= or +=) G * sum over slices of (sum - compensation), in FP64
+// What a combine does with g_k: store it, or take the adjoint one step
+// further back (backward recursion of host/adjoint.c), which saves the three
+// launches of 5 us each that the update, nu and the next bodies took.
+struct VjpStore {
+	float* g;
+	explicit VjpStore(const sf_vjp_epi& e) : g(e.g) {}
+	__device__ __forceinline__ void operator()(unsigned k, float gx, float gy, float gz) const {
+		g[3u * k + 0u] = gx;
+		g[3u * k + 1u] = gy;
+		g[3u * k + 2u] = gz;
+	}
+};
+
+__device__ __forceinline__ float4 weight(float coef, int acc_phys, float m, const float l[3]) {
+	const float f = acc_phys ? coef : coef * m;
+	return make_float4(f * l[0], f * l[1], f * l[2], 0.0f);
+}
+
+struct VjpStep {
+	sf_vjp_epi e;
+	explicit VjpStep(const sf_vjp_epi& v) : e(v) {}
+	__device__ __forceinline__ void operator()(unsigned k, float gx, float gy, float gz) const {
+		const float g[3] = {gx, gy, gz};
+		float lx[3], lv[3];
+#pragma unroll
+		for (unsigned u = 0; u < 3u; ++u) {
+			lx[u] = g[u] + e.lx[3u * k + u];
+			lv[u] = e.lv[3u * k + u];
+		}
+		if (e.gx0) {   // x_0: done
+#pragma unroll
+			for (unsigned u = 0; u < 3u; ++u) {
+				e.gx0[3u * k + u] = lx[u];
+				e.gv0[3u * k + u] = lv[u];
+			}
+			return;
+		}
+#pragma unroll
+		for (unsigned u = 0; u < 3u; ++u) {
+			lv[u] = __builtin_fmaf(e.dt, lx[u], lv[u]);
+			e.lx[3u * k + u] = lx[u];
+			e.lv[3u * k + u] = lv[u];
+		}
+		float4* body = reinterpret_cast<float4*>(e.body);
+		const float m = body[k].w;
+		reinterpret_cast<float4*>(e.nu)[k] = weight(e.coef, e.acc_phys, m, lv);
+		if (e.x) body[k] = make_float4(e.x[3u * k], e.x[3u * k + 1u], e.x[3u * k + 2u], m);
+	}
+};
+
+// g_k = G * sum over slices of (sum - compensation), in FP64
 // A block takes kCombI particles; its wavefronts take the slices s = w,
 // w + kCombG, ... (w = wavefront) and wavefront 0 adds their sums in order
 // (all lanes of one particle per slice would leave most CUs idle at small N).
 constexpr unsigned kCombI = 64;
 constexpr unsigned kCombG = kBlock / kCombI;
+template <class E>
 __global__ __launch_bounds__(kBlock) void k_vjp_combine(const float4* __restrict__ part, unsigned n_pad,
-                                                        unsigned slices, unsigned N, double G, int accumulate,
-                                                        float* __restrict__ g) {
+                                                        unsigned slices, unsigned N, double G, E epi) {
 	__shared__ double red[kCombG][3][kCombI];
 	const unsigned kl = threadIdx.x % kCombI, w = threadIdx.x / kCombI;
 	const unsigned k = blockIdx.x * kCombI + kl;   // < n_pad: the grid covers N in kCombI steps
@@ -307,24 +359,16 @@ __global__ __launch_bounds__(kBlock) void k_vjp_combine(const float4* __restrict
 		sy += red[q][1][kl];
 		sz += red[q][2][kl];
 	}
-	float gx = (float)(G * sx), gy = (float)(G * sy), gz = (float)(G * sz);
-	if (accumulate) {
-		gx += g[3u * k + 0u];
-		gy += g[3u * k + 1u];
-		gz += g[3u * k + 2u];
-	}
-	g[3u * k + 0u] = gx;
-	g[3u * k + 1u] = gy;
-	g[3u * k + 2u] = gz;
+	epi(k, (float)(G * sx), (float)(G * sy), (float)(G * sz));
 }
 
 // The same for a launch's planes of k_vjp_sym (one float4 per body and plane,
 // the k planes, then the j planes), added to the sums of the launches before
 // it (run, when !first), which all but the last keep there.
+template <class E>
 __global__ __launch_bounds__(kBlock) void k_vjp_sym_combine(const float4* __restrict__ part, unsigned n_pad,
                                                             unsigned planes, int first, int last,
-                                                            double4* __restrict__ run, unsigned N, double G,
-                                                            int accumulate, float* __restrict__ g) {
+                                                            double4* __restrict__ run, unsigned N, double G, E epi) {
 	__shared__ double red[kCombG][3][kCombI];
 	const unsigned kl = threadIdx.x % kCombI, w = threadIdx.x / kCombI;
 	const unsigned k = blockIdx.x * kCombI + kl;   // < n_pad: the grid covers N in kCombI steps
@@ -358,15 +402,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_combine(const float4* __rest
 		run[k] = make_double4(sx, sy, sz, 0.0);
 		return;
 	}
-	float gx = (float)(G * sx), gy = (float)(G * sy), gz = (float)(G * sz);
-	if (accumulate) {
-		gx += g[3u * k + 0u];
-		gy += g[3u * k + 1u];
-		gz += g[3u * k + 2u];
-	}
-	g[3u * k + 0u] = gx;
-	g[3u * k + 1u] = gy;
-	g[3u * k + 2u] = gz;
+	epi(k, (float)(G * sx), (float)(G * sy), (float)(G * sz));
 }
 
 // nu_i = coef * mu_i (physical) or coef * m_i * mu_i (reference); zero past N
@@ -375,31 +411,81 @@ __global__ __launch_bounds__(kBlock) void k_pack_nu(const float* __restrict__ mu
                                                     float4* __restrict__ nu) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
 	if (i >= n_pad) return;
+	float l[3] = {0.0f, 0.0f, 0.0f};
+	float m = 1.0f;
+	if (i < N) {
+		m = mas[i];
+#pragma unroll
+		for (unsigned u = 0; u < 3u; ++u) l[u] = mu[3u * i + u];
+	}
+	nu[i] = i < N ? weight(coef, acc_phys, m, l) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+// The state the forward integration starts from (positions into x too, when set)
+__global__ __launch_bounds__(kBlock) void k_adjoint_init(const float* __restrict__ x0, const float* __restrict__ v0,
+                                                         unsigned n3, double* __restrict__ x64,
+                                                         float* __restrict__ v, float* __restrict__ x) {
+	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+	if (i >= n3) return;
+	const float p = x0[i];
+	x64[i] = (double)p;
+	v[i] = v0[i];
+	if (x) x[i] = p;
+}
+
+// A segment from its checkpoint: x[0 .. 3N) its first positions; with steps,
+// also the first step's opening kick and drift (EpiKdk's), its positions into
+// x[3N .. 6N).  The last positions written go into the packed bodies.
+__global__ __launch_bounds__(kBlock) void k_adjoint_reopen(const double* __restrict__ ck_x64,
+                                                           const float* __restrict__ ck_v,
+                                                           const float* __restrict__ ck_a, unsigned N, float h,
+                                                           double dt, int steps, double* __restrict__ x64,
+                                                           float* __restrict__ v, float* __restrict__ x,
+                                                           float4* __restrict__ body) {
+	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+	if (i >= N) return;
+	float p[3];
+#pragma unroll
+	for (unsigned u = 0; u < 3u; ++u) {
+		const unsigned k = 3u * i + u;
+		double y = ck_x64[k];
+		p[u] = (float)y;
+		x[k] = p[u];
+		if (steps) {
+			const float w = __builtin_fmaf(h, ck_a[k], ck_v[k]);
+			y = __builtin_fma(dt, (double)w, y);
+			p[u] = (float)y;
+			v[k] = w;
+			x64[k] = y;
+			x[3u * (size_t)N + k] = p[u];
+		}
+	}
+	body[i] = make_float4(p[0], p[1], p[2], body[i].w);
+}
+
+// The cotangents the backward starts from (NULL: zero), the first VJP's nu
+// (zero past N) and its bodies.
+__global__ __launch_bounds__(kBlock) void k_adjoint_begin(const float* __restrict__ gx, const float* __restrict__ gv,
+                                                          const float* __restrict__ x, unsigned N, unsigned n_pad,
+                                                          float coef, int acc_phys, float* __restrict__ lx,
+                                                          float* __restrict__ lv, float4* __restrict__ body,
+                                                          float4* __restrict__ nu) {
+	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+	if (i >= n_pad) return;
 	if (i >= N) {
 		nu[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 		return;
 	}
-	const float f = acc_phys ? coef : coef * mas[i];
-	nu[i] = make_float4(f * mu[3u * i], f * mu[3u * i + 1u], f * mu[3u * i + 2u], 0.0f);
-}
-
-// y += a x over n floats
-__global__ __launch_bounds__(kBlock) void k_axpy(float* __restrict__ y, const float* __restrict__ x, unsigned n,
-                                                 float a) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	if (i < n) y[i] = __builtin_fmaf(a, x[i], y[i]);
-}
-
-__global__ __launch_bounds__(kBlock) void k_f32_to_f64(const float* __restrict__ x, unsigned n,
-                                                       double* __restrict__ y) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	if (i < n) y[i] = (double)x[i];
-}
-
-__global__ __launch_bounds__(kBlock) void k_f64_to_f32(const double* __restrict__ x, unsigned n,
-                                                       float* __restrict__ y) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	if (i < n) y[i] = (float)x[i];
+	float l[3];
+#pragma unroll
+	for (unsigned u = 0; u < 3u; ++u) {
+		lx[3u * i + u] = gx ? gx[3u * i + u] : 0.0f;
+		l[u] = gv ? gv[3u * i + u] : 0.0f;
+		lv[3u * i + u] = l[u];
+	}
+	const float m = body[i].w;
+	nu[i] = weight(coef, acc_phys, m, l);
+	body[i] = make_float4(x[3u * i], x[3u * i + 1u], x[3u * i + 2u], m);
 }
 
 __global__ __launch_bounds__(kBlock) void k_fill0(float* __restrict__ y, unsigned n) {
@@ -419,21 +505,27 @@ size_t sfd_vjp_part_bytes(unsigned n_pad, unsigned slices) {
 	return n_pad >= kSymMin ? sym_part_bytes(n_pad, false) : (size_t)slices * 2u * n_pad * 16u;
 }
 
-// g (=, or += when accumulate) G sum_j K(d_kj) (m_k nu_j - m_j nu_k) with
-// nu = coef mu (coef m mu): body is the packed (x, m) array of the force
-// kernel (n_pad entries), nu and part are scratch (n_pad float4 and
-// sfd_vjp_part_bytes).
-int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned N, unsigned n_pad, float eps2,
-                  double G, int acc_phys, float coef, float* nu, float* part, unsigned slices, int accumulate,
-                  float* g, hipStream_t s) {
+int sfd_pack_nu(const float* mu, const float* mas, unsigned N, unsigned n_pad, float coef, int acc_phys, float* nu,
+                hipStream_t s) {
+	if (N == 0) return 0;
+	hipLaunchKernelGGL(k_pack_nu, grid(n_pad), dim3(kBlock), 0, s, mu, mas, N, n_pad, coef, acc_phys,
+	                   reinterpret_cast<float4*>(nu));
+	return sf_hip_check(hipGetLastError(), "sfd_pack_nu", "launch");
+}
+
+// g = G sum_j K(d_kj) (m_k nu_j - m_j nu_k), then *epi: body is the packed
+// (x, m) array of the force kernel, nu the packed weights (both n_pad float4),
+// part scratch of sfd_vjp_part_bytes.
+int sfd_force_vjp(const float* body, const float* nu, unsigned N, unsigned n_pad, float eps2, double G, float* part,
+                  unsigned slices, const sf_vjp_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
 	if (n_pad % kBlock != 0 || slices == 0) return -1;
-	float4* nu4 = reinterpret_cast<float4*>(nu);
-	hipLaunchKernelGGL(k_pack_nu, grid(n_pad), dim3(kBlock), 0, s, mu, mas, N, n_pad, coef, acc_phys, nu4);
+	const float4* b4 = reinterpret_cast<const float4*>(body);
+	const float4* nu4 = reinterpret_cast<const float4*>(nu);
+	float4* p4 = reinterpret_cast<float4*>(part);
+	const dim3 cgrid((N + kCombI - 1) / kCombI);
 	if (n_pad >= kSymMin) {
 		const SymGeometry q = sym_geometry(n_pad, false);
-		const float4* b4 = reinterpret_cast<const float4*>(body);
-		float4* p4 = reinterpret_cast<float4*>(part);
 		double4* run = reinterpret_cast<double4*>(p4 + ((size_t)q.chunks + q.dchunks + q.per_launch) * n_pad);
 		for (unsigned d0 = 0; d0 < q.offsets; d0 += q.per_launch) {
 			const unsigned ch = d0 + q.per_launch < q.offsets ? q.per_launch : q.offsets - d0;
@@ -443,8 +535,12 @@ int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned
 			hipLaunchKernelGGL(k_vjp_sym, dim3(q.blocks * pi), dim3(kBlock), 0, s, b4, nu4, n_pad, q.blocks, d0, ch,
 			                   pi - ch, eps2, p4, p4 + (size_t)pi * n_pad);
 			sf_prof_end(tok, s);
-			hipLaunchKernelGGL(k_vjp_sym_combine, dim3((N + kCombI - 1) / kCombI), dim3(kBlock), 0, s, p4, n_pad,
-			                   pi + ch, first, last, run, N, G, accumulate, g);
+			if (epi->step)
+				hipLaunchKernelGGL(k_vjp_sym_combine<VjpStep>, cgrid, dim3(kBlock), 0, s, p4, n_pad, pi + ch, first,
+				                   last, run, N, G, VjpStep(*epi));
+			else
+				hipLaunchKernelGGL(k_vjp_sym_combine<VjpStore>, cgrid, dim3(kBlock), 0, s, p4, n_pad, pi + ch, first,
+				                   last, run, N, G, VjpStore(*epi));
 		}
 		return sf_hip_check(hipGetLastError(), "sfd_force_vjp", "launch");
 	}
@@ -455,30 +551,33 @@ int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned
 	slices = (n_pad + slice_len - 1u) / slice_len;
 	const unsigned grid_v = (n_pad / kBlock) * slices;
 	const int tok = sf_prof_begin("force_vjp", s);
-	hipLaunchKernelGGL(k_vjp, dim3(grid_v), dim3(kBlock), 0, s, reinterpret_cast<const float4*>(body), nu4, n_pad,
-	                   slices, slice_len, eps2, reinterpret_cast<float4*>(part));
+	hipLaunchKernelGGL(k_vjp, dim3(grid_v), dim3(kBlock), 0, s, b4, nu4, n_pad, slices, slice_len, eps2, p4);
 	sf_prof_end(tok, s);
-	hipLaunchKernelGGL(k_vjp_combine, dim3((N + kCombI - 1) / kCombI), dim3(kBlock), 0, s,
-	                   reinterpret_cast<const float4*>(part), n_pad, slices, N, G, accumulate, g);
+	if (epi->step)
+		hipLaunchKernelGGL(k_vjp_combine<VjpStep>, cgrid, dim3(kBlock), 0, s, p4, n_pad, slices, N, G, VjpStep(*epi));
+	else
+		hipLaunchKernelGGL(k_vjp_combine<VjpStore>, cgrid, dim3(kBlock), 0, s, p4, n_pad, slices, N, G,
+		                   VjpStore(*epi));
 	return sf_hip_check(hipGetLastError(), "sfd_force_vjp", "launch");
 }
 
-int sfd_axpy(float* y, const float* x, unsigned n, float a, hipStream_t s) {
-	if (n == 0) return 0;
-	hipLaunchKernelGGL(k_axpy, grid(n), dim3(kBlock), 0, s, y, x, n, a);
-	return sf_hip_check(hipGetLastError(), "sfd_axpy", "launch");
+int sfd_adjoint_init(const float* x0, const float* v0, unsigned N, double* x64, float* v, float* x, hipStream_t s) {
+	hipLaunchKernelGGL(k_adjoint_init, grid(3u * N), dim3(kBlock), 0, s, x0, v0, 3u * N, x64, v, x);
+	return sf_hip_check(hipGetLastError(), "sfd_adjoint_init", "launch");
 }
 
-int sfd_f32_to_f64(const float* x, unsigned n, double* y, hipStream_t s) {
-	if (n == 0) return 0;
-	hipLaunchKernelGGL(k_f32_to_f64, grid(n), dim3(kBlock), 0, s, x, n, y);
-	return sf_hip_check(hipGetLastError(), "sfd_f32_to_f64", "launch");
+int sfd_adjoint_reopen(const double* ck_x64, const float* ck_v, const float* ck_a, unsigned N, float h, double dt,
+                       int steps, double* x64, float* v, float* x, float* body, hipStream_t s) {
+	hipLaunchKernelGGL(k_adjoint_reopen, grid(N), dim3(kBlock), 0, s, ck_x64, ck_v, ck_a, N, h, dt, steps, x64, v, x,
+	                   reinterpret_cast<float4*>(body));
+	return sf_hip_check(hipGetLastError(), "sfd_adjoint_reopen", "launch");
 }
 
-int sfd_f64_to_f32(const double* x, unsigned n, float* y, hipStream_t s) {
-	if (n == 0) return 0;
-	hipLaunchKernelGGL(k_f64_to_f32, grid(n), dim3(kBlock), 0, s, x, n, y);
-	return sf_hip_check(hipGetLastError(), "sfd_f64_to_f32", "launch");
+int sfd_adjoint_begin(const float* gx, const float* gv, const float* x, unsigned N, unsigned n_pad, float coef,
+                      int acc_phys, float* lx, float* lv, float* body, float* nu, hipStream_t s) {
+	hipLaunchKernelGGL(k_adjoint_begin, grid(n_pad), dim3(kBlock), 0, s, gx, gv, x, N, n_pad, coef, acc_phys, lx, lv,
+	                   reinterpret_cast<float4*>(body), reinterpret_cast<float4*>(nu));
+	return sf_hip_check(hipGetLastError(), "sfd_adjoint_begin", "launch");
 }
 
 int sfd_fill0(float* y, unsigned n, hipStream_t s) {

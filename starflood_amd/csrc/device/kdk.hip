@@ -54,33 +54,24 @@ __global__ __launch_bounds__(kBlock) void k_x64_refresh(const float* __restrict_
 	if ((float)x64[k] != p) x64[k] = (double)p;
 }
 
-// refresh: first apply k_x64_refresh's rule to x64 (a caller that always
-// writes pos from x64 passes 0)
+// k_x64_refresh's rule first, then kick and drift
 __global__ __launch_bounds__(kBlock) void k_kick_drift_fast(float* __restrict__ vel, const float* __restrict__ acc,
                                                             double* __restrict__ x64, float* __restrict__ pos,
-                                                            unsigned n3, float half_dt, double dt, int refresh) {
+                                                            unsigned n3, float half_dt, double dt) {
 	const unsigned k = blockIdx.x * kBlock + threadIdx.x;
 	if (k >= n3) return;
 	const float v = __builtin_fmaf(half_dt, acc[k], vel[k]);
 	vel[k] = v;
 	double x0 = x64[k];
-	if (refresh) {
-		const float p = pos[k];
-		if ((float)x0 != p) x0 = (double)p;
-	}
+	const float p = pos[k];
+	if ((float)x0 != p) x0 = (double)p;
 	const double x = __builtin_fma(dt, (double)v, x0);
 	x64[k] = x;
 	pos[k] = (float)x;
 }
 
-__global__ __launch_bounds__(kBlock) void k_kick_fast(float* __restrict__ vel, const float* __restrict__ acc,
-                                                      unsigned n3, float half_dt) {
-	const unsigned k = blockIdx.x * kBlock + threadIdx.x;
-	if (k < n3) vel[k] = __builtin_fmaf(half_dt, acc[k], vel[k]);
-}
-
-// k_kick_fast followed by k_energy_terms, per particle, with the same
-// operations: one pass over vel instead of two launches.
+// The closing kick followed by k_energy_terms, per particle: one pass over
+// vel instead of two launches.
 __global__ __launch_bounds__(kBlock) void k_kick_energy_fast(float* __restrict__ vel, const float* __restrict__ acc,
                                                              const float* __restrict__ mas,
                                                              const float* __restrict__ pot, unsigned N, float half_dt,
@@ -206,11 +197,11 @@ extern "C" int sfd_x64_refresh(const float* pos, double* x64, unsigned n3, hipSt
 }
 
 extern "C" int sfd_kick_drift_fast(float* vel, const float* acc, double* x64, float* pos, unsigned n3,
-                                   float half_dt, double dt, int refresh, hipStream_t s) {
+                                   float half_dt, double dt, hipStream_t s) {
 	if (!n3) return 0;
 	const int tok = sf_prof_begin("kick_drift", s);
 	hipLaunchKernelGGL(k_kick_drift_fast, dim3(grid_for(n3)), dim3(kBlock), 0, s, vel, acc, x64, pos, n3, half_dt,
-	                   dt, refresh);
+	                   dt);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_kick_drift_fast", "launch");
 }
@@ -223,14 +214,6 @@ extern "C" int sfd_kick_energy_fast(float* vel, const float* acc, const float* m
 	                   pen);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_kick_energy_fast", "launch");
-}
-
-extern "C" int sfd_kick_fast(float* vel, const float* acc, unsigned n3, float half_dt, hipStream_t s) {
-	if (!n3) return 0;
-	const int tok = sf_prof_begin("kick", s);
-	hipLaunchKernelGGL(k_kick_fast, dim3(grid_for(n3)), dim3(kBlock), 0, s, vel, acc, n3, half_dt);
-	sf_prof_end(tok, s);
-	return sf_hip_check(hipGetLastError(), "sfd_kick_fast", "launch");
 }
 
 extern "C" unsigned sfd_reduce_scratch_doubles(unsigned N) {

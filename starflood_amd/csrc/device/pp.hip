@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "force_epi.h"
 #include "order_chain.h"
 #include "pp_sym.h"
 
@@ -292,10 +293,10 @@ __global__ __launch_bounds__(kBlock) void k_pp_fast(const float4* __restrict__ b
 // left most CUs idle at small N (64 blocks at N = 16384: 20 us).
 constexpr unsigned kCombI = 64;
 constexpr unsigned kCombG = kBlock / kCombI;
+template <class E>
 __global__ __launch_bounds__(kBlock) void k_pp_combine(const double4* __restrict__ part, unsigned n_pad,
-                                                       unsigned slices, const float4* __restrict__ body,
-                                                       unsigned N, double G, int acc_phys,
-                                                       float* __restrict__ acc, float* __restrict__ pot) {
+                                                       unsigned slices, float4* body, unsigned N, double G,
+                                                       int acc_phys, E epi) {
 	__shared__ double red[kCombG][4][kCombI];
 	const unsigned il = threadIdx.x % kCombI, g = threadIdx.x / kCombI;
 	const unsigned i = blockIdx.x * kCombI + il;   // < n_pad: the grid covers N in kCombI steps
@@ -321,45 +322,62 @@ __global__ __launch_bounds__(kBlock) void k_pp_combine(const double4* __restrict
 	}
 	// sum_j m_j (r_j - r_i)/s^3 = -sum_j m_j r_ij/s^3, so acc = G (m_i) * sum
 	const double f = acc_phys ? G : G * (double)body[i].w;
-	acc[3u * i + 0u] = (float)(f * sx);
-	acc[3u * i + 1u] = (float)(f * sy);
-	acc[3u * i + 2u] = (float)(f * sz);
-	if (pot) pot[i] = (float)(-G * sp);
+	epi(i, (float)(f * sx), (float)(f * sy), (float)(f * sz), (float)(-G * sp), body);
 }
 
-// Packs (x, y, z, m) per body, padding with zeros to n_pad, and finds
-// whether every mass has the bits of mas[0].  st[0] receives n_uni, the
-// whole SF_TJ tiles of [0, N) when they do, else 0 (padding bodies, mass 0,
-// are never in a uniform tile).  st[1] collects the blocks' differing-mass
-// flags and st[2] counts finished blocks; the last block to finish writes
-// st[0] and returns both to zero (atomicInc wraps at gridDim.x - 1), so
-// they start at zero on the next call without a clear.  The grid is capped
-// at kPackBlocks and strides over the bodies: the atomics on st[2] serialise
-// (one per block of 1024 measured 26 us at N = 262144).
-constexpr unsigned kPackBlocks = 128;
-__global__ __launch_bounds__(kBlock) void k_pack_bodies(const float* __restrict__ pos, const float* __restrict__ mas,
-                                                        unsigned N, unsigned n_pad, float4* __restrict__ body,
-                                                        unsigned* __restrict__ st) {
-	const unsigned m0 = N ? __float_as_uint(mas[0]) : 0u;
-	int d = 0;
-	for (unsigned i = blockIdx.x * kBlock + threadIdx.x; i < n_pad; i += gridDim.x * kBlock) {
-		if (i < N) {
-			const float m = mas[i];
-			body[i] = make_float4(pos[3u * i], pos[3u * i + 1u], pos[3u * i + 2u], m);
-			d |= __float_as_uint(m) != m0;
-		} else {
-			body[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-		}
-	}
+// The state words of the packed bodies (see pack_state): every mass has the
+// bits of mas[0] unless d; st[0] receives n_uni, the whole SF_TJ tiles of [0, N)
+// when they all do, else 0 (padding bodies, mass 0, are never in a uniform
+// tile).  st[1] collects the blocks' differing-mass flags and st[2] counts
+// finished blocks; the last block to finish writes st[0] and returns both to
+// zero (atomicInc wraps at gridDim.x - 1), so they start at zero on the next
+// call without a clear.  Only k_pp_fast and k_vjp read n_uni, below kSymMin
+// bodies (at most 36 blocks; the atomics on st[2] serialise: 1024 blocks
+// took 26 us).
+__device__ __forceinline__ void pack_state(int d, unsigned N, unsigned* __restrict__ st) {
 	d = __syncthreads_or(d);
-	if (threadIdx.x == 0) {
-		if (d) atomicOr(&st[1], 1u);
-		__threadfence();
-		if (atomicInc(&st[2], gridDim.x - 1u) == gridDim.x - 1u) {
-			const unsigned any = atomicExch(&st[1], 0u);
-			st[0] = any ? 0u : N / SF_TJ * SF_TJ;
-		}
+	if (threadIdx.x != 0) return;
+	if (d) atomicOr(&st[1], 1u);
+	__threadfence();
+	if (atomicInc(&st[2], gridDim.x - 1u) == gridDim.x - 1u) {
+		const unsigned any = atomicExch(&st[1], 0u);
+		st[0] = any ? 0u : N / SF_TJ * SF_TJ;
 	}
+}
+
+// Packs (x, y, z, m) per body, padding with zeros to n_pad.  STATE: below
+// kSymMin bodies.  KICK: first the opening kick and drift of the fast step,
+// with k_kick_drift_fast's operations (x64 restarts from pos where they differ).
+template <bool STATE, bool KICK>
+__global__ __launch_bounds__(kBlock) void k_pack_bodies(float* __restrict__ vel, const float* __restrict__ acc,
+                                                        double* __restrict__ x64, float* __restrict__ pos,
+                                                        const float* __restrict__ mas, unsigned N, unsigned n_pad,
+                                                        float half_dt, double dt, float4* __restrict__ body,
+                                                        unsigned* __restrict__ st) {
+	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+	int d = 0;
+	if (i < N) {
+		float p[3] = {pos[3u * i], pos[3u * i + 1u], pos[3u * i + 2u]};
+		if (KICK) {
+#pragma unroll
+			for (unsigned k = 0; k < 3u; ++k) {
+				const float v = __builtin_fmaf(half_dt, acc[3u * i + k], vel[3u * i + k]);
+				double x0 = x64[3u * i + k];
+				if ((float)x0 != p[k]) x0 = (double)p[k];
+				const double x = __builtin_fma(dt, (double)v, x0);
+				vel[3u * i + k] = v;
+				x64[3u * i + k] = x;
+				p[k] = (float)x;
+				pos[3u * i + k] = p[k];
+			}
+		}
+		const float m = mas[i];
+		body[i] = make_float4(p[0], p[1], p[2], m);
+		if (STATE) d = __float_as_uint(m) != __float_as_uint(mas[0]);
+	} else if (i < n_pad) {
+		body[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	}
+	if (STATE) pack_state(d, N, st);
 }
 
 // FP64 direct sum: one block per listed particle, lanes stride over j, then
@@ -409,13 +427,27 @@ __global__ __launch_bounds__(kBlock) void k_pp_f64(const float* __restrict__ pos
 
 }  // namespace
 
+template <bool KICK>
+static void launch_pack(float* vel, const float* acc, double* x64, float* pos, const float* mas, unsigned N,
+                        unsigned n_pad, float half_dt, double dt, float* body, hipStream_t s) {
+	unsigned* st = reinterpret_cast<unsigned*>(body + 4u * (size_t)n_pad);
+	auto k = n_pad < kSymMin ? k_pack_bodies<true, KICK> : k_pack_bodies<false, KICK>;
+	hipLaunchKernelGGL(k, dim3((n_pad + kBlock - 1) / kBlock), dim3(kBlock), 0, s, vel, acc, x64, pos, mas, N, n_pad,
+	                   half_dt, dt, reinterpret_cast<float4*>(body), st);
+}
+
 extern "C" int sfd_pack_bodies(const float* pos, const float* mas, unsigned N, unsigned n_pad, float* body,
                                hipStream_t s) {
-	const unsigned grid = min((n_pad + kBlock - 1) / kBlock, kPackBlocks);
-	unsigned* st = reinterpret_cast<unsigned*>(body + 4u * (size_t)n_pad);
-	hipLaunchKernelGGL(k_pack_bodies, dim3(grid), dim3(kBlock), 0, s, pos, mas, N, n_pad,
-	                   reinterpret_cast<float4*>(body), st);
+	launch_pack<false>(nullptr, nullptr, nullptr, const_cast<float*>(pos), mas, N, n_pad, 0.0f, 0.0, body, s);
 	return sf_hip_check(hipGetLastError(), "sfd_pack_bodies", "k_pack_bodies launch");
+}
+
+extern "C" int sfd_kick_drift_pack(float* vel, const float* acc, double* x64, float* pos, const float* mas, unsigned N,
+                                   unsigned n_pad, float half_dt, double dt, float* body, hipStream_t s) {
+	const int tok = sf_prof_begin("kick_drift", s);
+	launch_pack<true>(vel, acc, x64, pos, mas, N, n_pad, half_dt, dt, body, s);
+	sf_prof_end(tok, s);
+	return sf_hip_check(hipGetLastError(), "sfd_kick_drift_pack", "k_pack_bodies launch");
 }
 
 extern "C" int sfd_pp_exact(const float* pos, const float* mas, unsigned N, float eps2, float negG, int acc_phys,
@@ -456,34 +488,44 @@ extern "C" size_t sfd_pp_part_bytes(unsigned n_pad, unsigned slices) {
 }
 
 // device/pp_sym.hip
-extern "C" int sfd_pp_sym(const float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys,
-                          float* part, float* acc, float* pot, hipStream_t s);
+extern "C" int sfd_pp_sym(float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys, float* part,
+                          const sf_force_epi* epi, hipStream_t s);
 
-extern "C" int sfd_pp_fast(const float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys,
-                           float* part, unsigned slices, float* acc, float* pot, hipStream_t s) {
+extern "C" int sfd_pp_fast(float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys, float* part,
+                           unsigned slices, const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
 	if (n_pad % 64u != 0 || n_pad % SF_TJ != 0) {
 		sf_error("sfd_pp_fast", "n_pad %u is not a multiple of %u", n_pad, SF_TJ);
 		return -1;
 	}
 	// part holds sfd_pp_part_bytes(n_pad, slices)
-	if (n_pad >= kSymMin) return sfd_pp_sym(body, N, n_pad, eps2, G, acc_phys, part, acc, pot, s);
+	if (n_pad >= kSymMin) return sfd_pp_sym(body, N, n_pad, eps2, G, acc_phys, part, epi, s);
 	// one double4 plane per block slice
 	const PPGeometry g = pp_geometry(n_pad, slices);
 	const unsigned grid = (n_pad / 64u) * g.bslices;
 	double4* p4 = reinterpret_cast<double4*>(part);
-	const float4* b4 = reinterpret_cast<const float4*>(body);
+	float4* b4 = reinterpret_cast<float4*>(body);
+	const bool with_pot = epi->kind == SF_EPI_KICK || (epi->kind == SF_EPI_STORE && epi->pot);
 	const int tok = sf_prof_begin("pp_fast", s);
-	if (pot)
-		hipLaunchKernelGGL(k_pp_fast<true>, dim3(grid), dim3(kBlock), 0, s, b4, n_pad, g.bslices, g.sub_len, eps2, p4);
-	else
-		hipLaunchKernelGGL(k_pp_fast<false>, dim3(grid), dim3(kBlock), 0, s, b4, n_pad, g.bslices, g.sub_len, eps2,
-		                   p4);
+	hipLaunchKernelGGL(with_pot ? k_pp_fast<true> : k_pp_fast<false>, dim3(grid), dim3(kBlock), 0, s, b4, n_pad,
+	                   g.bslices, g.sub_len, eps2, p4);
 	sf_prof_end(tok, s);
 	if (sf_hip_check(hipGetLastError(), "sfd_pp_fast", "k_pp_fast launch")) return -1;
+	const dim3 cgrid((N + kCombI - 1) / kCombI);
 	const int tok2 = sf_prof_begin("pp_combine", s);
-	hipLaunchKernelGGL(k_pp_combine, dim3((N + kCombI - 1) / kCombI), dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4,
-	                   N, G, acc_phys, acc, pot);
+	switch (epi->kind) {
+	case SF_EPI_KICK:
+		hipLaunchKernelGGL(k_pp_combine<EpiKick>, cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4, N, G, acc_phys,
+		                   EpiKick(*epi));
+		break;
+	case SF_EPI_KDK:
+		hipLaunchKernelGGL(k_pp_combine<EpiKdk>, cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4, N, G, acc_phys,
+		                   EpiKdk(*epi));
+		break;
+	default:
+		hipLaunchKernelGGL(k_pp_combine<EpiStore>, cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4, N, G, acc_phys,
+		                   EpiStore(*epi));
+	}
 	sf_prof_end(tok2, s);
 	return sf_hip_check(hipGetLastError(), "sfd_pp_fast", "k_pp_combine launch");
 }

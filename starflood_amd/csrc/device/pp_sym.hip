@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "force_epi.h"
 #include "pp_sym.h"
 
 namespace {
@@ -68,6 +69,13 @@ struct Set {
 			m[k] = b.w;
 		}
 		clear();
+	}
+	// every mass of the wavefront's i has the bits of mu
+	__device__ __forceinline__ bool all_mass(float mu) const {
+		bool d = false;
+#pragma unroll
+		for (int k = 0; k < kPer; ++k) d |= __float_as_uint(m[k]) != __float_as_uint(mu);
+		return __ballot(d) == 0ull;
 	}
 };
 
@@ -155,13 +163,14 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 	Set a;
 	a.load(body, i0);
 	float sum[kPer][4], com[kPer][4];
+	bool pending = false, was_uni = false;   // plain sums not yet folded, and their kind
 #pragma unroll
 	for (int k = 0; k < kPer; ++k)
 #pragma unroll
 		for (int u = 0; u < 4; ++u) sum[k][u] = com[k][u] = 0.0f;
-	const unsigned n_uni = *reinterpret_cast<const unsigned*>(body + n_pad);
-	const bool i_uni = (ib + 1u) * kSymWide <= n_uni;
 	const float mu = body[0].w;
+	// one answer for the block: its wavefronts' j sums are added before they are scaled
+	const bool i_uni = !__syncthreads_or(!a.all_mass(mu));
 	for (unsigned u = t; u < 2u * kWaves * 2u * kSymTile; u += kBlock)
 		(&s_acc[0][0][0])[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	if (t < kSymTile && t0 < t1) {
@@ -170,6 +179,18 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 		s_j[0][t + kSymTile] = v;
 	}
 	__syncthreads();
+	auto fold = [&](bool uni) {
+		const float sc = uni ? mu : 1.0f;
+#pragma unroll
+		for (int k = 0; k < kPer; ++k) {
+			kahan_add(sum[k][0], com[k][0], sc * a.tx[k]);
+			kahan_add(sum[k][1], com[k][1], sc * a.ty[k]);
+			kahan_add(sum[k][2], com[k][2], sc * a.tz[k]);
+			if (POT) kahan_add(sum[k][3], com[k][3], sc * a.tp[k]);
+		}
+		a.clear();
+		pending = false;
+	};
 	unsigned buf = 0u;
 	for (unsigned tt = t0; tt < t1; tt += kSymTile) {
 		// the next tile, in flight during this one's arithmetic (past the
@@ -178,7 +199,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 		if (jn >= n_pad) jn -= n_pad;
 		float4 nv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 		if (t < kSymTile) nv = body[jn + t];
-		const bool uni = i_uni && j + kSymTile <= n_uni;
+		const bool uni = i_uni && __ballot(__float_as_uint(s_j[buf][lane].w) != __float_as_uint(mu)) == 0ull;
+		if (pending && uni != was_uni) fold(was_uni);
+		was_uni = uni;
 		if (sym) {
 			if (uni) sym_tile<POT, true, true>(s_j[buf], s_acc[buf][wv], lane, eps2, a);
 			else sym_tile<POT, false, true>(s_j[buf], s_acc[buf][wv], lane, eps2, a);
@@ -206,22 +229,13 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 			const double sc = uni ? (double)mu : 1.0;
 			part_j[((size_t)(tt / kSymWide) * n_pad + j) * 4u + t] = (float)(comp < 3u ? -sc * s : sc * s);
 		}
-		// fold the i sums at every 128 bodies: n_uni is a multiple of 128, so
-		// the tiles of one fold are all uniform or all not
-		if ((j & kSymTile) || tt + kSymTile >= t1) {
-			const float sc = uni ? mu : 1.0f;
-#pragma unroll
-			for (int k = 0; k < kPer; ++k) {
-				kahan_add(sum[k][0], com[k][0], sc * a.tx[k]);
-				kahan_add(sum[k][1], com[k][1], sc * a.ty[k]);
-				kahan_add(sum[k][2], com[k][2], sc * a.tz[k]);
-				if (POT) kahan_add(sum[k][3], com[k][3], sc * a.tp[k]);
-			}
-			a.clear();
-		}
+		// fold the i sums after two tiles of one kind
+		pending = !pending;
+		if (!pending) fold(uni);
 		buf ^= 1u;
 		j = jn;
 	}
+	if (pending) fold(was_uni);
 	const unsigned plane = sym ? c : chunks + c;
 #pragma unroll
 	for (int k = 0; k < kPer; ++k)   // Kahan's compensation holds the negated lost low part
@@ -261,9 +275,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const float4* __res
 	Set a;
 	a.load(body, ib * kSymNarrow + lane);
 	const float4 v = body[j + lane], zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-	const unsigned n_uni = *reinterpret_cast<const unsigned*>(body + n_pad);
-	const bool uni = (ib + 1u) * kSymNarrow <= n_uni && j + kSymTile <= n_uni;
 	const float mu = body[0].w;
+	const bool uni = a.all_mass(mu) && __ballot(__float_as_uint(v.w) != __float_as_uint(mu)) == 0ull;
 	float4* sj = s_mem[wv];
 	float4* acc = sj + 2u * kSymTile;
 	sj[lane] = sj[lane + kSymTile] = v;
@@ -305,12 +318,11 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const float4* __res
 // kept there or, at the last launch, written to acc and pot.  A block takes
 // 64 particles; its wavefronts take every fourth plane each.
 constexpr unsigned kCombI = 64;
+template <class E>
 __global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict__ part, unsigned n_pad,
                                                         unsigned planes, unsigned S, int last_offset, int first,
-                                                        int last, double4* __restrict__ run,
-                                                        const float4* __restrict__ body, unsigned N, double G,
-                                                        int acc_phys, float* __restrict__ acc,
-                                                        float* __restrict__ pot) {
+                                                        int last, double4* __restrict__ run, float4* body,
+                                                        unsigned N, double G, int acc_phys, E epi) {
 	__shared__ double red[kWaves][4][kCombI];
 	const unsigned il = threadIdx.x % kCombI, g = threadIdx.x / kCombI;
 	const unsigned i = blockIdx.x * kCombI + il;   // < n_pad: the grid covers N in kCombI steps
@@ -349,18 +361,31 @@ __global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict
 		return;
 	}
 	const double f = acc_phys ? G : G * (double)body[i].w;
-	acc[3u * i + 0u] = (float)(f * sx);
-	acc[3u * i + 1u] = (float)(f * sy);
-	acc[3u * i + 2u] = (float)(f * sz);
-	if (pot) pot[i] = (float)(-G * sp);
+	epi(i, (float)(f * sx), (float)(f * sy), (float)(f * sz), (float)(-G * sp), body);
+}
+
+struct CombineArgs {
+	const float4* part;
+	unsigned n_pad, planes, S;
+	int first, last;
+	double4* run;
+	float4* body;
+	unsigned N;
+	double G;
+	int acc_phys;
+};
+template <class E>
+void launch_combine(const CombineArgs& c, const sf_force_epi& epi, hipStream_t s) {
+	hipLaunchKernelGGL(k_sym_combine<E>, dim3((c.N + kCombI - 1u) / kCombI), dim3(kBlock), 0, s, c.part, c.n_pad,
+	                   c.planes, c.S, c.last, c.first, c.last, c.run, c.body, c.N, c.G, c.acc_phys, E(epi));
 }
 
 }  // namespace
 
-// acc and (unless NULL) pot from n_pad packed bodies (a multiple of 1024, at
-// least 2048); part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad)).
-extern "C" int sfd_pp_sym(const float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys,
-                          float* part, float* acc, float* pot, hipStream_t s) {
+// The force of n_pad packed bodies (a multiple of 1024, at least 2048), ended
+// by *epi; part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad)).
+extern "C" int sfd_pp_sym(float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys, float* part,
+                          const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
 	if (n_pad % kSymWide != 0 || n_pad < 2u * kSymWide || N > n_pad) {
 		sf_error("sfd_pp_sym", "n_pad %u does not fit N = %u", n_pad, N);
@@ -368,7 +393,8 @@ extern "C" int sfd_pp_sym(const float* body, unsigned N, unsigned n_pad, float e
 	}
 	const bool wide = sym_pp_wide(n_pad);
 	const SymGeometry g = sym_geometry(n_pad, wide);
-	const float4* b4 = reinterpret_cast<const float4*>(body);
+	float4* b4 = reinterpret_cast<float4*>(body);
+	const bool pot = epi->kind == SF_EPI_KICK || (epi->kind == SF_EPI_STORE && epi->pot);
 	float4* p4 = reinterpret_cast<float4*>(part);
 	double4* run = reinterpret_cast<double4*>(p4 + ((size_t)g.chunks + g.dchunks + g.per_launch) * n_pad);
 	for (unsigned d0 = 0; d0 < g.offsets; d0 += g.per_launch) {
@@ -391,8 +417,10 @@ extern "C" int sfd_pp_sym(const float* body, unsigned N, unsigned n_pad, float e
 		sf_prof_end(tok, s);
 		if (sf_hip_check(hipGetLastError(), "sfd_pp_sym", "k_pp_sym launch")) return -1;
 		const int tok2 = sf_prof_begin("pp_combine", s);
-		hipLaunchKernelGGL(k_sym_combine, dim3((N + kCombI - 1u) / kCombI), dim3(kBlock), 0, s, p4, n_pad,
-		                   pi + (d1 - d0), g.blocks, last, first, last, run, b4, N, G, acc_phys, acc, pot);
+		const CombineArgs ca{p4, n_pad, pi + (d1 - d0), g.blocks, first, last, run, b4, N, G, acc_phys};
+		if (epi->kind == SF_EPI_KICK) launch_combine<EpiKick>(ca, *epi, s);
+		else if (epi->kind == SF_EPI_KDK) launch_combine<EpiKdk>(ca, *epi, s);
+		else launch_combine<EpiStore>(ca, *epi, s);
 		sf_prof_end(tok2, s);
 		if (sf_hip_check(hipGetLastError(), "sfd_pp_sym", "k_sym_combine launch")) return -1;
 	}

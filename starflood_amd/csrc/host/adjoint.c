@@ -23,13 +23,16 @@
 #include "sf_host.h"
 
 /* kernels in device/adjoint.hip */
-int sfd_force_vjp(const float* body, const float* mas, const float* mu, unsigned int N, unsigned int n_pad,
-                  float eps2, double G, int acc_phys, float coef, float* nu, float* part, unsigned int slices,
-                  int accumulate, float* g, hipStream_t s);
+int sfd_pack_nu(const float* mu, const float* mas, unsigned int N, unsigned int n_pad, float coef, int acc_phys,
+                float* nu, hipStream_t s);
+int sfd_force_vjp(const float* body, const float* nu, unsigned int N, unsigned int n_pad, float eps2, double G,
+                  float* part, unsigned int slices, const sf_vjp_epi* epi, hipStream_t s);
 size_t sfd_vjp_part_bytes(unsigned int n_pad, unsigned int slices);
-int sfd_axpy(float* y, const float* x, unsigned int n, float a, hipStream_t s);
-int sfd_f32_to_f64(const float* x, unsigned int n, double* y, hipStream_t s);
-int sfd_f64_to_f32(const double* x, unsigned int n, float* y, hipStream_t s);
+int sfd_adjoint_init(const float* x0, const float* v0, unsigned int N, double* x64, float* v, float* x, hipStream_t s);
+int sfd_adjoint_reopen(const double* ck_x64, const float* ck_v, const float* ck_a, unsigned int N, float h, double dt,
+                       int steps, double* x64, float* v, float* x, float* body, hipStream_t s);
+int sfd_adjoint_begin(const float* gx, const float* gv, const float* x, unsigned int N, unsigned int n_pad, float coef,
+                      int acc_phys, float* lx, float* lv, float* body, float* nu, hipStream_t s);
 int sfd_fill0(float* y, unsigned int n, hipStream_t s);
 
 /* device scratch for one N: packed bodies, VJP weights, slice partials */
@@ -73,30 +76,21 @@ static int scratch_alloc(sf_pp_scratch* w, unsigned int N, const char* func) {
 
 static float eps2_of(const sf_params_t* p) { return (float)(p->epsilon * p->epsilon); }
 
-static int force(const sf_params_t* p, sf_pp_scratch* w, const float* x, const float* m, float* acc, float* pot,
-                 hipStream_t s) {
-	return sf_pp_force_arrays(p, w->N, w->n_pad, x, m, w->body, w->part, w->part_bytes, acc, pot, s);
-}
-
-/* g (=, or += when accumulate) J(x)^T (coef mu) */
-static int vjp(const sf_params_t* p, sf_pp_scratch* w, const float* x, const float* m, const float* mu, float coef,
-               int accumulate, float* g, hipStream_t s) {
-	if (sfd_pack_bodies(x, m, w->N, w->n_pad, w->body, s)) return -1;
-	return sfd_force_vjp(w->body, m, mu, w->N, w->n_pad, eps2_of(p), p->G, p->acc_mode == SF_ACC_PHYSICAL, coef, w->nu,
-	                     w->part, w->slices, accumulate, g, s);
+/* the VJP at the packed bodies and nu of w */
+static int vjp(const sf_params_t* p, sf_pp_scratch* w, const sf_vjp_epi* epi, hipStream_t s) {
+	return sfd_force_vjp(w->body, w->nu, w->N, w->n_pad, eps2_of(p), p->G, w->part, w->slices, epi, s);
 }
 
 struct sf_tape {
 	sf_params_t p;              /* epsilon, G, dt, acc_mode at the forward call */
 	unsigned int N, nsteps, ckpt, n_ckpt, last_start;
-	sf_pp_scratch w;
-	float* m;                   /* N (copy) */
+	sf_pp_scratch w;            /* its bodies keep the masses of the forward call */
 	double* ck_x64;             /* n_ckpt x 3N */
 	float* ck_v;                /* n_ckpt x 3N */
 	float* ck_a;                /* n_ckpt x 3N */
 	float* seg;                 /* (ckpt + 1) x 3N positions of one segment */
 	unsigned int seg_first;     /* step of seg[0] */
-	float *x, *v, *a, *lx, *lv; /* 3N each */
+	float *v, *lx, *lv;         /* 3N each */
 	double* x64;                /* 3N */
 	hipStream_t stream;         /* the stream of the tape's last call */
 	hipEvent_t done;            /* recorded there by sf_tape_free */
@@ -105,7 +99,7 @@ struct sf_tape {
 
 /* Device memory of a tape, released (hipFree waits for the device). */
 static void tape_release(sf_tape* t) {
-	void* ptrs[] = {t->m, t->ck_x64, t->ck_v, t->ck_a, t->seg, t->x, t->v, t->a, t->lx, t->lv, t->x64};
+	void* ptrs[] = {t->ck_x64, t->ck_v, t->ck_a, t->seg, t->v, t->lx, t->lv, t->x64};
 	for (size_t k = 0; k < sizeof(ptrs) / sizeof(ptrs[0]); ++k)
 		if (ptrs[k]) hipFree(ptrs[k]);
 	scratch_free(&t->w);
@@ -134,13 +128,16 @@ void sf_tape_free(sf_tape* t) {
    PyTorch's default stream, so work stays ordered with the caller's */
 static hipStream_t stream_of(void* stream) { return (hipStream_t)stream; }
 
-/* one KDK step from (x64, x, v, a) in place; a is the force at x on entry */
-static int kdk(sf_tape* t, hipStream_t s) {
-	const unsigned int n3 = 3u * t->N;
-	const float h = 0.5f * (float)t->p.dt;
-	if (sfd_kick_drift_fast(t->v, t->a, t->x64, t->x, n3, h, t->p.dt, 0, s)) return -1;
-	if (force(&t->p, &t->w, t->x, t->m, t->a, NULL, s)) return -1;
-	return sfd_kick_fast(t->v, t->a, n3, h, s);
+/* The force at the packed bodies (x_n), which ends one step and opens the
+   next (device/force_epi.h): one launch with the integration in its combine
+   where the kicks, the drift, the packing and the copies took five. */
+static int kdk(sf_tape* t, sf_force_epi* e, hipStream_t s) {
+	e->kind = SF_EPI_KDK;
+	e->h = 0.5f * (float)t->p.dt;
+	e->dt = t->p.dt;
+	e->v = t->v;
+	e->x64 = t->x64;
+	return sf_pp_force_packed(&t->p, t->w.N, t->w.n_pad, t->w.body, t->w.part, t->w.part_bytes, e, s);
 }
 
 static int forward_run(sf_tape* t, const float* x0, const float* v0, const float* m, float* xN, float* vN,
@@ -183,14 +180,11 @@ int sf_adjoint_forward(unsigned int N, const float* x0, const float* v0, const f
 	t->last_start = t->n_ckpt ? (t->n_ckpt - 1u) * t->ckpt : 0u;
 	t->have_done = hipEventCreateWithFlags(&t->done, hipEventDisableTiming) == hipSuccess;
 	int rc = scratch_alloc(&t->w, N, fn);
-	rc |= hipMalloc((void**)&t->m, (size_t)N * sizeof(float)) != hipSuccess;
 	rc |= hipMalloc((void**)&t->ck_x64, (t->n_ckpt ? t->n_ckpt : 1u) * n3 * sizeof(double)) != hipSuccess;
 	rc |= hipMalloc((void**)&t->ck_v, (t->n_ckpt ? t->n_ckpt : 1u) * f3) != hipSuccess;
 	rc |= hipMalloc((void**)&t->ck_a, (t->n_ckpt ? t->n_ckpt : 1u) * f3) != hipSuccess;
 	rc |= hipMalloc((void**)&t->seg, (t->ckpt + 1u) * f3) != hipSuccess;
-	rc |= hipMalloc((void**)&t->x, f3) != hipSuccess;
 	rc |= hipMalloc((void**)&t->v, f3) != hipSuccess;
-	rc |= hipMalloc((void**)&t->a, f3) != hipSuccess;
 	rc |= hipMalloc((void**)&t->lx, f3) != hipSuccess;
 	rc |= hipMalloc((void**)&t->lv, f3) != hipSuccess;
 	rc |= hipMalloc((void**)&t->x64, n3 * sizeof(double)) != hipSuccess;
@@ -213,32 +207,30 @@ static int forward_run(sf_tape* t, const float* x0, const float* v0, const float
 	const unsigned int N = t->N, nsteps = t->nsteps;
 	const size_t n3 = 3u * (size_t)N, f3 = n3 * sizeof(float);
 	int rc = 0;
-	rc |= hipMemcpyAsync(t->m, m, (size_t)N * sizeof(float), hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= hipMemcpyAsync(t->x, x0, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= hipMemcpyAsync(t->v, v0, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= sfd_f32_to_f64(t->x, (unsigned int)n3, t->x64, s);
-	const int tok = sf_prof_begin("adjoint_forward", s);
-	rc |= force(&t->p, &t->w, t->x, t->m, t->a, NULL, s);
-	for (unsigned int n = 0; n < nsteps && !rc; ++n) {
-		if (n % t->ckpt == 0u) {
-			const size_t c = n / t->ckpt;
-			rc |= hipMemcpyAsync(t->ck_x64 + c * n3, t->x64, n3 * sizeof(double), hipMemcpyDeviceToDevice, s) !=
-			      hipSuccess;
-			rc |= hipMemcpyAsync(t->ck_v + c * n3, t->v, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-			rc |= hipMemcpyAsync(t->ck_a + c * n3, t->a, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-		}
-		if (n >= t->last_start)
-			rc |= hipMemcpyAsync(t->seg + (n - t->last_start) * n3, t->x, f3, hipMemcpyDeviceToDevice, s) !=
-			      hipSuccess;
-		rc |= kdk(t, s);
-	}
-	if (nsteps && !rc)
-		rc |= hipMemcpyAsync(t->seg + (nsteps - t->last_start) * n3, t->x, f3, hipMemcpyDeviceToDevice, s) !=
-		      hipSuccess;
-	sf_prof_end(tok, s);
+	rc |= sfd_adjoint_init(x0, v0, N, t->x64, t->v, t->last_start == 0u ? t->seg : NULL, s);
+	rc |= sfd_pack_bodies(x0, m, N, t->w.n_pad, t->w.body, s);
 	t->seg_first = t->last_start;
-	rc |= hipMemcpyAsync(xN, t->x, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= hipMemcpyAsync(vN, t->v, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
+	const int tok = sf_prof_begin("adjoint_forward", s);
+	for (unsigned int n = 0; n <= nsteps && nsteps && !rc; ++n) {
+		sf_force_epi e = {.close = n > 0u, .open = n < nsteps};
+		if (e.open && n % t->ckpt == 0u) {
+			const size_t c = n / t->ckpt;
+			e.ck_x64 = t->ck_x64 + c * n3;
+			e.ck_v = t->ck_v + c * n3;
+			e.ck_a = t->ck_a + c * n3;
+		}
+		if (e.open && n + 1u >= t->last_start) e.x = t->seg + (n + 1u - t->last_start) * n3;
+		if (!e.open) {
+			e.xN = xN;
+			e.vN = vN;
+		}
+		rc |= kdk(t, &e, s);
+	}
+	sf_prof_end(tok, s);
+	if (nsteps == 0u) {
+		rc |= hipMemcpyAsync(xN, t->seg, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
+		rc |= hipMemcpyAsync(vN, t->v, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
+	}
 	if (rc || sf_hip_check(hipGetLastError(), fn, "launch")) {
 		sf_error(fn, "forward integration failed");
 		return -1;
@@ -249,23 +241,19 @@ static int forward_run(sf_tape* t, const float* x0, const float* v0, const float
 /* The positions of segment c that the backward reads, into t->seg:
    x_{start} .. x_{start+len-1}, and x_{start+len} too for the last segment.
    Only the last segment reads its end position, so the others take len - 1
-   steps (none with a checkpoint every step).  The forward leaves the last
+   steps (none with a checkpoint every step), and no force is needed at the
+   last position; the packed bodies hold it in the end.  The forward leaves the last
    segment on the tape; it is recomputed only when the tape's backward runs
    again. */
 static int recompute(sf_tape* t, unsigned int c, unsigned int len, hipStream_t s) {
-	const size_t n3 = 3u * (size_t)t->N, f3 = n3 * sizeof(float);
+	const size_t n3 = 3u * (size_t)t->N;
 	const unsigned int steps = c + 1u == t->n_ckpt ? len : len - 1u;
-	int rc = 0;
 	t->seg_first = c * t->ckpt;
-	if (steps == 0u) return sfd_f64_to_f32(t->ck_x64 + c * n3, (unsigned int)n3, t->seg, s);
-	rc |= hipMemcpyAsync(t->x64, t->ck_x64 + c * n3, n3 * sizeof(double), hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= hipMemcpyAsync(t->v, t->ck_v + c * n3, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= hipMemcpyAsync(t->a, t->ck_a + c * n3, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= sfd_f64_to_f32(t->x64, (unsigned int)n3, t->x, s);
-	rc |= hipMemcpyAsync(t->seg, t->x, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	for (unsigned int k = 1; k <= steps && !rc; ++k) {
-		rc |= kdk(t, s);
-		rc |= hipMemcpyAsync(t->seg + k * n3, t->x, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
+	int rc = sfd_adjoint_reopen(t->ck_x64 + c * n3, t->ck_v + c * n3, t->ck_a + c * n3, t->N,
+	                            0.5f * (float)t->p.dt, t->p.dt, steps > 0u, t->x64, t->v, t->seg, t->w.body, s);
+	for (unsigned int k = 1; k < steps && !rc; ++k) {
+		sf_force_epi e = {.close = 1, .open = 1, .x = t->seg + (k + 1u) * n3};
+		rc |= kdk(t, &e, s);
 	}
 	return rc;
 }
@@ -281,25 +269,40 @@ int sf_adjoint_backward(sf_tape* t, const float* gxN, const float* gvN, float* g
 	const unsigned int n3 = 3u * t->N;
 	const size_t f3 = (size_t)n3 * sizeof(float);
 	const float dt = (float)t->p.dt, h = 0.5f * dt;
+	const int phys = t->p.acc_mode == SF_ACC_PHYSICAL;
 	int rc = 0;
-	rc |= gxN ? hipMemcpyAsync(t->lx, gxN, f3, hipMemcpyDeviceToDevice, s) != hipSuccess : sfd_fill0(t->lx, n3, s);
-	rc |= gvN ? hipMemcpyAsync(t->lv, gvN, f3, hipMemcpyDeviceToDevice, s) != hipSuccess : sfd_fill0(t->lv, n3, s);
+	if (t->nsteps == 0u) {   /* x_K = x_0: the cotangents as they are */
+		rc |= gxN ? hipMemcpyAsync(t->lx, gxN, f3, hipMemcpyDeviceToDevice, s) != hipSuccess
+		          : sfd_fill0(t->lx, n3, s);
+		rc |= gvN ? hipMemcpyAsync(t->lv, gvN, f3, hipMemcpyDeviceToDevice, s) != hipSuccess
+		          : sfd_fill0(t->lv, n3, s);
+		rc |= hipMemcpyAsync(gx0, t->lx, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
+		rc |= hipMemcpyAsync(gv0, t->lv, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
+	}
 	const int tok = sf_prof_begin("adjoint_backward", s);
+	sf_vjp_epi e = {.step = 1, .lx = t->lx, .lv = t->lv, .dt = dt, .acc_phys = phys, .nu = t->w.nu, .body = t->w.body};
 	for (unsigned int c = t->n_ckpt; c-- > 0u && !rc;) {
 		const unsigned int start = c * t->ckpt;
 		const unsigned int len = (t->nsteps - start) < t->ckpt ? (t->nsteps - start) : t->ckpt;
 		if (t->seg_first != start) rc |= recompute(t, c, len, s);
 		/* the kick that ends the last step acts at x_K alone */
-		if (c == t->n_ckpt - 1u) rc |= vjp(&t->p, &t->w, t->seg + (size_t)len * n3, t->m, t->lv, h, 1, t->lx, s);
-		for (unsigned int k = len; k-- > 0u && !rc;) {
+		const int last = c == t->n_ckpt - 1u;
+		if (last)
+			rc |= sfd_adjoint_begin(gxN, gvN, t->seg + (size_t)len * n3, t->N, t->w.n_pad, h, phys, t->lx, t->lv,
+			                        t->w.body, t->w.nu, s);
+		for (unsigned int k = last ? len : len - 1u; !rc; --k) {
+			/* the VJP at x_{start+k}, then its epilogue: lv and the inputs of
+			   the one before (recompute leaves the bodies at a segment's end) */
 			const unsigned int n = start + k;
-			rc |= sfd_axpy(t->lv, t->lx, n3, dt, s);
-			rc |= vjp(&t->p, &t->w, t->seg + (size_t)k * n3, t->m, t->lv, n > 0u ? dt : h, 1, t->lx, s);
+			e.coef = n > 1u ? dt : h;
+			e.x = k > 0u ? t->seg + (size_t)(k - 1u) * n3 : NULL;
+			e.gx0 = n ? NULL : gx0;
+			e.gv0 = n ? NULL : gv0;
+			rc |= vjp(&t->p, &t->w, &e, s);
+			if (k == 0u) break;
 		}
 	}
 	sf_prof_end(tok, s);
-	rc |= hipMemcpyAsync(gx0, t->lx, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
-	rc |= hipMemcpyAsync(gv0, t->lv, f3, hipMemcpyDeviceToDevice, s) != hipSuccess;
 	if (rc || sf_hip_check(hipGetLastError(), fn, "launch")) {
 		sf_error(fn, "adjoint integration failed");
 		return STARFLOOD_FAILURE;
@@ -329,7 +332,8 @@ int sf_force_dev(unsigned int N, const float* x, const float* m, float* acc, flo
 	}
 	if (scratch_for(N, fn)) return STARFLOOD_FAILURE;
 	hipStream_t s = stream_of(stream);
-	if (force(sf_params(), &g_w, x, m, acc, pot, s)) return STARFLOOD_FAILURE;
+	if (sf_pp_force_arrays(sf_params(), N, g_w.n_pad, x, m, g_w.body, g_w.part, g_w.part_bytes, acc, pot, s))
+		return STARFLOOD_FAILURE;
 	return sf_hip_check(hipStreamSynchronize(s), fn, "sync") ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;
 }
 
@@ -342,6 +346,11 @@ int sf_force_vjp_dev(unsigned int N, const float* x, const float* m, const float
 	}
 	if (scratch_for(N, fn)) return STARFLOOD_FAILURE;
 	hipStream_t s = stream_of(stream);
-	if (vjp(sf_params(), &g_w, x, m, mu, 1.0f, 0, g, s)) return STARFLOOD_FAILURE;
+	const sf_params_t* p = sf_params();
+	const sf_vjp_epi epi = {.g = g};
+	if (sfd_pack_bodies(x, m, N, g_w.n_pad, g_w.body, s) ||
+	    sfd_pack_nu(mu, m, N, g_w.n_pad, 1.0f, p->acc_mode == SF_ACC_PHYSICAL, g_w.nu, s) ||
+	    vjp(p, &g_w, &epi, s))
+		return STARFLOOD_FAILURE;
 	return sf_hip_check(hipStreamSynchronize(s), fn, "sync") ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;
 }

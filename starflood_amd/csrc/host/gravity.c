@@ -25,39 +25,54 @@ static unsigned int pp_slices(unsigned int n_pad) {
 /* reference: (real)(EPSILON*EPSILON) is squared in double, then rounded */
 static float eps2_f32(double eps) { return (float)(eps * eps); }
 
-static int pp_on(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
-                 float* body, sf_ctx* c, float* acc, float* pot, hipStream_t s) {
-	const int phys = p->acc_mode == SF_ACC_PHYSICAL;
-	if (p->precision == SF_PRECISION_EXACT) {
-		return sfd_pp_exact(pos, mas, N, eps2_f32(p->epsilon), (float)(-p->G), phys, p->kahan_solver,
-		                    p->kahan_energy, acc, pot, s);
-	}
-	const unsigned int slices = pp_slices(n_pad);
-	if (sf_ctx_reserve_part(c, sf_pp_part_bytes(n_pad))) return -1;
-	if (sfd_pack_bodies(pos, mas, N, n_pad, body, s)) return -1;
-	return sfd_pp_fast(body, N, n_pad, eps2_f32(p->epsilon), p->G, phys, c->d_part, slices, acc, pot, s);
-}
-
 unsigned int sf_pp_slice_count(unsigned int n_pad) { return pp_slices(n_pad); }
 
 size_t sf_pp_part_bytes(unsigned int n_pad) { return sfd_pp_part_bytes(n_pad, pp_slices(n_pad)); }
 
-int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
-                       float* body, float* part, size_t part_bytes, float* acc, float* pot, hipStream_t s) {
+int sf_pp_force_packed(const sf_params_t* p, unsigned int N, unsigned int n_pad, float* body, float* part,
+                       size_t part_bytes, const sf_force_epi* epi, hipStream_t s) {
 	if (part_bytes < sf_pp_part_bytes(n_pad)) {
-		sf_error("sf_pp_force_arrays", "%zu bytes of slice partials, %zu needed", part_bytes, sf_pp_part_bytes(n_pad));
+		sf_error("sf_pp_force_packed", "%zu bytes of slice partials, %zu needed", part_bytes, sf_pp_part_bytes(n_pad));
 		return -1;
 	}
-	if (sfd_pack_bodies(pos, mas, N, n_pad, body, s)) return -1;
 	return sfd_pp_fast(body, N, n_pad, eps2_f32(p->epsilon), p->G, p->acc_mode == SF_ACC_PHYSICAL, part,
-	                   pp_slices(n_pad), acc, pot, s);
+	                   pp_slices(n_pad), epi, s);
+}
+
+int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
+                       float* body, float* part, size_t part_bytes, float* acc, float* pot, hipStream_t s) {
+	const sf_force_epi epi = {.kind = SF_EPI_STORE, .acc = acc, .pot = pot};
+	if (sfd_pack_bodies(pos, mas, N, n_pad, body, s)) return -1;
+	return sf_pp_force_packed(p, N, n_pad, body, part, part_bytes, &epi, s);
 }
 
 int sf_solve_gravity_pp(sf_ctx* c) {
 	const sf_params_t* p = sf_params();
 	const unsigned int N = c->N;
-	return pp_on(p, N, c->n_pad, sf_blk(c->d_mem, N, SF_E_POS), sf_blk(c->d_mem, N, SF_E_MAS), c->d_body, c,
-	             sf_blk(c->d_mem, N, SF_E_ACC), sf_blk(c->d_mem, N, SF_E_POT), c->stream);
+	const float *pos = sf_blk(c->d_mem, N, SF_E_POS), *mas = sf_blk(c->d_mem, N, SF_E_MAS);
+	float *acc = sf_blk(c->d_mem, N, SF_E_ACC), *pot = sf_blk(c->d_mem, N, SF_E_POT);
+	if (p->precision == SF_PRECISION_EXACT) {
+		return sfd_pp_exact(pos, mas, N, eps2_f32(p->epsilon), (float)(-p->G), p->acc_mode == SF_ACC_PHYSICAL,
+		                    p->kahan_solver, p->kahan_energy, acc, pot, c->stream);
+	}
+	const sf_force_epi epi = {.kind = SF_EPI_STORE, .acc = acc, .pot = pot};
+	if (sf_ctx_reserve_part(c, sf_pp_part_bytes(c->n_pad))) return -1;
+	if (sfd_pack_bodies(pos, mas, N, c->n_pad, c->d_body, c->stream)) return -1;
+	return sf_pp_force_packed(p, N, c->n_pad, c->d_body, c->d_part, c->part_bytes, &epi, c->stream);
+}
+
+int sf_step_gravity_pp(sf_ctx* c) {
+	const sf_params_t* p = sf_params();
+	const unsigned int N = c->N;
+	const float h = 0.5f * (float)p->dt;
+	float *vel = sf_blk(c->d_mem, N, SF_E_VEL), *acc = sf_blk(c->d_mem, N, SF_E_ACC);
+	const sf_force_epi epi = {.kind = SF_EPI_KICK, .acc = acc, .pot = sf_blk(c->d_mem, N, SF_E_POT), .h = h, .v = vel,
+	                          .ken = sf_blk(c->d_mem, N, SF_E_KEN), .pen = sf_blk(c->d_mem, N, SF_E_PEN)};
+	if (sf_ctx_reserve_part(c, sf_pp_part_bytes(c->n_pad))) return -1;
+	if (sfd_kick_drift_pack(vel, acc, c->d_x64, sf_blk(c->d_mem, N, SF_E_POS), sf_blk(c->d_mem, N, SF_E_MAS), N,
+	                        c->n_pad, h, p->dt, c->d_body, c->stream))
+		return -1;
+	return sf_pp_force_packed(p, N, c->n_pad, c->d_body, c->d_part, c->part_bytes, &epi, c->stream);
 }
 
 /* reference src/gravity.c:667-819: reads pos, mas; writes acc (assigned, not

@@ -11,12 +11,18 @@
 
 /* gravity.c: PP gravity from d_mem pos/mas into d_mem acc/pot */
 int sf_solve_gravity_pp(sf_ctx* c);
+/* gravity.c: a whole step of the fast policy with PP gravity and no SPH:
+   kick and drift, force, closing kick and energy terms, in three launches */
+int sf_step_gravity_pp(sf_ctx* c);
 /* gravity.c: j ranges of the fast PP kernel (and of the SPH all-pairs and
    VJP passes) for n_pad particles, the bytes of slice partials the fast PP
-   kernel writes, and the fast PP force on caller arrays (body: n_pad float4,
-   part: part_bytes >= sf_pp_part_bytes(n_pad), pot may be NULL) */
+   kernel writes, the fast PP force of packed bodies ended by *epi, and the
+   one of caller arrays (body: n_pad float4, part: part_bytes >=
+   sf_pp_part_bytes(n_pad), pot may be NULL) */
 unsigned int sf_pp_slice_count(unsigned int n_pad);
 size_t sf_pp_part_bytes(unsigned int n_pad);
+int sf_pp_force_packed(const sf_params_t* p, unsigned int N, unsigned int n_pad, float* body, float* part,
+                       size_t part_bytes, const sf_force_epi* epi, hipStream_t s);
 int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
                        float* body, float* part, size_t part_bytes, float* acc, float* pot, hipStream_t s);
 /* tree.c: bounds as src/simulation.c:245-301, build, then walk into acc/pot.

@@ -223,6 +223,9 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 	/* the cubic SPH model carries u: it is kicked with v, and the solve
 	   predicts v and u to the end of the step from the previous forces */
 	const int cubic = p->enable_sph && p->sph_model == SF_SPH_CUBIC_IDEAL;
+	/* PP gravity alone: the kicks and the drift ride on the force's own
+	   launches (the same operations; the log's timings need them apart) */
+	const int fused = N && !exact && !timing && !p->enable_tree && !p->enable_sph;
 	int rc = 0;
 
 	if (timing && !g_tev_ready) {
@@ -241,15 +244,15 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 		if (sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_0 */
 		if (timing) tev_record(1, s);
 		if (sfd_drift_exact(pos, vel, n3, dt, s)) return STARFLOOD_FAILURE;       /* drift */
-	} else {
+	} else if (!fused) {
 		/* x64 restarts from pos where a host-side change left them apart */
-		if (sfd_kick_drift_fast(vel, acc, c->d_x64, pos, n3, half_dt, p->dt, 1, s)) return STARFLOOD_FAILURE;
+		if (sfd_kick_drift_fast(vel, acc, c->d_x64, pos, n3, half_dt, p->dt, s)) return STARFLOOD_FAILURE;
 		if (timing) tev_record(1, s);
 	}
 	if (timing) tev_record(2, s);
 
 	/* acc still holds the force that kick_0 used: the previous evaluation */
-	if (sf_solve_all(c, &sim_ptr->tree, sim.step_number, cubic ? half_dt : 0.0f, 1)) {
+	if (fused ? sf_step_gravity_pp(c) : sf_solve_all(c, &sim_ptr->tree, sim.step_number, cubic ? half_dt : 0.0f, 1)) {
 		fprintf(stderr, "%s error: %s failed.\n", "sim_step()", "sim_solv()");
 		rc = -1;
 	}
@@ -257,7 +260,7 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 
 	if (exact) {
 		if (sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_1 */
-	} else {
+	} else if (!fused) {
 		/* kick_1 and the energy terms below, in one pass */
 		if (sfd_kick_energy_fast(vel, acc, mas, pot, N, half_dt, ken, pen, s)) return STARFLOOD_FAILURE;
 	}

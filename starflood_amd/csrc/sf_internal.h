@@ -92,8 +92,10 @@ void sf_prof_end(int token, hipStream_t s);
 /* ---------- device launchers (csrc/device) ---------- */
 #define SF_PP_TILE 256u      /* j padding granule of d_body */
 /* packed bodies: n_pad float4, then SF_BODY_STATE words that sfd_pack_bodies
-   reads and writes (the leading bodies that form whole tiles of equal mass,
-   and two block-count words that must be zero when the buffer is made) */
+   reads and writes below 10240 bodies (the leading bodies that form whole
+   tiles of equal mass, and two block-count words that must be zero when the
+   buffer is made; the kernels from 10240 bodies look at each tile's masses
+   themselves) */
 #define SF_BODY_STATE 64u
 #define SF_BODY_BYTES(n_pad) ((size_t)(n_pad) * 16u + SF_BODY_STATE * 4u)
 #define SF_RED_VALUES 16u    /* doubles per reduction partial */
@@ -101,17 +103,55 @@ void sf_prof_end(int token, hipStream_t s);
 /* body[i] = (pos_i, m_i) for i < N, zero for N <= i < n_pad */
 int sfd_pack_bodies(const float* pos, const float* mas, unsigned int N, unsigned int n_pad,
                     float* body, hipStream_t s);
+/* sfd_kick_drift_fast, then sfd_pack_bodies, in one pass */
+int sfd_kick_drift_pack(float* vel, const float* acc, double* x64, float* pos, const float* mas, unsigned int N,
+                        unsigned int n_pad, float half_dt, double dt, float* body, hipStream_t s);
 
 /* Reference-order PP gravity (src/gravity.c:693-812). */
 int sfd_pp_exact(const float* pos, const float* mas, unsigned int N, float eps2, float negG,
                  int acc_phys, int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s);
 
+/* What the fast force's combine does with each acceleration
+   (device/force_epi.h): SF_EPI_STORE writes acc and (unless NULL) pot;
+   SF_EPI_KICK also v += h a, ken and pen; SF_EPI_KDK takes the adjoint's
+   integration from one force to the next (no acc, no pot). */
+enum { SF_EPI_STORE = 0, SF_EPI_KICK, SF_EPI_KDK };
+typedef struct {
+	int kind;
+	float *acc, *pot;
+	float h;                       /* half a time step */
+	float *v, *ken, *pen;
+	double dt;                     /* SF_EPI_KDK from here */
+	double* x64;
+	float* x;                      /* copy of the opened step's positions, or NULL */
+	int close, open;
+	double* ck_x64;                /* checkpoint before the opening kick, or NULL */
+	float *ck_v, *ck_a;
+	float *xN, *vN;                /* the final state, or NULL */
+} sf_force_epi;
+
+/* What the force VJP's combine does with g (device/adjoint.hip): store it, or
+   (step) lx += g, then either write lx and lv to gx0 and gv0 (where set) or
+   lv += dt lx and the next VJP's inputs: nu = coef lv (coef m lv unless
+   acc_phys) and, unless NULL, the bodies at x. */
+typedef struct {
+	int step;
+	float* g;
+	float *lx, *lv;   /* step from here */
+	float dt, coef;
+	int acc_phys;
+	float *nu, *body;
+	const float* x;
+	float *gx0, *gv0;
+} sf_vjp_epi;
+
 /* Fast PP gravity: partial sums into part (sfd_pp_part_bytes of n_pad and
    slices), then a fixed-order FP64 combine into acc (AoS) and pot.  From
    10240 bodies each pair is evaluated once (device/pp_sym.hip); below, every
-   i against `slices` ranges of j.  pot may be NULL (skip). */
-int sfd_pp_fast(const float* body, unsigned int N, unsigned int n_pad, float eps2, double G,
-                int acc_phys, float* part, unsigned int slices, float* acc, float* pot, hipStream_t s);
+   i against `slices` ranges of j.  The combine ends with *epi (only
+   SF_EPI_KDK writes body). */
+int sfd_pp_fast(float* body, unsigned int N, unsigned int n_pad, float eps2, double G, int acc_phys, float* part,
+                unsigned int slices, const sf_force_epi* epi, hipStream_t s);
 size_t sfd_pp_part_bytes(unsigned int n_pad, unsigned int slices);
 
 /* FP64 direct sum for the listed particles (device idx list). */
@@ -131,12 +171,11 @@ size_t sfd_energy_scratch_bytes(unsigned int N);
 int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned int N, void* part, double* out, hipStream_t s);
 
 /* FAST KDK: kick + FP64 drift fused; x64 refreshed from pos where they
-   disagree (sfd_x64_refresh, or inside the drift with refresh = 1). */
+   disagree (sfd_x64_refresh, or inside the drift). */
 int sfd_x64_refresh(const float* pos, double* x64, unsigned int n3, hipStream_t s);
 int sfd_kick_drift_fast(float* vel, const float* acc, double* x64, float* pos, unsigned int n3,
-                        float half_dt, double dt, int refresh, hipStream_t s);
-int sfd_kick_fast(float* vel, const float* acc, unsigned int n3, float half_dt, hipStream_t s);
-/* sfd_kick_fast then sfd_energy_terms in one pass over the particles */
+                        float half_dt, double dt, hipStream_t s);
+/* v += half_dt a, then sfd_energy_terms, in one pass over the particles */
 int sfd_kick_energy_fast(float* vel, const float* acc, const float* mas, const float* pot, unsigned int N,
                          float half_dt, float* ken, float* pen, hipStream_t s);
 /* sph.hip: u += half_dt du/dt (cubic SPH model) */
