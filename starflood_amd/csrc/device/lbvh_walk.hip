@@ -11,9 +11,18 @@
 // side of the node's particle box), a "leaf" summed particle by particle when
 // the node holds at most leaf_size particles, otherwise opened (its two
 // children are pushed).  Cells and leaf particles are queued in LDS and
-// evaluated 64 at a time by every lane with the PP kernel's 13-VALU + rsqrt
-// interaction; leaf particles are gathered 64 at a time with one vector load,
-// so the tree logic and memory latency are amortised over 64 interactions.
+// evaluated 64 at a time with a 14-VALU + rsqrt interaction; leaf particles
+// are gathered 64 at a time with one vector load, so the tree logic and
+// memory latency are amortised over 64 interactions.
+//
+// The evaluation is bound by VALU issue.  Groups hold 44 particles on
+// average, so with one particle per lane a third of it went to idle lanes.
+// Instead each row of 16 lanes takes every fourth entry and each lane up to
+// four particles (Slots): (cnt + 15) / 16 interactions per lane for four
+// entries, 0.8 of the work on average, a quarter of the LDS reads and four
+// independent chains.  KDK step, before -> after: 65537 particles (monopole,
+// theta 0.5) 266 -> 236 us, 1M 2116 -> 1876 us; 4M quadrupoles under the
+// relative test, more of it tree logic, 5474 -> 5300 us.
 //
 // Options: quadrupole cells (the 34-VALU interact_quad), and the relative
 // opening test, which also requires G M l^p <= alpha |a|min d^(p+2) of a
@@ -56,20 +65,24 @@ constexpr float kMonoBeta = 0.2f;
 
 __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
+// the same on every lane: kept in a scalar register
+__device__ __forceinline__ float uniform(float v) {
+	return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+
 __device__ __forceinline__ float wave_min(float v) {
 	for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-	return v;
+	return uniform(v);
 }
 __device__ __forceinline__ float wave_max(float v) {
 	for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-	return v;
+	return uniform(v);
 }
 
-struct Acc {
-	float tx, ty, tz, tp;   // partial sums of the current batch of 64
-	float sx, sy, sz, sp;   // running sums
-	float cx, cy, cz, cp;   // Kahan compensations
-};
+// The lists' entries are taken four at a time, one by each row of 16 lanes;
+// lane 16 r + p sums entries 4 k + r for the particles p, p + 16, p + 32 and
+// p + 48 of the group, as many of these slots as the group fills.
+constexpr int kWays = 4;
 
 __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	const float y = x - c;
@@ -78,48 +91,48 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	s = t;
 }
 
-__device__ __forceinline__ void fold(Acc& a) {
-	kahan_add(a.sx, a.cx, a.tx);
-	kahan_add(a.sy, a.cy, a.ty);
-	kahan_add(a.sz, a.cz, a.tz);
-	kahan_add(a.sp, a.cp, a.tp);
-	a.tx = a.ty = a.tz = a.tp = 0.0f;
+struct Slots {
+	float x[kWays], y[kWays], z[kWays];
+	float t[kWays][4];   // plain sums of at most 64 terms
+	float s[4], c[4];    // running Kahan sums of particle `lane`
+	int terms;           // in t, per lane
+};
+
+// a of the upper 32 lanes with b of the lower ones, and the same for odd and even rows
+__device__ __forceinline__ float swap_add32(float a, float b) {
+	const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+	return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b) {
+	const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+	return __uint_as_float(v[0]) + __uint_as_float(v[1]);
 }
 
-// UNIFORM: every q has the same mass, left out of the sums (the caller
-// scales the partial by it before the fold)
-template <bool UNIFORM = false>
-__device__ __forceinline__ void interact(Acc& a, float xi, float yi, float zi, float4 bj, float eps2) {
+// Adds t over the rows, slot r's sum to row r: lane l then holds particle l's.
+__device__ __forceinline__ void fold(Slots& a) {
+#pragma unroll
+	for (int u = 0; u < 4; ++u) {
+		const float lo = swap_add32(a.t[0][u], a.t[2][u]);   // lower half: slot 0, upper: slot 2
+		const float hi = swap_add32(a.t[1][u], a.t[3][u]);
+		kahan_add(a.s[u], a.c[u], swap_add16(lo, hi));
+#pragma unroll
+		for (int j = 0; j < kWays; ++j) a.t[j][u] = 0.0f;
+	}
+	a.terms = 0;
+}
+
+__device__ __forceinline__ void interact(float t[4], float xi, float yi, float zi, float4 bj, float eps2) {
 	const float dx = bj.x - xi, dy = bj.y - yi, dz = bj.z - zi;
 	float r2 = __builtin_fmaf(dx, dx, eps2);
 	r2 = __builtin_fmaf(dy, dy, r2);
 	r2 = __builtin_fmaf(dz, dz, r2);
 	const float inv = __builtin_amdgcn_rsqf(r2);
-	const float mi = UNIFORM ? inv : bj.w * inv;
+	const float mi = bj.w * inv;
 	const float w = mi * (inv * inv);
-	a.tx = __builtin_fmaf(w, dx, a.tx);
-	a.ty = __builtin_fmaf(w, dy, a.ty);
-	a.tz = __builtin_fmaf(w, dz, a.tz);
-	a.tp += mi;
-}
-
-// Interactions with q[0 .. n), n <= 64, read from LDS by every lane.
-template <bool UNIFORM = false>
-__device__ __forceinline__ void eval_list(Acc& a, float xi, float yi, float zi, const float4* q, int n, float eps2,
-                                          float m = 1.0f) {
-	if (n == 64) {
-#pragma unroll 8
-		for (int k = 0; k < 64; ++k) interact<UNIFORM>(a, xi, yi, zi, q[k], eps2);
-	} else {
-		for (int k = 0; k < n; ++k) interact<UNIFORM>(a, xi, yi, zi, q[k], eps2);
-	}
-	if (UNIFORM) {
-		a.tx *= m;
-		a.ty *= m;
-		a.tz *= m;
-		a.tp *= m;
-	}
-	fold(a);
+	t[0] = __builtin_fmaf(w, dx, t[0]);
+	t[1] = __builtin_fmaf(w, dy, t[1]);
+	t[2] = __builtin_fmaf(w, dz, t[2]);
+	t[3] += mi;
 }
 
 // Monopole plus traceless quadrupole of a cell with e = com - x:
@@ -129,7 +142,7 @@ __device__ __forceinline__ void eval_list(Acc& a, float xi, float yi, float zi, 
 // gradient), Plummer-softened through r^2 = |e|^2 + eps^2.  Qt is
 // (q0 = Qxx, Qxy, Qxz, Qyy; q1 = Qyz, Qzz), Qzz = -Qxx - Qyy stored with the
 // queued cell.  34 VALU operations plus the rsqrt.
-__device__ __forceinline__ void interact_quad(Acc& a, float xi, float yi, float zi, float4 c, float4 q0, float2 q1,
+__device__ __forceinline__ void interact_quad(float t[4], float xi, float yi, float zi, float4 c, float4 q0, float2 q1,
                                               float eps2) {
 	const float ex = c.x - xi, ey = c.y - yi, ez = c.z - zi;
 	float r2 = __builtin_fmaf(ex, ex, eps2);
@@ -144,31 +157,74 @@ __device__ __forceinline__ void interact_quad(Acc& a, float xi, float yi, float 
 	const float qy = __builtin_fmaf(q0.y, ex, __builtin_fmaf(q0.w, ey, q1.x * ez));
 	const float qz = __builtin_fmaf(q0.z, ex, __builtin_fmaf(q1.x, ey, q1.y * ez));
 	const float eqe = __builtin_fmaf(ex, qx, __builtin_fmaf(ey, qy, ez * qz));
-	const float t = eqe * inv5;
-	const float w = __builtin_fmaf(2.5f, t * inv2, m3);
-	a.tx = __builtin_fmaf(w, ex, __builtin_fmaf(-inv5, qx, a.tx));
-	a.ty = __builtin_fmaf(w, ey, __builtin_fmaf(-inv5, qy, a.ty));
-	a.tz = __builtin_fmaf(w, ez, __builtin_fmaf(-inv5, qz, a.tz));
-	a.tp = __builtin_fmaf(0.5f, t, a.tp) + mi;
+	const float v = eqe * inv5;
+	const float w = __builtin_fmaf(2.5f, v * inv2, m3);
+	t[0] = __builtin_fmaf(w, ex, __builtin_fmaf(-inv5, qx, t[0]));
+	t[1] = __builtin_fmaf(w, ey, __builtin_fmaf(-inv5, qy, t[1]));
+	t[2] = __builtin_fmaf(w, ez, __builtin_fmaf(-inv5, qz, t[2]));
+	t[3] = __builtin_fmaf(0.5f, v, t[3]) + mi;
 }
 
-__device__ __forceinline__ void eval_list_quad(Acc& a, float xi, float yi, float zi, const float4* c, const float4* q0,
-                                               const float2* q1, int n, float eps2) {
+// Interactions of P slots with the entries q[0 .. n), n <= 64, read from LDS.
+template <int P>
+__device__ __forceinline__ void eval_slots(Slots& a, const float4* q, int n, int row, float eps2) {
 	if (n == 64) {
-#pragma unroll 4
-		for (int k = 0; k < 64; ++k) interact_quad(a, xi, yi, zi, c[k], q0[k], q1[k], eps2);
+#pragma unroll (8 / P)
+		for (int k = 0; k < 64; k += kWays) {
+			const float4 b = q[k + row];
+#pragma unroll
+			for (int j = 0; j < P; ++j) interact(a.t[j], a.x[j], a.y[j], a.z[j], b, eps2);
+		}
 	} else {
-		for (int k = 0; k < n; ++k) interact_quad(a, xi, yi, zi, c[k], q0[k], q1[k], eps2);
+		for (int k = row; k < n; k += kWays) {
+			const float4 b = q[k];
+#pragma unroll
+			for (int j = 0; j < P; ++j) interact(a.t[j], a.x[j], a.y[j], a.z[j], b, eps2);
+		}
 	}
-	fold(a);
 }
 
-// 5 wavefronts per SIMD (96 VGPRs): the monopole walk fits without spills
-// and runs 7% faster at 4M than at 4 per SIMD; the quadrupole walk spills 11
-// VGPRs, and at 4 per SIMD without spills it was 3.4% slower.
+template <int P>
+__device__ __forceinline__ void eval_slots_quad(Slots& a, const float4* c, const float4* q0, const float2* q1, int n,
+                                                int row, float eps2) {
+	for (int k = row; k < n; k += kWays) {
+		const float4 b = c[k], r0 = q0[k];
+		const float2 r1 = q1[k];
+#pragma unroll
+		for (int j = 0; j < P; ++j) interact_quad(a.t[j], a.x[j], a.y[j], a.z[j], b, r0, r1, eps2);
+	}
+}
+
+// slots: (particles of the group + 15) / 16
+__device__ __forceinline__ void eval_list(Slots& a, int slots, const float4* q, int n, int row, float eps2) {
+	switch (slots) {
+	case 1: eval_slots<1>(a, q, n, row, eps2); break;
+	case 2: eval_slots<2>(a, q, n, row, eps2); break;
+	case 3: eval_slots<3>(a, q, n, row, eps2); break;
+	default: eval_slots<4>(a, q, n, row, eps2);
+	}
+	a.terms += (n + kWays - 1) / kWays;
+	if (a.terms > 48) fold(a);
+}
+
+__device__ __forceinline__ void eval_list_quad(Slots& a, int slots, const float4* c, const float4* q0,
+                                               const float2* q1, int n, int row, float eps2) {
+	switch (slots) {
+	case 1: eval_slots_quad<1>(a, c, q0, q1, n, row, eps2); break;
+	case 2: eval_slots_quad<2>(a, c, q0, q1, n, row, eps2); break;
+	case 3: eval_slots_quad<3>(a, c, q0, q1, n, row, eps2); break;
+	default: eval_slots_quad<4>(a, c, q0, q1, n, row, eps2);
+	}
+	a.terms += (n + kWays - 1) / kWays;
+	if (a.terms > 48) fold(a);
+}
+
+// Monopole walk: 5 wavefronts per SIMD (96 VGPRs, no spills) run the 1M step
+// in 1876 us, 4 in 2016.  Quadrupole walk: 4 (128 VGPRs) and 5 (34 spilled)
+// measure the same.
 // QUAD: cells carry traceless quadrupoles (node_q0, node_q1).
 template <bool QUAD>
-__global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ body, const unsigned* __restrict__ order,
+__global__ __launch_bounds__(kBlock, QUAD ? 4 : 5) void k_walk(const float4* __restrict__ body, const unsigned* __restrict__ order,
                                                  int N, const unsigned* __restrict__ group_start,
                                                  const float4* __restrict__ rec_a,
                                                  const float4* __restrict__ node_q0, const float* __restrict__ node_q1,
@@ -184,7 +240,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 	__shared__ float2 s_q1[kWaves][QUAD ? kList : 1];
 	constexpr int kTop = QUAD ? kTopQuad : kTopMono;
 	__shared__ int s_top[kWaves][kTop];
-	const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+	const unsigned lane = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int row = (int)(lane >> 4);
 	float4* cq0 = s_q0[w];
 	float2* cq1 = s_q1[w];
 	int* stack = gstack + (size_t)(blockIdx.x * kWaves + w) * kStack;
@@ -195,7 +252,6 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 	float4* part = s_part[w];
 	const unsigned long long lt = (1ull << lane) - 1ull;
 	const int n_nodes = 2 * N - 1;
-	const float m0 = body[0].w;   // the mass of the equal-mass leaf batches
 	const unsigned budget = 2u * (unsigned)n_nodes + 64u;
 	unsigned long long n_cell_tot = 0, n_part_tot = 0, n_batch = 0;
 	unsigned bad = 0;
@@ -206,7 +262,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 	for (;;) {
 		unsigned long long cw = 0;
 		if (lane == 0) cw = atomicAdd(&counters[5], 1ull);
-		const unsigned c = (unsigned)__shfl(cw, 0);
+		const unsigned c = __builtin_amdgcn_readfirstlane((unsigned)cw);
 		if (c >= n_chunks) break;
 		// the groups that start in sorted positions [64c, 64c + 64); each ends at
 		// the next start flag, at most 64 positions later (start[N] is set)
@@ -227,10 +283,33 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 			}
 			const int p = base + (int)lane;
 			const bool live = (int)lane < cnt;
-			const float4 me = body[live ? p : base];
-			const float xi = me.x, yi = me.y, zi = me.z;
-			const float gx0 = wave_min(xi), gy0 = wave_min(yi), gz0 = wave_min(zi);
-			const float gx1 = wave_max(xi), gy1 = wave_max(yi), gz1 = wave_max(zi);
+			const int slots = (cnt + 15) / 16;
+			Slots a;
+			float gx0 = 3.0e38f, gy0 = 3.0e38f, gz0 = 3.0e38f, gx1 = -3.0e38f, gy1 = -3.0e38f, gz1 = -3.0e38f;
+#pragma unroll
+			for (int j = 0; j < kWays; ++j) {
+				const float4 b = body[base + min(16 * j + (int)(lane & 15u), cnt - 1)];
+				a.x[j] = b.x;
+				a.y[j] = b.y;
+				a.z[j] = b.z;
+				gx0 = fminf(gx0, b.x);
+				gy0 = fminf(gy0, b.y);
+				gz0 = fminf(gz0, b.z);
+				gx1 = fmaxf(gx1, b.x);
+				gy1 = fmaxf(gy1, b.y);
+				gz1 = fmaxf(gz1, b.z);
+#pragma unroll
+				for (int u = 0; u < 4; ++u) a.t[j][u] = 0.0f;
+			}
+#pragma unroll
+			for (int u = 0; u < 4; ++u) a.s[u] = a.c[u] = 0.0f;
+			a.terms = 0;
+			gx0 = wave_min(gx0);
+			gy0 = wave_min(gy0);
+			gz0 = wave_min(gz0);
+			gx1 = wave_max(gx1);
+			gy1 = wave_max(gy1);
+			gz1 = wave_max(gz1);
 			// relative opening test: am = alpha / G times the smallest previous
 			// |a| of the group (0: theta test alone; also when no particle has a
 			// positive finite previous acceleration)
@@ -241,14 +320,12 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 					const unsigned i0 = order[p];
 					const float ax = acc[3u * i0], ay = acc[3u * i0 + 1u], az = acc[3u * i0 + 2u];
 					const float a = sqrtf(ax * ax + ay * ay + az * az);
-					amag = acc_phys ? a : a / me.w;   // the reference's acc is m a
+					amag = acc_phys ? a : a / body[p].w;   // the reference's acc is m a
 				}
 				amag = wave_min(amag);   // fminf drops NaN
 				am = (amag > 0.0f && amag < 3.0e38f) ? alpha_g * amag : 0.0f;
 			}
 
-			Acc a;
-			a.tx = a.ty = a.tz = a.tp = a.sx = a.sy = a.sz = a.sp = a.cx = a.cy = a.cz = a.cp = 0.0f;
 			unsigned long long n_cell = 0, n_part = 0, n_mono = 0;
 			unsigned popped = 0;
 			// pending nodes: nt in the LDS top, ng in the global stack
@@ -353,8 +430,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 				// monopoles
 				if (nc >= 64 || (drain && nc > 0)) {
 					const int take = min(nc, 64);
-					if (QUAD) eval_list_quad(a, xi, yi, zi, cells, cq0, cq1, take, eps2);
-					else eval_list(a, xi, yi, zi, cells, take, eps2);
+					if (QUAD) eval_list_quad(a, slots, cells, cq0, cq1, take, row, eps2);
+					else eval_list(a, slots, cells, take, row, eps2);
 					n_cell += (unsigned long long)take;
 					wave_fence();
 					if ((int)lane < nc - take) {
@@ -387,7 +464,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 							}
 							const bool fits = li < nl && npid + incl <= kList;
 							const int k = __popcll(__ballot(fits));
-							const int total = __shfl(incl, k - 1);
+							const int total = __builtin_amdgcn_readlane(incl, k - 1);
 							if (fits) {
 								const int at = npid + incl - lf.y;
 								for (int j = 0; j < lf.y; ++j) pid[at + j] = lf.x + j;
@@ -398,20 +475,12 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 						wave_fence();
 						if (npid >= 64 || (drain && q == nl && npid > 0)) {
 							const int take = min(npid, 64);
-							float pm = m0;
 							if ((int)lane < take) {
 								const int id = pid[lane];
-								const float4 pb = (!QUAD || id >= 0) ? body[id] : rec_a[~id];
-								part[lane] = pb;
-								pm = pb.w;
+								part[lane] = (!QUAD || id >= 0) ? body[id] : rec_a[~id];
 							}
 							wave_fence();
-							// particles of one mass (the common case) leave the
-							// per-pair mass product out
-							if (__ballot(__float_as_uint(pm) != __float_as_uint(m0)) == 0ull)
-								eval_list<true>(a, xi, yi, zi, part, take, eps2, m0);
-							else
-								eval_list(a, xi, yi, zi, part, take, eps2);
+							eval_list(a, slots, part, take, row, eps2);
 							n_part += (unsigned long long)take;
 							wave_fence();
 							if ((int)lane < npid - take) pid[lane] = pid[take + (int)lane];
@@ -427,11 +496,12 @@ __global__ __launch_bounds__(kBlock, 5) void k_walk(const float4* __restrict__ b
 					wave_fence();
 				}
 			}
+			fold(a);
 			if (live) {
 				const unsigned i = order[p];
-				const double sx = (double)a.sx - (double)a.cx, sy = (double)a.sy - (double)a.cy,
-				             sz = (double)a.sz - (double)a.cz, sp2 = (double)a.sp - (double)a.cp;
-				const double f = acc_phys ? G : G * (double)me.w;
+				const double sx = (double)a.s[0] - (double)a.c[0], sy = (double)a.s[1] - (double)a.c[1],
+				             sz = (double)a.s[2] - (double)a.c[2], sp2 = (double)a.s[3] - (double)a.c[3];
+				const double f = acc_phys ? G : G * (double)body[p].w;
 				acc[3u * i + 0u] = (float)(f * sx);
 				acc[3u * i + 1u] = (float)(f * sy);
 				acc[3u * i + 2u] = (float)(f * sz);
