@@ -34,13 +34,9 @@ constexpr unsigned kBlock = 256;
 constexpr unsigned kTile = 4096;          // radix sort tile (256 threads x 16)
 constexpr unsigned kRadixRounds = kTile / kBlock;
 
-__global__ __launch_bounds__(kBlock) void k_fill_u32(unsigned* __restrict__ p, unsigned n, unsigned v) {
+__global__ __launch_bounds__(kBlock) void k_fill_u64(unsigned long long* __restrict__ p, unsigned n) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	if (i < n) p[i] = v;
-}
-
-__global__ void k_fill_u64(unsigned long long* __restrict__ p, unsigned n) {
-	if (threadIdx.x < n) p[threadIdx.x] = 0ull;
+	if (i < n) p[i] = 0ull;
 }
 
 // ---------------------------------------------------------------- bbox
@@ -684,7 +680,7 @@ constexpr int kBoxLevels = 7;
 constexpr unsigned kBoxWaves = kBlock / 64;
 static_assert(kAabbNode == 64, "the walk groups hold at most 64 particles");
 __global__ __launch_bounds__(kBlock) void k_group_boxes(const float4* __restrict__ body, int N,
-                                                        const unsigned* __restrict__ start,
+                                                        const unsigned long long* __restrict__ start,
                                                         const int2* __restrict__ node_range,
                                                         float4* __restrict__ node_cell) {
 	// one table at a time (the minima, then the maxima): 7 KiB per wavefront
@@ -695,8 +691,7 @@ __global__ __launch_bounds__(kBlock) void k_group_boxes(const float4* __restrict
 	// the groups that start in the chunk; each ends at the next start flag,
 	// at most 64 positions later (start[N] is set)
 	const unsigned at = 64u * c + lane;
-	const unsigned long long e1 = __ballot(start[at] != 0u);
-	const unsigned long long e2 = __ballot(start[at + 64u] != 0u);
+	const unsigned long long e1 = start[c], e2 = start[c + 1u];
 	unsigned long long rem = e1 & __ballot(at < (unsigned)N);
 	if (!rem) return;
 	// the bodies and node ranges of the chunk and of the part of the next one
@@ -807,15 +802,15 @@ __global__ __launch_bounds__(kBlock) void k_records(int N, const int2* __restric
 
 // Walk groups: the maximal subtrees holding at most `cap` particles.  They
 // partition the sorted order into runs of at most cap particles that each lie
-// inside one Morton cell; start[p] = 1 where a run begins, start[N] = 1 ends
+// inside one Morton cell; bit p of start is set where a run begins, bit N ends
 // the last run.  `start` is zero beforehand.
 __global__ __launch_bounds__(kBlock) void k_group_flags(int N, const int2* __restrict__ node_lr,
                                                         const int2* __restrict__ node_range, int cap,
-                                                        unsigned* __restrict__ start) {
+                                                        unsigned long long* __restrict__ start) {
 	const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
 	if (i == 0) {
-		start[N] = 1u;
-		if (N <= cap) start[0] = 1u;   // the root (a single leaf when N == 1) is the only group
+		atomicOr(&start[N >> 6], 1ull << (N & 63));
+		if (N <= cap) atomicOr(&start[0], 1ull);   // the root (a single leaf when N == 1) is the only group
 	}
 	if (i >= N - 1) return;
 	if (node_range[i].y <= cap) return;
@@ -824,28 +819,67 @@ __global__ __launch_bounds__(kBlock) void k_group_flags(int N, const int2* __res
 	for (int k = 0; k < 2; ++k) {
 		const int c = child[k];
 		const int2 rg = c >= N - 1 ? make_int2(c - (N - 1), 1) : node_range[c];
-		if (rg.y <= cap) start[rg.x] = 1u;
+		if (rg.y <= cap) atomicOr(&start[rg.x >> 6], 1ull << (rg.x & 63));
 	}
+}
+
+// The set bits of start in order, as a list (the last is N, the end of the last
+// group), and the number of groups.  A block takes 1024 words; each adds up the
+// words before its own itself, 256 KiB on average at 4M particles, instead of a
+// scan in launches of its own.
+constexpr unsigned kListBlock = 1024;
+__global__ __launch_bounds__(kListBlock) void k_group_list(const unsigned long long* __restrict__ start,
+                                                           unsigned words, unsigned* __restrict__ list,
+                                                           unsigned* __restrict__ n_groups) {
+	__shared__ unsigned s_sum[2][kListBlock / 64];
+	const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6, first = blockIdx.x * kListBlock;
+	unsigned before = 0;
+	for (unsigned i = t; i < first; i += kListBlock) before += (unsigned)__popcll(start[i]);
+	const unsigned long long v = first + t < words ? start[first + t] : 0ull;
+	const unsigned n = (unsigned)__popcll(v);
+	unsigned incl = n;
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1) {
+		const unsigned up = __shfl_up(incl, (unsigned)o);
+		if ((int)lane >= o) incl += up;
+	}
+	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+	if (lane == 63u) s_sum[0][w] = incl;
+	if (lane == 0u) s_sum[1][w] = before;
+	__syncthreads();
+	unsigned at = incl - n;
+	for (unsigned k = 0; k < kListBlock / 64; ++k) at += s_sum[1][k] + (k < w ? s_sum[0][k] : 0u);
+	for (unsigned long long rem = v; rem; rem &= rem - 1ull) list[at++] = 64u * (first + t) + (unsigned)__builtin_ctzll(rem);
+	if (v && first + t + 1u == words) *n_groups = at - 1u;   // the last word holds bit N alone or last
 }
 
 }  // namespace
 
 extern "C" {
 
-unsigned sfd_lbvh_group_flag_len(unsigned N) { return (N + 63u) / 64u * 64u + 64u; }
+unsigned sfd_lbvh_group_words(unsigned N) { return N / 64u + 2u; }
 
-int sfd_lbvh_groups(unsigned N, const void* node_lr, const void* node_range, int cap, unsigned* start,
-                    hipStream_t s) {
+int sfd_lbvh_groups(unsigned N, const void* node_lr, const void* node_range, int cap,
+                    unsigned long long* start, hipStream_t s) {
 	if (N == 0 || cap < 1 || cap > 64) return -1;
-	const unsigned len = sfd_lbvh_group_flag_len(N);
-	hipLaunchKernelGGL(k_fill_u32, dim3((len + kBlock - 1) / kBlock), dim3(kBlock), 0, s, start, len, 0u);
+	const unsigned words = sfd_lbvh_group_words(N);
+	hipLaunchKernelGGL(k_fill_u64, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s, start, words);
 	const unsigned threads = N > 1 ? N - 1 : 1;
 	hipLaunchKernelGGL(k_group_flags, dim3((threads + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (int)N,
 	                   static_cast<const int2*>(node_lr), static_cast<const int2*>(node_range), cap, start);
 	return sf_hip_check(hipGetLastError(), "sfd_lbvh_groups", "launch");
 }
 
-int sfd_lbvh_group_boxes(unsigned N, const void* body, const unsigned* start, const void* node_range,
+int sfd_lbvh_group_list(unsigned N, const unsigned long long* start, unsigned* list, unsigned* n_groups,
+                        hipStream_t s) {
+	if (N == 0) return 0;
+	const unsigned words = N / 64u + 1u;   // bit N is in the last of them
+	hipLaunchKernelGGL(k_group_list, dim3((words + kListBlock - 1u) / kListBlock), dim3(kListBlock), 0, s, start, words,
+	                   list, n_groups);
+	return sf_hip_check(hipGetLastError(), "sfd_lbvh_group_list", "launch");
+}
+
+int sfd_lbvh_group_boxes(unsigned N, const void* body, const unsigned long long* start, const void* node_range,
                          void* node_cell, hipStream_t s) {
 	if (N < 2) return 0;
 	const unsigned chunks = (N + 63u) / 64u;

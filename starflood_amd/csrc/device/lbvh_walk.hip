@@ -30,12 +30,18 @@
 // walk then sums the cells that meet the monopole form of that bound (scaled
 // by kMonoBeta) as monopoles, through the leaf particles' queue.
 //
-// The grid is persistent and sized to the wavefronts resident at once; each
-// wavefront takes runs of 64 sorted positions from a shared counter, walks
-// the groups that start in each, and owns a node stack: its top in LDS, the
-// rest in global memory (deep enough that the 64-wide pops rarely have to
-// narrow).  The self pair is included in leaf sums, as in the reference's PP
-// sum.
+// The grid is persistent and sized to the wavefronts resident at once, or to
+// N / 32 if that is less.  Each wavefront walks the group of its own rank and
+// then takes further ones from a shared counter, and owns a node stack: its top
+// in LDS, the rest in global memory (deep enough that the 64-wide pops rarely
+// have to narrow).  Groups are taken one by one from a list of them: taken by
+// runs of 64 sorted positions, a wavefront had up to three in series while
+// others had none, which at 65537 particles (1570 groups on 1024 SIMDs) was
+// most of the walk: 394 -> 222 us (step 646 -> 487 us alone); 1M step 2661 ->
+// 2518 us alone, 4M quadrupole walk 4 % faster.  A block walking a group
+// together (shared frontier, two barriers a round) took 273 us at 65537 and
+// half as long again at 1M.  The self pair is included in leaf sums, as in the
+// reference's PP sum.
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
@@ -45,6 +51,7 @@ namespace {
 
 constexpr unsigned kBlock = 256;
 constexpr int kWaves = kBlock / 64;
+constexpr unsigned kSpan = 32;      // particles per wavefront of the grid: fewer than an average group's 44
 constexpr int kList = 128;          // queued cells / leaves / particle ids per wavefront
 constexpr int kStack = 8192;        // node ids per wavefront (global memory)
 constexpr int kHead = 160;          // room for a depth-first descent (tree depth <= 96)
@@ -225,13 +232,14 @@ __device__ __forceinline__ void eval_list_quad(Slots& a, int slots, const float4
 // QUAD: cells carry traceless quadrupoles (node_q0, node_q1).
 template <bool QUAD>
 __global__ __launch_bounds__(kBlock, QUAD ? 4 : 5) void k_walk(const float4* __restrict__ body, const unsigned* __restrict__ order,
-                                                 int N, const unsigned* __restrict__ group_start,
+                                                 int N, const unsigned* __restrict__ groups,
+                                                 const unsigned* __restrict__ group_count,
                                                  const float4* __restrict__ rec_a,
                                                  const float4* __restrict__ node_q0, const float* __restrict__ node_q1,
                                                  const int4* __restrict__ rec_b, float alpha_g, float eps2, double G, int acc_phys,
                                                  float* __restrict__ acc, float* __restrict__ pot,
-                                                 unsigned long long* __restrict__ counters, int* __restrict__ gstack,
-                                                 unsigned n_chunks) {
+                                                 unsigned long long* __restrict__ counters,
+                                                 int* __restrict__ gstack) {
 	__shared__ float4 s_cell[kWaves][kList];
 	__shared__ int2 s_leaf[kWaves][kList];
 	__shared__ int s_pid[kWaves][kList];
@@ -256,260 +264,248 @@ __global__ __launch_bounds__(kBlock, QUAD ? 4 : 5) void k_walk(const float4* __r
 	unsigned long long n_cell_tot = 0, n_part_tot = 0, n_batch = 0;
 	unsigned bad = 0;
 
-	// chunks of 64 sorted positions are taken from a shared counter, one
-	// atomic per chunk: walk groups differ in cost (more so under the
-	// relative opening test), and a static split leaves waves idle at the end
-	for (;;) {
-		unsigned long long cw = 0;
-		if (lane == 0) cw = atomicAdd(&counters[5], 1ull);
-		const unsigned c = __builtin_amdgcn_readfirstlane((unsigned)cw);
-		if (c >= n_chunks) break;
-		// the groups that start in sorted positions [64c, 64c + 64); each ends at
-		// the next start flag, at most 64 positions later (start[N] is set)
-		const unsigned at = 64u * c + lane;
-		const unsigned long long e1 = __ballot(group_start[at] != 0u);
-		const unsigned long long e2 = __ballot(group_start[at + 64u] != 0u);
-		unsigned long long rem = e1 & __ballot(at < (unsigned)N);
-		while (rem) {
-			const int s0 = __builtin_ctzll(rem);
-			rem &= rem - 1ull;
-			const unsigned long long above = s0 < 63 ? e1 & (~0ull << (s0 + 1)) : 0ull;
-			const int e0 = above ? __builtin_ctzll(above) : (e2 ? 64 + __builtin_ctzll(e2) : 128);
-			const int base = 64 * (int)c + s0;
-			int cnt = e0 - s0;
-			if (cnt > 64 || cnt > N - base) {   // only a malformed start array gets here
-				bad = 1u;
-				cnt = min(64, N - base);
-			}
-			const int p = base + (int)lane;
-			const bool live = (int)lane < cnt;
-			const int slots = (cnt + 15) / 16;
-			Slots a;
-			float gx0 = 3.0e38f, gy0 = 3.0e38f, gz0 = 3.0e38f, gx1 = -3.0e38f, gy1 = -3.0e38f, gz1 = -3.0e38f;
+	// Each wavefront has a first group of its own and takes further ones from
+	// a shared counter: groups differ in cost (more so under the relative
+	// opening test), and a static split leaves wavefronts idle at the end.
+	const unsigned n_waves = gridDim.x * kWaves, n_groups = *group_count;
+	for (unsigned g = blockIdx.x * kWaves + w; g < n_groups;) {
+		const int base = (int)groups[g];
+		int cnt = (int)groups[g + 1u] - base;
+		if (cnt < 1 || cnt > 64 || base + cnt > N) {   // only a malformed list gets here
+			bad = 1u;
+			break;
+		}
+		const int p = base + (int)lane;
+		const bool live = (int)lane < cnt;
+		const int slots = (cnt + 15) / 16;
+		Slots a;
+		float gx0, gy0, gz0, gx1, gy1, gz1;   // the group's box
 #pragma unroll
-			for (int j = 0; j < kWays; ++j) {
-				const float4 b = body[base + min(16 * j + (int)(lane & 15u), cnt - 1)];
-				a.x[j] = b.x;
-				a.y[j] = b.y;
-				a.z[j] = b.z;
-				gx0 = fminf(gx0, b.x);
-				gy0 = fminf(gy0, b.y);
-				gz0 = fminf(gz0, b.z);
-				gx1 = fmaxf(gx1, b.x);
-				gy1 = fmaxf(gy1, b.y);
-				gz1 = fmaxf(gz1, b.z);
+		for (int j = 0; j < kWays; ++j) {
+			const float4 b = body[base + min(16 * j + (int)(lane & 15u), cnt - 1)];
+			a.x[j] = b.x;
+			a.y[j] = b.y;
+			a.z[j] = b.z;
+			gx0 = j ? fminf(gx0, b.x) : b.x;
+			gy0 = j ? fminf(gy0, b.y) : b.y;
+			gz0 = j ? fminf(gz0, b.z) : b.z;
+			gx1 = j ? fmaxf(gx1, b.x) : b.x;
+			gy1 = j ? fmaxf(gy1, b.y) : b.y;
+			gz1 = j ? fmaxf(gz1, b.z) : b.z;
 #pragma unroll
-				for (int u = 0; u < 4; ++u) a.t[j][u] = 0.0f;
-			}
+			for (int u = 0; u < 4; ++u) a.t[j][u] = 0.0f;
+		}
 #pragma unroll
-			for (int u = 0; u < 4; ++u) a.s[u] = a.c[u] = 0.0f;
-			a.terms = 0;
-			gx0 = wave_min(gx0);
-			gy0 = wave_min(gy0);
-			gz0 = wave_min(gz0);
-			gx1 = wave_max(gx1);
-			gy1 = wave_max(gy1);
-			gz1 = wave_max(gz1);
-			// relative opening test: am = alpha / G times the smallest previous
-			// |a| of the group (0: theta test alone; also when no particle has a
-			// positive finite previous acceleration)
-			float am = 0.0f;
-			if (alpha_g > 0.0f) {
-				float amag = 3.0e38f;
-				if (live) {
-					const unsigned i0 = order[p];
-					const float ax = acc[3u * i0], ay = acc[3u * i0 + 1u], az = acc[3u * i0 + 2u];
-					const float a = sqrtf(ax * ax + ay * ay + az * az);
-					amag = acc_phys ? a : a / body[p].w;   // the reference's acc is m a
-				}
-				amag = wave_min(amag);   // fminf drops NaN
-				am = (amag > 0.0f && amag < 3.0e38f) ? alpha_g * amag : 0.0f;
+		for (int u = 0; u < 4; ++u) a.s[u] = a.c[u] = 0.0f;
+		a.terms = 0;
+		gx0 = wave_min(gx0);
+		gy0 = wave_min(gy0);
+		gz0 = wave_min(gz0);
+		gx1 = wave_max(gx1);
+		gy1 = wave_max(gy1);
+		gz1 = wave_max(gz1);
+		// relative opening test: am = alpha / G times the smallest previous
+		// |a| of the group (0: theta test alone; also when no particle has a
+		// positive finite previous acceleration)
+		float am = 0.0f;
+		if (alpha_g > 0.0f) {
+			float amag = 3.0e38f;
+			if (live) {
+				const unsigned i0 = order[p];
+				const float ax = acc[3u * i0], ay = acc[3u * i0 + 1u], az = acc[3u * i0 + 2u];
+				const float a = sqrtf(ax * ax + ay * ay + az * az);
+				amag = acc_phys ? a : a / body[p].w;   // the reference's acc is m a
 			}
+			amag = wave_min(amag);   // fminf drops NaN
+			am = (amag > 0.0f && amag < 3.0e38f) ? alpha_g * amag : 0.0f;
+		}
 
-			unsigned long long n_cell = 0, n_part = 0, n_mono = 0;
-			unsigned popped = 0;
-			// pending nodes: nt in the LDS top, ng in the global stack
-			int nt = 1, ng = 0, nc = 0, nl = 0, npid = 0;
-			if (lane == 0) top[0] = 0;   // root: internal node 0, or the only leaf when N == 1
-			wave_fence();
+		unsigned long long n_cell = 0, n_part = 0, n_mono = 0;
+		unsigned popped = 0;
+		// pending nodes: nt in the LDS top, ng in the global stack
+		int nt = 1, ng = 0, nc = 0, nl = 0, npid = 0;
+		if (lane == 0) top[0] = 0;   // root: internal node 0, or the only leaf when N == 1
+		wave_fence();
 
-			while (nt + ng > 0 || nc > 0 || nl > 0 || npid > 0) {
-				if (nt + ng > 0) {
-					// pops come from the LDS top first; the global stack grows by at
-					// most 2 k per batch, and by one per batch in the narrow regime
-					const int k = (ng + 128 <= kStack - kHead) ? min(64, nt + ng) : 1;
-					const int kt = min(k, nt);
-					int node = -1;
-					if ((int)lane < kt) node = top[nt - 1 - (int)lane];
-					else if ((int)lane < k) node = stack[ng - 1 - ((int)lane - kt)];
-					nt -= kt;
-					ng -= k - kt;
-					popped += (unsigned)k;
-					++n_batch;
-					wave_fence();
-					if (node >= n_nodes) {
-						node = -1;   // only a malformed tree gets here
-						bad = 1u;
+		while (nt + ng > 0 || nc > 0 || nl > 0 || npid > 0) {
+			if (nt + ng > 0) {
+				// pops come from the LDS top first; the global stack grows by at
+				// most 2 k per batch, and by one per batch in the narrow regime
+				const int k = (ng + 128 <= kStack - kHead) ? min(64, nt + ng) : 1;
+				const int kt = min(k, nt);
+				int node = -1;
+				if ((int)lane < kt) node = top[nt - 1 - (int)lane];
+				else if ((int)lane < k) node = stack[ng - 1 - ((int)lane - kt)];
+				nt -= kt;
+				ng -= k - kt;
+				popped += (unsigned)k;
+				++n_batch;
+				wave_fence();
+				if (node >= n_nodes) {
+					node = -1;   // only a malformed tree gets here
+					bad = 1u;
+				}
+				int cls = 0;   // 0 none, 1 cell, 2 leaf, 3 open, 4 monopole of a quadrupole walk
+				float4 ra = make_float4(0.f, 0.f, 0.f, 0.f);
+				int4 rb = make_int4(0, 0, 0, 0);
+				if (node >= 0) {
+					ra = rec_a[node];
+					rb = rec_b[node];
+					const float dx = fmaxf(fmaxf(gx0 - ra.x, ra.x - gx1), 0.0f);
+					const float dy = fmaxf(fmaxf(gy0 - ra.y, ra.y - gy1), 0.0f);
+					const float dz = fmaxf(fmaxf(gz0 - ra.z, ra.z - gz1), 0.0f);
+					const float d2 = dx * dx + dy * dy + dz * dz;
+					// the sign bit of the r_crit^2 word marks a (first, count) record
+					const bool leafy = rb.x < 0;
+					// relative test: G M l^p <= alpha |a| d^(p+2), p = 2 for a
+					// monopole and 3 for a quadrupole (l = the record's size).  A
+					// quadrupole walk takes a cell that meets the p = 2 bound
+					// (scaled by kMonoBeta) as a monopole, for 13 VALU instead of 34.
+					bool rel = true, mono = false;
+					if (am > 0.0f) {
+						const float l = __int_as_float(rb.w), d4 = d2 * d2;
+						const float ml2 = ra.w * l * l;
+						mono = ml2 <= (QUAD ? kMonoBeta : 1.0f) * am * d4;
+						rel = QUAD ? ml2 * l <= am * d4 * sqrtf(d2) : mono;
 					}
-					int cls = 0;   // 0 none, 1 cell, 2 leaf, 3 open, 4 monopole of a quadrupole walk
-					float4 ra = make_float4(0.f, 0.f, 0.f, 0.f);
-					int4 rb = make_int4(0, 0, 0, 0);
-					if (node >= 0) {
-						ra = rec_a[node];
-						rb = rec_b[node];
-						const float dx = fmaxf(fmaxf(gx0 - ra.x, ra.x - gx1), 0.0f);
-						const float dy = fmaxf(fmaxf(gy0 - ra.y, ra.y - gy1), 0.0f);
-						const float dz = fmaxf(fmaxf(gz0 - ra.z, ra.z - gz1), 0.0f);
-						const float d2 = dx * dx + dy * dy + dz * dz;
-						// the sign bit of the r_crit^2 word marks a (first, count) record
-						const bool leafy = rb.x < 0;
-						// relative test: G M l^p <= alpha |a| d^(p+2), p = 2 for a
-						// monopole and 3 for a quadrupole (l = the record's size).  A
-						// quadrupole walk takes a cell that meets the p = 2 bound
-						// (scaled by kMonoBeta) as a monopole, for 13 VALU instead of 34.
-						bool rel = true, mono = false;
-						if (am > 0.0f) {
-							const float l = __int_as_float(rb.w), d4 = d2 * d2;
-							const float ml2 = ra.w * l * l;
-							mono = ml2 <= (QUAD ? kMonoBeta : 1.0f) * am * d4;
-							rel = QUAD ? ml2 * l <= am * d4 * sqrtf(d2) : mono;
-						}
-						// a cell holds at least two particles (every internal node does)
-						if (d2 > __int_as_float(rb.x & 0x7fffffff) && (!leafy || rb.z > 1) && rel)
-							cls = (QUAD && mono) ? 4 : 1;
-						else if (leafy) cls = 2;
-						else cls = 3;
-					}
-					const unsigned long long m_cell = __ballot(cls == 1);
-					const unsigned long long m_leaf = __ballot(cls == 2);
-					const unsigned long long m_open = __ballot(cls == 3);
-					// monopoles of a quadrupole walk join the particle queue as
-					// negative ids (npid < 64 here, so 64 more fit in pid[])
-					const unsigned long long m_mono = QUAD ? __ballot(cls == 4) : 0ull;
-					if (QUAD && cls == 4) pid[npid + __popcll(m_mono & lt)] = ~node;
-					if (cls == 1) {
-						const int at = nc + __popcll(m_cell & lt);
-						cells[at] = ra;
-						if (QUAD) {
-							const float4 q0 = node_q0[node];
-							cq0[at] = q0;
-							cq1[at] = make_float2(node_q1[node], -q0.x - q0.w);
-						}
-					}
-					if (cls == 2) leaves[nl + __popcll(m_leaf & lt)] = make_int2(rb.y, rb.z);
-					if (cls == 3) {
-						// children fill the LDS top; what does not fit goes to the
-						// global stack
-						const int at = nt + 2 * __popcll(m_open & lt);
-#pragma unroll
-						for (int h = 0; h < 2; ++h) {
-							const int child = h ? rb.z : rb.y;
-							if (at + h < kTop) {
-								top[at + h] = child;
-							} else {
-								const int gi = ng + at + h - kTop;
-								if (gi < kStack) stack[gi] = child;   // always: see kHead
-								else bad = 1u;
-							}
-						}
-					}
-					nc += __popcll(m_cell);
-					nl += __popcll(m_leaf);
-					npid += __popcll(m_mono);
-					n_mono += (unsigned long long)__popcll(m_mono);
-					const int pushed = nt + 2 * __popcll(m_open);
-					ng = min(ng + max(pushed - kTop, 0), kStack);
-					nt = min(pushed, kTop);
-					wave_fence();
-					if (popped > budget) {   // a tree visits each node at most once per group
-						bad = 1u;
-						nt = ng = 0;
+					// a cell holds at least two particles (every internal node does)
+					if (d2 > __int_as_float(rb.x & 0x7fffffff) && (!leafy || rb.z > 1) && rel)
+						cls = (QUAD && mono) ? 4 : 1;
+					else if (leafy) cls = 2;
+					else cls = 3;
+				}
+				const unsigned long long m_cell = __ballot(cls == 1);
+				const unsigned long long m_leaf = __ballot(cls == 2);
+				const unsigned long long m_open = __ballot(cls == 3);
+				// monopoles of a quadrupole walk join the particle queue as
+				// negative ids (npid < 64 here, so 64 more fit in pid[])
+				const unsigned long long m_mono = QUAD ? __ballot(cls == 4) : 0ull;
+				if (QUAD && cls == 4) pid[npid + __popcll(m_mono & lt)] = ~node;
+				if (cls == 1) {
+					const int at = nc + __popcll(m_cell & lt);
+					cells[at] = ra;
+					if (QUAD) {
+						const float4 q0 = node_q0[node];
+						cq0[at] = q0;
+						cq1[at] = make_float2(node_q1[node], -q0.x - q0.w);
 					}
 				}
-				const bool drain = nt + ng == 0;
-				// monopoles
-				if (nc >= 64 || (drain && nc > 0)) {
-					const int take = min(nc, 64);
-					if (QUAD) eval_list_quad(a, slots, cells, cq0, cq1, take, row, eps2);
-					else eval_list(a, slots, cells, take, row, eps2);
-					n_cell += (unsigned long long)take;
-					wave_fence();
-					if ((int)lane < nc - take) {
-						cells[lane] = cells[take + lane];
-						if (QUAD) {
-							cq0[lane] = cq0[take + lane];
-							cq1[lane] = cq1[take + lane];
+				if (cls == 2) leaves[nl + __popcll(m_leaf & lt)] = make_int2(rb.y, rb.z);
+				if (cls == 3) {
+					// children fill the LDS top; what does not fit goes to the
+					// global stack
+					const int at = nt + 2 * __popcll(m_open & lt);
+#pragma unroll
+					for (int h = 0; h < 2; ++h) {
+						const int child = h ? rb.z : rb.y;
+						if (at + h < kTop) {
+							top[at + h] = child;
+						} else {
+							const int gi = ng + at + h - kTop;
+							if (gi < kStack) stack[gi] = child;   // always: see kHead
+							else bad = 1u;
 						}
 					}
-					nc -= take;
-					wave_fence();
 				}
-				// leaves: expand into particle ids, then gather and sum 64 at a time
-				if (nl >= 64 || npid >= 64 || (drain && (nl > 0 || npid > 0))) {
-					int q = 0;
-					while (q < nl || npid >= 64 || (drain && npid > 0)) {
-						if (q < nl && npid < 64) {
-							// up to 64 leaves at once, one per lane: an inclusive scan of
-							// their counts places each leaf's particle ids after the
-							// previous ones; the leaves that fit in pid[] (a prefix, the
-							// scan being nondecreasing, and at least the first: counts
-							// are at most 64 and npid < 64) are taken
-							const int li = q + (int)lane;
-							const int2 lf = li < nl ? leaves[li] : make_int2(0, 0);
-							int incl = lf.y;
+				nc += __popcll(m_cell);
+				nl += __popcll(m_leaf);
+				npid += __popcll(m_mono);
+				n_mono += (unsigned long long)__popcll(m_mono);
+				const int pushed = nt + 2 * __popcll(m_open);
+				ng = min(ng + max(pushed - kTop, 0), kStack);
+				nt = min(pushed, kTop);
+				wave_fence();
+				if (popped > budget) {   // a tree visits each node at most once per group
+					bad = 1u;
+					nt = ng = 0;
+				}
+			}
+			const bool drain = nt + ng == 0;
+			// monopoles
+			if (nc >= 64 || (drain && nc > 0)) {
+				const int take = min(nc, 64);
+				if (QUAD) eval_list_quad(a, slots, cells, cq0, cq1, take, row, eps2);
+				else eval_list(a, slots, cells, take, row, eps2);
+				n_cell += (unsigned long long)take;
+				wave_fence();
+				if ((int)lane < nc - take) {
+					cells[lane] = cells[take + lane];
+					if (QUAD) {
+						cq0[lane] = cq0[take + lane];
+						cq1[lane] = cq1[take + lane];
+					}
+				}
+				nc -= take;
+				wave_fence();
+			}
+			// leaves: expand into particle ids, then gather and sum 64 at a time
+			if (nl >= 64 || npid >= 64 || (drain && (nl > 0 || npid > 0))) {
+				int q = 0;
+				while (q < nl || npid >= 64 || (drain && npid > 0)) {
+					if (q < nl && npid < 64) {
+						// up to 64 leaves at once, one per lane: an inclusive scan of
+						// their counts places each leaf's particle ids after the
+						// previous ones; the leaves that fit in pid[] (a prefix, the
+						// scan being nondecreasing, and at least the first: counts
+						// are at most 64 and npid < 64) are taken
+						const int li = q + (int)lane;
+						const int2 lf = li < nl ? leaves[li] : make_int2(0, 0);
+						int incl = lf.y;
 #pragma unroll
-							for (int o = 1; o < 64; o <<= 1) {
-								const int v = __shfl_up(incl, (unsigned)o);
-								if ((int)lane >= o) incl += v;
-							}
-							const bool fits = li < nl && npid + incl <= kList;
-							const int k = __popcll(__ballot(fits));
-							const int total = __builtin_amdgcn_readlane(incl, k - 1);
-							if (fits) {
-								const int at = npid + incl - lf.y;
-								for (int j = 0; j < lf.y; ++j) pid[at + j] = lf.x + j;
-							}
-							npid += total;
-							q += k;
+						for (int o = 1; o < 64; o <<= 1) {
+							const int v = __shfl_up(incl, (unsigned)o);
+							if ((int)lane >= o) incl += v;
+						}
+						const bool fits = li < nl && npid + incl <= kList;
+						const int k = __popcll(__ballot(fits));
+						const int total = __builtin_amdgcn_readlane(incl, k - 1);
+						if (fits) {
+							const int at = npid + incl - lf.y;
+							for (int j = 0; j < lf.y; ++j) pid[at + j] = lf.x + j;
+						}
+						npid += total;
+						q += k;
+					}
+					wave_fence();
+					if (npid >= 64 || (drain && q == nl && npid > 0)) {
+						const int take = min(npid, 64);
+						if ((int)lane < take) {
+							const int id = pid[lane];
+							part[lane] = (!QUAD || id >= 0) ? body[id] : rec_a[~id];
 						}
 						wave_fence();
-						if (npid >= 64 || (drain && q == nl && npid > 0)) {
-							const int take = min(npid, 64);
-							if ((int)lane < take) {
-								const int id = pid[lane];
-								part[lane] = (!QUAD || id >= 0) ? body[id] : rec_a[~id];
-							}
-							wave_fence();
-							eval_list(a, slots, part, take, row, eps2);
-							n_part += (unsigned long long)take;
-							wave_fence();
-							if ((int)lane < npid - take) pid[lane] = pid[take + (int)lane];
-							npid -= take;
-							wave_fence();
-						} else {
-							break;
-						}
+						eval_list(a, slots, part, take, row, eps2);
+						n_part += (unsigned long long)take;
+						wave_fence();
+						if ((int)lane < npid - take) pid[lane] = pid[take + (int)lane];
+						npid -= take;
+						wave_fence();
+					} else {
+						break;
 					}
-					wave_fence();
-					if ((int)lane < nl - q) leaves[lane] = leaves[q + (int)lane];
-					nl -= q;
-					wave_fence();
 				}
+				wave_fence();
+				if ((int)lane < nl - q) leaves[lane] = leaves[q + (int)lane];
+				nl -= q;
+				wave_fence();
 			}
-			fold(a);
-			if (live) {
-				const unsigned i = order[p];
-				const double sx = (double)a.s[0] - (double)a.c[0], sy = (double)a.s[1] - (double)a.c[1],
-				             sz = (double)a.s[2] - (double)a.c[2], sp2 = (double)a.s[3] - (double)a.c[3];
-				const double f = acc_phys ? G : G * (double)body[p].w;
-				acc[3u * i + 0u] = (float)(f * sx);
-				acc[3u * i + 1u] = (float)(f * sy);
-				acc[3u * i + 2u] = (float)(f * sz);
-				pot[i] = (float)(-G * sp2);
-			}
-			n_cell_tot += (n_cell + n_mono) * (unsigned long long)cnt;
-			n_part_tot += (n_part - n_mono) * (unsigned long long)cnt;
 		}
+		fold(a);
+		if (live) {
+			const unsigned i = order[p];
+			const double sx = (double)a.s[0] - (double)a.c[0], sy = (double)a.s[1] - (double)a.c[1],
+			             sz = (double)a.s[2] - (double)a.c[2], sp2 = (double)a.s[3] - (double)a.c[3];
+			const double f = acc_phys ? G : G * (double)body[p].w;
+			acc[3u * i + 0u] = (float)(f * sx);
+			acc[3u * i + 1u] = (float)(f * sy);
+			acc[3u * i + 2u] = (float)(f * sz);
+			pot[i] = (float)(-G * sp2);
+		}
+		n_cell_tot += (n_cell + n_mono) * (unsigned long long)cnt;
+		n_part_tot += (n_part - n_mono) * (unsigned long long)cnt;
+		if (n_groups <= n_waves) break;
+		if (lane == 0) g = n_waves + (unsigned)atomicAdd(&counters[5], 1ull);
+		g = __builtin_amdgcn_readfirstlane(g);
 	}
 	const bool any_bad = __ballot(bad != 0u) != 0ull;
 	if (counters && lane == 0) {
@@ -556,29 +552,28 @@ extern "C" {
 
 size_t sfd_lbvh_walk_stack_bytes(void) { return (size_t)resident_blocks() * kWaves * kStack * sizeof(int); }
 
-int sfd_lbvh_walk(const void* body, const unsigned* order, unsigned N, const unsigned* group_start,
+int sfd_lbvh_walk(const void* body, const unsigned* order, unsigned N, const unsigned* groups, const unsigned* n_groups,
                   const void* node_cm, const void* node_q0, const float* node_q1, const void* rec_b,
                   float alpha_g, float eps2, double G, int acc_phys, float* acc, float* pot,
                   unsigned long long* counters, int* gstack, hipStream_t s) {
 	if (N == 0) return 0;
-	if (!counters || !gstack || !group_start) return -1;
+	if (!counters || !gstack || !groups || !n_groups) return -1;
 	const bool quad = node_q0 && node_q1;
-	const unsigned chunks = (N + 63) / 64;   // group_start holds 64 * (chunks + 1) flags
-	unsigned blocks = (chunks + kWaves - 1) / kWaves;
 	const unsigned resident = quad ? resident_blocks_of<true>() : resident_blocks_of<false>();
+	unsigned blocks = (N + kWaves * kSpan - 1u) / (kWaves * kSpan);
 	if (blocks > resident) blocks = resident;   // gstack holds resident_blocks() >= resident slots
 	hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, s, counters);
 	const int tok = sf_prof_begin("lbvh_walk", s);
 	if (quad)
 		hipLaunchKernelGGL(k_walk<true>, dim3(blocks), dim3(kBlock), 0, s, static_cast<const float4*>(body), order,
-		                   (int)N, group_start, static_cast<const float4*>(node_cm),
+		                   (int)N, groups, n_groups, static_cast<const float4*>(node_cm),
 		                   static_cast<const float4*>(node_q0), node_q1, static_cast<const int4*>(rec_b),
-		                   alpha_g, eps2, G, acc_phys, acc, pot, counters, gstack, chunks);
+		                   alpha_g, eps2, G, acc_phys, acc, pot, counters, gstack);
 	else
 		hipLaunchKernelGGL(k_walk<false>, dim3(blocks), dim3(kBlock), 0, s, static_cast<const float4*>(body), order,
-		                   (int)N, group_start, static_cast<const float4*>(node_cm), (const float4*)nullptr,
+		                   (int)N, groups, n_groups, static_cast<const float4*>(node_cm), (const float4*)nullptr,
 		                   (const float*)nullptr, static_cast<const int4*>(rec_b), alpha_g, eps2, G, acc_phys,
-		                   acc, pot, counters, gstack, chunks);
+		                   acc, pot, counters, gstack);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_lbvh_walk", "launch");
 }

@@ -107,14 +107,15 @@ int sfd_lbvh_records(unsigned int N, const void* node_lr, const void* node_range
 /* lbvh_walk.hip.  counters (6 x u64; all but the fifth zeroed here): cell
    interactions, particle interactions, wavefronts that met a malformed tree,
    node batches; the fifth adds the third up over walks until the host clears
-   it; the sixth hands out the chunks of 64 sorted positions.
+   it; the sixth hands out the groups (sfd_lbvh_group_list's).
    gstack: sfd_lbvh_walk_stack_bytes() of scratch.  alpha_g > 0 adds the
    relative opening test M l^p <= alpha_g |a|_min d^(p+2) (l the records'
    size, p = 2 for monopole cells and 3 for quadrupole cells; a quadrupole
    walk takes the cells that meet p = 2 as monopoles), |a|_min over each
    group's previous acc. */
 size_t sfd_lbvh_walk_stack_bytes(void);
-int sfd_lbvh_walk(const void* body, const unsigned int* order, unsigned int N, const unsigned int* group_start,
+int sfd_lbvh_walk(const void* body, const unsigned int* order, unsigned int N, const unsigned int* groups,
+                  const unsigned int* n_groups,
                   const void* node_cm, const void* node_q0, const float* node_q1, const void* rec_b,
                   float alpha_g, float eps2, double G, int acc_phys, float* acc, float* pot,
                   unsigned long long* counters, int* gstack, hipStream_t s);
@@ -126,16 +127,19 @@ int sfd_lbvh_quadrupoles(unsigned int N, const void* body, const void* node_rang
                          const double* box, void* prefix2, void* tile_sum2, double* ref, void* node_q0,
                          float* node_q1, hipStream_t s);
 
-/* walk groups: start[p] = 1 where a maximal subtree of at most cap (<= 64)
-   particles begins in sorted order, and start[N] = 1; start holds
-   sfd_lbvh_group_flag_len(N) entries (lbvh.hip) */
-unsigned int sfd_lbvh_group_flag_len(unsigned int N);
-int sfd_lbvh_groups(unsigned int N, const void* node_lr, const void* node_range, int cap, unsigned int* start,
+/* walk groups: bit p of start is set where a maximal subtree of at most cap
+   (<= 64) particles begins in sorted order, and bit N; start holds
+   sfd_lbvh_group_words(N) words (lbvh.hip) */
+unsigned int sfd_lbvh_group_words(unsigned int N);
+int sfd_lbvh_groups(unsigned int N, const void* node_lr, const void* node_range, int cap, unsigned long long* start,
                     hipStream_t s);
+/* the set bits of start in order (groups + 1 <= max(2, N) entries) and the number of groups */
+int sfd_lbvh_group_list(unsigned int N, const unsigned long long* start, unsigned int* list, unsigned int* n_groups,
+                        hipStream_t s);
 /* the particle boxes of the internal nodes of at most 64 particles into
    node_cell (their other entries come from sfd_lbvh_topology); start: the
    groups of sfd_lbvh_groups with cap 64 */
-int sfd_lbvh_group_boxes(unsigned int N, const void* body, const unsigned int* start, const void* node_range,
+int sfd_lbvh_group_boxes(unsigned int N, const void* body, const unsigned long long* start, const void* node_range,
                          void* node_cell, hipStream_t s);
 
 #ifdef __cplusplus

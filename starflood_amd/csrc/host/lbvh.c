@@ -19,7 +19,7 @@ struct sf_lbvh {
 	unsigned long long* key0;
 	unsigned long long* key1;
 	unsigned int* val0;
-	unsigned int* val1;
+	unsigned int* val1;       /* after the build: the walk groups' first sorted positions, then N */
 	unsigned int* hist;
 	double* bbox_part;
 	double* box;
@@ -32,10 +32,11 @@ struct sf_lbvh {
 	void* node_cell;          /* 2N-1 float4: Morton cell centre, side */
 	void* rec_b;              /* 2N-1 int4 */
 	unsigned long long* counters;   /* 6: the walk's four (zeroed per walk), the sticky guard count, the
-	                                   walk's chunk counter (zeroed per walk) */
+	                                   walk's group counter (zeroed per walk) */
 	unsigned long long* h_counters; /* pinned */
 	int* gstack;                    /* walk node stacks, one per wavefront slot */
-	unsigned int* group_start;      /* walk group starts in sorted order */
+	unsigned long long* group_start;   /* bits: walk group starts in sorted order */
+	unsigned int* n_groups;
 	/* quadrupoles (allocated on first use) */
 	void* prefix2;                  /* N x 6 doubles: inclusive m x' x'^T sums */
 	void* tile_sum2;
@@ -48,7 +49,7 @@ struct sf_lbvh {
 static void free_buffers(sf_lbvh* t) {
 	void* ptrs[] = {t->key0, t->key1, t->val0, t->val1, t->hist, t->bbox_part, t->box, t->body, t->node_lr,
 	                t->node_range, t->prefix, t->tile_sum, t->node_cm, t->node_cell, t->rec_b, t->counters,
-	                t->gstack, t->group_start, t->prefix2, t->tile_sum2, t->quad_ref, t->node_q0, t->node_q1};
+	                t->gstack, t->group_start, t->n_groups, t->prefix2, t->tile_sum2, t->quad_ref, t->node_q0, t->node_q1};
 	for (size_t k = 0; k < sizeof(ptrs) / sizeof(ptrs[0]); ++k)
 		if (ptrs[k]) hipFree(ptrs[k]);
 	if (t->h_counters) hipHostFree(t->h_counters);
@@ -98,7 +99,8 @@ static int ensure(sf_lbvh** st, unsigned int N) {
 	rc |= alloc(&t->rec_b, nn * 16u);
 	rc |= alloc((void**)&t->counters, 6u * 8u);
 	rc |= alloc((void**)&t->gstack, sfd_lbvh_walk_stack_bytes());
-	rc |= alloc((void**)&t->group_start, (size_t)sfd_lbvh_group_flag_len(N) * 4u);
+	rc |= alloc((void**)&t->n_groups, 4u);
+	rc |= alloc((void**)&t->group_start, (size_t)sfd_lbvh_group_words(N) * 8u);
 	if (!rc && hipHostMalloc((void**)&t->h_counters, 5u * 8u, hipHostMallocDefault) != hipSuccess) rc = -1;
 	/* the sticky guard count starts at zero (the walk resets only the first four) */
 	if (!rc && (hipMemset(t->counters, 0, 6u * 8u) != hipSuccess || hipDeviceSynchronize() != hipSuccess)) rc = -1;
@@ -160,6 +162,8 @@ int sf_lbvh_build(sf_lbvh** st, unsigned int N, const float* pos, const float* m
 	                      t->node_cm, t->node_cell, s))
 		return -1;
 	if (sfd_lbvh_groups(N, t->node_lr, t->node_range, SF_LBVH_GROUP, t->group_start, s)) return -1;
+	/* the sort is done with val1 */
+	if (sfd_lbvh_group_list(N, t->group_start, t->val1, t->n_groups, s)) return -1;
 	if (sfd_lbvh_group_boxes(N, t->body, t->group_start, t->node_range, t->node_cell, s)) return -1;
 	if (quadrupole) {
 		if (sfd_lbvh_quadrupoles(N, t->body, t->node_range, t->prefix, t->box, t->prefix2, t->tile_sum2, t->quad_ref,
@@ -193,7 +197,7 @@ int sf_lbvh_walk(sf_lbvh* t, unsigned int N, const float* pos, const float* mas,
 		return -1;
 	/* G M l^p <= alpha |a| d^(p+2)  <=>  M l^p <= (alpha / G) |a| d^(p+2) */
 	const float alpha_g = (prev_acc && p->mac_alpha > 0.0) ? (float)(p->mac_alpha / p->G) : 0.0f;
-	return sfd_lbvh_walk(t->body, t->val0, N, t->group_start, t->node_cm, quad ? t->node_q0 : NULL,
+	return sfd_lbvh_walk(t->body, t->val0, N, t->val1, t->n_groups, t->node_cm, quad ? t->node_q0 : NULL,
 	                     quad ? t->node_q1 : NULL, t->rec_b, alpha_g, (float)(p->epsilon * p->epsilon),
 	                     p->G, p->acc_mode == SF_ACC_PHYSICAL, acc, pot, t->counters, t->gstack, s);
 }

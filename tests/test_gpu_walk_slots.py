@@ -37,3 +37,29 @@ def test_slots_close_to_fp64(N, quad, acc_mode):
         assert np.abs(acc[i] - w @ d).max() <= 2e-6 * (w * np.sqrt((d * d).sum(1))).sum(), i
         p = (m / np.sqrt(s2)).sum()
         assert abs(pot[i] + p) <= 2e-6 * p, i
+
+
+@pytest.mark.parametrize("N", [65535, 65536, 65537, 131072, 230001, 400000])
+def test_every_group_is_walked(N):
+    """The group list at the edges of its blocks (65536 positions) and with
+    more groups than wavefronts.  A cell is accepted from d > l / theta + its
+    centre's offset, so its monopole is wrong by at most 3 (theta / 2)^2 =
+    0.12 of its size; a particle of a group left out would keep pot = 0."""
+    print(f"walk groups N={N}", flush=True)
+    rng = np.random.default_rng(N)
+    with Simulation(N, enable_tree=1, tree_mode=L.SF_TREE_LBVH, theta=0.4, leaf_size=3, logging=0, epsilon=EPS,
+                    precision=L.SF_PRECISION_FAST, acc_mode=L.SF_ACC_PHYSICAL) as s:
+        s.pos[:] = rng.normal(size=(N, 3)).astype(np.float32)
+        s.mas[:] = np.float32(1.0 / N)
+        s.solve()
+        x, m = s.pos.astype(np.float64), s.mas.astype(np.float64)
+        acc, pot = s.acc.astype(np.float64), s.pot.astype(np.float64)
+    L.set_params()
+    assert pot.max() < 0.0
+    for i in np.linspace(0, N - 1, 24).astype(int):
+        d = x - x[i]
+        s2 = (d * d).sum(1) + EPS * EPS
+        w = m * s2 ** -1.5
+        assert np.abs(acc[i] - w @ d).max() <= 0.12 * (w * np.sqrt((d * d).sum(1))).sum(), i
+        p = (m / np.sqrt(s2)).sum()
+        assert abs(pot[i] + p) <= 0.12 * p, i
