@@ -31,8 +31,7 @@
 namespace {
 
 constexpr unsigned kBlock = 256;
-constexpr unsigned kTile = 4096;          // radix sort tile (256 threads x 16)
-constexpr unsigned kRadixRounds = kTile / kBlock;
+constexpr unsigned kTile = 4096;          // radix sorts take multiples of this
 
 __global__ __launch_bounds__(kBlock) void k_fill_u64(unsigned long long* __restrict__ p, unsigned n) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
@@ -141,143 +140,123 @@ __global__ __launch_bounds__(kBlock) void k_morton(const float* __restrict__ pos
 }
 
 // ---------------------------------------------------------------- radix sort
-__global__ __launch_bounds__(kBlock) void k_radix_hist(const unsigned long long* __restrict__ key, unsigned shift,
-                                                       unsigned ntiles, unsigned* __restrict__ hist) {
-	__shared__ unsigned h[256];
-	h[threadIdx.x] = 0;
+// Stable LSD sort on 8-bit digits: k_radix_digits counts every pass's digits
+// at once, k_radix_offsets turns the counts into each digit's first position,
+// and one k_radix_pass per digit ranks, exchanges its tile counts and
+// scatters.  A pass of histogram, scan and scatter launches took 20.3 us at
+// 65536 pairs, 35 at 1M and 60 at 4M; k_radix_pass takes 8.1, 20 and 44, the
+// two launches before the passes together 9, 16 and 29.  At 65536 pairs a pass
+// is the latency of its chain (load, rank, post, collect, write); from 1M on
+// the collection is a third of it: every tile running at once looks back at
+// those before it (two at a time; 1 and 4 take 21 us at 1M, 8 take 21.3, 32
+// take 27).
+
+// A block's digit counts for the first `passes` digits, and the state of the
+// first pass cleared.
+constexpr unsigned kDigitBlocks = 256, kDigitThreads = 1024;
+__global__ __launch_bounds__(kDigitThreads) void k_radix_digits(const unsigned long long* __restrict__ key, unsigned n,
+                                                         unsigned passes, unsigned* __restrict__ part,
+                                                         unsigned long long* __restrict__ state, unsigned state_len,
+                                                         unsigned* __restrict__ tickets) {
+	__shared__ unsigned h[8][256];
+	const unsigned t = threadIdx.x, first = blockIdx.x * kDigitThreads + t, stride = gridDim.x * kDigitThreads;
+	for (unsigned i = t; i < passes * 256u; i += kDigitThreads) (&h[0][0])[i] = 0u;
+	if (blockIdx.x == 0u && t < 8u) tickets[t] = 0u;
+	for (unsigned i = first; i < state_len; i += stride) state[i] = 0ull;
 	__syncthreads();
-	const unsigned base = blockIdx.x * kTile;
-	for (unsigned r = 0; r < kRadixRounds; ++r) {
-		const unsigned d = (unsigned)(key[base + r * kBlock + threadIdx.x] >> shift) & 255u;
-		atomicAdd(&h[d], 1u);
+	for (unsigned i = first; i < n; i += stride) {
+		const unsigned long long k = key[i];
+		for (unsigned p = 0; p < passes; ++p) {
+			const unsigned d = (unsigned)(k >> (8u * p)) & 255u;
+			// the high digits are often the same on every lane
+			const unsigned long long on = __ballot(true);
+			if (__ballot(d == __builtin_amdgcn_readfirstlane(d)) == on) {
+				if (t % 64u == (unsigned)__builtin_ctzll(on)) atomicAdd(&h[p][d], (unsigned)__popcll(on));
+			} else {
+				atomicAdd(&h[p][d], 1u);
+			}
+		}
 	}
 	__syncthreads();
-	hist[threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+	for (unsigned i = t; i < passes * 256u; i += kDigitThreads)
+		part[(i / 256u * gridDim.x + blockIdx.x) * 256u + i % 256u] = (&h[0][0])[i];
 }
 
-// Exclusive scan of the digit-major histogram (256 * ntiles entries) in three
-// passes: per-chunk totals (k_scan_u32_sums), an exclusive scan of the chunk
-// totals in one block (k_radix_scan), and the scan of each chunk from its
-// offset (k_scan_u32_down).  A chunk is 4096 entries, 16 per thread.
-constexpr unsigned kScanU32Per = 16;
-constexpr unsigned kScanU32Chunk = kBlock * kScanU32Per;
-
-__global__ __launch_bounds__(kBlock) void k_scan_u32_sums(const unsigned* __restrict__ data, unsigned n,
-                                                          unsigned* __restrict__ sums) {
+// One block per pass: the digits' exclusive prefix over all blocks' counts.
+__global__ __launch_bounds__(kBlock) void k_radix_offsets(const unsigned* __restrict__ part, unsigned rows,
+                                                          unsigned* __restrict__ offs) {
 	__shared__ unsigned ws[kBlock / 64];
-	const unsigned base = blockIdx.x * kScanU32Chunk + threadIdx.x * kScanU32Per;
-	unsigned s = 0;
-#pragma unroll
-	for (unsigned k = 0; k < kScanU32Per; ++k) s += base + k < n ? data[base + k] : 0u;
-	for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-	if ((threadIdx.x & 63u) == 0) ws[threadIdx.x >> 6] = s;
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		unsigned t = 0;
-		for (unsigned q = 0; q < kBlock / 64; ++q) t += ws[q];
-		sums[blockIdx.x] = t;
-	}
-}
-
-__global__ __launch_bounds__(kBlock) void k_scan_u32_down(unsigned* __restrict__ data, unsigned n,
-                                                          const unsigned* __restrict__ offs) {
-	__shared__ unsigned ws[kBlock / 64];
-	const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-	const unsigned base = blockIdx.x * kScanU32Chunk + threadIdx.x * kScanU32Per;
-	unsigned v[kScanU32Per];
-	unsigned s = 0;
-#pragma unroll
-	for (unsigned k = 0; k < kScanU32Per; ++k) {
-		v[k] = base + k < n ? data[base + k] : 0u;
-		s += v[k];
-	}
-	unsigned inc = s;
+	const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
+	unsigned n = 0;
+#pragma unroll 16
+	for (unsigned r = 0; r < rows; ++r) n += part[(blockIdx.x * rows + r) * 256u + t];
+	unsigned inc = n;
 	for (int o = 1; o < 64; o <<= 1) {
-		const unsigned t = __shfl_up(inc, o);
-		if ((int)lane >= o) inc += t;
+		const unsigned v = __shfl_up(inc, (unsigned)o);
+		if ((int)lane >= o) inc += v;
 	}
 	if (lane == 63u) ws[w] = inc;
 	__syncthreads();
-	unsigned run = offs[blockIdx.x] + inc - s;
-	for (unsigned q = 0; q < w; ++q) run += ws[q];
-#pragma unroll
-	for (unsigned k = 0; k < kScanU32Per; ++k) {
-		if (base + k < n) data[base + k] = run;
-		run += v[k];
-	}
+	unsigned excl = inc - n;
+	for (unsigned q = 0; q < w; ++q) excl += ws[q];
+	offs[blockIdx.x * 256u + t] = excl;
 }
 
-// Exclusive scan of n entries in one block: each thread scans a contiguous
-// chunk, then the chunk totals (the top level of the histogram scan).
-__global__ __launch_bounds__(1024) void k_radix_scan(unsigned* __restrict__ hist, unsigned n) {
-	__shared__ unsigned tot[1024];
-	const unsigned chunk = (n + 1023) / 1024;
-	const unsigned b = threadIdx.x * chunk, e = min(b + chunk, n);
-	unsigned s = 0;
-	for (unsigned k = b; k < e; ++k) s += hist[k];
-	tot[threadIdx.x] = s;
-	__syncthreads();
-	for (unsigned off = 1; off < 1024; off <<= 1) {
-		const unsigned v = threadIdx.x >= off ? tot[threadIdx.x - off] : 0u;
-		__syncthreads();
-		tot[threadIdx.x] += v;
-		__syncthreads();
-	}
-	unsigned run = threadIdx.x ? tot[threadIdx.x - 1] : 0u;
-	for (unsigned k = b; k < e; ++k) {
-		const unsigned v = hist[k];
-		hist[k] = run;
-		run += v;
-	}
+// State word of a tile's digit: nothing yet, the tile's own count, or the
+// count of the tile and all before it.
+constexpr unsigned long long kOwn = 1ull << 32, kAll = 2ull << 32;
+
+__device__ __forceinline__ unsigned long long peek(const unsigned long long* p) {
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void post(unsigned long long* p, unsigned long long v) {
+	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Stable scatter of one 4096-element tile.  Each wavefront ranks its 1024
+// One digit's pass over a tile of 256 PER pairs.  Each wavefront ranks its
 // consecutive elements in index order (a 64-lane match mask from eight
-// ballots per round, and per-wave running digit counts in LDS), the tile is
-// staged in LDS in sorted order, and it is written out by consecutive
-// threads, so that each digit's run goes to consecutive global addresses.
-// The tile's digit counts are differences of consecutive entries of the
-// scanned histogram (offs[256 * ntiles] would be n_total).
-constexpr unsigned kScatterPer = kTile / kBlock;          // elements per thread
-constexpr unsigned kWaveSpan = kTile / (kBlock / 64);     // elements per wavefront
-
-__global__ __launch_bounds__(kBlock) void k_radix_scatter(const unsigned long long* __restrict__ key_in,
-                                                          const unsigned* __restrict__ val_in, unsigned shift,
-                                                          unsigned ntiles, const unsigned* __restrict__ offs,
-                                                          unsigned n_total, unsigned long long* __restrict__ key_out,
-                                                          unsigned* __restrict__ val_out) {
-	__shared__ unsigned long long s_key[kTile];
-	__shared__ unsigned s_val[kTile];
+// ballots per round, and per-wave running digit counts in LDS); the tile's
+// counts are posted, the counts of the tiles before it collected (thread t:
+// digit t), the tile is staged in LDS in sorted order and written out by
+// consecutive threads, so that each digit's run goes to consecutive global
+// addresses.
+// Tiles are numbered by a ticket taken when a block starts, so the tiles
+// before one's own belong to blocks that have started; a block posts its own
+// counts before it waits for anything, so every wait ends.
+template <unsigned PER>
+__global__ __launch_bounds__(kBlock) void k_radix_pass(const unsigned long long* __restrict__ key_in,
+                                                       const unsigned* __restrict__ val_in, unsigned shift,
+                                                       const unsigned* __restrict__ offs,
+                                                       unsigned long long* state, unsigned long long* state_next,
+                                                       unsigned* ticket, unsigned long long* __restrict__ key_out,
+                                                       unsigned* __restrict__ val_out) {
+	constexpr unsigned kLook = 2;   // tiles looked back at once
+	__shared__ unsigned long long s_key[kBlock * PER];
+	__shared__ unsigned s_val[kBlock * PER];
 	__shared__ unsigned s_wcnt[kBlock / 64][256];   // running counts, then each wave's prefix
 	__shared__ unsigned s_start[256];               // the digit's first slot in the tile
 	__shared__ unsigned s_base[256];                // the digit's first global position of this tile
 	__shared__ unsigned s_wsum[kBlock / 64];
+	__shared__ unsigned s_tile;
 	const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
-	const unsigned at = t * ntiles + blockIdx.x;
-	const unsigned o = offs[at];
-	const unsigned cnt = (at + 1u < 256u * ntiles ? offs[at + 1u] : n_total) - o;
-	s_base[t] = o;
-	// exclusive scan of the tile's 256 digit counts
-	unsigned inc = cnt;
-	for (int k = 1; k < 64; k <<= 1) {
-		const unsigned v = __shfl_up(inc, (unsigned)k);
-		if ((int)lane >= k) inc += v;
-	}
-	if (lane == 63u) s_wsum[w] = inc;
-	for (unsigned q = 0; q < kBlock / 64; ++q) s_wcnt[q][t] = 0;
+	if (t == 0u) s_tile = atomicAdd(ticket, 1u);
+	for (unsigned q = 0; q < kBlock / 64; ++q) s_wcnt[q][t] = 0u;
 	__syncthreads();
-	unsigned excl = inc - cnt;
-	for (unsigned q = 0; q < w; ++q) excl += s_wsum[q];
-	s_start[t] = excl;
-	// rank: element r of this thread is tile element w * kWaveSpan + 64 r + lane
+	const unsigned tile = __builtin_amdgcn_readfirstlane(s_tile);
+	state_next[(size_t)tile * 256u + t] = 0ull;
+	// rank: element r of this thread is tile element (w PER + r) 64 + lane
 	const unsigned long long lt = (1ull << lane) - 1ull;
-	const unsigned g0 = blockIdx.x * kTile + w * kWaveSpan + lane;
-	unsigned long long kr[kScatterPer];
-	unsigned vr[kScatterPer], pk[kScatterPer];
+	const size_t g0 = (size_t)tile * (kBlock * PER) + w * (64u * PER) + lane;
+	unsigned long long kr[PER];
+	unsigned vr[PER], pk[PER];
 #pragma unroll
-	for (unsigned r = 0; r < kScatterPer; ++r) {
-		const unsigned long long k = key_in[g0 + 64u * r];
-		const unsigned d = (unsigned)(k >> shift) & 255u;
+	for (unsigned r = 0; r < PER; ++r) {
+		kr[r] = key_in[g0 + 64u * r];
+		vr[r] = val_in[g0 + 64u * r];
+	}
+#pragma unroll
+	for (unsigned r = 0; r < PER; ++r) {
+		const unsigned d = (unsigned)(kr[r] >> shift) & 255u;
 		unsigned long long match = ~0ull;
 		for (int bit = 0; bit < 8; ++bit) {
 			const unsigned long long b = __ballot((d >> bit) & 1u);
@@ -288,21 +267,51 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const unsigned long lo
 		const unsigned rank = __popcll(match & lt);
 		if (rank == 0u) s_wcnt[w][d] = before + (unsigned)__popcll(match);
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-		kr[r] = k;
-		vr[r] = val_in[g0 + 64u * r];
-		pk[r] = (d << 16) | (before + rank);   // before + rank < kWaveSpan
+		pk[r] = (d << 16) | (before + rank);   // before + rank < 64 PER
 	}
 	__syncthreads();
-	// each wave's offset within every digit
-	unsigned run = 0;
+	// each wave's offset within every digit, and the tile's count
+	unsigned cnt = 0;
 	for (unsigned q = 0; q < kBlock / 64; ++q) {
 		const unsigned c = s_wcnt[q][t];
-		s_wcnt[q][t] = run;
-		run += c;
+		s_wcnt[q][t] = cnt;
+		cnt += c;
 	}
+	unsigned long long* mine = state + (size_t)tile * 256u + t;
+	post(mine, (tile ? kOwn : kAll) | cnt);
+	// exclusive scan of the tile's 256 digit counts
+	unsigned inc = cnt;
+	for (int k = 1; k < 64; k <<= 1) {
+		const unsigned v = __shfl_up(inc, (unsigned)k);
+		if ((int)lane >= k) inc += v;
+	}
+	if (lane == 63u) s_wsum[w] = inc;
+	unsigned prior = 0;
+	for (int j = (int)tile - 1; j >= 0;) {
+		unsigned long long v[kLook];
+#pragma unroll
+		for (unsigned q = 0; q < kLook; ++q)
+			v[q] = j >= (int)q ? peek(state + (size_t)(j - (int)q) * 256u + t) : kAll;
+		bool done = false;
+#pragma unroll
+		for (unsigned q = 0; q < kLook; ++q) {
+			if (done || j < (int)q) continue;
+			while (v[q] == 0ull) v[q] = peek(state + (size_t)(j - (int)q) * 256u + t);
+			prior += (unsigned)v[q];
+			done = v[q] >= kAll;
+		}
+		if (done) break;
+		j -= (int)kLook;
+	}
+	if (tile) post(mine, kAll | (unsigned long long)(prior + cnt));
+	s_base[t] = offs[t] + prior;
+	__syncthreads();
+	unsigned excl = inc - cnt;
+	for (unsigned q = 0; q < w; ++q) excl += s_wsum[q];
+	s_start[t] = excl;
 	__syncthreads();
 #pragma unroll
-	for (unsigned r = 0; r < kScatterPer; ++r) {
+	for (unsigned r = 0; r < PER; ++r) {
 		const unsigned d = pk[r] >> 16;
 		const unsigned slot = s_start[d] + s_wcnt[w][d] + (pk[r] & 0xFFFFu);
 		s_key[slot] = kr[r];
@@ -310,7 +319,7 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const unsigned long lo
 	}
 	__syncthreads();
 #pragma unroll
-	for (unsigned r = 0; r < kScatterPer; ++r) {
+	for (unsigned r = 0; r < PER; ++r) {
 		const unsigned slot = r * kBlock + t;
 		const unsigned long long k = s_key[slot];
 		const unsigned d = (unsigned)(k >> shift) & 255u;
@@ -904,44 +913,45 @@ int sfd_lbvh_keys(const float* pos, const float* mas, unsigned N, unsigned n_sor
 
 unsigned sfd_radix_tile(void) { return kTile; }
 
+// Tiles of 1024 pairs up to this many, for sorts that leave most CUs idle (a
+// pass over 65536 pairs: 512 pairs 10.7 us, 1024 9.2, 2048 9.1), and of 4096
+// above, where each tile's collection costs more (1M: 1024 pairs 38 us, 2048
+// 26, 4096 21, 6144 21; 4M: 101, 64, 47, 44; the choices compared at 8 tiles
+// looked back).
+constexpr unsigned kSmallSort = 1u << 19, kPerSmall = 4, kPerLarge = 16;
+static unsigned radix_tiles(unsigned n_sort) { return n_sort / (kBlock * (n_sort <= kSmallSort ? kPerSmall : kPerLarge)); }
+
+// two passes' state words, the blocks' digit counts and offsets of 8 passes, tickets
 unsigned sfd_radix_hist_entries(unsigned n_sort) {
-	const unsigned nh = 256u * (n_sort / kTile);
-	return nh + (nh + kScanU32Chunk - 1u) / kScanU32Chunk;
+	// no fewer than any smaller sort's
+	const unsigned ntiles = max(radix_tiles(n_sort), radix_tiles(min(n_sort, kSmallSort)));
+	return 2u * 2u * 256u * ntiles + 8u * 256u * (kDigitBlocks + 1u) + 8u;
 }
 
 unsigned sfd_lbvh_scan_tiles(unsigned N) { return (N + kScanTile - 1) / kScanTile; }
 
-// Histograms of up to this many entries (128 tiles, 524288 keys) are scanned
-// by one block in one launch instead of three.
-constexpr unsigned kRadixScanOneBlock = 32768;
-
 // Sorts n_sort (a multiple of the tile) pairs on the low 8 * passes key bits;
 // the result ends in (key0, val0) after an even number of passes and in
-// (key1, val1) after an odd one.
+// (key1, val1) after an odd one.  hist: sfd_radix_hist_entries(n_sort), 8-byte
+// aligned.
 int sfd_radix_sort_passes(unsigned long long* key0, unsigned* val0, unsigned long long* key1, unsigned* val1,
                           unsigned n_sort, unsigned* hist, unsigned passes, hipStream_t s) {
 	if (n_sort % kTile != 0 || passes > 8u) return -1;
-	const unsigned ntiles = n_sort / kTile;
-	const unsigned nh = 256u * ntiles;
-	const unsigned nchunks = (nh + kScanU32Chunk - 1u) / kScanU32Chunk;
-	unsigned* chunk_sums = hist + nh;   // sfd_radix_hist_entries() leaves room for them
-	if (ntiles == 0) return 0;
+	if (n_sort == 0 || passes == 0) return 0;
+	const unsigned ntiles = radix_tiles(n_sort), len = 256u * ntiles;
+	unsigned long long* state = reinterpret_cast<unsigned long long*>(hist);
+	unsigned* part = hist + 4u * (size_t)len;
+	const unsigned rows = min(kDigitBlocks, (n_sort + kDigitThreads - 1u) / kDigitThreads);
+	unsigned* offs = part + 8u * 256u * kDigitBlocks;
+	unsigned* tickets = offs + 8u * 256u;
+	hipLaunchKernelGGL(k_radix_digits, dim3(rows), dim3(kDigitThreads), 0, s, key0, n_sort, passes, part, state, len, tickets);
+	hipLaunchKernelGGL(k_radix_offsets, dim3(passes), dim3(kBlock), 0, s, part, rows, offs);
 	for (unsigned pass = 0; pass < passes; ++pass) {
-		const unsigned shift = 8u * pass;
-		unsigned long long* kin = (pass & 1) ? key1 : key0;
-		unsigned* vin = (pass & 1) ? val1 : val0;
-		unsigned long long* kout = (pass & 1) ? key0 : key1;
-		unsigned* vout = (pass & 1) ? val0 : val1;
-		hipLaunchKernelGGL(k_radix_hist, dim3(ntiles), dim3(kBlock), 0, s, kin, shift, ntiles, hist);
-		if (nh <= kRadixScanOneBlock) {
-			hipLaunchKernelGGL(k_radix_scan, dim3(1), dim3(1024), 0, s, hist, nh);
-		} else {
-			hipLaunchKernelGGL(k_scan_u32_sums, dim3(nchunks), dim3(kBlock), 0, s, hist, nh, chunk_sums);
-			hipLaunchKernelGGL(k_radix_scan, dim3(1), dim3(1024), 0, s, chunk_sums, nchunks);
-			hipLaunchKernelGGL(k_scan_u32_down, dim3(nchunks), dim3(kBlock), 0, s, hist, nh, chunk_sums);
-		}
-		hipLaunchKernelGGL(k_radix_scatter, dim3(ntiles), dim3(kBlock), 0, s, kin, vin, shift, ntiles, hist, n_sort,
-		                   kout, vout);
+		const bool odd = pass & 1u;
+		hipLaunchKernelGGL((n_sort <= kSmallSort ? k_radix_pass<kPerSmall> : k_radix_pass<kPerLarge>), dim3(ntiles), dim3(kBlock), 0, s,
+		                   odd ? key1 : key0, odd ? val1 : val0, 8u * pass, offs + 256u * pass,
+		                   state + (odd ? len : 0u), state + (odd ? 0u : len), tickets + pass, odd ? key0 : key1,
+		                   odd ? val0 : val1);
 	}
 	return sf_hip_check(hipGetLastError(), "sfd_radix_sort", "launch");
 }
@@ -949,19 +959,6 @@ int sfd_radix_sort_passes(unsigned long long* key0, unsigned* val0, unsigned lon
 int sfd_radix_sort(unsigned long long* key0, unsigned* val0, unsigned long long* key1, unsigned* val1,
                    unsigned n_sort, unsigned* hist, hipStream_t s) {
 	return sfd_radix_sort_passes(key0, val0, key1, val1, n_sort, hist, 8u, s);
-}
-
-unsigned sfd_scan_u32_sums_len(unsigned n) { return (n + kScanU32Chunk - 1u) / kScanU32Chunk; }
-
-// In-place exclusive scan of n u32 entries; sums holds
-// sfd_scan_u32_sums_len(n) entries of scratch.
-int sfd_scan_u32_exclusive(unsigned* data, unsigned n, unsigned* sums, hipStream_t s) {
-	if (n == 0) return 0;
-	const unsigned nchunks = sfd_scan_u32_sums_len(n);
-	hipLaunchKernelGGL(k_scan_u32_sums, dim3(nchunks), dim3(kBlock), 0, s, data, n, sums);
-	hipLaunchKernelGGL(k_radix_scan, dim3(1), dim3(1024), 0, s, sums, nchunks);
-	hipLaunchKernelGGL(k_scan_u32_down, dim3(nchunks), dim3(kBlock), 0, s, data, n, sums);
-	return sf_hip_check(hipGetLastError(), "sfd_scan_u32_exclusive", "launch");
 }
 
 // prefix: N records of 4 doubles; tile_sum: sfd_lbvh_scan_tiles(N) records

@@ -74,7 +74,7 @@ int sfd_tree_walk_ref(const float* pos, const float* mas, unsigned int N, const 
    device, passed untyped through C --- */
 unsigned int sfd_lbvh_bbox_blocks(void);
 unsigned int sfd_radix_tile(void);
-/* u32 entries of the radix-sort histogram scratch for n_sort keys */
+/* u32 entries of the radix sort's scratch for n_sort keys (8-byte aligned) */
 unsigned int sfd_radix_hist_entries(unsigned int n_sort);
 /* bbox (FP64), then 63-bit Morton keys and identity values for n_sort
    (a multiple of the radix tile) entries; padding keys are all ones.
@@ -89,10 +89,6 @@ int sfd_radix_sort(unsigned long long* key0, unsigned int* val0, unsigned long l
    (key1, val1) for an odd one */
 int sfd_radix_sort_passes(unsigned long long* key0, unsigned int* val0, unsigned long long* key1, unsigned int* val1,
                           unsigned int n_sort, unsigned int* hist, unsigned int passes, hipStream_t s);
-/* in-place exclusive scan of n u32 entries with sfd_scan_u32_sums_len(n)
-   entries of scratch */
-unsigned int sfd_scan_u32_sums_len(unsigned int n);
-int sfd_scan_u32_exclusive(unsigned int* data, unsigned int n, unsigned int* sums, hipStream_t s);
 /* tiles of the FP64 moment scan (records of 4 doubles each) */
 unsigned int sfd_lbvh_scan_tiles(unsigned int N);
 /* sorted bodies, radix tree, FP64 prefix moments (N records of 4 doubles),
