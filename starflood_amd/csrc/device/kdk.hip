@@ -70,35 +70,20 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift_fast(float* __restrict__ 
 	pos[k] = (float)x;
 }
 
-// The closing kick followed by k_energy_terms, per particle: one pass over
-// vel instead of two launches.
-__global__ __launch_bounds__(kBlock) void k_kick_energy_fast(float* __restrict__ vel, const float* __restrict__ acc,
-                                                             const float* __restrict__ mas,
-                                                             const float* __restrict__ pot, unsigned N, float half_dt,
-                                                             float* __restrict__ ken, float* __restrict__ pen) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	if (i >= N) return;
-	const float vx = __builtin_fmaf(half_dt, acc[3u * i], vel[3u * i]);
-	const float vy = __builtin_fmaf(half_dt, acc[3u * i + 1u], vel[3u * i + 1u]);
-	const float vz = __builtin_fmaf(half_dt, acc[3u * i + 2u], vel[3u * i + 2u]);
-	vel[3u * i] = vx;
-	vel[3u * i + 1u] = vy;
-	vel[3u * i + 2u] = vz;
-	const float m = mas[i];
-	const float v2 = (vx * vx + vy * vy) + vz * vz;
-	ken[i] = 0.5f * m * v2;
-	pen[i] = m * pot[i];
-}
-
 constexpr int kRedQ = 11;   // T, V, W, U, Px, Py, Pz, Lx, Ly, Lz, K
 
 // Per-block partial sums with a fixed grid-stride assignment and a fixed
-// LDS tree, so the result does not depend on scheduling.
+// LDS tree, so the result does not depend on scheduling.  KICK: first the
+// fast policy's closing kick and k_energy_terms, particle by particle, in the
+// same pass (a launch of its own cost 5 us, 41 at 4M particles).
+template <bool KICK>
 __global__ __launch_bounds__(kBlock) void k_reduce_state(const float* __restrict__ pos, const double* __restrict__ x64,
-                                                         const float* __restrict__ vel, const float* __restrict__ mas,
-                                                         const float* __restrict__ pot, const float* __restrict__ ken,
-                                                         const float* __restrict__ pen, const float* __restrict__ u,
-                                                         unsigned N, double G, double eps, double* __restrict__ red) {
+                                                         float* __restrict__ vel, const float* __restrict__ mas,
+                                                         const float* __restrict__ pot, float* __restrict__ ken,
+                                                         float* __restrict__ pen, const float* __restrict__ u,
+                                                         unsigned N, double G, double eps,
+                                                         const float* __restrict__ acc, float half_dt,
+                                                         double* __restrict__ red) {
 	__shared__ double sh[kRedQ][kBlock];
 	double q[kRedQ];
 #pragma unroll
@@ -112,9 +97,26 @@ __global__ __launch_bounds__(kBlock) void k_reduce_state(const float* __restrict
 		} else {
 			x = pos[3u * i]; y = pos[3u * i + 1u]; z = pos[3u * i + 2u];
 		}
-		const double vx = vel[3u * i], vy = vel[3u * i + 1u], vz = vel[3u * i + 2u];
-		q[0] += (double)ken[i];
-		q[1] += (double)pen[i];
+		float wx = vel[3u * i], wy = vel[3u * i + 1u], wz = vel[3u * i + 2u], ke, pe;
+		if (KICK) {
+			wx = __builtin_fmaf(half_dt, acc[3u * i], wx);
+			wy = __builtin_fmaf(half_dt, acc[3u * i + 1u], wy);
+			wz = __builtin_fmaf(half_dt, acc[3u * i + 2u], wz);
+			vel[3u * i] = wx;
+			vel[3u * i + 1u] = wy;
+			vel[3u * i + 2u] = wz;
+			const float v2 = (wx * wx + wy * wy) + wz * wz;
+			ke = 0.5f * mas[i] * v2;
+			pe = mas[i] * pot[i];
+			ken[i] = ke;
+			pen[i] = pe;
+		} else {
+			ke = ken[i];
+			pe = pen[i];
+		}
+		const double vx = wx, vy = wy, vz = wz;
+		q[0] += (double)ke;
+		q[1] += (double)pe;
 		q[2] += 0.5 * m * ((double)pot[i] + self * m);
 		if (u) q[3] += m * (double)u[i];
 		q[4] += m * vx;
@@ -206,31 +208,35 @@ extern "C" int sfd_kick_drift_fast(float* vel, const float* acc, double* x64, fl
 	return sf_hip_check(hipGetLastError(), "sfd_kick_drift_fast", "launch");
 }
 
-extern "C" int sfd_kick_energy_fast(float* vel, const float* acc, const float* mas, const float* pot, unsigned N,
-                                    float half_dt, float* ken, float* pen, hipStream_t s) {
-	if (!N) return 0;
-	const int tok = sf_prof_begin("kick", s);
-	hipLaunchKernelGGL(k_kick_energy_fast, dim3(grid_for(N)), dim3(kBlock), 0, s, vel, acc, mas, pot, N, half_dt, ken,
-	                   pen);
-	sf_prof_end(tok, s);
-	return sf_hip_check(hipGetLastError(), "sfd_kick_energy_fast", "launch");
-}
-
 extern "C" unsigned sfd_reduce_scratch_doubles(unsigned N) {
 	(void)N;
 	return (kRedBlocks + 1u) * SF_RED_VALUES;
 }
 
-extern "C" int sfd_reduce_state(const float* pos, const double* x64, const float* vel, const float* mas,
-                                const float* pot, const float* ken, const float* pen, const float* u, unsigned N,
-                                double G, double eps, double* red, hipStream_t s) {
+static int reduce(bool kick, const float* pos, const double* x64, float* vel, const float* mas, const float* pot,
+                  float* ken, float* pen, const float* u, unsigned N, double G, double eps, const float* acc,
+                  float half_dt, double* red, hipStream_t s) {
 	unsigned nb = grid_for(N);
 	if (nb > kRedBlocks) nb = kRedBlocks;
 	if (nb == 0) nb = 1;
-	const int tok = sf_prof_begin("reduce_state", s);
-	hipLaunchKernelGGL(k_reduce_state, dim3(nb), dim3(kBlock), 0, s, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps,
-	                   red);
+	const int tok = sf_prof_begin(kick ? "kick_reduce_state" : "reduce_state", s);
+	hipLaunchKernelGGL((kick ? k_reduce_state<true> : k_reduce_state<false>), dim3(nb), dim3(kBlock), 0, s, pos, x64, vel,
+	                   mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red);
 	hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, s, red, nb, red + (size_t)kRedBlocks * SF_RED_VALUES);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_reduce_state", "launch");
+}
+
+extern "C" int sfd_reduce_state(const float* pos, const double* x64, const float* vel, const float* mas,
+                                const float* pot, const float* ken, const float* pen, const float* u, unsigned N,
+                                double G, double eps, double* red, hipStream_t s) {
+	// not written without the kick
+	return reduce(false, pos, x64, const_cast<float*>(vel), mas, pot, const_cast<float*>(ken), const_cast<float*>(pen), u,
+	              N, G, eps, nullptr, 0.0f, red, s);
+}
+
+extern "C" int sfd_kick_reduce_state(const float* pos, const double* x64, float* vel, const float* acc,
+                                     const float* mas, const float* pot, float half_dt, float* ken, float* pen,
+                                     const float* u, unsigned N, double G, double eps, double* red, hipStream_t s) {
+	return reduce(true, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red, s);
 }

@@ -33,11 +33,6 @@ namespace {
 constexpr unsigned kBlock = 256;
 constexpr unsigned kTile = 4096;          // radix sorts take multiples of this
 
-__global__ __launch_bounds__(kBlock) void k_fill_u64(unsigned long long* __restrict__ p, unsigned n) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	if (i < n) p[i] = 0ull;
-}
-
 // ---------------------------------------------------------------- bbox
 __global__ __launch_bounds__(kBlock) void k_bbox_partial(const float* __restrict__ pos, unsigned N,
                                                          double* __restrict__ part) {
@@ -183,20 +178,26 @@ __global__ __launch_bounds__(kDigitThreads) void k_radix_digits(const unsigned l
 }
 
 // One block per pass: the digits' exclusive prefix over all blocks' counts.
-__global__ __launch_bounds__(kBlock) void k_radix_offsets(const unsigned* __restrict__ part, unsigned rows,
-                                                          unsigned* __restrict__ offs) {
-	__shared__ unsigned ws[kBlock / 64];
-	const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
+constexpr unsigned kOffsThreads = 1024;
+__global__ __launch_bounds__(kOffsThreads) void k_radix_offsets(const unsigned* __restrict__ part, unsigned rows,
+                                                                unsigned* __restrict__ offs) {
+	__shared__ unsigned cnt[kOffsThreads], ws[4];
+	const unsigned t = threadIdx.x, d = t % 256u, lane = t & 63u, w = t >> 6;
 	unsigned n = 0;
-#pragma unroll 16
-	for (unsigned r = 0; r < rows; ++r) n += part[(blockIdx.x * rows + r) * 256u + t];
+#pragma unroll 8
+	for (unsigned r = t / 256u; r < rows; r += kOffsThreads / 256u) n += part[(blockIdx.x * rows + r) * 256u + d];
+	cnt[t] = n;
+	__syncthreads();
+	n = 0;
+	for (unsigned q = d; q < kOffsThreads; q += 256u) n += cnt[q];
 	unsigned inc = n;
 	for (int o = 1; o < 64; o <<= 1) {
 		const unsigned v = __shfl_up(inc, (unsigned)o);
 		if ((int)lane >= o) inc += v;
 	}
-	if (lane == 63u) ws[w] = inc;
+	if (lane == 63u && w < 4u) ws[w] = inc;
 	__syncthreads();
+	if (w >= 4u) return;
 	unsigned excl = inc - n;
 	for (unsigned q = 0; q < w; ++q) excl += ws[q];
 	offs[blockIdx.x * 256u + t] = excl;
@@ -332,8 +333,10 @@ __global__ __launch_bounds__(kBlock) void k_radix_pass(const unsigned long long*
 // ---------------------------------------------------------------- tree
 __global__ __launch_bounds__(kBlock) void k_gather_sorted(const float4* __restrict__ packed,
                                                           const unsigned* __restrict__ order, unsigned N,
-                                                          float4* __restrict__ body) {
+                                                          float4* __restrict__ body,
+                                                          unsigned long long* __restrict__ start, unsigned words) {
 	const unsigned p = blockIdx.x * kBlock + threadIdx.x;
+	if (p < words) start[p] = 0ull;   // for k_group_flags (words <= the grid's threads)
 	if (p >= N) return;
 	body[p] = packed[order[p]];
 }
@@ -345,25 +348,45 @@ __device__ __forceinline__ int delta(const unsigned long long* __restrict__ key,
 	return 64 + __clz((int)((unsigned)i ^ (unsigned)j));
 }
 
+// delta(i, j) > d as two comparisons, for -1 <= d <= 95: the keys (63 bits)
+// agree in more than d bits, and if d >= 64 so do the indexes.
+struct Longer {
+	unsigned long long key_i, below;
+	unsigned i, upto;
+	int N;
+	__device__ __forceinline__ Longer(unsigned long long key_i_, int i_, int N_, int d)
+	    : key_i(key_i_), below(d < 0 ? ~0ull : (d < 64 ? 1ull << (63 - d) : 1ull)), i((unsigned)i_),
+	      upto(d < 64 ? ~0u : (1u << (95 - d)) - 1u), N(N_) {}
+	__device__ __forceinline__ bool operator()(const unsigned long long* __restrict__ key, int j) const {
+		return j >= 0 && j < N && (key[j] ^ key_i) < below && (i ^ (unsigned)j) <= upto;
+	}
+};
+
 // Internal nodes 0..N-2; node id >= N-1 is the leaf of sorted particle
 // id - (N-1).  node_lr holds (left, right), node_range (first, count).
+// Bound by issue: a wavefront takes as many probes as its largest node, a
+// couple of dozen.  Comparisons in place of a count of leading bits per probe:
+// 65537 particles 17.3 -> 14.0 us, 1M 45 -> 36, 4M 132 -> 105.  Keeping the keys
+// around a block in LDS changed nothing.
 __global__ __launch_bounds__(kBlock) void k_karras(const unsigned long long* __restrict__ key, int N,
                                                    int2* __restrict__ node_lr, int2* __restrict__ node_range) {
 	const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
 	if (i >= N - 1) return;
-	const int d = (delta(key, N, i, i + 1) - delta(key, N, i, i - 1)) >= 0 ? 1 : -1;
-	const int dmin = delta(key, N, i, i - d);
+	const unsigned long long ki = key[i];
+	const int up = delta(key, N, i, i + 1), down = delta(key, N, i, i - 1);
+	const int d = up - down >= 0 ? 1 : -1;
+	const Longer of_node(ki, i, N, min(up, down));
 	int lmax = 2;
-	while (delta(key, N, i, i + lmax * d) > dmin) lmax <<= 1;
+	while (of_node(key, i + lmax * d)) lmax <<= 1;
 	int l = 0;
 	for (int t = lmax >> 1; t >= 1; t >>= 1)
-		if (delta(key, N, i, i + (l + t) * d) > dmin) l += t;
+		if (of_node(key, i + (l + t) * d)) l += t;
 	const int j = i + l * d;
-	const int dnode = delta(key, N, i, j);
+	const Longer of_child(ki, i, N, delta(key, N, i, j));
 	int s = 0;
-	for (int div = 2;; div <<= 1) {
-		const int t = (l + div - 1) / div;
-		if (delta(key, N, i, i + (s + t) * d) > dnode) s += t;
+	for (int k = 1;; ++k) {
+		const int t = (l + (1 << k) - 1) >> k;
+		if (of_child(key, i + (s + t) * d)) s += t;
 		if (t <= 1) break;
 	}
 	const int gamma = i + s * d + min(d, 0);
@@ -416,8 +439,9 @@ struct d6 {   // xx, xy, xz, yy, yz, zz
 };
 
 constexpr unsigned kScanPer = 16;
-constexpr unsigned kScanTile = kBlock * kScanPer;
-constexpr unsigned kScanWaveSpan = kScanTile / (kBlock / 64);   // consecutive elements per wavefront
+constexpr unsigned kScanSpan = 64 * kScanPer;   // consecutive elements summed by a wavefront
+constexpr unsigned kScanSpans = 4;              // in a tile
+constexpr unsigned kScanTile = kScanSpans * kScanSpan;
 
 template <class R>
 __device__ R block_exclusive_scan(R v, R* sh) {
@@ -435,13 +459,17 @@ __device__ R block_exclusive_scan(R v, R* sh) {
 	return excl;
 }
 
-// Sum of a wavefront's kScanWaveSpan consecutive elements (read 64
-// consecutive at a time), reduced across lanes in a fixed order; every lane
-// returns it.
+// Span sums, and tile sums from them: a wavefront reads its span 64
+// consecutive elements at a time and adds its lanes in a fixed order, then
+// wave 0 adds the tile's spans in order.
 template <class R>
-__device__ R wave_span_sum(const float4* __restrict__ body, unsigned N, const double* __restrict__ ref,
-                           unsigned first) {
-	const unsigned lane = threadIdx.x & 63u;
+__global__ __launch_bounds__(kBlock) void k_scan_tiles(const float4* __restrict__ body, unsigned N,
+                                                       const double* __restrict__ ref, R* __restrict__ tile_sum,
+                                                       R* __restrict__ span_sum) {
+	static_assert(kScanSpans == kBlock / 64, "a wavefront per span");
+	__shared__ R sh[kScanSpans];
+	const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+	const unsigned first = blockIdx.x * kScanTile + w * kScanSpan;
 	R s = R::zero();
 	for (unsigned r = 0; r < kScanPer; ++r) {
 		const unsigned i = first + 64u * r + lane;
@@ -451,22 +479,14 @@ __device__ R wave_span_sum(const float4* __restrict__ body, unsigned N, const do
 		const R t = s.shfl_up(o);
 		if (lane >= o) s = s + t;
 	}
-	return s.shfl(63);
-}
-
-// Tile sums: each wavefront sums its kScanWaveSpan elements, then wave 0 adds
-// the four in order.
-template <class R>
-__global__ __launch_bounds__(kBlock) void k_scan_tiles(const float4* __restrict__ body, unsigned N,
-                                                       const double* __restrict__ ref, R* __restrict__ tile_sum) {
-	__shared__ R sh[kBlock / 64];
-	const unsigned w = threadIdx.x >> 6;
-	const R s = wave_span_sum<R>(body, N, ref, blockIdx.x * kScanTile + w * kScanWaveSpan);
-	if ((threadIdx.x & 63u) == 0u) sh[w] = s;
+	if (lane == 63u) {
+		sh[w] = s;
+		span_sum[blockIdx.x * kScanSpans + w] = s;
+	}
 	__syncthreads();
 	if (threadIdx.x == 0) {
 		R t = sh[0];
-		for (unsigned q = 1; q < kBlock / 64; ++q) t = t + sh[q];
+		for (unsigned q = 1; q < kScanSpans; ++q) t = t + sh[q];
 		tile_sum[blockIdx.x] = t;
 	}
 }
@@ -486,31 +506,41 @@ __global__ __launch_bounds__(kBlock) void k_scan_tile_sums(R* __restrict__ tile_
 	}
 }
 
-// Inclusive prefix of a tile: each wavefront starts from the tile offset plus
-// the sums of the wavefronts before it, and scans its elements 64 at a time
-// (a lane scan, then the round's total carried to the next round), so that
-// reads and writes are of consecutive records.
+// Inclusive prefix of a span: each wavefront scans four of its sixteen 64s
+// (interleaved: a lane scan is a chain of six exchanges), which start from the
+// tile's offset, the spans before and the 64s before, added in order.  (One
+// wavefront taking all sixteen in turn, after summing the span again for the
+// offsets, took 18.4 us at 65537 particles and 56 at 4M, 83 with second
+// moments; this 7.0, 45 and 67.)
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_scan_write(const float4* __restrict__ body, unsigned N,
                                                        const double* __restrict__ ref, const R* __restrict__ tile_off,
-                                                       R* __restrict__ prefix) {
-	__shared__ R sh[kBlock / 64];
+                                                       const R* __restrict__ span_sum, R* __restrict__ prefix) {
+	constexpr unsigned kRounds = kScanPer / (kBlock / 64);
+	__shared__ R sh[kScanPer];
 	const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-	const unsigned first = blockIdx.x * kScanTile + w * kScanWaveSpan;
-	const R total = wave_span_sum<R>(body, N, ref, first);
-	if (lane == 0u) sh[w] = total;
-	__syncthreads();
-	R run = tile_off[blockIdx.x];
-	for (unsigned q = 0; q < w; ++q) run = run + sh[q];
-	for (unsigned r = 0; r < kScanPer; ++r) {
-		const unsigned i = first + 64u * r + lane;
-		R v = i < N ? R::of(body[i], ref) : R::zero();
-		for (unsigned o = 1; o < 64; o <<= 1) {
-			const R t = v.shfl_up(o);
-			if (lane >= o) v = v + t;
+	const unsigned tile = blockIdx.x / kScanSpans, span = blockIdx.x % kScanSpans;
+	const unsigned first = blockIdx.x * kScanSpan + w * 64u * kRounds + lane;
+	R v[kRounds];
+#pragma unroll
+	for (unsigned k = 0; k < kRounds; ++k) v[k] = first + 64u * k < N ? R::of(body[first + 64u * k], ref) : R::zero();
+	for (unsigned o = 1; o < 64; o <<= 1) {
+#pragma unroll
+		for (unsigned k = 0; k < kRounds; ++k) {
+			const R t = v[k].shfl_up(o);
+			if (lane >= o) v[k] = v[k] + t;
 		}
-		if (i < N) prefix[i] = run + v;   // inclusive
-		run = run + v.shfl(63);
+	}
+	if (lane == 63u)
+		for (unsigned k = 0; k < kRounds; ++k) sh[w * kRounds + k] = v[k];
+	R run = tile_off[tile];
+	for (unsigned q = 0; q < span; ++q) run = run + span_sum[tile * kScanSpans + q];
+	__syncthreads();
+	for (unsigned q = 0; q < w * kRounds; ++q) run = run + sh[q];
+#pragma unroll
+	for (unsigned k = 0; k < kRounds; ++k) {
+		if (first + 64u * k < N) prefix[first + 64u * k] = run + v[k];   // inclusive
+		run = run + sh[w * kRounds + k];
 	}
 }
 
@@ -554,9 +584,7 @@ __global__ __launch_bounds__(kBlock) void k_node_quad(int N, const int2* __restr
 	const int2 rg = node_range[n];
 	const int f = rg.x, l = rg.x + rg.y - 1;
 	const d4 a = f > 0 ? prefix[f - 1] : d4::zero();
-	const d6 a2 = f > 0 ? prefix2[f - 1] : d6::zero();
 	const d4 b = prefix[l];
-	const d6 b2 = prefix2[l];
 	const double M = b.m - a.m;
 	if (!(M > 0.0)) {
 		q0[n] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -591,6 +619,7 @@ __global__ __launch_bounds__(kBlock) void k_node_quad(int N, const int2* __restr
 		qyz -= sm * cy * cz;
 		qzz -= sm * cz * cz;
 	} else {
+		const d6 a2 = f > 0 ? prefix2[f - 1] : d6::zero(), b2 = prefix2[l];
 		// centre of mass relative to ref
 		const double cx = (b.x - a.x) / M - ref[0], cy = (b.y - a.y) / M - ref[1], cz = (b.z - a.z) / M - ref[2];
 		qxx = (b2.v[0] - a2.v[0]) - M * cx * cx;
@@ -787,8 +816,11 @@ __global__ __launch_bounds__(kBlock) void k_records(int N, const int2* __restric
                                                     const int2* __restrict__ node_range,
                                                     const float4* __restrict__ node_cm,
                                                     const float4* __restrict__ node_cell, float inv_theta,
-                                                    int leaf_size, int4* __restrict__ rec_b) {
+                                                    int leaf_size, int4* __restrict__ rec_b,
+                                                    unsigned long long* __restrict__ counters) {
 	const int n = (int)(blockIdx.x * kBlock + threadIdx.x);
+	// the walk's counters, but the fifth, which lasts until the host clears it
+	if (blockIdx.x == 0u && threadIdx.x < 6u && threadIdx.x != 4u) counters[threadIdx.x] = 0ull;
 	if (n >= 2 * N - 1) return;
 	int first, count, l = -1, r = -1;
 	if (n < N - 1) {
@@ -871,8 +903,6 @@ unsigned sfd_lbvh_group_words(unsigned N) { return N / 64u + 2u; }
 int sfd_lbvh_groups(unsigned N, const void* node_lr, const void* node_range, int cap,
                     unsigned long long* start, hipStream_t s) {
 	if (N == 0 || cap < 1 || cap > 64) return -1;
-	const unsigned words = sfd_lbvh_group_words(N);
-	hipLaunchKernelGGL(k_fill_u64, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s, start, words);
 	const unsigned threads = N > 1 ? N - 1 : 1;
 	hipLaunchKernelGGL(k_group_flags, dim3((threads + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (int)N,
 	                   static_cast<const int2*>(node_lr), static_cast<const int2*>(node_range), cap, start);
@@ -928,7 +958,8 @@ unsigned sfd_radix_hist_entries(unsigned n_sort) {
 	return 2u * 2u * 256u * ntiles + 8u * 256u * (kDigitBlocks + 1u) + 8u;
 }
 
-unsigned sfd_lbvh_scan_tiles(unsigned N) { return (N + kScanTile - 1) / kScanTile; }
+static unsigned scan_tiles(unsigned N) { return (N + kScanTile - 1) / kScanTile; }
+unsigned sfd_lbvh_scan_records(unsigned N) { return (1u + kScanSpans) * scan_tiles(N); }
 
 // Sorts n_sort (a multiple of the tile) pairs on the low 8 * passes key bits;
 // the result ends in (key0, val0) after an even number of passes and in
@@ -945,7 +976,7 @@ int sfd_radix_sort_passes(unsigned long long* key0, unsigned* val0, unsigned lon
 	unsigned* offs = part + 8u * 256u * kDigitBlocks;
 	unsigned* tickets = offs + 8u * 256u;
 	hipLaunchKernelGGL(k_radix_digits, dim3(rows), dim3(kDigitThreads), 0, s, key0, n_sort, passes, part, state, len, tickets);
-	hipLaunchKernelGGL(k_radix_offsets, dim3(passes), dim3(kBlock), 0, s, part, rows, offs);
+	hipLaunchKernelGGL(k_radix_offsets, dim3(passes), dim3(kOffsThreads), 0, s, part, rows, offs);
 	for (unsigned pass = 0; pass < passes; ++pass) {
 		const bool odd = pass & 1u;
 		hipLaunchKernelGGL((n_sort <= kSmallSort ? k_radix_pass<kPerSmall> : k_radix_pass<kPerLarge>), dim3(ntiles), dim3(kBlock), 0, s,
@@ -961,26 +992,28 @@ int sfd_radix_sort(unsigned long long* key0, unsigned* val0, unsigned long long*
 	return sfd_radix_sort_passes(key0, val0, key1, val1, n_sort, hist, 8u, s);
 }
 
-// prefix: N records of 4 doubles; tile_sum: sfd_lbvh_scan_tiles(N) records
+// prefix: N records of 4 doubles; tile_sum: sfd_lbvh_scan_records(N) records
 int sfd_lbvh_topology(const unsigned long long* key, const unsigned* order, unsigned N, const double* box, void* body,
                       void* node_lr, void* node_range, void* prefix, void* tile_sum, void* node_cm, void* node_cell,
-                      hipStream_t s) {
+                      unsigned long long* start, hipStream_t s) {
 	const unsigned g = (N + kBlock - 1) / kBlock;
 	float4* b4 = static_cast<float4*>(body);
 	int2* rg = static_cast<int2*>(node_range);
 	d4* pre = static_cast<d4*>(prefix);
 	d4* ts = static_cast<d4*>(tile_sum);
-	const unsigned ntiles = sfd_lbvh_scan_tiles(N);
+	const unsigned ntiles = scan_tiles(N), nspans = (N + kScanSpan - 1u) / kScanSpan;
 	const int tok = sf_prof_begin("lbvh_topology", s);
 	// the packed records of sfd_lbvh_keys, in the prefix buffer until the scan overwrites it
 	hipLaunchKernelGGL(k_gather_sorted, dim3(g), dim3(kBlock), 0, s, reinterpret_cast<const float4*>(prefix), order, N,
-	                   b4);
+	                   b4, start, sfd_lbvh_group_words(N));
 	if (N > 1)
 		hipLaunchKernelGGL(k_karras, dim3((N - 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, key, (int)N,
 		                   static_cast<int2*>(node_lr), rg);
-	hipLaunchKernelGGL(k_scan_tiles<d4>, dim3(ntiles), dim3(kBlock), 0, s, b4, N, (const double*)nullptr, ts);
+	hipLaunchKernelGGL(k_scan_tiles<d4>, dim3(ntiles), dim3(kBlock), 0, s, b4, N, (const double*)nullptr, ts,
+	                   ts + ntiles);
 	hipLaunchKernelGGL(k_scan_tile_sums<d4>, dim3(1), dim3(kBlock), 0, s, ts, ntiles);
-	hipLaunchKernelGGL(k_scan_write<d4>, dim3(ntiles), dim3(kBlock), 0, s, b4, N, (const double*)nullptr, ts, pre);
+	hipLaunchKernelGGL(k_scan_write<d4>, dim3(nspans), dim3(kBlock), 0, s, b4, N, (const double*)nullptr, ts,
+	                   ts + ntiles, pre);
 	const unsigned nn = 2u * N - 1u;
 	hipLaunchKernelGGL(k_node_moments, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0, s, b4, (int)N, key, rg, pre,
 	                   box, static_cast<float4*>(node_cm), static_cast<float4*>(node_cell));
@@ -989,7 +1022,7 @@ int sfd_lbvh_topology(const unsigned long long* key, const unsigned* order, unsi
 }
 
 // Traceless quadrupoles of every node (after sfd_lbvh_topology): prefix2 is
-// N records of 6 doubles, tile_sum2 sfd_lbvh_scan_tiles(N) of them, ref 3
+// N records of 6 doubles, tile_sum2 sfd_lbvh_scan_records(N) of them, ref 3
 // doubles; node_q0 / node_q1 are 2N-1 float4 / float.
 int sfd_lbvh_quadrupoles(unsigned N, const void* body, const void* node_range, const void* prefix, const double* box,
                          void* prefix2, void* tile_sum2, double* ref, void* node_q0, float* node_q1, hipStream_t s) {
@@ -998,11 +1031,13 @@ int sfd_lbvh_quadrupoles(unsigned N, const void* body, const void* node_range, c
 	const float4* b4 = static_cast<const float4*>(body);
 	d6* pre2 = static_cast<d6*>(prefix2);
 	d6* ts2 = static_cast<d6*>(tile_sum2);
-	const unsigned ntiles = sfd_lbvh_scan_tiles(N);
+	const unsigned ntiles = scan_tiles(N), nspans = (N + kScanSpan - 1u) / kScanSpan;
 	hipLaunchKernelGGL(k_quad_ref, dim3(1), dim3(64), 0, s, static_cast<const d4*>(prefix), N, ref);
-	hipLaunchKernelGGL(k_scan_tiles<d6>, dim3(ntiles), dim3(kBlock), 0, s, b4, N, (const double*)ref, ts2);
+	hipLaunchKernelGGL(k_scan_tiles<d6>, dim3(ntiles), dim3(kBlock), 0, s, b4, N, (const double*)ref, ts2,
+	                   ts2 + ntiles);
 	hipLaunchKernelGGL(k_scan_tile_sums<d6>, dim3(1), dim3(kBlock), 0, s, ts2, ntiles);
-	hipLaunchKernelGGL(k_scan_write<d6>, dim3(ntiles), dim3(kBlock), 0, s, b4, N, (const double*)ref, ts2, pre2);
+	hipLaunchKernelGGL(k_scan_write<d6>, dim3(nspans), dim3(kBlock), 0, s, b4, N, (const double*)ref, ts2,
+	                   ts2 + ntiles, pre2);
 	const unsigned nn = 2u * N - 1u;
 	hipLaunchKernelGGL(k_node_quad, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (int)N,
 	                   static_cast<const int2*>(node_range), b4, static_cast<const d4*>(prefix), pre2,
@@ -1011,13 +1046,14 @@ int sfd_lbvh_quadrupoles(unsigned N, const void* body, const void* node_range, c
 }
 
 int sfd_lbvh_records(unsigned N, const void* node_lr, const void* node_range, const void* node_cm,
-                     const void* node_cell, float theta, int leaf_size, void* rec_b, hipStream_t s) {
+                     const void* node_cell, float theta, int leaf_size, void* rec_b,
+                     unsigned long long* counters, hipStream_t s) {
 	const unsigned nn = 2u * N - 1u;
 	const float inv_theta = theta > 0.0f ? 1.0f / theta : 3.0e38f;
 	hipLaunchKernelGGL(k_records, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (int)N,
 	                   static_cast<const int2*>(node_lr), static_cast<const int2*>(node_range),
 	                   static_cast<const float4*>(node_cm), static_cast<const float4*>(node_cell), inv_theta,
-	                   leaf_size, static_cast<int4*>(rec_b));
+	                   leaf_size, static_cast<int4*>(rec_b), counters);
 	return sf_hip_check(hipGetLastError(), "sfd_lbvh_records", "launch");
 }
 

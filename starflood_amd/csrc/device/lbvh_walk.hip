@@ -519,10 +519,6 @@ __global__ __launch_bounds__(kBlock, QUAD ? 4 : 5) void k_walk(const float4* __r
 	}
 }
 
-__global__ void k_walk_reset(unsigned long long* __restrict__ counters) {
-	if (threadIdx.x < 6 && threadIdx.x != 4) counters[threadIdx.x] = 0ull;
-}
-
 // Blocks that are resident at once, the size of the persistent grid: every
 // wavefront runs from the start and takes chunks until none are left
 // (cached after the first call).
@@ -562,7 +558,6 @@ int sfd_lbvh_walk(const void* body, const unsigned* order, unsigned N, const uns
 	const unsigned resident = quad ? resident_blocks_of<true>() : resident_blocks_of<false>();
 	unsigned blocks = (N + kWaves * kSpan - 1u) / (kWaves * kSpan);
 	if (blocks > resident) blocks = resident;   // gstack holds resident_blocks() >= resident slots
-	hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, s, counters);
 	const int tok = sf_prof_begin("lbvh_walk", s);
 	if (quad)
 		hipLaunchKernelGGL(k_walk<true>, dim3(blocks), dim3(kBlock), 0, s, static_cast<const float4*>(body), order,

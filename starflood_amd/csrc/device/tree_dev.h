@@ -89,18 +89,21 @@ int sfd_radix_sort(unsigned long long* key0, unsigned int* val0, unsigned long l
    (key1, val1) for an odd one */
 int sfd_radix_sort_passes(unsigned long long* key0, unsigned int* val0, unsigned long long* key1, unsigned int* val1,
                           unsigned int n_sort, unsigned int* hist, unsigned int passes, hipStream_t s);
-/* tiles of the FP64 moment scan (records of 4 doubles each) */
-unsigned int sfd_lbvh_scan_tiles(unsigned int N);
+/* scratch records of the FP64 moment scans (4 or 6 doubles each) */
+unsigned int sfd_lbvh_scan_records(unsigned int N);
 /* sorted bodies, radix tree, FP64 prefix moments (N records of 4 doubles),
    node monopoles (2N-1 float4) and Morton cells (2N-1 float4: centre, side;
    internal nodes of at most 64 particles are left to sfd_lbvh_group_boxes).
-   prefix holds sfd_lbvh_keys' packed records on entry */
+   prefix holds sfd_lbvh_keys' packed records on entry; start is cleared for
+   sfd_lbvh_groups */
 int sfd_lbvh_topology(const unsigned long long* key, const unsigned int* order, unsigned int N, const double* box,
                       void* body, void* node_lr, void* node_range, void* prefix, void* tile_sum, void* node_cm,
-                      void* node_cell, hipStream_t s);
+                      void* node_cell, unsigned long long* start, hipStream_t s);
 int sfd_lbvh_records(unsigned int N, const void* node_lr, const void* node_range, const void* node_cm,
-                     const void* node_cell, float theta, int leaf_size, void* rec_b, hipStream_t s);
-/* lbvh_walk.hip.  counters (6 x u64; all but the fifth zeroed here): cell
+                     const void* node_cell, float theta, int leaf_size, void* rec_b,
+                     unsigned long long* counters, hipStream_t s);
+/* lbvh_walk.hip.  counters (6 x u64; all but the fifth zeroed by
+   sfd_lbvh_records): cell
    interactions, particle interactions, wavefronts that met a malformed tree,
    node batches; the fifth adds the third up over walks until the host clears
    it; the sixth hands out the groups (sfd_lbvh_group_list's).
@@ -117,14 +120,14 @@ int sfd_lbvh_walk(const void* body, const unsigned int* order, unsigned int N, c
                   unsigned long long* counters, int* gstack, hipStream_t s);
 /* traceless quadrupoles (node_q0 2N-1 float4, node_q1 2N-1 float) from a
    second FP64 prefix scan (prefix2: N x 6 doubles, tile_sum2:
-   sfd_lbvh_scan_tiles(N) x 6 doubles, ref: 3 doubles); NULL node_q0 in
+   sfd_lbvh_scan_records(N) x 6 doubles, ref: 3 doubles); NULL node_q0 in
    sfd_lbvh_walk selects the monopole walk */
 int sfd_lbvh_quadrupoles(unsigned int N, const void* body, const void* node_range, const void* prefix,
                          const double* box, void* prefix2, void* tile_sum2, double* ref, void* node_q0,
                          float* node_q1, hipStream_t s);
 
 /* walk groups: bit p of start is set where a maximal subtree of at most cap
-   (<= 64) particles begins in sorted order, and bit N; start holds
+   (<= 64) particles begins in sorted order, and bit N; start, clear on entry, holds
    sfd_lbvh_group_words(N) words (lbvh.hip) */
 unsigned int sfd_lbvh_group_words(unsigned int N);
 int sfd_lbvh_groups(unsigned int N, const void* node_lr, const void* node_range, int cap, unsigned long long* start,

@@ -27,7 +27,7 @@ struct sf_lbvh {
 	void* node_lr;            /* N-1 int2 */
 	void* node_range;         /* N-1 int2 */
 	void* prefix;             /* N x 4 doubles: inclusive (m, mx, my, mz) sums */
-	void* tile_sum;           /* scan tiles x 4 doubles */
+	void* tile_sum;           /* the scan's tiles and spans x 4 doubles */
 	void* node_cm;            /* 2N-1 float4: com, mass */
 	void* node_cell;          /* 2N-1 float4: Morton cell centre, side */
 	void* rec_b;              /* 2N-1 int4 */
@@ -93,7 +93,7 @@ static int ensure(sf_lbvh** st, unsigned int N) {
 	rc |= alloc(&t->node_lr, (size_t)N * 8u);
 	rc |= alloc(&t->node_range, (size_t)N * 8u);
 	rc |= alloc(&t->prefix, (size_t)N * 32u);
-	rc |= alloc(&t->tile_sum, (size_t)sfd_lbvh_scan_tiles(N) * 32u);
+	rc |= alloc(&t->tile_sum, (size_t)sfd_lbvh_scan_records(N) * 32u);
 	rc |= alloc(&t->node_cm, nn * 16u);
 	rc |= alloc(&t->node_cell, nn * 16u);
 	rc |= alloc(&t->rec_b, nn * 16u);
@@ -130,7 +130,7 @@ static int ensure_quad(sf_lbvh* t) {
 	const size_t N = t->n_alloc, nn = 2u * N;
 	int rc = 0;
 	rc |= alloc(&t->prefix2, N * 48u);
-	rc |= alloc(&t->tile_sum2, (size_t)sfd_lbvh_scan_tiles((unsigned int)N) * 48u);
+	rc |= alloc(&t->tile_sum2, (size_t)sfd_lbvh_scan_records((unsigned int)N) * 48u);
 	rc |= alloc((void**)&t->quad_ref, 3u * 8u);
 	rc |= alloc(&t->node_q0, nn * 16u);
 	rc |= alloc((void**)&t->node_q1, nn * 4u);
@@ -159,7 +159,7 @@ int sf_lbvh_build(sf_lbvh** st, unsigned int N, const float* pos, const float* m
 	if (sfd_lbvh_keys(pos, mas, N, t->n_sort, t->bbox_part, t->box, t->key0, t->val0, t->prefix, s)) return -1;
 	if (sfd_radix_sort(t->key0, t->val0, t->key1, t->val1, t->n_sort, t->hist, s)) return -1;
 	if (sfd_lbvh_topology(t->key0, t->val0, N, t->box, t->body, t->node_lr, t->node_range, t->prefix, t->tile_sum,
-	                      t->node_cm, t->node_cell, s))
+	                      t->node_cm, t->node_cell, t->group_start, s))
 		return -1;
 	if (sfd_lbvh_groups(N, t->node_lr, t->node_range, SF_LBVH_GROUP, t->group_start, s)) return -1;
 	/* the sort is done with val1 */
@@ -193,7 +193,7 @@ int sf_lbvh_walk(sf_lbvh* t, unsigned int N, const float* pos, const float* mas,
 		return -1;
 	}
 	if (sfd_lbvh_records(N, t->node_lr, t->node_range, t->node_cm, t->node_cell, (float)p->theta, (int)p->leaf_size,
-	                     t->rec_b, s))
+	                     t->rec_b, t->counters, s))
 		return -1;
 	/* G M l^p <= alpha |a| d^(p+2)  <=>  M l^p <= (alpha / G) |a| d^(p+2) */
 	const float alpha_g = (prev_acc && p->mac_alpha > 0.0) ? (float)(p->mac_alpha / p->G) : 0.0f;

@@ -258,18 +258,14 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 	}
 	if (timing) tev_record(3, s);
 
-	if (exact) {
-		if (sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_1 */
-	} else if (!fused) {
-		/* kick_1 and the energy terms below, in one pass */
-		if (sfd_kick_energy_fast(vel, acc, mas, pot, N, half_dt, ken, pen, s)) return STARFLOOD_FAILURE;
-	}
+	if (exact && sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_1 */
 	if (cubic && sfd_sph_u_kick(c->d_u, c->d_dudt, N, half_dt, s)) return STARFLOOD_FAILURE;
-	if (timing) tev_record(4, s);
-	if (exact && sfd_energy_terms(vel, mas, pot, N, ken, pen, s)) return STARFLOOD_FAILURE;
 
 	double* red_out = c->d_red + (size_t)(sfd_reduce_scratch_doubles(N) - SF_RED_VALUES);
+	const float* u = c->have_u ? c->d_u : NULL;
 	if (exact) {
+		if (timing) tev_record(4, s);
+		if (sfd_energy_terms(vel, mas, pot, N, ken, pen, s)) return STARFLOOD_FAILURE;
 		/* ken_sum and pen_sum in one pass (its time is logged as ken_sum's) */
 		if (sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
 		if (timing) {
@@ -277,11 +273,15 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 			tev_record(6, s);
 		}
 	}
-	/* FP64 W, P, L (and T, V in the fast policy) */
-	if (sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, c->have_u ? c->d_u : NULL, N, p->G,
-	                     p->epsilon, c->d_red, s))
+	/* FP64 W, P, L (and T, V in the fast policy, whose kick_1 and energy terms
+	   are in the same pass: its time is logged as kick_1's) */
+	if (exact || fused ? sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, u, N, p->G, p->epsilon,
+	                                      c->d_red, s)
+	                   : sfd_kick_reduce_state(pos, c->d_x64, vel, acc, mas, pot, half_dt, ken, pen, u, N, p->G,
+	                                           p->epsilon, c->d_red, s))
 		return STARFLOOD_FAILURE;
 	if (!exact && timing) {
+		tev_record(4, s);
 		tev_record(5, s);
 		tev_record(6, s);
 	}

@@ -175,9 +175,6 @@ int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned int N, vo
 int sfd_x64_refresh(const float* pos, double* x64, unsigned int n3, hipStream_t s);
 int sfd_kick_drift_fast(float* vel, const float* acc, double* x64, float* pos, unsigned int n3,
                         float half_dt, double dt, hipStream_t s);
-/* v += half_dt a, then sfd_energy_terms, in one pass over the particles */
-int sfd_kick_energy_fast(float* vel, const float* acc, const float* mas, const float* pot, unsigned int N,
-                         float half_dt, float* ken, float* pen, hipStream_t s);
 /* sph.hip: u += half_dt du/dt (cubic SPH model) */
 int sfd_sph_u_kick(float* u, const float* dudt, unsigned int N, float half_dt, hipStream_t s);
 
@@ -188,6 +185,10 @@ unsigned int sfd_reduce_scratch_doubles(unsigned int N);
 int sfd_reduce_state(const float* pos, const double* x64, const float* vel, const float* mas,
                      const float* pot, const float* ken, const float* pen, const float* u,
                      unsigned int N, double G, double eps, double* red, hipStream_t s);
+/* v += half_dt a and sfd_energy_terms first, in the same pass */
+int sfd_kick_reduce_state(const float* pos, const double* x64, float* vel, const float* acc, const float* mas,
+                          const float* pot, float half_dt, float* ken, float* pen, const float* u, unsigned int N,
+                          double G, double eps, double* red, hipStream_t s);
 
 #ifdef __cplusplus
 }
