@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "lookback.h"
 #include "tree_dev.h"
 
 namespace {
@@ -203,17 +204,6 @@ __global__ __launch_bounds__(kOffsThreads) void k_radix_offsets(const unsigned* 
 	offs[blockIdx.x * 256u + t] = excl;
 }
 
-// State word of a tile's digit: nothing yet, the tile's own count, or the
-// count of the tile and all before it.
-constexpr unsigned long long kOwn = 1ull << 32, kAll = 2ull << 32;
-
-__device__ __forceinline__ unsigned long long peek(const unsigned long long* p) {
-	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void post(unsigned long long* p, unsigned long long v) {
-	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // One digit's pass over a tile of 256 PER pairs.  Each wavefront ranks its
 // consecutive elements in index order (a 64-lane match mask from eight
 // ballots per round, and per-wave running digit counts in LDS); the tile's
@@ -221,15 +211,13 @@ __device__ __forceinline__ void post(unsigned long long* p, unsigned long long v
 // digit t), the tile is staged in LDS in sorted order and written out by
 // consecutive threads, so that each digit's run goes to consecutive global
 // addresses.
-// Tiles are numbered by a ticket taken when a block starts, so the tiles
-// before one's own belong to blocks that have started; a block posts its own
-// counts before it waits for anything, so every wait ends.
+// State words and tickets as in lookback.h.
 template <unsigned PER>
 __global__ __launch_bounds__(kBlock) void k_radix_pass(const unsigned long long* __restrict__ key_in,
                                                        const unsigned* __restrict__ val_in, unsigned shift,
                                                        const unsigned* __restrict__ offs,
                                                        unsigned long long* state, unsigned long long* state_next,
-                                                       unsigned* ticket, unsigned long long* __restrict__ key_out,
+                                                       unsigned* tickets, unsigned long long* __restrict__ key_out,
                                                        unsigned* __restrict__ val_out) {
 	constexpr unsigned kLook = 2;   // tiles looked back at once
 	__shared__ unsigned long long s_key[kBlock * PER];
@@ -240,10 +228,8 @@ __global__ __launch_bounds__(kBlock) void k_radix_pass(const unsigned long long*
 	__shared__ unsigned s_wsum[kBlock / 64];
 	__shared__ unsigned s_tile;
 	const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
-	if (t == 0u) s_tile = atomicAdd(ticket, 1u);
 	for (unsigned q = 0; q < kBlock / 64; ++q) s_wcnt[q][t] = 0u;
-	__syncthreads();
-	const unsigned tile = __builtin_amdgcn_readfirstlane(s_tile);
+	const unsigned tile = look::ticket(tickets, s_tile);   // past its barrier s_wcnt is clear
 	state_next[(size_t)tile * 256u + t] = 0ull;
 	// rank: element r of this thread is tile element (w PER + r) 64 + lane
 	const unsigned long long lt = (1ull << lane) - 1ull;
@@ -279,7 +265,7 @@ __global__ __launch_bounds__(kBlock) void k_radix_pass(const unsigned long long*
 		cnt += c;
 	}
 	unsigned long long* mine = state + (size_t)tile * 256u + t;
-	post(mine, (tile ? kOwn : kAll) | cnt);
+	look::post(mine, (tile ? look::kOwn : look::kAll) | cnt);
 	// exclusive scan of the tile's 256 digit counts
 	unsigned inc = cnt;
 	for (int k = 1; k < 64; k <<= 1) {
@@ -292,19 +278,19 @@ __global__ __launch_bounds__(kBlock) void k_radix_pass(const unsigned long long*
 		unsigned long long v[kLook];
 #pragma unroll
 		for (unsigned q = 0; q < kLook; ++q)
-			v[q] = j >= (int)q ? peek(state + (size_t)(j - (int)q) * 256u + t) : kAll;
+			v[q] = j >= (int)q ? look::peek(state + (size_t)(j - (int)q) * 256u + t) : look::kAll;
 		bool done = false;
 #pragma unroll
 		for (unsigned q = 0; q < kLook; ++q) {
 			if (done || j < (int)q) continue;
-			while (v[q] == 0ull) v[q] = peek(state + (size_t)(j - (int)q) * 256u + t);
+			while (v[q] == 0ull) v[q] = look::peek(state + (size_t)(j - (int)q) * 256u + t);
 			prior += (unsigned)v[q];
-			done = v[q] >= kAll;
+			done = v[q] >= look::kAll;
 		}
 		if (done) break;
 		j -= (int)kLook;
 	}
-	if (tile) post(mine, kAll | (unsigned long long)(prior + cnt));
+	if (tile) look::post(mine, look::kAll | (unsigned long long)(prior + cnt));
 	s_base[t] = offs[t] + prior;
 	__syncthreads();
 	unsigned excl = inc - cnt;

@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "exact_inv.h"
 #include "force_epi.h"
 #include "order_chain.h"
 #include "pp_sym.h"
@@ -52,27 +53,6 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	c = z - y;
 	s = t;
 }
-
-// 1 / s and 1 / sqrt(s) with the IEEE quotient's and square root's bits (each
-// rounded to nearest, the second from the rounded root), in 11 operations and
-// one v_rsq_f32 instead of two divisions and a square root of about 45:
-// Newton steps whose last operation is an FMA (Markstein's scheme).
-// Compared with 1.0f / s and 1.0f / sqrtf(s) on the device for every float
-// in [2^-96, 2^97): they differ only where the significand of s is all ones
-// or within one of it (1/s or 1/root then lies next to a rounding boundary).
-// kRootBits tells those, and kTopBits the values above the range.
-__device__ __forceinline__ void exact_inverses(float s, float& inv_s, float& inv_root) {
-	const float r = __builtin_amdgcn_rsqf(s);
-	const float g = s * r, h = 0.5f * r;
-	const float root = __builtin_fmaf(__builtin_fmaf(-g, g, s), h, g);
-	inv_root = __builtin_fmaf(r, __builtin_fmaf(-root, r, 1.0f), r);
-	const float q = r * r;
-	const float e = __builtin_fmaf(-s, q, 1.0f);
-	inv_s = __builtin_fmaf(q, __builtin_fmaf(e, e, e), q);
-}
-constexpr unsigned kRootBits = 0xFFFFFFFEu;   // bits(s) | 0xFF800000 at or above this: IEEE operations
-constexpr unsigned kTopBits = 0x6F800000u;    // bits(s) at or above this (2^96, inf, NaN): IEEE operations
-constexpr float kExactMinEps2 = 0x1p-96f;     // s >= eps2: below this, IEEE operations throughout
 
 // The terms of the reference's pair (src/gravity.c:709-769) and its sums:
 // the model that order_chain.h runs, components x, y, z and the potential.

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "exact_inv.h"
 #include "tree_dev.h"
 
 namespace {
@@ -131,28 +132,34 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	s = t;
 }
 
+__device__ __forceinline__ float mean_width(const float* bmin, const float* bmax) {
+	const float third = (float)(1.0 / 3.0);
+	return third * (((bmax[0] - bmin[0]) + (bmax[1] - bmin[1])) + (bmax[2] - bmin[2]));
+}
+
 // The opening test of src/gravity.c:334-357 for a node of more than eight
 // bodies: open iff theta <= (mean width)^2 / (distance to the centre)^2.
 __device__ __forceinline__ bool opens(const float* bmin, const float* bmax, const float* ri, float theta) {
-	const float third = (float)(1.0 / 3.0);
 	float off[3];
 	for (int a = 0; a < 3; ++a) off[a] = 0.5f * (bmin[a] + bmax[a]) - ri[a];
 	const float d2 = (off[0] * off[0] + off[1] * off[1]) + off[2] * off[2];
-	const float w = third * (((bmax[0] - bmin[0]) + (bmax[1] - bmin[1])) + (bmax[2] - bmin[2]));
+	const float w = mean_width(bmin, bmax);
 	const float ratio = 0.0f < d2 ? (w * w) / d2 : 0.0f;
 	return theta <= ratio;
 }
 
-// The node as one monopole, less particle i when the node's box holds it
-// (src/gravity.c:380-640), added into the (Kahan) sums.
+// The node as one monopole, less particle i when the node's box holds it and
+// other bodies (holds; src/gravity.c:380-640), added into the (Kahan) sums.
+__device__ __forceinline__ bool in_box(const float* b, const float* ri) {   // b: the lower corner, then the upper
+	return b[0] <= ri[0] && ri[0] <= b[3] && b[1] <= ri[1] && ri[1] <= b[4] && b[2] <= ri[2] && ri[2] <= b[5];
+}
+
 template <bool KAHAN_ACC, bool KAHAN_POT>
-__device__ __forceinline__ void add_monopole(const sf_node* __restrict__ nd, unsigned bodies, const float* bmin,
-                                             const float* bmax, const float* ri, float mi, float eps2, float* sum,
-                                             float* com) {
-	float rj[3] = {nd->params[0], nd->params[1], nd->params[2]};
-	float mj = nd->params[3];
-	if (bmin[0] <= ri[0] && ri[0] <= bmax[0] && bmin[1] <= ri[1] && ri[1] <= bmax[1] && bmin[2] <= ri[2] &&
-	    ri[2] <= bmax[2] && 1u < bodies) {
+__device__ __forceinline__ void add_monopole(const float* params, bool holds, const float* ri, float mi, float eps2,
+                                             float* sum, float* com) {
+	float rj[3] = {params[0], params[1], params[2]};
+	float mj = params[3];
+	if (holds) {
 		for (int a = 0; a < 3; ++a) rj[a] = rj[a] * mj;
 		for (int a = 0; a < 3; ++a) rj[a] = rj[a] - mi * ri[a];
 		mj = mj - mi;
@@ -160,8 +167,8 @@ __device__ __forceinline__ void add_monopole(const sf_node* __restrict__ nd, uns
 	}
 	const float rx = ri[0] - rj[0], ry = ri[1] - rj[1], rz = ri[2] - rj[2];
 	const float r2 = (rx * rx + ry * ry) + rz * rz;
-	const float inv_r2 = 1.0f / (r2 + eps2);
-	const float inv_r1 = 1.0f / sqrtf(r2 + eps2);
+	float inv_r2, inv_r1;
+	checked_inverses(r2 + eps2, inv_r2, inv_r1);
 	const float pj = mj * inv_r1;
 	const float f[3] = {pj * inv_r2 * rx, pj * inv_r2 * ry, pj * inv_r2 * rz};
 	for (int a = 0; a < 3; ++a) {
@@ -241,27 +248,58 @@ __global__ __launch_bounds__(kBlock) void k_tree_walk_ref(const float* __restric
 				continue;
 			}
 		}
-		add_monopole<KAHAN_ACC, KAHAN_POT>(nd, bodies, bmin, bmax, ri, mi, eps2, sum, com);
+		add_monopole<KAHAN_ACC, KAHAN_POT>(nd->params, 1u < bodies && in_box(nd->bounds, ri), ri, mi, eps2, sum, com);
 		next_node = parent;
 		cur_depth -= 1;
 	}
 	store_walk<PHYS>(idx, mi, negG, sum, acc, pot);
 }
 
-// The same walk over threaded links: down[n] is n's first non-empty child,
-// next[n] the first non-empty node after n's subtree in the walk's order
+// The same walk over threaded links: down is the node's first non-empty child,
+// next the first non-empty node after its subtree in the walk's order
 // (children in octant order), kEnd past the last.  It visits the reference
 // walk's non-empty nodes in its order without the returns to the parent;
 // empty nodes add nothing there.  For a complete tree the reference walk
 // takes 16 (opened nodes) + 1 <= 2 num_nodes - 1 iterations, below its cap,
 // so the two walks add the same terms in the same order.
+//
+// Bound by the divergent loads: 64 lanes at as many nodes take a look-up in L1
+// each per 16 bytes, and a CU's four wavefronts share it.  A visit reads a
+// 48-byte record, and the node's box itself only where the particle may lie in
+// it; the next record is loaded as soon as the opening test has chosen it,
+// before the monopole's arithmetic, which has no divisions left (opens_at,
+// checked_inverses).  A Plummer sphere of 65536: 308 us instead of 353 with the
+// node's own 80 bytes and its links, and IEEE divisions; with 64-byte records
+// 345, with the record after next loaded ahead as well 397.  Visiting the
+// union of a wavefront's nodes in step, with scalar loads, took 1144.
 constexpr unsigned kEnd = 0xFFFFFFFFu;
+
+struct alignas(16) WalkRec {
+	float centre[3], width2;   // (mean width)^2, the dividend of the opening test
+	unsigned down, next, bodies;
+	float reach;               // beyond this distance from the centre on an axis lies outside the box
+	float params[4];
+};
+static_assert(sizeof(WalkRec) == SF_WALK_REC_BYTES, "the host allocates the records");
+
+// opens() of a record: the quotient's side of theta is clear from an
+// approximation within 2^-20 of it, or it is divided.
+__device__ __forceinline__ bool opens_at(float width2, const float* off, float theta) {
+	const float d2 = (off[0] * off[0] + off[1] * off[1]) + off[2] * off[2];
+	if (d2 > 1.0e-37f && d2 < 1.0e37f && theta > 1.0e-30f) {
+		const float about = width2 * __builtin_amdgcn_rcpf(d2);
+		if (about > theta * 1.000001f && about < 3.0e38f) return true;
+		if (about < theta * 0.999999f) return false;
+	}
+	const float ratio = 0.0f < d2 ? width2 / d2 : 0.0f;
+	return theta <= ratio;
+}
 
 template <bool KAHAN_ACC, bool KAHAN_POT, bool PHYS>
 __global__ __launch_bounds__(kBlock) void k_tree_walk_thr(const float* __restrict__ pos, const float* __restrict__ mas,
                                                           unsigned N, const unsigned* __restrict__ order,
                                                           const sf_node* __restrict__ node,
-                                                          const uint2* __restrict__ link, float eps2, float theta,
+                                                          const WalkRec* __restrict__ recs, float eps2, float theta,
                                                           float negG, float* __restrict__ acc,
                                                           float* __restrict__ pot) {
 	const unsigned lane_id = blockIdx.x * kBlock + threadIdx.x;
@@ -270,28 +308,31 @@ __global__ __launch_bounds__(kBlock) void k_tree_walk_thr(const float* __restric
 	float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f}, com[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 	const float ri[3] = {pos[3u * idx], pos[3u * idx + 1u], pos[3u * idx + 2u]};
 	const float mi = mas[idx];
-	unsigned n = node[0].bodies ? 0u : kEnd;
+	WalkRec w = recs[0];
+	unsigned n = w.bodies ? 0u : kEnd;
 	while (n != kEnd) {
-		const sf_node* nd = &node[n];
-		const uint2 ln = link[n];   // (down, next)
-		const unsigned bodies = nd->bodies;
-		const float bmin[3] = {nd->bounds[0], nd->bounds[1], nd->bounds[2]};
-		const float bmax[3] = {nd->bounds[3], nd->bounds[4], nd->bounds[5]};
-		if (bodies > 8u && opens(bmin, bmax, ri, theta)) {
-			n = ln.x;
-			continue;
+		float off[3];
+		for (int a = 0; a < 3; ++a) off[a] = w.centre[a] - ri[a];
+		const bool open = w.bodies > 8u && opens_at(w.width2, off, theta);
+		const unsigned here = n;
+		n = open ? w.down : w.next;
+		WalkRec v = w;
+		if (n != kEnd) v = recs[n];
+		if (!open) {
+			// not beyond reach (NaN included): the box decides
+			const bool holds = 1u < w.bodies && !(fabsf(off[0]) > w.reach || fabsf(off[1]) > w.reach ||
+			                                      fabsf(off[2]) > w.reach) && in_box(node[here].bounds, ri);
+			add_monopole<KAHAN_ACC, KAHAN_POT>(w.params, holds, ri, mi, eps2, sum, com);
 		}
-		add_monopole<KAHAN_ACC, KAHAN_POT>(nd, bodies, bmin, bmax, ri, mi, eps2, sum, com);
-		n = ln.y;
+		w = v;
 	}
 	store_walk<PHYS>(idx, mi, negG, sum, acc, pot);
 }
 
-// link[t] = (first non-empty child, first non-empty node after t's subtree)
-// for the num_nodes nodes of a complete tree.  Walking up through last
-// children takes at most the tree depth (16) steps.
+// The walk records of the num_nodes nodes of a complete tree.  Walking up
+// through last children takes at most the tree depth (16) steps.
 __global__ __launch_bounds__(kBlock) void k_tree_links(const sf_node* __restrict__ node, const unsigned* __restrict__ meta,
-                                                       uint2* __restrict__ link) {
+                                                       WalkRec* __restrict__ recs) {
 	const unsigned t = blockIdx.x * kBlock + threadIdx.x;
 	const unsigned num_nodes = meta[0];
 	if (t >= num_nodes) return;
@@ -317,7 +358,22 @@ __global__ __launch_bounds__(kBlock) void k_tree_links(const sf_node* __restrict
 		if (next != kEnd) break;
 		n = par;
 	}
-	link[t] = make_uint2(down, next);
+	const sf_node nd = node[t];
+	WalkRec w;
+	float half = 0.0f;
+	for (int a = 0; a < 3; ++a) {
+		w.centre[a] = 0.5f * (nd.bounds[a] + nd.bounds[3 + a]);
+		half = fmaxf(half, fmaxf(fabsf(nd.bounds[a] - w.centre[a]), fabsf(nd.bounds[3 + a] - w.centre[a])));
+	}
+	const float width = mean_width(nd.bounds, nd.bounds + 3);
+	w.width2 = width * width;
+	w.bodies = nd.bodies;
+	// wider than the box by more than the rounding of a distance from its centre
+	w.reach = half * 1.00001f;
+	for (int k = 0; k < 4; ++k) w.params[k] = nd.params[k];
+	w.down = down;
+	w.next = next;
+	recs[t] = w;
 }
 
 }  // namespace
@@ -363,7 +419,7 @@ extern "C" int sfd_tree_links(const sf_node* node, const unsigned* meta, unsigne
                               hipStream_t s) {
 	const unsigned grid = (max_nodes + kBlock - 1) / kBlock;
 	hipLaunchKernelGGL(k_tree_links, dim3(grid ? grid : 1), dim3(kBlock), 0, s, node, meta,
-	                   static_cast<uint2*>(link));
+	                   static_cast<WalkRec*>(link));
 	return sf_hip_check(hipGetLastError(), "sfd_tree_links", "launch");
 }
 
@@ -372,12 +428,12 @@ extern "C" int sfd_tree_walk_thr(const float* pos, const float* mas, unsigned N,
                                  int acc_phys, int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s) {
 	if (N == 0) return 0;
 	const dim3 grid((N + kBlock - 1) / kBlock), block(kBlock);
-	const uint2* ln = static_cast<const uint2*>(link);
+	const WalkRec* recs = static_cast<const WalkRec*>(link);
 	const int sel = (kahan_acc ? 4 : 0) | (kahan_pot ? 2 : 0) | (acc_phys ? 1 : 0);
 	const int tok = sf_prof_begin("tree_walk_ref", s);
 #define SF_WALK(A, B, C)                                                                                         \
-	hipLaunchKernelGGL((k_tree_walk_thr<A, B, C>), grid, block, 0, s, pos, mas, N, order, node, ln, eps2, theta, negG, \
-	                   acc, pot)
+	hipLaunchKernelGGL((k_tree_walk_thr<A, B, C>), grid, block, 0, s, pos, mas, N, order, node, recs, eps2, theta,      \
+	                   negG, acc, pot)
 	switch (sel) {
 	case 0: SF_WALK(false, false, false); break;
 	case 1: SF_WALK(false, false, true); break;

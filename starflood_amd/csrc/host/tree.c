@@ -35,7 +35,7 @@ struct sf_tree_dev {
 	double* d_radius;        /* partial sums of the reference bounds' mean radius */
 	unsigned int* d_order;   /* walk order of the last parallel build (N entries) */
 	unsigned int order_n;    /* its N, 0 when the last build was serial */
-	void* d_link;            /* threaded links of the last complete parallel build (max_nodes x 2 u32) */
+	void* d_link;            /* walk records of the last complete parallel build */
 	sf_lbvh* lbvh;           /* SF_TREE_LBVH state (lbvh.c) */
 };
 
@@ -146,7 +146,9 @@ static int is_device_pointer(const void* p) {
 
 /* Reference-mode build from device pos/mas into d->d_node; reports the
    reference's errors (src/tree.c:180-189) after a synchronisation. */
-static int build_ref(sf_tree_dev* d, tree_t* t, unsigned int N, const float* pos, const float* mas, hipStream_t s) {
+/* Queues the reference build on s; d->order_n = N when the parallel build made
+   the tree (d->par.ev[0] marks its end on s). */
+static int build_ref(sf_tree_dev* d, unsigned int N, const float* pos, const float* mas, hipStream_t s) {
 	const sf_params_t* p = sf_params();
 	/* 0: serial build only (also for no particles: the root alone) */
 	const size_t need = N ? sfd_tree_par_bytes(N, d->max_nodes) : 0u;
@@ -177,14 +179,27 @@ static int build_ref(sf_tree_dev* d, tree_t* t, unsigned int N, const float* pos
 	                                             (int)p->tree_depth_max, d->d_node, d->d_meta, d->d_order, s)
 	                    : 1;
 	if (rc == 0) {
-		if (!d->d_link) SF_HIP(hipMalloc(&d->d_link, (size_t)d->max_nodes * 2u * sizeof(unsigned int)), "tree_build");
+		if (!d->d_link) SF_HIP(hipMalloc(&d->d_link, (size_t)d->max_nodes * SF_WALK_REC_BYTES), "tree_build");
 		if (sfd_tree_links(d->d_node, d->d_meta, d->max_nodes, d->d_link, s)) return -1;
+		SF_HIP(hipEventRecord(d->par.ev[0], s), "tree_build");
 		d->order_n = N;
 	}
 	if (rc < 0) return -1;
 	if (rc > 0 &&
 	    sfd_tree_build_ref(pos, mas, N, d->d_bounds, d->max_nodes, (int)p->tree_depth_max, d->d_node, d->d_meta, s))
 		return -1;
+	return 0;
+}
+
+/* num_nodes, the host's nodes (mirror mode) and the build's result.  After a
+   parallel build the copies run on its side stream, beside what s does next
+   (the walk). */
+static int finish_ref(sf_tree_dev* d, tree_t* t, hipStream_t s) {
+	const sf_params_t* p = sf_params();
+	if (d->order_n) {
+		SF_HIP(hipStreamWaitEvent(d->par.side, d->par.ev[0], 0), "tree_build");
+		s = d->par.side;
+	}
 	SF_HIP(hipMemcpyAsync(d->h_meta, d->d_meta, 2u * sizeof(unsigned int), hipMemcpyDeviceToHost, s), "tree_build");
 	SF_HIP(hipStreamSynchronize(s), "tree_build");
 	t->num_nodes = d->h_meta[0];
@@ -233,7 +248,8 @@ int tree_build(tree_t* SF_RESTRICT tree_ptr, unsigned int num_parts, const real*
 	SF_HIP(hipMemcpyAsync(d->d_bounds, tree_ptr->bounds, 6u * sizeof(float), hipMemcpyHostToDevice, s), "tree_build");
 	int rc;
 	if (p->tree_mode == SF_TREE_REFERENCE) {
-		rc = build_ref(d, tree_ptr, num_parts, dpos, dmas, s);
+		rc = build_ref(d, num_parts, dpos, dmas, s);
+		if (!rc) rc = finish_ref(d, tree_ptr, s);
 	} else {
 		rc = sf_lbvh_build(&d->lbvh, num_parts, dpos, dmas, sf_params()->quadrupole, s);
 		if (!rc) tree_ptr->num_nodes = num_parts ? 2u * num_parts - 1u : 0u;
@@ -286,12 +302,15 @@ int sf_solve_gravity_tree(sf_ctx* c, tree_t* tree, unsigned int step_number, int
 		if (!d->d_radius)
 			SF_HIP(hipMalloc((void**)&d->d_radius, 2u * SF_RADIUS_PARTIALS * sizeof(double)), "solve_gravity_part_tree");
 		if (N && sfd_tree_bounds_ref(pos, N, jit, d->d_radius, d->d_bounds, s)) return -1;
-		const int rc = build_ref(d, tree, N, pos, mas, s);
-		SF_HIP(hipMemcpyAsync(tree->bounds, d->d_bounds, 6u * sizeof(float), hipMemcpyDeviceToHost, s),
-		       "solve_gravity_part_tree");
+		int rc = build_ref(d, N, pos, mas, s);
 		/* the reference walks the tree even after a failed build */
-		if (walk_ref(d, N, pos, mas, eps2, acc, pot, s)) return -1;
-		return rc;
+		const int walked = rc ? 0 : walk_ref(d, N, pos, mas, eps2, acc, pot, s);
+		if (!rc) rc = finish_ref(d, tree, s);
+		SF_HIP(hipMemcpyAsync(tree->bounds, d->d_bounds, 6u * sizeof(float), hipMemcpyDeviceToHost,
+		                      d->order_n ? d->par.side : s),
+		       "solve_gravity_part_tree");
+		if (d->order_n) SF_HIP(hipStreamSynchronize(d->par.side), "solve_gravity_part_tree");
+		return walked ? -1 : rc;
 	}
 	if (sf_lbvh_build(&d->lbvh, N, pos, mas, p->quadrupole, s)) return -1;
 	tree->num_nodes = N ? 2u * N - 1u : 0u;
