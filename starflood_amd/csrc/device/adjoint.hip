@@ -12,12 +12,11 @@
 // pair (j = k, where K = I/eps^3 is largest) cancels exactly.
 //
 // Per pair: 26 VALU operations and one v_rsq_f32 (the force takes 13), with
-// the same layout as the fast PP kernel: one lane per k, the j stream
-// wavefront-uniform (scalar loads), j split into slices over the grid with
-// Kahan-folded partial sums per tile, and a fixed-order FP64 combine.  The
-// whole tiles of equal-mass particles that sfd_pack_bodies finds form
-// w = m (nu_j - nu_k) instead (23 VALU operations; still exactly zero for
-// j == k), scaling each tile partial by m.
+// the same layout as pp.hip's kernel of small states: one lane per k, tiles of
+// 64 j staged in LDS, j split over wavefronts, Kahan-folded sums per tile, and
+// a fixed-order FP64 combine.  Tiles of one mass form w = m (nu_j - nu_k)
+// instead (23 VALU operations; still exactly zero for j == k), scaling each
+// tile's sums by m.
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
@@ -26,9 +25,6 @@
 namespace {
 
 constexpr unsigned kBlock = 256;
-constexpr unsigned kTile = 128;
-constexpr int kPrefetch = 4;   // j records per scalar-load group
-static_assert(kTile % kPrefetch == 0, "tiles hold whole prefetch groups");
 
 __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	const float y = x - c;
@@ -38,105 +34,91 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 	s = t;
 }
 
-// One tile of kTile pairs, j from jt; nbb/nbn hold the tile's first
-// kPrefetch j records on entry and the next tile's on exit.  UNIFORM: every
-// mass of the tile and of k equals m, and the sums leave it out.
+// Pairs of k with a tile's 64 bodies and weights in LDS, read by every lane.
+// UNIFORM: every mass of the tile and of k is the same, and the sums leave it
+// out.
 template <bool UNIFORM>
-__device__ __forceinline__ void vjp_tile(const float4* __restrict__ body, const float4* __restrict__ nu, unsigned jt,
-                                         unsigned j1, float4 (&nbb)[kPrefetch], float4 (&nbn)[kPrefetch],
+__device__ __forceinline__ void vjp_tile(const float4* __restrict__ body, const float4* __restrict__ nu,
                                          const float4& bk, const float4& nk, float eps2, float& tx, float& ty,
                                          float& tz) {
-	for (unsigned j = jt; j < jt + kTile; j += kPrefetch) {
-		float4 cbb[kPrefetch], cbn[kPrefetch];
-#pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) {
-			cbb[u] = nbb[u];
-			cbn[u] = nbn[u];
-		}
-		const unsigned jn = (j + kPrefetch < j1) ? j + kPrefetch : j;   // in bounds
-#pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) {
-			nbb[u] = body[jn + u];
-			nbn[u] = nu[jn + u];
-		}
-#pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) {
-			const float4 bj = cbb[u];
-			const float4 nj = cbn[u];
-			const float dx = bk.x - bj.x, dy = bk.y - bj.y, dz = bk.z - bj.z;
-			float r2 = __builtin_fmaf(dx, dx, eps2);
-			r2 = __builtin_fmaf(dy, dy, r2);
-			r2 = __builtin_fmaf(dz, dz, r2);
-			const float inv = __builtin_amdgcn_rsqf(r2);
-			const float inv2 = inv * inv;
-			const float inv3 = inv2 * inv;
-			const float i5_3 = inv3 * (3.0f * inv2);
-			// exactly zero when j == k: a difference of equal values, or of two
-			// equal rounded products
-			const float wx = UNIFORM ? nj.x - nk.x : bk.w * nj.x - bj.w * nk.x;
-			const float wy = UNIFORM ? nj.y - nk.y : bk.w * nj.y - bj.w * nk.y;
-			const float wz = UNIFORM ? nj.z - nk.z : bk.w * nj.z - bj.w * nk.z;
-			const float dw = __builtin_fmaf(dz, wz, __builtin_fmaf(dy, wy, dx * wx));
-			const float q = i5_3 * dw;
-			tx = __builtin_fmaf(-q, dx, __builtin_fmaf(inv3, wx, tx));
-			ty = __builtin_fmaf(-q, dy, __builtin_fmaf(inv3, wy, ty));
-			tz = __builtin_fmaf(-q, dz, __builtin_fmaf(inv3, wz, tz));
-		}
+#pragma unroll 8
+	for (unsigned j = 0; j < kSymTile; ++j) {
+		const float4 bj = body[j], nj = nu[j];
+		const float dx = bk.x - bj.x, dy = bk.y - bj.y, dz = bk.z - bj.z;
+		float r2 = __builtin_fmaf(dx, dx, eps2);
+		r2 = __builtin_fmaf(dy, dy, r2);
+		r2 = __builtin_fmaf(dz, dz, r2);
+		const float inv = __builtin_amdgcn_rsqf(r2);
+		const float inv2 = inv * inv;
+		const float inv3 = inv2 * inv;
+		const float i5_3 = inv3 * (3.0f * inv2);
+		// exactly zero when j == k: a difference of equal values, or of two
+		// equal rounded products
+		const float wx = UNIFORM ? nj.x - nk.x : bk.w * nj.x - bj.w * nk.x;
+		const float wy = UNIFORM ? nj.y - nk.y : bk.w * nj.y - bj.w * nk.y;
+		const float wz = UNIFORM ? nj.z - nk.z : bk.w * nj.z - bj.w * nk.z;
+		const float dw = __builtin_fmaf(dz, wz, __builtin_fmaf(dy, wy, dx * wx));
+		const float q = i5_3 * dw;
+		tx = __builtin_fmaf(-q, dx, __builtin_fmaf(inv3, wx, tx));
+		ty = __builtin_fmaf(-q, dy, __builtin_fmaf(inv3, wy, ty));
+		tz = __builtin_fmaf(-q, dz, __builtin_fmaf(inv3, wz, tz));
 	}
 }
 
-// body = (x, y, z, m) and nu = (nu, 0) for n_pad entries (m = nu = 0 past
-// N); the word after the n_pad bodies holds n_uni, the leading bodies that
-// form whole tiles of one mass, body[0].w (sfd_pack_bodies)
+// body = (x, y, z, m) and nu = (nu, 0) for n_pad entries (m = nu = 0 past N).
+// Block b owns 64 k (the same in its wavefronts) and a j slice, as k_pp_few.
+// With the j stream in scalar loads a VJP with its launches and the wait for it
+// took 64 us up to 1000 bodies, 54 at 3000 and 67 at 6000; now 33, 40 and 61.
+constexpr unsigned kVjpWaves = kBlock / 64;
 __global__ __launch_bounds__(kBlock) void k_vjp(const float4* __restrict__ body, const float4* __restrict__ nu,
-                                                unsigned n_pad, unsigned slices, unsigned slice_len, float eps2,
-                                                float4* __restrict__ part) {
-	static_assert(kTile == 128u, "n_uni counts whole tiles of 128 bodies");
-	const unsigned b = blockIdx.x;
-	const unsigned sl = b % slices;
-	const unsigned k = (b / slices) * kBlock + threadIdx.x;
-	const float4 bk = body[k];
-	const float4 nk = nu[k];
-	float Sx = 0.0f, Sy = 0.0f, Sz = 0.0f, Cx = 0.0f, Cy = 0.0f, Cz = 0.0f;
-	// one group of kPrefetch j records in flight, as in the fast PP kernel
-	const unsigned j0 = sl * slice_len;
-	const unsigned j1 = min(j0 + slice_len, n_pad);
-	const unsigned n_uni = *reinterpret_cast<const unsigned*>(body + n_pad);
-	const unsigned ju = min(j1, max(j0, n_uni));
+                                                unsigned n_pad, unsigned slices, unsigned per, float eps2,
+                                                double4* __restrict__ part) {
+	__shared__ float4 s_body[kVjpWaves][2][kSymTile], s_nu[kVjpWaves][2][kSymTile];
+	__shared__ double red[kVjpWaves][3][64];
+	const unsigned sl = blockIdx.x % slices;
+	const unsigned lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const unsigned k = (blockIdx.x / slices) * 64u + lane;
+	const unsigned j0 = min((sl * kVjpWaves + wv) * per * kSymTile, n_pad), j1 = min(j0 + per * kSymTile, n_pad);
+	const float4 bk = body[k], nk = nu[k], zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	float4 vb = j0 < j1 ? body[j0 + lane] : zero, vn = j0 < j1 ? nu[j0 + lane] : zero;
 	const float mu = body[0].w;
-	float4 nbb[kPrefetch], nbn[kPrefetch];
-#pragma unroll
-	for (int u = 0; u < kPrefetch; ++u) {
-		nbb[u] = body[j0 + u];
-		nbn[u] = nu[j0 + u];
-	}
-	unsigned jt = j0;
-	// the equal-mass tiles need m_k = m too: k beyond n_uni (padding, or a
-	// partial tile) takes the general sum throughout.  n_uni is a multiple of
-	// 128 and a wavefront's 64 k are aligned, so the test is the same on every
-	// lane; lane 0's k keeps the branch (and the j stream) scalar.
-	if (__builtin_amdgcn_readfirstlane(k) < n_uni) {
-		for (; jt < ju; jt += kTile) {
-			float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-			vjp_tile<true>(body, nu, jt, j1, nbb, nbn, bk, nk, eps2, tx, ty, tz);
-			kahan_add(Sx, Cx, mu * tx);
-			kahan_add(Sy, Cy, mu * ty);
-			kahan_add(Sz, Cz, mu * tz);
+	const bool k_uni = __ballot(__float_as_uint(bk.w) != __float_as_uint(mu)) == 0ull;
+	float sum[3] = {0.0f, 0.0f, 0.0f}, com[3] = {0.0f, 0.0f, 0.0f};
+	unsigned buf = 0u;
+	for (unsigned j = j0; j < j1; j += kSymTile) {
+		s_body[wv][buf][lane] = vb;
+		s_nu[wv][buf][lane] = vn;
+		const bool uni = k_uni && __ballot(__float_as_uint(vb.w) != __float_as_uint(mu)) == 0ull;
+		if (j + kSymTile < j1) {
+			vb = body[j + kSymTile + lane];
+			vn = nu[j + kSymTile + lane];
 		}
+		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+		float t[3] = {0.0f, 0.0f, 0.0f};
+		if (uni) vjp_tile<true>(s_body[wv][buf], s_nu[wv][buf], bk, nk, eps2, t[0], t[1], t[2]);
+		else vjp_tile<false>(s_body[wv][buf], s_nu[wv][buf], bk, nk, eps2, t[0], t[1], t[2]);
+		const float sc = uni ? mu : 1.0f;
+#pragma unroll
+		for (int u = 0; u < 3; ++u) kahan_add(sum[u], com[u], sc * t[u]);
+		buf ^= 1u;
 	}
-	for (; jt < j1; jt += kTile) {
-		float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-		vjp_tile<false>(body, nu, jt, j1, nbb, nbn, bk, nk, eps2, tx, ty, tz);
-		kahan_add(Sx, Cx, tx);
-		kahan_add(Sy, Cy, ty);
-		kahan_add(Sz, Cz, tz);
+	// Kahan's compensation holds the negated lost low part
+#pragma unroll
+	for (int u = 0; u < 3; ++u) red[wv][u][lane] = (double)sum[u] - (double)com[u];
+	__syncthreads();
+	if (wv != 0) return;
+	double4 t = make_double4(red[0][0][lane], red[0][1][lane], red[0][2][lane], 0.0);
+#pragma unroll
+	for (unsigned q = 1; q < kVjpWaves; ++q) {
+		t.x += red[q][0][lane];
+		t.y += red[q][1][lane];
+		t.z += red[q][2][lane];
 	}
-	part[(size_t)(2u * sl) * n_pad + k] = make_float4(Sx, Sy, Sz, 0.0f);
-	part[(size_t)(2u * sl + 1u) * n_pad + k] = make_float4(Cx, Cy, Cz, 0.0f);
+	part[(size_t)sl * n_pad + k] = t;
 }
 
 // ------------------------------------------------- each pair once (pp_sym.h)
-// From kSymMin bodies: w = m_k nu_j - m_j nu_k changes sign with the pair's
+// From kVjpSymMin bodies: w = m_k nu_j - m_j nu_k changes sign with the pair's
 // order and K does not, so a pair's term goes to k as it is and to j negated:
 // 29 VALU operations and one rsq with equal masses (35 with general ones) for
 // both, where the one-sided kernel takes 46 and two (52).  The layout is
@@ -329,25 +311,24 @@ struct VjpStep {
 	}
 };
 
-// g_k = G * sum over slices of (sum - compensation), in FP64
+// g_k = G * sum over slices, in FP64
 // A block takes kCombI particles; its wavefronts take the slices s = w,
 // w + kCombG, ... (w = wavefront) and wavefront 0 adds their sums in order
 // (all lanes of one particle per slice would leave most CUs idle at small N).
 constexpr unsigned kCombI = 64;
 constexpr unsigned kCombG = kBlock / kCombI;
 template <class E>
-__global__ __launch_bounds__(kBlock) void k_vjp_combine(const float4* __restrict__ part, unsigned n_pad,
+__global__ __launch_bounds__(kBlock) void k_vjp_combine(const double4* __restrict__ part, unsigned n_pad,
                                                         unsigned slices, unsigned N, double G, E epi) {
 	__shared__ double red[kCombG][3][kCombI];
 	const unsigned kl = threadIdx.x % kCombI, w = threadIdx.x / kCombI;
 	const unsigned k = blockIdx.x * kCombI + kl;   // < n_pad: the grid covers N in kCombI steps
 	double sx = 0.0, sy = 0.0, sz = 0.0;
 	for (unsigned s = w; s < slices; s += kCombG) {
-		const float4 a = part[(size_t)(2u * s) * n_pad + k];
-		const float4 c = part[(size_t)(2u * s + 1u) * n_pad + k];
-		sx += (double)a.x - (double)c.x;
-		sy += (double)a.y - (double)c.y;
-		sz += (double)a.z - (double)c.z;
+		const double4 a = part[(size_t)s * n_pad + k];
+		sx += a.x;
+		sy += a.y;
+		sz += a.z;
 	}
 	red[w][0][kl] = sx;
 	red[w][1][kl] = sy;
@@ -499,10 +480,10 @@ inline dim3 grid(unsigned n) { return dim3((n + kBlock - 1u) / kBlock); }
 
 extern "C" {
 
-// bytes of part for sfd_force_vjp: k_vjp_sym's planes, or below kSymMin
-// bodies slices x 2 x n_pad float4
-size_t sfd_vjp_part_bytes(unsigned n_pad, unsigned slices) {
-	return n_pad >= kSymMin ? sym_part_bytes(n_pad, false) : (size_t)slices * 2u * n_pad * 16u;
+// bytes of part for sfd_force_vjp: k_vjp_sym's planes, or below kVjpSymMin
+// bodies k_vjp's
+size_t sfd_vjp_part_bytes(unsigned n_pad) {
+	return n_pad >= kVjpSymMin ? sym_part_bytes(n_pad, false) : (size_t)few_geometry(n_pad).bslices * n_pad * 32u;
 }
 
 int sfd_pack_nu(const float* mu, const float* mas, unsigned N, unsigned n_pad, float coef, int acc_phys, float* nu,
@@ -517,14 +498,14 @@ int sfd_pack_nu(const float* mu, const float* mas, unsigned N, unsigned n_pad, f
 // (x, m) array of the force kernel, nu the packed weights (both n_pad float4),
 // part scratch of sfd_vjp_part_bytes.
 int sfd_force_vjp(const float* body, const float* nu, unsigned N, unsigned n_pad, float eps2, double G, float* part,
-                  unsigned slices, const sf_vjp_epi* epi, hipStream_t s) {
+                  const sf_vjp_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
-	if (n_pad % kBlock != 0 || slices == 0) return -1;
+	if (n_pad == 0 || n_pad % 1024u != 0) return -1;
 	const float4* b4 = reinterpret_cast<const float4*>(body);
 	const float4* nu4 = reinterpret_cast<const float4*>(nu);
 	float4* p4 = reinterpret_cast<float4*>(part);
 	const dim3 cgrid((N + kCombI - 1) / kCombI);
-	if (n_pad >= kSymMin) {
+	if (n_pad >= kVjpSymMin) {
 		const SymGeometry q = sym_geometry(n_pad, false);
 		double4* run = reinterpret_cast<double4*>(p4 + ((size_t)q.chunks + q.dchunks + q.per_launch) * n_pad);
 		for (unsigned d0 = 0; d0 < q.offsets; d0 += q.per_launch) {
@@ -544,19 +525,17 @@ int sfd_force_vjp(const float* body, const float* nu, unsigned N, unsigned n_pad
 		}
 		return sf_hip_check(hipGetLastError(), "sfd_force_vjp", "launch");
 	}
-	// whole tiles per slice, every slice non-empty (at most the requested count)
-	const unsigned tiles = n_pad / kTile;
-	if (slices > tiles) slices = tiles;
-	const unsigned slice_len = (tiles + slices - 1u) / slices * kTile;
-	slices = (n_pad + slice_len - 1u) / slice_len;
-	const unsigned grid_v = (n_pad / kBlock) * slices;
+	const FewGeometry g = few_geometry(n_pad);
+	double4* p8 = reinterpret_cast<double4*>(part);
 	const int tok = sf_prof_begin("force_vjp", s);
-	hipLaunchKernelGGL(k_vjp, dim3(grid_v), dim3(kBlock), 0, s, b4, nu4, n_pad, slices, slice_len, eps2, p4);
+	hipLaunchKernelGGL(k_vjp, dim3((n_pad / 64u) * g.bslices), dim3(kBlock), 0, s, b4, nu4, n_pad, g.bslices, g.per, eps2,
+	                   p8);
 	sf_prof_end(tok, s);
 	if (epi->step)
-		hipLaunchKernelGGL(k_vjp_combine<VjpStep>, cgrid, dim3(kBlock), 0, s, p4, n_pad, slices, N, G, VjpStep(*epi));
+		hipLaunchKernelGGL(k_vjp_combine<VjpStep>, cgrid, dim3(kBlock), 0, s, p8, n_pad, g.bslices, N, G,
+		                   VjpStep(*epi));
 	else
-		hipLaunchKernelGGL(k_vjp_combine<VjpStore>, cgrid, dim3(kBlock), 0, s, p4, n_pad, slices, N, G,
+		hipLaunchKernelGGL(k_vjp_combine<VjpStore>, cgrid, dim3(kBlock), 0, s, p8, n_pad, g.bslices, N, G,
 		                   VjpStore(*epi));
 	return sf_hip_check(hipGetLastError(), "sfd_force_vjp", "launch");
 }

@@ -4,13 +4,11 @@
 // cannot allocate (code under stream capture, allocation-free serving
 // loops).  No counterpart in the reference.
 //
-// scratch holds the packed bodies (n_pad float4, then the pack kernel's
-// SF_BODY_STATE words) and, from the next 256-byte boundary, the force
-// kernel's partial sums.  It is sized for every N up to SF_NOALLOC_MAX_N:
-// 256 KiB + 256 B of bodies and 16.3 MiB of partials (65 planes of one float4
-// per body at the largest n_pad).  Each device
-// holds its own copy; its address comes from hipGetSymbolAddress, once per
-// device, on the first call with that device current.
+// scratch holds the force kernels' partial sums.  It is sized for every N up to
+// SF_NOALLOC_MAX_N: 16.3 MiB (65 planes of one float4 per body at the largest
+// n_pad).  Each device holds its own copy; its address comes from
+// hipGetSymbolAddress, once per device, on the first call with that device
+// current.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -22,28 +20,24 @@ extern "C" {
 size_t sf_pp_part_bytes(unsigned int n_pad);
 int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
                        float* body, float* part, size_t part_bytes, float* acc, float* pot, hipStream_t s);
-int sfd_fill0(float* y, unsigned int n, hipStream_t s);
 }
 
 namespace {
 
 constexpr unsigned kMaxN = SF_NOALLOC_MAX_N;
-constexpr size_t kAlign = 256;
-constexpr size_t align_up(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
-constexpr size_t kBodyBytes = align_up(SF_BODY_BYTES(kMaxN));
-// the largest partial sums over the sizes: sym_part_bytes from kSymMin
-// bodies; below, k_pp_fast's block slices (at most one double4 plane per 1024 bodies)
+// the largest partial sums over the sizes
 constexpr size_t max_part_bytes() {
 	size_t most = 0;
 	for (unsigned n = 1024u; n <= kMaxN; n += 1024u) {
-		const size_t b = n >= kSymMin ? sym_part_bytes(n, sym_pp_wide(n)) : (size_t)(n / 1024u) * n * 32u;
+		const size_t b = pp_part_bytes(n);
 		if (b > most) most = b;
 	}
 	return most;
 }
+static_assert(!sym_pp_wide(kMaxN), "the kernels read the caller's arrays: no packed bodies");
 constexpr size_t kPartBytes = max_part_bytes();
 
-static __device__ __align__(256) unsigned char scratch[kBodyBytes + kPartBytes];
+static __device__ __align__(256) unsigned char scratch[kPartBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_lock;
@@ -83,22 +77,15 @@ extern "C" int sf_force_dev_noalloc(unsigned int N, const float* x, const float*
 	}
 	// the layout sf_force_dev allocates: n_pad a multiple of 1024
 	const unsigned n_pad = (N + 1023u) / 1024u * 1024u;
-	const size_t body_bytes = align_up(SF_BODY_BYTES(n_pad));
 	const size_t part_bytes = sf_pp_part_bytes(n_pad);
-	if (body_bytes + part_bytes > sizeof(scratch)) {
-		sf_error(fn, "N = %u needs %zu scratch bytes, more than the %zu available", N, body_bytes + part_bytes,
-		         sizeof(scratch));
+	if (part_bytes > sizeof(scratch)) {
+		sf_error(fn, "N = %u needs %zu scratch bytes, more than the %zu available", N, part_bytes, sizeof(scratch));
 		return STARFLOOD_FAILURE;
 	}
 	unsigned char* base = scratch_ptr(fn);
 	if (!base) return STARFLOOD_FAILURE;
-	float* body = reinterpret_cast<float*>(base);
-	float* part = reinterpret_cast<float*>(base + body_bytes);
-	hipStream_t s = static_cast<hipStream_t>(stream);
-	// The pack kernel's state words follow the n_pad bodies, so they move
-	// with N and may hold an earlier call's bodies: clear them (a kernel, not
-	// a memset node, so the call can be captured).
-	if (sfd_fill0(body + 4u * (size_t)n_pad, SF_BODY_STATE, s)) return STARFLOOD_FAILURE;
-	return sf_pp_force_arrays(sf_params(), N, n_pad, x, m, body, part, part_bytes, acc, pot, s) ? STARFLOOD_FAILURE
-	                                                                                           : STARFLOOD_SUCCESS;
+	return sf_pp_force_arrays(sf_params(), N, n_pad, x, m, nullptr, reinterpret_cast<float*>(base), part_bytes, acc, pot,
+	                          static_cast<hipStream_t>(stream))
+	           ? STARFLOOD_FAILURE
+	           : STARFLOOD_SUCCESS;
 }

@@ -14,24 +14,21 @@
 // bit-identical to the CPU path.  The terms of a tile of j are made by some of
 // a block's wavefronts while others run the chains of sums.
 //
-// k_pp_fast is the throughput kernel below 10240 bodies (from there
-// pp_sym.hip evaluates each pair once): 13 VALU operations plus one
-// v_rsq_f32 per interaction, one i per lane, j fetched with scalar loads,
-// partial sums per tile of SF_TJ interactions folded into a
-// Kahan-compensated running sum, and the j range split into slices so the
-// grid fills the CUs.
-// When every particle has the same mass m (k_pack_bodies checks the bits of
-// each mass on the device), the whole tiles of real particles drop the
-// per-pair mass product: they sum 1/s^3 (r_j - r_i) and 1/s with 12 VALU
-// operations plus the rsqrt, and the tile partial is scaled by m before the
-// fold.  A block's four wavefronts hold the same 64 particles and split its
-// slice into four sub-slices; their sums meet in LDS in FP64, in wavefront
+// k_pp_few is the throughput kernel of small states (from kSymMin bodies
+// pp_sym.hip evaluates each pair once): 13 VALU operations plus one v_rsq_f32
+// per interaction, one i per lane, tiles of 64 j staged in LDS, their plain
+// partial sums folded into a Kahan-compensated running sum, and the j range
+// split over wavefronts so that the grid fills the CUs.  Where a tile's masses
+// all have the bits of the first body's, the per-pair mass product is left out
+// and the tile's sums are scaled before the fold.  A block's four wavefronts
+// hold the same 64 particles; their sums meet in LDS in FP64, in wavefront
 // order, so a block writes one double4 per particle.
 // A second kernel adds the slice partials per i in fixed order in FP64,
 // which keeps the result deterministic.
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "bodies.h"
 #include "exact_inv.h"
 #include "force_epi.h"
 #include "order_chain.h"
@@ -40,9 +37,6 @@
 namespace {
 
 constexpr unsigned kBlock = 256;
-constexpr unsigned SF_TJ = 128;   // interactions per plain-FP32 partial sum
-constexpr int kPrefetch = 4;      // bodies per scalar-load group (one s_load_dwordx16)
-static_assert(SF_TJ % kPrefetch == 0, "tiles hold whole prefetch groups");
 
 // One step of Kahan summation (reference src/gravity.c:771-784):
 // y = x - c; t = s + y; c = (t - s) - y; s = t.
@@ -150,109 +144,72 @@ void launch_exact(int sel, const float* pos, const float* mas, unsigned N, float
 	                   pot);
 }
 
-// One tile of SF_TJ interactions, j from jt.  nb holds the tile's first
-// kPrefetch bodies on entry and the next tile's first ones on exit (the
-// group after the range's last is its own first again: in bounds; the
-// compiler then issues the four loads as separate dwordx4 into fresh
-// registers, early in the group -- measured faster than one dwordx16 into
-// the registers being consumed).  UNIFORM: every mass of the tile equals m,
-// and the sums leave it out (sum_j (r_j - r_i)/s^3 and sum_j 1/s).
+// Interactions with a tile's 64 bodies q in LDS, read by every lane.  UNIFORM:
+// every mass is the same, and the sums leave it out.
 template <bool WITH_POT, bool UNIFORM>
-__device__ __forceinline__ void pp_tile(const float4* __restrict__ body, unsigned jt, unsigned j1,
-                                        float4 (&nb)[kPrefetch], float xi, float yi, float zi, float eps2, float& tx,
-                                        float& ty, float& tz, float& tp) {
-	for (unsigned j = jt; j < jt + SF_TJ; j += kPrefetch) {
-		float4 cb[kPrefetch];
-#pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) cb[u] = nb[u];
-		const unsigned jn = (j + kPrefetch < j1) ? j + kPrefetch : j;
-#pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) nb[u] = body[jn + u];
-#pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) {
-			const float4 bj = cb[u];
-			const float dx = bj.x - xi;
-			const float dy = bj.y - yi;
-			const float dz = bj.z - zi;
-			float r2 = __builtin_fmaf(dx, dx, eps2);
-			r2 = __builtin_fmaf(dy, dy, r2);
-			r2 = __builtin_fmaf(dz, dz, r2);
-			const float inv = __builtin_amdgcn_rsqf(r2);
-			const float mi = UNIFORM ? inv : bj.w * inv;
-			const float inv2 = inv * inv;
-			const float w = mi * inv2;
-			tx = __builtin_fmaf(w, dx, tx);
-			ty = __builtin_fmaf(w, dy, ty);
-			tz = __builtin_fmaf(w, dz, tz);
-			if (WITH_POT) tp += mi;
-		}
+__device__ __forceinline__ void few_tile(const float4* __restrict__ q, float xi, float yi, float zi, float eps2,
+                                         float& tx, float& ty, float& tz, float& tp) {
+#pragma unroll 16
+	for (unsigned k = 0; k < kSymTile; ++k) {
+		const float4 bj = q[k];
+		const float dx = bj.x - xi;
+		const float dy = bj.y - yi;
+		const float dz = bj.z - zi;
+		float r2 = __builtin_fmaf(dx, dx, eps2);
+		r2 = __builtin_fmaf(dy, dy, r2);
+		r2 = __builtin_fmaf(dz, dz, r2);
+		const float inv = __builtin_amdgcn_rsqf(r2);
+		const float mi = UNIFORM ? inv : bj.w * inv;
+		const float inv2 = inv * inv;
+		const float w = mi * inv2;
+		tx = __builtin_fmaf(w, dx, tx);
+		ty = __builtin_fmaf(w, dy, ty);
+		tz = __builtin_fmaf(w, dz, tz);
+		if (WITH_POT) tp += mi;
 	}
 }
 
 // Block b owns the 64 particles i of i-block b / slices (one per lane, the
-// same in each of its kWavesPP wavefronts) and j slice b % slices, which its
-// wavefronts split into kWavesPP consecutive sub-slices of sub_len bodies.
-// Each wavefront accumulates sum_j m_j (r_j - r_i) / s^3 and sum_j m_j / s
-// over its sub-slice: plain FP32 sums over tiles of SF_TJ interactions,
-// folded into Kahan-compensated running sums.  The wavefronts' compensated
-// sums (s - c) are then added in FP64 in wavefront order through LDS, and
-// the block writes one double4 per particle: part[slice][i].  The word
-// after the n_pad bodies holds n_uni: the bodies [0, n_uni) are whole tiles
-// of particles of one mass, body[0].w (0 when the masses differ).
+// same in each of its wavefronts) and j slice b % slices, of which each
+// wavefront takes `per` consecutive tiles.
+// Bound by a wavefront's chain at small sizes (a lone wavefront issues one
+// instruction in 2.5 ns) and by issue from about 6000 bodies on.  With the j
+// stream in scalar loads, four bodies ahead of their use, each wavefront waited
+// for most of them, 24 us whatever the size; now 6.7 us at 1000 bodies, 8.3 at
+// 3000, 19.5 at 6000, 28 at 8192.  With the bodies read from the caller's arrays
+// a force up to 1000 bodies takes 22.8 us instead of 44, 3000 24.6, 6000 34.1
+// (42.8), 9216 47.6 (54.3).
 constexpr unsigned kWavesPP = kBlock / 64;
-template <bool WITH_POT>
-__global__ __launch_bounds__(kBlock) void k_pp_fast(const float4* __restrict__ body, unsigned n_pad,
-                                                    unsigned slices, unsigned sub_len, float eps2,
-                                                    double4* __restrict__ part) {
+template <bool WITH_POT, class L>
+__global__ __launch_bounds__(kBlock) void k_pp_few(const L bodies, unsigned n_pad, unsigned slices, unsigned per,
+                                                   float eps2, double4* __restrict__ part) {
+	__shared__ float4 s_j[kWavesPP][2][kSymTile];
 	__shared__ double red[kWavesPP][4][64];
-	const unsigned b = blockIdx.x;
-	const unsigned s = b % slices;
-	// the wavefront index is uniform per wavefront: readfirstlane tells the
-	// compiler, so the j stream stays in scalar loads and SGPRs
+	const unsigned s = blockIdx.x % slices;
 	const unsigned lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const unsigned i = (b / slices) * 64u + lane;
-	const float4 bi = body[i];
-	const float xi = bi.x, yi = bi.y, zi = bi.z;
-	float Sx = 0.0f, Sy = 0.0f, Sz = 0.0f, Sp = 0.0f;
-	float Cx = 0.0f, Cy = 0.0f, Cz = 0.0f, Cp = 0.0f;
-
-	// The j stream keeps one group of kPrefetch bodies in flight: the scalar
-	// loads of the next group are issued before the current group's
-	// arithmetic, so their latency overlaps it.  The equal-mass tiles come
-	// first in a loop of their own: one loop with a branch per tile made the
-	// compiler carry the j stream in VGPRs (measured 8 % slower).
-	const unsigned j0 = min((s * kWavesPP + wv) * sub_len, n_pad);
-	const unsigned j1 = min(j0 + sub_len, n_pad);
-	if (j0 < j1) {
-		const unsigned n_uni = *reinterpret_cast<const unsigned*>(body + n_pad);
-		const unsigned ju = min(j1, max(j0, n_uni));
-		const float mu = body[0].w;
-		float4 nb[kPrefetch];
+	const unsigned i = (blockIdx.x / slices) * 64u + lane;
+	const unsigned j0 = min((s * kWavesPP + wv) * per * kSymTile, n_pad), j1 = min(j0 + per * kSymTile, n_pad);
+	const float4 bi = bodies(i);
+	float4 v = j0 < j1 ? bodies(j0 + lane) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	const float mu = bodies.mass(0u);
+	float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f}, com[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+	unsigned buf = 0u;
+	for (unsigned j = j0; j < j1; j += kSymTile) {
+		s_j[wv][buf][lane] = v;
+		const bool uni = __ballot(__float_as_uint(v.w) != __float_as_uint(mu)) == 0ull;
+		if (j + kSymTile < j1) v = bodies(j + kSymTile + lane);
+		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+		float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+		if (uni) few_tile<WITH_POT, true>(s_j[wv][buf], bi.x, bi.y, bi.z, eps2, t[0], t[1], t[2], t[3]);
+		else few_tile<WITH_POT, false>(s_j[wv][buf], bi.x, bi.y, bi.z, eps2, t[0], t[1], t[2], t[3]);
+		const float sc = uni ? mu : 1.0f;
 #pragma unroll
-		for (int u = 0; u < kPrefetch; ++u) nb[u] = body[j0 + u];
-		unsigned jt = j0;
-		for (; jt < ju; jt += SF_TJ) {
-			float tx = 0.0f, ty = 0.0f, tz = 0.0f, tp = 0.0f;
-			pp_tile<WITH_POT, true>(body, jt, j1, nb, xi, yi, zi, eps2, tx, ty, tz, tp);
-			kahan_add(Sx, Cx, mu * tx);
-			kahan_add(Sy, Cy, mu * ty);
-			kahan_add(Sz, Cz, mu * tz);
-			if (WITH_POT) kahan_add(Sp, Cp, mu * tp);
-		}
-		for (; jt < j1; jt += SF_TJ) {
-			float tx = 0.0f, ty = 0.0f, tz = 0.0f, tp = 0.0f;
-			pp_tile<WITH_POT, false>(body, jt, j1, nb, xi, yi, zi, eps2, tx, ty, tz, tp);
-			kahan_add(Sx, Cx, tx);
-			kahan_add(Sy, Cy, ty);
-			kahan_add(Sz, Cz, tz);
-			if (WITH_POT) kahan_add(Sp, Cp, tp);
-		}
+		for (int u = 0; u < (WITH_POT ? 4 : 3); ++u) kahan_add(sum[u], com[u], sc * t[u]);
+		buf ^= 1u;
 	}
 	// Kahan's compensation c holds the negated lost low part: each sum is s - c
-	red[wv][0][lane] = (double)Sx - (double)Cx;
-	red[wv][1][lane] = (double)Sy - (double)Cy;
-	red[wv][2][lane] = (double)Sz - (double)Cz;
-	red[wv][3][lane] = (double)Sp - (double)Cp;
+#pragma unroll
+	for (int u = 0; u < 4; ++u) red[wv][u][lane] = (double)sum[u] - (double)com[u];
 	__syncthreads();
 	if (wv != 0) return;
 	double4 t = make_double4(red[0][0][lane], red[0][1][lane], red[0][2][lane], red[0][3][lane]);
@@ -273,10 +230,10 @@ __global__ __launch_bounds__(kBlock) void k_pp_fast(const float4* __restrict__ b
 // left most CUs idle at small N (64 blocks at N = 16384: 20 us).
 constexpr unsigned kCombI = 64;
 constexpr unsigned kCombG = kBlock / kCombI;
-template <class E>
+template <class E, class L>
 __global__ __launch_bounds__(kBlock) void k_pp_combine(const double4* __restrict__ part, unsigned n_pad,
-                                                       unsigned slices, float4* body, unsigned N, double G,
-                                                       int acc_phys, E epi) {
+                                                       unsigned slices, const L bodies, float4* body, unsigned N,
+                                                       double G, int acc_phys, E epi) {
 	__shared__ double red[kCombG][4][kCombI];
 	const unsigned il = threadIdx.x % kCombI, g = threadIdx.x / kCombI;
 	const unsigned i = blockIdx.x * kCombI + il;   // < n_pad: the grid covers N in kCombI steps
@@ -301,63 +258,39 @@ __global__ __launch_bounds__(kBlock) void k_pp_combine(const double4* __restrict
 		sp += red[q][3][il];
 	}
 	// sum_j m_j (r_j - r_i)/s^3 = -sum_j m_j r_ij/s^3, so acc = G (m_i) * sum
-	const double f = acc_phys ? G : G * (double)body[i].w;
+	const double f = acc_phys ? G : G * (double)bodies.mass(i);
 	epi(i, (float)(f * sx), (float)(f * sy), (float)(f * sz), (float)(-G * sp), body);
 }
 
-// The state words of the packed bodies (see pack_state): every mass has the
-// bits of mas[0] unless d; st[0] receives n_uni, the whole SF_TJ tiles of [0, N)
-// when they all do, else 0 (padding bodies, mass 0, are never in a uniform
-// tile).  st[1] collects the blocks' differing-mass flags and st[2] counts
-// finished blocks; the last block to finish writes st[0] and returns both to
-// zero (atomicInc wraps at gridDim.x - 1), so they start at zero on the next
-// call without a clear.  Only k_pp_fast and k_vjp read n_uni, below kSymMin
-// bodies (at most 36 blocks; the atomics on st[2] serialise: 1024 blocks
-// took 26 us).
-__device__ __forceinline__ void pack_state(int d, unsigned N, unsigned* __restrict__ st) {
-	d = __syncthreads_or(d);
-	if (threadIdx.x != 0) return;
-	if (d) atomicOr(&st[1], 1u);
-	__threadfence();
-	if (atomicInc(&st[2], gridDim.x - 1u) == gridDim.x - 1u) {
-		const unsigned any = atomicExch(&st[1], 0u);
-		st[0] = any ? 0u : N / SF_TJ * SF_TJ;
-	}
-}
-
-// Packs (x, y, z, m) per body, padding with zeros to n_pad.  STATE: below
-// kSymMin bodies.  KICK: first the opening kick and drift of the fast step,
-// with k_kick_drift_fast's operations (x64 restarts from pos where they differ).
-template <bool STATE, bool KICK>
+// Packs (x, y, z, m) per body, padding with zeros to n_pad.  KICK: first the
+// opening kick and drift of the fast step, with k_kick_drift_fast's operations
+// (x64 restarts from pos where they differ).
+template <bool KICK>
 __global__ __launch_bounds__(kBlock) void k_pack_bodies(float* __restrict__ vel, const float* __restrict__ acc,
                                                         double* __restrict__ x64, float* __restrict__ pos,
                                                         const float* __restrict__ mas, unsigned N, unsigned n_pad,
-                                                        float half_dt, double dt, float4* __restrict__ body,
-                                                        unsigned* __restrict__ st) {
+                                                        float half_dt, double dt, float4* __restrict__ body) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	int d = 0;
-	if (i < N) {
-		float p[3] = {pos[3u * i], pos[3u * i + 1u], pos[3u * i + 2u]};
-		if (KICK) {
-#pragma unroll
-			for (unsigned k = 0; k < 3u; ++k) {
-				const float v = __builtin_fmaf(half_dt, acc[3u * i + k], vel[3u * i + k]);
-				double x0 = x64[3u * i + k];
-				if ((float)x0 != p[k]) x0 = (double)p[k];
-				const double x = __builtin_fma(dt, (double)v, x0);
-				vel[3u * i + k] = v;
-				x64[3u * i + k] = x;
-				p[k] = (float)x;
-				pos[3u * i + k] = p[k];
-			}
-		}
-		const float m = mas[i];
-		body[i] = make_float4(p[0], p[1], p[2], m);
-		if (STATE) d = __float_as_uint(m) != __float_as_uint(mas[0]);
-	} else if (i < n_pad) {
+	if (i >= n_pad) return;
+	if (i >= N) {
 		body[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+		return;
 	}
-	if (STATE) pack_state(d, N, st);
+	float p[3] = {pos[3u * i], pos[3u * i + 1u], pos[3u * i + 2u]};
+	if (KICK) {
+#pragma unroll
+		for (unsigned k = 0; k < 3u; ++k) {
+			const float v = __builtin_fmaf(half_dt, acc[3u * i + k], vel[3u * i + k]);
+			double x0 = x64[3u * i + k];
+			if ((float)x0 != p[k]) x0 = (double)p[k];
+			const double x = __builtin_fma(dt, (double)v, x0);
+			vel[3u * i + k] = v;
+			x64[3u * i + k] = x;
+			p[k] = (float)x;
+			pos[3u * i + k] = p[k];
+		}
+	}
+	body[i] = make_float4(p[0], p[1], p[2], mas[i]);
 }
 
 // FP64 direct sum: one block per listed particle, lanes stride over j, then
@@ -410,10 +343,8 @@ __global__ __launch_bounds__(kBlock) void k_pp_f64(const float* __restrict__ pos
 template <bool KICK>
 static void launch_pack(float* vel, const float* acc, double* x64, float* pos, const float* mas, unsigned N,
                         unsigned n_pad, float half_dt, double dt, float* body, hipStream_t s) {
-	unsigned* st = reinterpret_cast<unsigned*>(body + 4u * (size_t)n_pad);
-	auto k = n_pad < kSymMin ? k_pack_bodies<true, KICK> : k_pack_bodies<false, KICK>;
-	hipLaunchKernelGGL(k, dim3((n_pad + kBlock - 1) / kBlock), dim3(kBlock), 0, s, vel, acc, x64, pos, mas, N, n_pad,
-	                   half_dt, dt, reinterpret_cast<float4*>(body), st);
+	hipLaunchKernelGGL(k_pack_bodies<KICK>, dim3((n_pad + kBlock - 1) / kBlock), dim3(kBlock), 0, s, vel, acc, x64, pos,
+	                   mas, N, n_pad, half_dt, dt, reinterpret_cast<float4*>(body));
 }
 
 extern "C" int sfd_pack_bodies(const float* pos, const float* mas, unsigned N, unsigned n_pad, float* body,
@@ -441,71 +372,57 @@ extern "C" int sfd_pp_exact(const float* pos, const float* mas, unsigned N, floa
 	return sf_hip_check(hipGetLastError(), "sfd_pp_exact", "k_pp_exact launch");
 }
 
-// The slice geometry of k_pp_fast for n_pad bodies and `slices` j ranges
-// (whole SF_TJ tiles, every one non-empty): sub-slice length, and block
-// slices (kWavesPP sub-slices each), one double4 plane each.
-struct PPGeometry {
-	unsigned sub_len, bslices;
-};
-static PPGeometry pp_geometry(unsigned n_pad, unsigned slices) {
-	const unsigned tiles = n_pad / SF_TJ;
-	// a multiple of the wavefronts per block: a wavefront without a j range
-	// would wait at the block's barrier and hold its slot (at N = 4M, two
-	// ranges left half of every block idle: the force took 6.7 s, not 4.5 s)
-	slices = (max(slices, 1u) + kWavesPP - 1u) / kWavesPP * kWavesPP;
-	if (slices > tiles) slices = tiles;
-	if (slices < 1u) slices = 1u;
-	PPGeometry g;
-	g.sub_len = (tiles + slices - 1) / slices * SF_TJ;
-	const unsigned subs = (n_pad + g.sub_len - 1) / g.sub_len;
-	g.bslices = (subs + kWavesPP - 1) / kWavesPP;
-	return g;
-}
-
-extern "C" size_t sfd_pp_part_bytes(unsigned n_pad, unsigned slices) {
-	if (n_pad >= kSymMin) return sym_part_bytes(n_pad, sym_pp_wide(n_pad));
-	return n_pad ? (size_t)pp_geometry(n_pad, slices).bslices * n_pad * sizeof(double4) : 0u;
-}
+extern "C" size_t sfd_pp_part_bytes(unsigned n_pad) { return pp_part_bytes(n_pad); }
 
 // device/pp_sym.hip
-extern "C" int sfd_pp_sym(float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys, float* part,
-                          const sf_force_epi* epi, hipStream_t s);
+extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsigned N, unsigned n_pad, float eps2,
+                          double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s);
 
-extern "C" int sfd_pp_fast(float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys, float* part,
-                           unsigned slices, const sf_force_epi* epi, hipStream_t s) {
+extern "C" int sfd_pp_fast(const float* pos, const float* mas, float* body, unsigned N, unsigned n_pad, float eps2,
+                           double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
-	if (n_pad % 64u != 0 || n_pad % SF_TJ != 0) {
-		sf_error("sfd_pp_fast", "n_pad %u is not a multiple of %u", n_pad, SF_TJ);
+	if (n_pad % 1024u != 0 || N > n_pad || (pos && epi->kind != SF_EPI_STORE)) {
+		sf_error("sfd_pp_fast", "n_pad %u does not fit N = %u", n_pad, N);
 		return -1;
 	}
-	// part holds sfd_pp_part_bytes(n_pad, slices)
-	if (n_pad >= kSymMin) return sfd_pp_sym(body, N, n_pad, eps2, G, acc_phys, part, epi, s);
-	// one double4 plane per block slice
-	const PPGeometry g = pp_geometry(n_pad, slices);
-	const unsigned grid = (n_pad / 64u) * g.bslices;
+	// part holds sfd_pp_part_bytes(n_pad)
+	if (n_pad >= kSymMin) {
+		if (pos && sym_pp_wide(n_pad)) {
+			if (sfd_pack_bodies(pos, mas, N, n_pad, body, s)) return -1;
+			pos = mas = nullptr;
+		}
+		return sfd_pp_sym(pos, mas, body, N, n_pad, eps2, G, acc_phys, part, epi, s);
+	}
+	const FewGeometry g = few_geometry(n_pad);
+	const dim3 grid((n_pad / 64u) * g.bslices), cgrid((N + kCombI - 1) / kCombI);
 	double4* p4 = reinterpret_cast<double4*>(part);
 	float4* b4 = reinterpret_cast<float4*>(body);
-	const bool with_pot = epi->kind == SF_EPI_KICK || (epi->kind == SF_EPI_STORE && epi->pot);
+	const PackedBodies packed{b4};
+	const ArrayBodies arrays{pos, mas, N};
+	const bool pot = epi->kind == SF_EPI_KICK || (epi->kind == SF_EPI_STORE && epi->pot);
 	const int tok = sf_prof_begin("pp_fast", s);
-	hipLaunchKernelGGL(with_pot ? k_pp_fast<true> : k_pp_fast<false>, dim3(grid), dim3(kBlock), 0, s, b4, n_pad,
-	                   g.bslices, g.sub_len, eps2, p4);
-	sf_prof_end(tok, s);
-	if (sf_hip_check(hipGetLastError(), "sfd_pp_fast", "k_pp_fast launch")) return -1;
-	const dim3 cgrid((N + kCombI - 1) / kCombI);
-	const int tok2 = sf_prof_begin("pp_combine", s);
-	switch (epi->kind) {
-	case SF_EPI_KICK:
-		hipLaunchKernelGGL(k_pp_combine<EpiKick>, cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4, N, G, acc_phys,
-		                   EpiKick(*epi));
-		break;
-	case SF_EPI_KDK:
-		hipLaunchKernelGGL(k_pp_combine<EpiKdk>, cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4, N, G, acc_phys,
-		                   EpiKdk(*epi));
-		break;
-	default:
-		hipLaunchKernelGGL(k_pp_combine<EpiStore>, cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, b4, N, G, acc_phys,
-		                   EpiStore(*epi));
+	if (pos) {
+		auto k = pot ? k_pp_few<true, ArrayBodies> : k_pp_few<false, ArrayBodies>;
+		hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, arrays, n_pad, g.bslices, g.per, eps2, p4);
+	} else {
+		auto k = pot ? k_pp_few<true, PackedBodies> : k_pp_few<false, PackedBodies>;
+		hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, packed, n_pad, g.bslices, g.per, eps2, p4);
 	}
+	sf_prof_end(tok, s);
+	if (sf_hip_check(hipGetLastError(), "sfd_pp_fast", "k_pp_few launch")) return -1;
+	const int tok2 = sf_prof_begin("pp_combine", s);
+	if (epi->kind == SF_EPI_KICK)
+		hipLaunchKernelGGL((k_pp_combine<EpiKick, PackedBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, packed,
+		                   b4, N, G, acc_phys, EpiKick(*epi));
+	else if (epi->kind == SF_EPI_KDK)
+		hipLaunchKernelGGL((k_pp_combine<EpiKdk, PackedBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, packed,
+		                   b4, N, G, acc_phys, EpiKdk(*epi));
+	else if (pos)
+		hipLaunchKernelGGL((k_pp_combine<EpiStore, ArrayBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, arrays,
+		                   b4, N, G, acc_phys, EpiStore(*epi));
+	else
+		hipLaunchKernelGGL((k_pp_combine<EpiStore, PackedBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices,
+		                   packed, b4, N, G, acc_phys, EpiStore(*epi));
 	sf_prof_end(tok2, s);
 	return sf_hip_check(hipGetLastError(), "sfd_pp_fast", "k_pp_combine launch");
 }

@@ -25,11 +25,12 @@
 
 constexpr unsigned kSymTile = 64;                      // j per tile
 constexpr unsigned kSymNarrow = 256, kSymWide = 1024;  // bodies per set
-// Below 10240 bodies the one-sided kernel (k_pp_fast) is as fast: at 8192 it
-// takes 29.8 us with its combine, the narrow layout 30.8 (its 544 blocks
-// leave half of the wavefront slots empty); at 9217 43.6 and 36.7 us, at
-// 10007 41.9 and 35.1, at 16384 80 and 67.
+// Below kSymMin bodies the one-sided kernel (k_pp_few).  A force with its combine
+// and the wait for it, general masses: 9216 bodies one-sided 47.6 us, each pair
+// once 52.6; 10240 56.4 and 56.2; 11264 61.8 and 55.7; 12288 71.6 and 62.6.
 constexpr unsigned kSymMin = 10240;
+// The same line for the force VJP (k_vjp, k_vjp_sym).
+constexpr unsigned kVjpSymMin = 10240;
 // The wide layout from here: at 16384 bodies it takes 75.5 us and the narrow
 // one 73.9, at 24576 146 and 140, at 32768 226 and 230, at 65536 832 and 845.
 constexpr unsigned kSymWideMin = 25600;
@@ -89,5 +90,24 @@ constexpr size_t sym_part_bytes(unsigned n_pad, bool wide) {
 
 // the layout of the force kernel
 constexpr bool sym_pp_wide(unsigned n_pad) { return n_pad >= kSymWideMin; }
+
+// k_pp_few: 64 i and 64 per j per wavefront, four wavefronts to a block; as many
+// j tiles per wavefront as leave about eight wavefronts per SIMD (a force of
+// 9216 bodies: four 54.1 us, eight 47.7, sixteen 48.8).
+struct FewGeometry {
+	unsigned per;       // j tiles per wavefront
+	unsigned bslices;   // blocks (planes of partial sums) per 64 i
+};
+constexpr FewGeometry few_geometry(unsigned n_pad) {
+	const unsigned long long t = n_pad / kSymTile;
+	const unsigned per = (unsigned)((t * t + 8191u) / 8192u);
+	const unsigned waves = (unsigned)((t + per - 1u) / per), slices = (waves + 3u) / 4u;
+	return {(unsigned)((t + 4u * slices - 1u) / (4u * slices)), slices};
+}
+// bytes of partial sums of the fast PP force
+constexpr size_t pp_part_bytes(unsigned n_pad) {
+	return n_pad == 0u ? 0u : (n_pad >= kSymMin ? sym_part_bytes(n_pad, sym_pp_wide(n_pad))
+	                                            : (size_t)few_geometry(n_pad).bslices * n_pad * 32u);
+}
 
 #endif

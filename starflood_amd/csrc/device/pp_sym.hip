@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "bodies.h"
 #include "force_epi.h"
 #include "pp_sym.h"
 
@@ -59,10 +60,11 @@ struct Set {
 #pragma unroll
 		for (int k = 0; k < kPer; ++k) tx[k] = ty[k] = tz[k] = tp[k] = 0.0f;
 	}
-	__device__ __forceinline__ void load(const float4* __restrict__ body, unsigned i0) {
+	template <class L>
+	__device__ __forceinline__ void load(const L& bodies, unsigned i0) {
 #pragma unroll
 		for (int k = 0; k < kPer; ++k) {
-			const float4 b = body[i0 + 64u * k];
+			const float4 b = bodies(i0 + 64u * k);
 			x[k] = b.x;
 			y[k] = b.y;
 			z[k] = b.z;
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 	if (j >= n_pad) j -= n_pad;
 	const unsigned i0 = ib * kSymWide + wv * kSet + lane;
 	Set a;
-	a.load(body, i0);
+	a.load(PackedBodies{body}, i0);
 	float sum[kPer][4], com[kPer][4];
 	bool pending = false, was_uni = false;   // plain sums not yet folded, and their kind
 #pragma unroll
@@ -251,9 +253,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 // wavefronts' i sums meet in LDS at the end.
 // One tile per wavefront needs no compensated sums: 94 VGPRs, 5 per SIMD (4
 // and 6 measured the same).
-template <bool POT>
-__global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const float4* __restrict__ body, unsigned n_pad,
-                                                             unsigned S, unsigned d0, unsigned chunks, unsigned dchunks,
+template <bool POT, class L>
+__global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const L bodies, unsigned n_pad, unsigned S,
+                                                             unsigned d0, unsigned chunks, unsigned dchunks,
                                                              float eps2, float4* __restrict__ part_i,
                                                              float4* __restrict__ part_j) {
 	__shared__ float4 s_mem[kWaves][4u * kSymTile];   // a wavefront's j and j sums, then its i sums
@@ -273,9 +275,9 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const float4* __res
 	if (jb >= S) jb -= S;
 	const unsigned j = jb * kSymNarrow + wv * kSymTile;
 	Set a;
-	a.load(body, ib * kSymNarrow + lane);
-	const float4 v = body[j + lane], zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-	const float mu = body[0].w;
+	a.load(bodies, ib * kSymNarrow + lane);
+	const float4 v = bodies(j + lane), zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	const float mu = bodies.mass(0u);
 	const bool uni = a.all_mass(mu) && __ballot(__float_as_uint(v.w) != __float_as_uint(mu)) == 0ull;
 	float4* sj = s_mem[wv];
 	float4* acc = sj + 2u * kSymTile;
@@ -318,11 +320,11 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const float4* __res
 // kept there or, at the last launch, written to acc and pot.  A block takes
 // 64 particles; its wavefronts take every fourth plane each.
 constexpr unsigned kCombI = 64;
-template <class E>
+template <class E, class L>
 __global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict__ part, unsigned n_pad,
                                                         unsigned planes, unsigned S, int last_offset, int first,
-                                                        int last, double4* __restrict__ run, float4* body,
-                                                        unsigned N, double G, int acc_phys, E epi) {
+                                                        int last, double4* __restrict__ run, const L bodies,
+                                                        float4* body, unsigned N, double G, int acc_phys, E epi) {
 	__shared__ double red[kWaves][4][kCombI];
 	const unsigned il = threadIdx.x % kCombI, g = threadIdx.x / kCombI;
 	const unsigned i = blockIdx.x * kCombI + il;   // < n_pad: the grid covers N in kCombI steps
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict
 		run[i] = make_double4(sx, sy, sz, sp);
 		return;
 	}
-	const double f = acc_phys ? G : G * (double)body[i].w;
+	const double f = acc_phys ? G : G * (double)bodies.mass(i);
 	epi(i, (float)(f * sx), (float)(f * sy), (float)(f * sz), (float)(-G * sp), body);
 }
 
@@ -374,26 +376,29 @@ struct CombineArgs {
 	double G;
 	int acc_phys;
 };
-template <class E>
-void launch_combine(const CombineArgs& c, const sf_force_epi& epi, hipStream_t s) {
-	hipLaunchKernelGGL(k_sym_combine<E>, dim3((c.N + kCombI - 1u) / kCombI), dim3(kBlock), 0, s, c.part, c.n_pad,
-	                   c.planes, c.S, c.last, c.first, c.last, c.run, c.body, c.N, c.G, c.acc_phys, E(epi));
+template <class E, class L>
+void launch_combine(const CombineArgs& c, const L& bodies, const sf_force_epi& epi, hipStream_t s) {
+	hipLaunchKernelGGL((k_sym_combine<E, L>), dim3((c.N + kCombI - 1u) / kCombI), dim3(kBlock), 0, s, c.part, c.n_pad,
+	                   c.planes, c.S, c.last, c.first, c.last, c.run, bodies, c.body, c.N, c.G, c.acc_phys, E(epi));
 }
 
 }  // namespace
 
-// The force of n_pad packed bodies (a multiple of 1024, at least 2048), ended
-// by *epi; part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad)).
-extern "C" int sfd_pp_sym(float* body, unsigned N, unsigned n_pad, float eps2, double G, int acc_phys, float* part,
-                          const sf_force_epi* epi, hipStream_t s) {
+// The force of n_pad bodies (a multiple of 1024, at least 2048), ended by *epi:
+// of the caller's arrays where pos is set (the narrow layout only), else of the
+// packed bodies; part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad)).
+extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsigned N, unsigned n_pad, float eps2,
+                          double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
-	if (n_pad % kSymWide != 0 || n_pad < 2u * kSymWide || N > n_pad) {
+	const bool wide = sym_pp_wide(n_pad);
+	if (n_pad % kSymWide != 0 || n_pad < 2u * kSymWide || N > n_pad || (pos && (wide || epi->kind != SF_EPI_STORE))) {
 		sf_error("sfd_pp_sym", "n_pad %u does not fit N = %u", n_pad, N);
 		return -1;
 	}
-	const bool wide = sym_pp_wide(n_pad);
 	const SymGeometry g = sym_geometry(n_pad, wide);
 	float4* b4 = reinterpret_cast<float4*>(body);
+	const PackedBodies packed{b4};
+	const ArrayBodies arrays{pos, mas, N};
 	const bool pot = epi->kind == SF_EPI_KICK || (epi->kind == SF_EPI_STORE && epi->pot);
 	float4* p4 = reinterpret_cast<float4*>(part);
 	double4* run = reinterpret_cast<double4*>(p4 + ((size_t)g.chunks + g.dchunks + g.per_launch) * n_pad);
@@ -410,17 +415,21 @@ extern "C" int sfd_pp_sym(float* body, unsigned N, unsigned n_pad, float eps2, d
 			auto k = pot ? k_pp_sym<true> : k_pp_sym<false>;
 			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, b4, n_pad, g.blocks, d0, d1, g.tiles, ch, dch, eps2, p4,
 			                   reinterpret_cast<float*>(pj));
+		} else if (pos) {
+			auto k = pot ? k_pp_sym_narrow<true, ArrayBodies> : k_pp_sym_narrow<false, ArrayBodies>;
+			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, arrays, n_pad, g.blocks, d0, ch, dch, eps2, p4, pj);
 		} else {
-			auto k = pot ? k_pp_sym_narrow<true> : k_pp_sym_narrow<false>;
-			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, b4, n_pad, g.blocks, d0, ch, dch, eps2, p4, pj);
+			auto k = pot ? k_pp_sym_narrow<true, PackedBodies> : k_pp_sym_narrow<false, PackedBodies>;
+			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, packed, n_pad, g.blocks, d0, ch, dch, eps2, p4, pj);
 		}
 		sf_prof_end(tok, s);
 		if (sf_hip_check(hipGetLastError(), "sfd_pp_sym", "k_pp_sym launch")) return -1;
 		const int tok2 = sf_prof_begin("pp_combine", s);
 		const CombineArgs ca{p4, n_pad, pi + (d1 - d0), g.blocks, first, last, run, b4, N, G, acc_phys};
-		if (epi->kind == SF_EPI_KICK) launch_combine<EpiKick>(ca, *epi, s);
-		else if (epi->kind == SF_EPI_KDK) launch_combine<EpiKdk>(ca, *epi, s);
-		else launch_combine<EpiStore>(ca, *epi, s);
+		if (epi->kind == SF_EPI_KICK) launch_combine<EpiKick>(ca, packed, *epi, s);
+		else if (epi->kind == SF_EPI_KDK) launch_combine<EpiKdk>(ca, packed, *epi, s);
+		else if (pos) launch_combine<EpiStore>(ca, arrays, *epi, s);
+		else launch_combine<EpiStore>(ca, packed, *epi, s);
 		sf_prof_end(tok2, s);
 		if (sf_hip_check(hipGetLastError(), "sfd_pp_sym", "k_sym_combine launch")) return -1;
 	}

@@ -26,8 +26,8 @@
 int sfd_pack_nu(const float* mu, const float* mas, unsigned int N, unsigned int n_pad, float coef, int acc_phys,
                 float* nu, hipStream_t s);
 int sfd_force_vjp(const float* body, const float* nu, unsigned int N, unsigned int n_pad, float eps2, double G,
-                  float* part, unsigned int slices, const sf_vjp_epi* epi, hipStream_t s);
-size_t sfd_vjp_part_bytes(unsigned int n_pad, unsigned int slices);
+                  float* part, const sf_vjp_epi* epi, hipStream_t s);
+size_t sfd_vjp_part_bytes(unsigned int n_pad);
 int sfd_adjoint_init(const float* x0, const float* v0, unsigned int N, double* x64, float* v, float* x, hipStream_t s);
 int sfd_adjoint_reopen(const double* ck_x64, const float* ck_v, const float* ck_a, unsigned int N, float h, double dt,
                        int steps, double* x64, float* v, float* x, float* body, hipStream_t s);
@@ -35,9 +35,9 @@ int sfd_adjoint_begin(const float* gx, const float* gv, const float* x, unsigned
                       int acc_phys, float* lx, float* lv, float* body, float* nu, hipStream_t s);
 int sfd_fill0(float* y, unsigned int n, hipStream_t s);
 
-/* device scratch for one N: packed bodies, VJP weights, slice partials */
+/* device scratch for one N: packed bodies, VJP weights, partial sums */
 typedef struct {
-	unsigned int N, n_pad, slices;
+	unsigned int N, n_pad;
 	float* body;   /* n_pad float4 */
 	float* nu;     /* n_pad float4 */
 	float* part;   /* the partial sums of the force and of its VJP */
@@ -54,20 +54,13 @@ static void scratch_free(sf_pp_scratch* w) {
 static int scratch_alloc(sf_pp_scratch* w, unsigned int N, const char* func) {
 	w->N = N;
 	w->n_pad = ((N ? N : 1u) + 1023u) / 1024u * 1024u;
-	w->slices = sf_pp_slice_count(w->n_pad);
 	const size_t plane = (size_t)w->n_pad * 4u * sizeof(float), pp_bytes = sf_pp_part_bytes(w->n_pad);
-	w->part_bytes = sfd_vjp_part_bytes(w->n_pad, w->slices);
+	w->part_bytes = sfd_vjp_part_bytes(w->n_pad);
 	if (w->part_bytes < pp_bytes) w->part_bytes = pp_bytes;
-	if (hipMalloc((void**)&w->body, SF_BODY_BYTES(w->n_pad)) != hipSuccess ||
+	if (hipMalloc((void**)&w->body, plane) != hipSuccess ||
 	    hipMalloc((void**)&w->nu, plane) != hipSuccess ||
 	    hipMalloc((void**)&w->part, w->part_bytes) != hipSuccess) {
 		sf_error(func, "device allocation for N = %u failed", N);
-		scratch_free(w);
-		return -1;
-	}
-	/* the packed-body state words start at zero (set-up only, then synchronised) */
-	if (hipMemset(w->body, 0, SF_BODY_BYTES(w->n_pad)) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
-		sf_error(func, "clearing the body buffer for N = %u failed", N);
 		scratch_free(w);
 		return -1;
 	}
@@ -78,7 +71,7 @@ static float eps2_of(const sf_params_t* p) { return (float)(p->epsilon * p->epsi
 
 /* the VJP at the packed bodies and nu of w */
 static int vjp(const sf_params_t* p, sf_pp_scratch* w, const sf_vjp_epi* epi, hipStream_t s) {
-	return sfd_force_vjp(w->body, w->nu, w->N, w->n_pad, eps2_of(p), p->G, w->part, w->slices, epi, s);
+	return sfd_force_vjp(w->body, w->nu, w->N, w->n_pad, eps2_of(p), p->G, w->part, epi, s);
 }
 
 struct sf_tape {

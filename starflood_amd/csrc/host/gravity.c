@@ -8,8 +8,8 @@
 
 #include "sf_host.h"
 
-/* j slices of the one-sided kernels (PP below 10240 bodies, the SPH all-pairs
-   passes): enough blocks to give every CU several waves */
+/* j slices of the one-sided kernels (the force VJP below 10240 bodies, the SPH
+   all-pairs passes): enough blocks to give every CU several waves */
 static unsigned int pp_slices(unsigned int n_pad) {
 	/* one j range per wavefront of 64 i; about 128k wavefronts, while each
 	   range keeps at least 256 j */
@@ -27,23 +27,27 @@ static float eps2_f32(double eps) { return (float)(eps * eps); }
 
 unsigned int sf_pp_slice_count(unsigned int n_pad) { return pp_slices(n_pad); }
 
-size_t sf_pp_part_bytes(unsigned int n_pad) { return sfd_pp_part_bytes(n_pad, pp_slices(n_pad)); }
+size_t sf_pp_part_bytes(unsigned int n_pad) { return sfd_pp_part_bytes(n_pad); }
+
+static int force(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
+                 float* body, float* part, size_t part_bytes, const sf_force_epi* epi, hipStream_t s) {
+	if (part_bytes < sf_pp_part_bytes(n_pad)) {
+		sf_error("sfd_pp_fast", "%zu bytes of partial sums, %zu needed", part_bytes, sf_pp_part_bytes(n_pad));
+		return -1;
+	}
+	return sfd_pp_fast(pos, mas, body, N, n_pad, eps2_f32(p->epsilon), p->G, p->acc_mode == SF_ACC_PHYSICAL, part, epi,
+	                   s);
+}
 
 int sf_pp_force_packed(const sf_params_t* p, unsigned int N, unsigned int n_pad, float* body, float* part,
                        size_t part_bytes, const sf_force_epi* epi, hipStream_t s) {
-	if (part_bytes < sf_pp_part_bytes(n_pad)) {
-		sf_error("sf_pp_force_packed", "%zu bytes of slice partials, %zu needed", part_bytes, sf_pp_part_bytes(n_pad));
-		return -1;
-	}
-	return sfd_pp_fast(body, N, n_pad, eps2_f32(p->epsilon), p->G, p->acc_mode == SF_ACC_PHYSICAL, part,
-	                   pp_slices(n_pad), epi, s);
+	return force(p, N, n_pad, NULL, NULL, body, part, part_bytes, epi, s);
 }
 
 int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad, const float* pos, const float* mas,
                        float* body, float* part, size_t part_bytes, float* acc, float* pot, hipStream_t s) {
 	const sf_force_epi epi = {.kind = SF_EPI_STORE, .acc = acc, .pot = pot};
-	if (sfd_pack_bodies(pos, mas, N, n_pad, body, s)) return -1;
-	return sf_pp_force_packed(p, N, n_pad, body, part, part_bytes, &epi, s);
+	return force(p, N, n_pad, pos, mas, body, part, part_bytes, &epi, s);
 }
 
 int sf_solve_gravity_pp(sf_ctx* c) {
@@ -55,10 +59,8 @@ int sf_solve_gravity_pp(sf_ctx* c) {
 		return sfd_pp_exact(pos, mas, N, eps2_f32(p->epsilon), (float)(-p->G), p->acc_mode == SF_ACC_PHYSICAL,
 		                    p->kahan_solver, p->kahan_energy, acc, pot, c->stream);
 	}
-	const sf_force_epi epi = {.kind = SF_EPI_STORE, .acc = acc, .pot = pot};
 	if (sf_ctx_reserve_part(c, sf_pp_part_bytes(c->n_pad))) return -1;
-	if (sfd_pack_bodies(pos, mas, N, c->n_pad, c->d_body, c->stream)) return -1;
-	return sf_pp_force_packed(p, N, c->n_pad, c->d_body, c->d_part, c->part_bytes, &epi, c->stream);
+	return sf_pp_force_arrays(p, N, c->n_pad, pos, mas, c->d_body, c->d_part, c->part_bytes, acc, pot, c->stream);
 }
 
 int sf_step_gravity_pp(sf_ctx* c) {

@@ -40,7 +40,7 @@ typedef struct sf_ctx {
 	unsigned int dof;        /* reals per particle in sim.mem */
 	unsigned int n_pad;      /* N rounded up to the PP j tile */
 	float* d_mem;            /* device copy of sim.mem, same layout */
-	float* d_body;           /* SF_BODY_BYTES(n_pad): x, y, z, m (pad: m = 0), then SF_BODY_STATE words */
+	float* d_body;           /* n_pad x 4: x, y, z, m (pad: m = 0) */
 	double* d_x64;           /* 3N FP64 positions for the FAST drift */
 	float* d_part;           /* partial sums of the PP and the SPH all-pairs passes */
 	size_t part_bytes;
@@ -90,14 +90,6 @@ int sf_prof_begin(const char* name, hipStream_t s);
 void sf_prof_end(int token, hipStream_t s);
 
 /* ---------- device launchers (csrc/device) ---------- */
-#define SF_PP_TILE 256u      /* j padding granule of d_body */
-/* packed bodies: n_pad float4, then SF_BODY_STATE words that sfd_pack_bodies
-   reads and writes below 10240 bodies (the leading bodies that form whole
-   tiles of equal mass, and two block-count words that must be zero when the
-   buffer is made; the kernels from 10240 bodies look at each tile's masses
-   themselves) */
-#define SF_BODY_STATE 64u
-#define SF_BODY_BYTES(n_pad) ((size_t)(n_pad) * 16u + SF_BODY_STATE * 4u)
 #define SF_RED_VALUES 16u    /* doubles per reduction partial */
 
 /* body[i] = (pos_i, m_i) for i < N, zero for N <= i < n_pad */
@@ -145,14 +137,14 @@ typedef struct {
 	float *gx0, *gv0;
 } sf_vjp_epi;
 
-/* Fast PP gravity: partial sums into part (sfd_pp_part_bytes of n_pad and
-   slices), then a fixed-order FP64 combine into acc (AoS) and pot.  From
-   10240 bodies each pair is evaluated once (device/pp_sym.hip); below, every
-   i against `slices` ranges of j.  The combine ends with *epi (only
-   SF_EPI_KDK writes body). */
-int sfd_pp_fast(float* body, unsigned int N, unsigned int n_pad, float eps2, double G, int acc_phys, float* part,
-                unsigned int slices, const sf_force_epi* epi, hipStream_t s);
-size_t sfd_pp_part_bytes(unsigned int n_pad, unsigned int slices);
+/* Fast PP gravity of the n_pad packed bodies (a multiple of 1024), or of pos
+   and mas where pos is set (SF_EPI_STORE only; body is then scratch): partial
+   sums into part (sfd_pp_part_bytes), then a fixed-order FP64 combine that ends
+   with *epi (only SF_EPI_KDK writes body).  From kSymMin bodies each pair is
+   evaluated once (device/pp_sym.hip); below, every i against every j. */
+int sfd_pp_fast(const float* pos, const float* mas, float* body, unsigned int N, unsigned int n_pad, float eps2,
+                double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s);
+size_t sfd_pp_part_bytes(unsigned int n_pad);
 
 /* FP64 direct sum for the listed particles (device idx list). */
 int sfd_pp_f64(const float* pos, const float* mas, unsigned int N, double eps2, double G, int acc_phys,
