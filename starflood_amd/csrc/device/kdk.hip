@@ -24,6 +24,20 @@ __global__ __launch_bounds__(kBlock) void k_kick_exact(float* __restrict__ vel, 
 	if (k < n3) vel[k] = vel[k] + half_dt * acc[k];
 }
 
+// Both, component by component: the same two roundings in one launch.  Here and
+// in k_reduce_state the step's updates ride on other passes, 93 -> 84 us a step
+// at 1000 bodies; the separate kernels serve the step times log, whose columns
+// need them apart.
+__global__ __launch_bounds__(kBlock) void k_kick_drift_exact(float* __restrict__ vel, const float* __restrict__ acc,
+                                                             float* __restrict__ pos, unsigned n3, float half_dt,
+                                                             float dt) {
+	const unsigned k = blockIdx.x * kBlock + threadIdx.x;
+	if (k >= n3) return;
+	const float v = vel[k] + half_dt * acc[k];
+	vel[k] = v;
+	pos[k] = pos[k] + dt * v;
+}
+
 // pos[k] += dt vel[k]  (src/simulation.c:394)
 __global__ __launch_bounds__(kBlock) void k_drift_exact(float* __restrict__ pos, const float* __restrict__ vel,
                                                         unsigned n3, float dt) {
@@ -74,9 +88,12 @@ constexpr int kRedQ = 11;   // T, V, W, U, Px, Py, Pz, Lx, Ly, Lz, K
 
 // Per-block partial sums with a fixed grid-stride assignment and a fixed
 // LDS tree, so the result does not depend on scheduling.  KICK: first the
-// fast policy's closing kick and k_energy_terms, particle by particle, in the
-// same pass (a launch of its own cost 5 us, 41 at 4M particles).
-template <bool KICK>
+// closing kick (with the fast policy's rounding, or k_kick_exact's) and
+// k_energy_terms, particle by particle, in the same pass (a launch of its own
+// cost 5 us, 41 at 4M particles).
+enum Kick { kNoKick, kFastKick, kExactKick };
+
+template <Kick KICK>
 __global__ __launch_bounds__(kBlock) void k_reduce_state(const float* __restrict__ pos, const double* __restrict__ x64,
                                                          float* __restrict__ vel, const float* __restrict__ mas,
                                                          const float* __restrict__ pot, float* __restrict__ ken,
@@ -98,10 +115,11 @@ __global__ __launch_bounds__(kBlock) void k_reduce_state(const float* __restrict
 			x = pos[3u * i]; y = pos[3u * i + 1u]; z = pos[3u * i + 2u];
 		}
 		float wx = vel[3u * i], wy = vel[3u * i + 1u], wz = vel[3u * i + 2u], ke, pe;
-		if (KICK) {
-			wx = __builtin_fmaf(half_dt, acc[3u * i], wx);
-			wy = __builtin_fmaf(half_dt, acc[3u * i + 1u], wy);
-			wz = __builtin_fmaf(half_dt, acc[3u * i + 2u], wz);
+		if (KICK != kNoKick) {
+			const float ax = acc[3u * i], ay = acc[3u * i + 1u], az = acc[3u * i + 2u];
+			wx = KICK == kExactKick ? wx + half_dt * ax : __builtin_fmaf(half_dt, ax, wx);
+			wy = KICK == kExactKick ? wy + half_dt * ay : __builtin_fmaf(half_dt, ay, wy);
+			wz = KICK == kExactKick ? wz + half_dt * az : __builtin_fmaf(half_dt, az, wz);
 			vel[3u * i] = wx;
 			vel[3u * i + 1u] = wy;
 			vel[3u * i + 2u] = wz;
@@ -183,6 +201,15 @@ extern "C" int sfd_drift_exact(float* pos, const float* vel, unsigned n3, float 
 	return sf_hip_check(hipGetLastError(), "sfd_drift_exact", "launch");
 }
 
+extern "C" int sfd_kick_drift_exact(float* vel, const float* acc, float* pos, unsigned n3, float half_dt, float dt,
+                                    hipStream_t s) {
+	if (!n3) return 0;
+	const int tok = sf_prof_begin("kick_drift", s);
+	hipLaunchKernelGGL(k_kick_drift_exact, dim3(grid_for(n3)), dim3(kBlock), 0, s, vel, acc, pos, n3, half_dt, dt);
+	sf_prof_end(tok, s);
+	return sf_hip_check(hipGetLastError(), "sfd_kick_drift_exact", "launch");
+}
+
 extern "C" int sfd_energy_terms(const float* vel, const float* mas, const float* pot, unsigned N, float* ken,
                                 float* pen, hipStream_t s) {
 	if (!N) return 0;
@@ -213,15 +240,18 @@ extern "C" unsigned sfd_reduce_scratch_doubles(unsigned N) {
 	return (kRedBlocks + 1u) * SF_RED_VALUES;
 }
 
-static int reduce(bool kick, const float* pos, const double* x64, float* vel, const float* mas, const float* pot,
+static int reduce(Kick kick, const float* pos, const double* x64, float* vel, const float* mas, const float* pot,
                   float* ken, float* pen, const float* u, unsigned N, double G, double eps, const float* acc,
                   float half_dt, double* red, hipStream_t s) {
 	unsigned nb = grid_for(N);
 	if (nb > kRedBlocks) nb = kRedBlocks;
 	if (nb == 0) nb = 1;
-	const int tok = sf_prof_begin(kick ? "kick_reduce_state" : "reduce_state", s);
-	hipLaunchKernelGGL((kick ? k_reduce_state<true> : k_reduce_state<false>), dim3(nb), dim3(kBlock), 0, s, pos, x64, vel,
-	                   mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red);
+	const auto kernel = kick == kNoKick     ? k_reduce_state<kNoKick>
+	                    : kick == kFastKick ? k_reduce_state<kFastKick>
+	                                        : k_reduce_state<kExactKick>;
+	const int tok = sf_prof_begin(kick == kNoKick ? "reduce_state" : "kick_reduce_state", s);
+	hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, s, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc,
+	                   half_dt, red);
 	hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, s, red, nb, red + (size_t)kRedBlocks * SF_RED_VALUES);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_reduce_state", "launch");
@@ -231,12 +261,12 @@ extern "C" int sfd_reduce_state(const float* pos, const double* x64, const float
                                 const float* pot, const float* ken, const float* pen, const float* u, unsigned N,
                                 double G, double eps, double* red, hipStream_t s) {
 	// not written without the kick
-	return reduce(false, pos, x64, const_cast<float*>(vel), mas, pot, const_cast<float*>(ken), const_cast<float*>(pen), u,
+	return reduce(kNoKick, pos, x64, const_cast<float*>(vel), mas, pot, const_cast<float*>(ken), const_cast<float*>(pen), u,
 	              N, G, eps, nullptr, 0.0f, red, s);
 }
 
 extern "C" int sfd_kick_reduce_state(const float* pos, const double* x64, float* vel, const float* acc,
                                      const float* mas, const float* pot, float half_dt, float* ken, float* pen,
                                      const float* u, unsigned N, double G, double eps, double* red, hipStream_t s) {
-	return reduce(true, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red, s);
+	return reduce(x64 ? kFastKick : kExactKick, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red, s);
 }

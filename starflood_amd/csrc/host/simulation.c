@@ -240,9 +240,11 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 
 	if (cubic && (sf_ctx_ensure_u(c) || sfd_sph_u_kick(c->d_u, c->d_dudt, N, half_dt, s))) return STARFLOOD_FAILURE;
 	if (timing) tev_record(0, s);
-	if (exact) {
+	if (exact && !timing) {
+		if (sfd_kick_drift_exact(vel, acc, pos, n3, half_dt, dt, s)) return STARFLOOD_FAILURE;
+	} else if (exact) {
 		if (sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_0 */
-		if (timing) tev_record(1, s);
+		tev_record(1, s);
 		if (sfd_drift_exact(pos, vel, n3, dt, s)) return STARFLOOD_FAILURE;       /* drift */
 	} else if (!fused) {
 		/* x64 restarts from pos where a host-side change left them apart */
@@ -258,27 +260,30 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 	}
 	if (timing) tev_record(3, s);
 
-	if (exact && sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_1 */
 	if (cubic && sfd_sph_u_kick(c->d_u, c->d_dudt, N, half_dt, s)) return STARFLOOD_FAILURE;
 
 	double* red_out = c->d_red + (size_t)(sfd_reduce_scratch_doubles(N) - SF_RED_VALUES);
 	const float* u = c->have_u ? c->d_u : NULL;
-	if (exact) {
-		if (timing) tev_record(4, s);
+	const int apart = exact && timing;
+	if (apart) {
+		if (sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_1 */
+		tev_record(4, s);
 		if (sfd_energy_terms(vel, mas, pot, N, ken, pen, s)) return STARFLOOD_FAILURE;
 		/* ken_sum and pen_sum in one pass (its time is logged as ken_sum's) */
 		if (sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
-		if (timing) {
-			tev_record(5, s);
-			tev_record(6, s);
-		}
+		tev_record(5, s);
+		tev_record(6, s);
 	}
-	/* FP64 W, P, L (and T, V in the fast policy, whose kick_1 and energy terms
-	   are in the same pass: its time is logged as kick_1's) */
-	if (exact || fused ? sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, u, N, p->G, p->epsilon,
+	/* FP64 W, P, L (and T, V in the fast policy), with kick_1 and the energy
+	   terms in the same pass: the fast policy's time is logged as kick_1's, the
+	   exact policy's log has them apart */
+	if (apart || fused ? sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, u, N, p->G, p->epsilon,
 	                                      c->d_red, s)
 	                   : sfd_kick_reduce_state(pos, c->d_x64, vel, acc, mas, pot, half_dt, ken, pen, u, N, p->G,
 	                                           p->epsilon, c->d_red, s))
+		return STARFLOOD_FAILURE;
+	if (exact && !apart &&
+	    sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s))
 		return STARFLOOD_FAILURE;
 	if (!exact && timing) {
 		tev_record(4, s);

@@ -153,6 +153,8 @@ int sfd_pp_f64(const float* pos, const float* mas, unsigned int N, double eps2, 
 /* Reference KDK pieces (src/simulation.c:381-451), FP32, no contraction. */
 int sfd_kick_exact(float* vel, const float* acc, unsigned int n3, float half_dt, hipStream_t s);
 int sfd_drift_exact(float* pos, const float* vel, unsigned int n3, float dt, hipStream_t s);
+int sfd_kick_drift_exact(float* vel, const float* acc, float* pos, unsigned int n3, float half_dt, float dt,
+                         hipStream_t s);
 /* ken_i = (0.5 m_i) |v_i|^2, pen_i = m_i pot_i */
 int sfd_energy_terms(const float* vel, const float* mas, const float* pot, unsigned int N,
                      float* ken, float* pen, hipStream_t s);
@@ -177,7 +179,8 @@ unsigned int sfd_reduce_scratch_doubles(unsigned int N);
 int sfd_reduce_state(const float* pos, const double* x64, const float* vel, const float* mas,
                      const float* pot, const float* ken, const float* pen, const float* u,
                      unsigned int N, double G, double eps, double* red, hipStream_t s);
-/* v += half_dt a and sfd_energy_terms first, in the same pass */
+/* v += half_dt a (the exact policy's roundings without x64) and
+   sfd_energy_terms first, in the same pass */
 int sfd_kick_reduce_state(const float* pos, const double* x64, float* vel, const float* acc, const float* mas,
                           const float* pot, float half_dt, float* ken, float* pen, const float* u, unsigned int N,
                           double G, double eps, double* red, hipStream_t s);
