@@ -72,6 +72,7 @@ sf_ctx* sf_ctx_create(void* host_mem, unsigned int N, unsigned int dof) {
 	                                     sfd_energy_scratch_bytes(N)) != hipSuccess)
 		goto fail;
 	if (hipHostMalloc((void**)&c->h_red, SF_RED_VALUES * sizeof(double), hipHostMallocDefault) != hipSuccess) goto fail;
+	if (hipHostGetDevicePointer((void**)&c->h_red_dev, c->h_red, 0) != hipSuccess) goto fail;
 	if (hipMemsetAsync(c->d_mem, 0, (nm ? nm : 1u) * sizeof(float), c->stream) != hipSuccess) goto fail;
 	if (hipMemsetAsync(c->d_body, 0, (size_t)c->n_pad * 4u * sizeof(float), c->stream) != hipSuccess) goto fail;
 	if (hipMemsetAsync(c->d_x64, 0, ((size_t)N * 3u + 1u) * sizeof(double), c->stream) != hipSuccess) goto fail;
@@ -115,22 +116,48 @@ int sf_ctx_reserve_part(sf_ctx* c, size_t bytes) {
 	return 0;
 }
 
-int sf_upload_blocks(sf_ctx* c, unsigned int e0, unsigned int count) {
-	if (sf_params()->mem_mode != SF_MEM_MIRROR || c->N == 0 || count == 0) return 0;
-	const size_t off = (size_t)c->N * e0, n = (size_t)c->N * count;
-	SF_HIP(hipMemcpyAsync(c->d_mem + off, (float*)c->host_mem + off, n * sizeof(float), hipMemcpyHostToDevice,
-	                      c->stream),
-	       "sf_upload_blocks");
-	return 0;
+/* Transfers of up to this many bytes go by kernel: it starts and ends in stream
+   order, while the copy engine's signals cost about 10 us a copy.  With larger
+   ones the engine's rate wins: 0.26 to 0.85 MB are faster by kernel (a step of
+   16384 bodies 371 us instead of 402), 1.6 MB slower (a frame of 65536 bodies
+   816 us instead of 805). */
+#define SF_KERNEL_COPY_MAX 1310720u
+
+static int move_blocks(sf_ctx* c, const sf_blocks* span, unsigned int spans, int to_device, const double* red) {
+	const char* func = to_device ? "sf_upload_blocks" : "sf_download_blocks";
+	sf_copy_range range[SF_COPY_RANGES];
+	unsigned int ranges = 0;
+	if (sf_params()->mem_mode != SF_MEM_MIRROR || c->N == 0) spans = 0;
+	for (unsigned int k = 0; k < spans; ++k) {
+		const size_t off = (size_t)c->N * span[k].e0, n = (size_t)c->N * span[k].count;
+		if (c->host_dev && n * sizeof(float) <= SF_KERNEL_COPY_MAX) {
+			range[ranges].dst = (to_device ? c->d_mem : c->host_dev) + off;
+			range[ranges].src = (to_device ? c->host_dev : c->d_mem) + off;
+			range[ranges++].words = n;
+		} else if (to_device) {
+			SF_HIP(hipMemcpyAsync(c->d_mem + off, (float*)c->host_mem + off, n * sizeof(float), hipMemcpyHostToDevice,
+			                      c->stream),
+			       func);
+		} else {
+			SF_HIP(hipMemcpyAsync((float*)c->host_mem + off, c->d_mem + off, n * sizeof(float), hipMemcpyDeviceToHost,
+			                      c->stream),
+			       func);
+		}
+	}
+	if (red) {
+		range[ranges].dst = c->h_red_dev;
+		range[ranges].src = red;
+		range[ranges++].words = SF_RED_VALUES * sizeof(double) / 4u;
+	}
+	return sfd_copy_ranges(range, ranges, c->stream);
 }
 
-int sf_download_blocks(sf_ctx* c, unsigned int e0, unsigned int count) {
-	if (sf_params()->mem_mode != SF_MEM_MIRROR || c->N == 0 || count == 0) return 0;
-	const size_t off = (size_t)c->N * e0, n = (size_t)c->N * count;
-	SF_HIP(hipMemcpyAsync((float*)c->host_mem + off, c->d_mem + off, n * sizeof(float), hipMemcpyDeviceToHost,
-	                      c->stream),
-	       "sf_download_blocks");
-	return 0;
+int sf_upload_blocks(sf_ctx* c, const sf_blocks* span, unsigned int spans) {
+	return move_blocks(c, span, spans, 1, NULL);
+}
+
+int sf_download_blocks(sf_ctx* c, const sf_blocks* span, unsigned int spans, const double* red) {
+	return move_blocks(c, span, spans, 0, red);
 }
 
 int sf_finish(sf_ctx* c, const char* func) {

@@ -83,9 +83,9 @@ int solve_gravity_part_part(const sim_t* SF_RESTRICT sim_ptr) {
 	if (!sim_ptr) return STARFLOOD_FAILURE;
 	sf_ctx* c = sf_ctx_lookup(sim_ptr->mem, "solve_gravity_part_part");
 	if (!c) return STARFLOOD_FAILURE;
-	if (sf_upload_blocks(c, SF_E_POS, 3u) || sf_upload_blocks(c, SF_E_MAS, 1u)) return STARFLOOD_FAILURE;
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 3u}, {SF_E_MAS, 1u}))) return STARFLOOD_FAILURE;
 	int rc = sf_solve_gravity_pp(c);
-	if (sf_download_blocks(c, SF_E_ACC, 3u) || sf_download_blocks(c, SF_E_POT, 1u)) rc = -1;
+	if (sf_download_blocks(c, SF_SPANS({SF_E_ACC, 3u}, {SF_E_POT, 1u}), NULL)) rc = -1;
 	if (sf_finish(c, "solve_gravity_part_part")) rc = -1;
 	return rc ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;
 }
@@ -103,7 +103,7 @@ int sf_pp_direct_f64(const sim_t* sim_ptr, const unsigned int* idx, unsigned int
 		}
 	}
 	const sf_params_t* p = sf_params();
-	if (sf_upload_blocks(c, SF_E_POS, 3u) || sf_upload_blocks(c, SF_E_MAS, 1u)) return STARFLOOD_FAILURE;
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 3u}, {SF_E_MAS, 1u}))) return STARFLOOD_FAILURE;
 	unsigned int* d_idx = NULL;
 	double* d_out = NULL;
 	int rc = 0;

@@ -13,11 +13,6 @@
 #include "sf_host.h"
 
 #define SF_ALIGNMENT 4194304u   /* STARFLOOD_ALIGNMENT, config.h:230 */
-/* smaller sim.mem stays ordinary memory: copies from page-locked memory go
-   through the DMA engine, whose per-copy latency costs more than its rate
-   gains on a few-MB state (N = 65536: reference-tree solve 3.2 -> 4.0 ms),
-   while a 13.6 MB state (N = 262144) steps 2.7 % faster in mirror mode */
-#define SF_PIN_MIN_BYTES 8388608u
 
 /* statistics.csv and timings_sim_step.csv (src/simulation.c:24-30,58-76) */
 static FILE* g_log_statistics = NULL;
@@ -79,13 +74,13 @@ int sim_init(sim_t* SF_RESTRICT sim_ptr, unsigned int N) {
 	sim_t sim = *sim_ptr;
 	const unsigned int dof = sf_sim_dof();
 	const size_t mem_size = sizeof(real) * (size_t)N * (size_t)dof;
-	/* page-locked (the mirror-mode copies then run at full PCIe rate), still
-	   SF_ALIGNMENT aligned inside the allocation; ordinary aligned memory,
-	   as the reference's, for small systems or when pinning fails */
+	/* page-locked (the mirror-mode copies then run at full PCIe rate, small ones
+	   by a kernel), still SF_ALIGNMENT aligned inside the allocation (0.3 to
+	   0.8 ms of the call's 3 to 4 where its pages are new); ordinary aligned
+	   memory, as the reference's, when pinning fails */
 	void* mem = NULL;
 	void* pinned = NULL;
-	if (mem_size >= SF_PIN_MIN_BYTES &&
-	    hipHostMalloc(&pinned, mem_size + SF_ALIGNMENT, hipHostMallocDefault) == hipSuccess && pinned) {
+	if (hipHostMalloc(&pinned, mem_size + SF_ALIGNMENT, hipHostMallocDefault) == hipSuccess && pinned) {
 		mem = (void*)(((uintptr_t)pinned + (SF_ALIGNMENT - 1u)) & ~(uintptr_t)(SF_ALIGNMENT - 1u));
 	} else {
 		(void)hipGetLastError();
@@ -107,6 +102,10 @@ int sim_init(sim_t* SF_RESTRICT sim_ptr, unsigned int N) {
 		return STARFLOOD_FAILURE;
 	}
 	c->host_pinned_base = pinned;
+	if (pinned && hipHostGetDevicePointer((void**)&c->host_dev, mem, 0) != hipSuccess) {
+		(void)hipGetLastError();
+		c->host_dev = NULL;
+	}
 
 	if (p->verbose) {
 		printf("Simulation Memory Addresses:\n  mem: %p (%zu bytes)\n\n", mem, mem_size);
@@ -150,17 +149,13 @@ int sim_free(sim_t* SF_RESTRICT sim_ptr) {
 
 /* blocks a solve reads / writes in mirror mode */
 static int upload_solver_inputs(sf_ctx* c) {
-	if (sf_upload_blocks(c, SF_E_POS, 3u)) return -1;
-	if (sf_upload_blocks(c, SF_E_MAS, 1u)) return -1;
-	if (sf_params()->enable_sph && sf_upload_blocks(c, SF_E_RAD, 1u)) return -1;
-	return 0;
+	const sf_blocks span[] = {{SF_E_POS, 3u}, {SF_E_MAS, 1u}, {SF_E_RAD, 1u}};
+	return sf_upload_blocks(c, span, sf_params()->enable_sph ? 3u : 2u);
 }
 
 static int download_solver_outputs(sf_ctx* c) {
-	if (sf_download_blocks(c, SF_E_ACC, 3u)) return -1;
-	if (sf_download_blocks(c, SF_E_POT, 1u)) return -1;
-	if (sf_params()->enable_sph && sf_download_blocks(c, SF_E_RHO, 2u)) return -1;
-	return 0;
+	const sf_blocks span[] = {{SF_E_ACC, 3u}, {SF_E_POT, 1u}, {SF_E_RHO, 2u}};
+	return sf_download_blocks(c, span, sf_params()->enable_sph ? 3u : 2u, NULL);
 }
 
 /* Solver sequence of src/simulation.c:231-345 on device state. */
@@ -235,8 +230,8 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 	}
 
 	/* mirror mode: pos, vel, acc, mas (+ rad) are read */
-	if (sf_upload_blocks(c, SF_E_POS, 10u)) return STARFLOOD_FAILURE;
-	if (p->enable_sph && sf_upload_blocks(c, SF_E_RAD, 1u)) return STARFLOOD_FAILURE;
+	const sf_blocks in[] = {{SF_E_POS, 10u}, {SF_E_RAD, 1u}};
+	if (sf_upload_blocks(c, in, p->enable_sph ? 2u : 1u)) return STARFLOOD_FAILURE;
 
 	if (cubic && (sf_ctx_ensure_u(c) || sfd_sph_u_kick(c->d_u, c->d_dudt, N, half_dt, s))) return STARFLOOD_FAILURE;
 	if (timing) tev_record(0, s);
@@ -291,14 +286,11 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 		tev_record(6, s);
 	}
 
-	/* mirror mode: pos, vel, acc, mas, pot, ken, pen (+ rho, prs) are written */
-	if (sf_download_blocks(c, SF_E_POS, 13u)) return STARFLOOD_FAILURE;
-	if (p->enable_sph && sf_download_blocks(c, SF_E_RHO, 2u)) return STARFLOOD_FAILURE;
-
 	const int need_host = p->mem_mode == SF_MEM_MIRROR || p->logging || p->verbose;
+	/* mirror mode: pos, vel, acc, mas, pot, ken, pen (+ rho, prs) are written */
+	const sf_blocks written[] = {{SF_E_POS, 13u}, {SF_E_RHO, 2u}};
+	if (sf_download_blocks(c, written, p->enable_sph ? 2u : 1u, need_host ? red_out : NULL)) return STARFLOOD_FAILURE;
 	if (need_host) {
-		SF_HIP(hipMemcpyAsync(c->h_red, red_out, SF_RED_VALUES * sizeof(double), hipMemcpyDeviceToHost, s),
-		       "sim_step");
 		if (sf_finish(c, "sim_step")) return STARFLOOD_FAILURE;
 		/* the step synchronises here anyway: report a tree walk cut short */
 		if (p->enable_tree && N && sf_tree_check(&sim_ptr->tree, s, "sim_step")) rc = -1;
@@ -345,7 +337,7 @@ int sf_get_stats(const sim_t* sim_ptr, sf_stats_t* out) {
 	const unsigned int N = c->N;
 	const int exact = p->precision == SF_PRECISION_EXACT;
 	hipStream_t s = c->stream;
-	if (p->mem_mode == SF_MEM_MIRROR && sf_upload_blocks(c, SF_E_POS, 13u)) return STARFLOOD_FAILURE;
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 13u}))) return STARFLOOD_FAILURE;
 	float* ken = sf_blk(c->d_mem, N, SF_E_KEN);
 	float* pen = sf_blk(c->d_mem, N, SF_E_PEN);
 	double* red_out = c->d_red + (size_t)(sfd_reduce_scratch_doubles(N) - SF_RED_VALUES);
@@ -355,8 +347,7 @@ int sf_get_stats(const sim_t* sim_ptr, sf_stats_t* out) {
 	                     c->have_u ? c->d_u : NULL, N, p->G, p->epsilon, c->d_red, s))
 		return STARFLOOD_FAILURE;
 	if (exact && sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
-	SF_HIP(hipMemcpyAsync(c->h_red, red_out, SF_RED_VALUES * sizeof(double), hipMemcpyDeviceToHost, s),
-	       "sf_get_stats");
+	if (sf_download_blocks(c, NULL, 0u, red_out)) return STARFLOOD_FAILURE;
 	if (sf_finish(c, "sf_get_stats")) return STARFLOOD_FAILURE;
 	const double* r = c->h_red;
 	out->T = exact ? r[12] : r[0];

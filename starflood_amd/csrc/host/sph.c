@@ -83,10 +83,10 @@ int solve_sph(const sim_t* SF_RESTRICT sim_ptr) {
 		return STARFLOOD_FAILURE;
 	}
 	/* pos, vel, acc, mas, then rad */
-	if (sf_upload_blocks(c, SF_E_POS, 10u) || sf_upload_blocks(c, SF_E_RAD, 1u)) return STARFLOOD_FAILURE;
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 10u}, {SF_E_RAD, 1u}))) return STARFLOOD_FAILURE;
 	int rc = sf_sph_prepare(c, 0.0f);
 	if (!rc) rc = sf_solve_sph(c);
-	if (sf_download_blocks(c, SF_E_ACC, 3u) || sf_download_blocks(c, SF_E_RHO, 2u)) rc = -1;
+	if (sf_download_blocks(c, SF_SPANS({SF_E_ACC, 3u}, {SF_E_RHO, 2u}), NULL)) rc = -1;
 	if (sf_finish(c, "solve_sph")) rc = -1;
 	return rc ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;
 }
@@ -117,8 +117,7 @@ int sf_sph_direct_f64(const sim_t* sim_ptr, const unsigned int* idx, unsigned in
 			return STARFLOOD_FAILURE;
 		}
 	}
-	if (sf_upload_blocks(c, SF_E_POS, 2u * 3u) || sf_upload_blocks(c, SF_E_MAS, 1u) ||
-	    sf_upload_blocks(c, SF_E_RAD, 1u) || sf_ctx_ensure_u(c))
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 2u * 3u}, {SF_E_MAS, 1u}, {SF_E_RAD, 1u})) || sf_ctx_ensure_u(c))
 		return STARFLOOD_FAILURE;
 	unsigned int* d_idx = NULL;
 	double* d_buf = NULL;   /* rho (N), P/rho^2 (N), 4 per listed particle */

@@ -359,7 +359,7 @@ static int gravity_part_tree(const sim_t* SF_RESTRICT sim_ptr) {
 	const sf_params_t* p = sf_params();
 	const unsigned int N = c->N;
 	hipStream_t s = c->stream;
-	if (sf_upload_blocks(c, SF_E_POS, 3u) || sf_upload_blocks(c, SF_E_MAS, 1u)) return STARFLOOD_FAILURE;
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 3u}, {SF_E_MAS, 1u}))) return STARFLOOD_FAILURE;
 	/* order the tree's stream before the simulation's */
 	SF_HIP(hipStreamSynchronize(d->stream), "solve_gravity_part_tree");
 	const float* pos = sf_blk(c->d_mem, N, SF_E_POS);
@@ -377,7 +377,7 @@ static int gravity_part_tree(const sim_t* SF_RESTRICT sim_ptr) {
 		if (!d->lbvh) sf_error("solve_gravity_part_tree", "no tree was built");
 		if (!rc && lbvh_check(d, s, "solve_gravity_part_tree")) rc = -1;
 	}
-	if (sf_download_blocks(c, SF_E_ACC, 3u) || sf_download_blocks(c, SF_E_POT, 1u)) rc = -1;
+	if (sf_download_blocks(c, SF_SPANS({SF_E_ACC, 3u}, {SF_E_POT, 1u}), NULL)) rc = -1;
 	if (sf_finish(c, "solve_gravity_part_tree")) rc = -1;
 	return rc ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;
 }

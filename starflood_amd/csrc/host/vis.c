@@ -204,7 +204,7 @@ int vis_draw(const vis_t* SF_RESTRICT vis_ptr, const sim_t* SF_RESTRICT sim_ptr)
 	const unsigned int N = c->N;
 	hipStream_t s = c->stream;
 	/* pos, vel (blocks 0..5) and pot */
-	if (sf_upload_blocks(c, SF_E_POS, 6u) || sf_upload_blocks(c, SF_E_POT, 1u)) return STARFLOOD_FAILURE;
+	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 6u}, {SF_E_POT, 1u}))) return STARFLOOD_FAILURE;
 	const float* pos = sf_blk(c->d_mem, N, SF_E_POS);
 	double average_radius = 1.0;
 	if (N) {

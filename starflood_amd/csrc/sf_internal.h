@@ -36,6 +36,7 @@ typedef struct sf_tree_dev sf_tree_dev;   /* host/tree.c */
 typedef struct sf_ctx {
 	void* host_mem;          /* key: sim_t.mem */
 	void* host_pinned_base;  /* the page-locked allocation holding sim_t.mem, or NULL (ordinary memory) */
+	float* host_dev;         /* sim_t.mem as the device sees it, or NULL (ordinary memory) */
 	unsigned int N;
 	unsigned int dof;        /* reals per particle in sim.mem */
 	unsigned int n_pad;      /* N rounded up to the PP j tile */
@@ -46,6 +47,7 @@ typedef struct sf_ctx {
 	size_t part_bytes;
 	double* d_red;           /* reduction scratch (blocks * SF_RED_VALUES), then the exact energy sums' */
 	double* h_red;           /* pinned host mirror of the reduction result */
+	double* h_red_dev;       /* the same as the device sees it */
 	float* d_u;              /* SPH specific internal energy (N) */
 	float* d_dudt;           /* its derivative (N) */
 	float* d_sph_tmp;        /* SPH scratch (packed records, 12 n_pad floats) */
@@ -79,9 +81,17 @@ static inline float* sf_blk(float* base, unsigned int N, unsigned int e) { retur
 #define SF_E_RHO 14u
 #define SF_E_PRS 15u
 
-/* mirror-mode transfers of blocks [e0, e0+count) (no-ops in RESIDENT mode) */
-int sf_upload_blocks(sf_ctx* c, unsigned int e0, unsigned int count);
-int sf_download_blocks(sf_ctx* c, unsigned int e0, unsigned int count);
+/* mirror-mode transfers of blocks [e0, e0+count) (no-ops in RESIDENT mode), three
+   of them at most; red (may be NULL, any mode): the
+   SF_RED_VALUES results of a reduction, to h_red */
+typedef struct sf_blocks {
+	unsigned int e0, count;
+} sf_blocks;
+/* the two middle arguments, from a list of {e0, count} */
+#define SF_SPANS(...) \
+	(const sf_blocks[]){__VA_ARGS__}, (unsigned int)(sizeof((const sf_blocks[]){__VA_ARGS__}) / sizeof(sf_blocks))
+int sf_upload_blocks(sf_ctx* c, const sf_blocks* span, unsigned int spans);
+int sf_download_blocks(sf_ctx* c, const sf_blocks* span, unsigned int spans, const double* red);
 int sf_finish(sf_ctx* c, const char* func);   /* synchronise the stream, report errors */
 
 /* ---------- kernel timing (host/prof.c) ---------- */
@@ -92,6 +102,16 @@ void sf_prof_end(int token, hipStream_t s);
 /* ---------- device launchers (csrc/device) ---------- */
 #define SF_RED_VALUES 16u    /* doubles per reduction partial */
 
+/* `words` 32-bit words between device memory and page-locked host memory; dst
+   and src are word aligned, at the same offset from a 16-byte boundary */
+typedef struct sf_copy_range {
+	void* dst;
+	const void* src;
+	size_t words;
+} sf_copy_range;
+#define SF_COPY_RANGES 4u
+/* up to SF_COPY_RANGES of them by one kernel (host_copy.hip) */
+int sfd_copy_ranges(const sf_copy_range* range, unsigned int count, hipStream_t s);
 /* body[i] = (pos_i, m_i) for i < N, zero for N <= i < n_pad */
 int sfd_pack_bodies(const float* pos, const float* mas, unsigned int N, unsigned int n_pad,
                     float* body, hipStream_t s);
