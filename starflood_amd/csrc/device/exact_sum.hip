@@ -30,11 +30,12 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "state_fold.h"
 #include "tree_dev.h"
 
 namespace {
 
-constexpr unsigned kBlock = 256;
+constexpr unsigned kBlock = fold::kThreads;
 constexpr unsigned kPer = 16;                  // terms per thread
 constexpr unsigned kChunk = kBlock * kPer;     // terms per block
 constexpr int kSpan = 27;                      // exponents kept in one integer: |m| 2^27 < 2^51
@@ -138,10 +139,16 @@ __device__ void finish_sum(const float* __restrict__ x, unsigned N, const Partia
 }
 
 // Blocks (chunk, array): array 0 is x0, array 1 is x1.  A single chunk is
-// finished here, more by k_exact_finish.
+// finished here, more by k_exact_finish.  A block of a third row folds the
+// partials of the state's reduction (a launch of its own took 3 us).
 __global__ __launch_bounds__(kBlock) void k_exact_chunks(const float* __restrict__ x0, const float* __restrict__ x1,
                                                          unsigned N, Partial* __restrict__ part,
-                                                         double* __restrict__ out) {
+                                                         double* __restrict__ out, double* __restrict__ red,
+                                                         unsigned red_blocks) {
+	if (blockIdx.y == 2u) {
+		if (blockIdx.x == 0u) fold::state(red, red_blocks);
+		return;
+	}
 	__shared__ int s_lo[kBlock / 64], s_hi[kBlock / 64];
 	__shared__ long long s_sum[kBlock / 64];
 	const float* __restrict__ x = blockIdx.y ? x1 : x0;
@@ -311,11 +318,12 @@ extern "C" size_t sfd_energy_scratch_bytes(unsigned N) {
 }
 
 extern "C" int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned N, void* part, double* out,
-                                     hipStream_t s) {
+                                     double* red, hipStream_t s) {
 	const unsigned np = N ? (N + kChunk - 1u) / kChunk : 1u;
 	Partial* p = static_cast<Partial*>(part);
 	const int tok = sf_prof_begin("energy_sum_seq", s);
-	hipLaunchKernelGGL(k_exact_chunks, dim3(np, 2), dim3(kBlock), 0, s, ken, pen, N, p, out);
+	hipLaunchKernelGGL(k_exact_chunks, dim3(np, red ? 3 : 2), dim3(kBlock), 0, s, ken, pen, N, p, out, red,
+	                   fold::blocks(N));
 	if (np > 1u) hipLaunchKernelGGL(k_exact_finish, dim3(2), dim3(kBlock), 0, s, ken, pen, N, p, np, out);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_energy_sums_exact", "launch");

@@ -9,11 +9,13 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "state_fold.h"
 
 namespace {
 
-constexpr unsigned kBlock = 256;
-constexpr unsigned kRedBlocks = 512;   // fixed grid of the state reduction
+constexpr unsigned kBlock = fold::kThreads;
+using fold::kRedBlocks;
+using fold::kRedQ;
 
 inline unsigned grid_for(unsigned n) { return (n + kBlock - 1) / kBlock; }
 
@@ -83,8 +85,6 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift_fast(float* __restrict__ 
 	x64[k] = x;
 	pos[k] = (float)x;
 }
-
-constexpr int kRedQ = 11;   // T, V, W, U, Px, Py, Pz, Lx, Ly, Lz, K
 
 // Per-block partial sums with a fixed grid-stride assignment and a fixed
 // LDS tree, so the result does not depend on scheduling.  KICK: first the
@@ -158,29 +158,8 @@ __global__ __launch_bounds__(kBlock) void k_reduce_state(const float* __restrict
 	if (threadIdx.x < kRedQ) red[(size_t)blockIdx.x * SF_RED_VALUES + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-// Second stage: one block folds the block partials in a fixed tree and
-// writes the totals to red[0 .. SF_RED_VALUES) (after the partials region).
-__global__ __launch_bounds__(kBlock) void k_reduce_final(double* __restrict__ red, unsigned nblocks,
-                                                         double* __restrict__ out) {
-	__shared__ double sh[kRedQ][kBlock];
-	double q[kRedQ];
-#pragma unroll
-	for (int t = 0; t < kRedQ; ++t) q[t] = 0.0;
-	for (unsigned b = threadIdx.x; b < nblocks; b += kBlock) {
-#pragma unroll
-		for (int t = 0; t < kRedQ; ++t) q[t] += red[(size_t)b * SF_RED_VALUES + t];
-	}
-#pragma unroll
-	for (int t = 0; t < kRedQ; ++t) sh[t][threadIdx.x] = q[t];
-	__syncthreads();
-	for (unsigned h = kBlock / 2; h > 0; h >>= 1) {
-		if (threadIdx.x < h) {
-#pragma unroll
-			for (int t = 0; t < kRedQ; ++t) sh[t][threadIdx.x] += sh[t][threadIdx.x + h];
-		}
-		__syncthreads();
-	}
-	if (threadIdx.x < (unsigned)kRedQ) out[threadIdx.x] = sh[threadIdx.x][0];
+__global__ __launch_bounds__(kBlock) void k_reduce_final(double* __restrict__ red, unsigned nblocks) {
+	fold::state(red, nblocks);
 }
 
 }  // namespace
@@ -243,16 +222,15 @@ extern "C" unsigned sfd_reduce_scratch_doubles(unsigned N) {
 static int reduce(Kick kick, const float* pos, const double* x64, float* vel, const float* mas, const float* pot,
                   float* ken, float* pen, const float* u, unsigned N, double G, double eps, const float* acc,
                   float half_dt, double* red, hipStream_t s) {
-	unsigned nb = grid_for(N);
-	if (nb > kRedBlocks) nb = kRedBlocks;
-	if (nb == 0) nb = 1;
+	const unsigned nb = fold::blocks(N);
 	const auto kernel = kick == kNoKick     ? k_reduce_state<kNoKick>
 	                    : kick == kFastKick ? k_reduce_state<kFastKick>
 	                                        : k_reduce_state<kExactKick>;
 	const int tok = sf_prof_begin(kick == kNoKick ? "reduce_state" : "kick_reduce_state", s);
 	hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, s, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc,
 	                   half_dt, red);
-	hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, s, red, nb, red + (size_t)kRedBlocks * SF_RED_VALUES);
+	// the exact policy's sums follow and fold the partials too
+	if (kick != kExactKick) hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, s, red, nb);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_reduce_state", "launch");
 }
@@ -268,5 +246,11 @@ extern "C" int sfd_reduce_state(const float* pos, const double* x64, const float
 extern "C" int sfd_kick_reduce_state(const float* pos, const double* x64, float* vel, const float* acc,
                                      const float* mas, const float* pot, float half_dt, float* ken, float* pen,
                                      const float* u, unsigned N, double G, double eps, double* red, hipStream_t s) {
-	return reduce(x64 ? kFastKick : kExactKick, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red, s);
+	return reduce(kFastKick, pos, x64, vel, mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red, s);
+}
+
+extern "C" int sfd_kick_reduce_exact(const float* pos, float* vel, const float* acc, const float* mas, const float* pot,
+                                     float half_dt, float* ken, float* pen, const float* u, unsigned N, double G,
+                                     double eps, double* red, hipStream_t s) {
+	return reduce(kExactKick, pos, nullptr, vel, mas, pot, ken, pen, u, N, G, eps, acc, half_dt, red, s);
 }

@@ -265,21 +265,24 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 		tev_record(4, s);
 		if (sfd_energy_terms(vel, mas, pot, N, ken, pen, s)) return STARFLOOD_FAILURE;
 		/* ken_sum and pen_sum in one pass (its time is logged as ken_sum's) */
-		if (sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
+		if (sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, NULL, s)) return STARFLOOD_FAILURE;
 		tev_record(5, s);
 		tev_record(6, s);
 	}
 	/* FP64 W, P, L (and T, V in the fast policy), with kick_1 and the energy
 	   terms in the same pass: the fast policy's time is logged as kick_1's, the
 	   exact policy's log has them apart */
-	if (apart || fused ? sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, u, N, p->G, p->epsilon,
-	                                      c->d_red, s)
-	                   : sfd_kick_reduce_state(pos, c->d_x64, vel, acc, mas, pot, half_dt, ken, pen, u, N, p->G,
-	                                           p->epsilon, c->d_red, s))
+	if (apart || fused) {
+		if (sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, u, N, p->G, p->epsilon, c->d_red, s))
+			return STARFLOOD_FAILURE;
+	} else if (exact) {
+		if (sfd_kick_reduce_exact(pos, vel, acc, mas, pot, half_dt, ken, pen, u, N, p->G, p->epsilon, c->d_red, s) ||
+		    sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, c->d_red, s))
+			return STARFLOOD_FAILURE;
+	} else if (sfd_kick_reduce_state(pos, c->d_x64, vel, acc, mas, pot, half_dt, ken, pen, u, N, p->G, p->epsilon,
+	                                 c->d_red, s)) {
 		return STARFLOOD_FAILURE;
-	if (exact && !apart &&
-	    sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s))
-		return STARFLOOD_FAILURE;
+	}
 	if (!exact && timing) {
 		tev_record(4, s);
 		tev_record(5, s);
@@ -346,7 +349,8 @@ int sf_get_stats(const sim_t* sim_ptr, sf_stats_t* out) {
 	                     sf_blk(c->d_mem, N, SF_E_MAS), sf_blk(c->d_mem, N, SF_E_POT), ken, pen,
 	                     c->have_u ? c->d_u : NULL, N, p->G, p->epsilon, c->d_red, s))
 		return STARFLOOD_FAILURE;
-	if (exact && sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, s)) return STARFLOOD_FAILURE;
+	if (exact && sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, NULL, s))
+		return STARFLOOD_FAILURE;
 	if (sf_download_blocks(c, NULL, 0u, red_out)) return STARFLOOD_FAILURE;
 	if (sf_finish(c, "sf_get_stats")) return STARFLOOD_FAILURE;
 	const double* r = c->h_red;

@@ -180,9 +180,11 @@ int sfd_energy_terms(const float* vel, const float* mas, const float* pot, unsig
                      float* ken, float* pen, hipStream_t s);
 /* exact_sum.hip: the sequential FP64 Kahan sums of ken and pen in index order
    (src/simulation.c:455-497), bit for bit, into out[0] and out[1]; part is
-   scratch of sfd_energy_scratch_bytes(N). */
+   scratch of sfd_energy_scratch_bytes(N).  red (may be NULL): partials that
+   sfd_kick_reduce_exact left, folded in the same launch. */
 size_t sfd_energy_scratch_bytes(unsigned int N);
-int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned int N, void* part, double* out, hipStream_t s);
+int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned int N, void* part, double* out, double* red,
+                          hipStream_t s);
 
 /* FAST KDK: kick + FP64 drift fused; x64 refreshed from pos where they
    disagree (sfd_x64_refresh, or inside the drift). */
@@ -199,11 +201,15 @@ unsigned int sfd_reduce_scratch_doubles(unsigned int N);
 int sfd_reduce_state(const float* pos, const double* x64, const float* vel, const float* mas,
                      const float* pot, const float* ken, const float* pen, const float* u,
                      unsigned int N, double G, double eps, double* red, hipStream_t s);
-/* v += half_dt a (the exact policy's roundings without x64) and
-   sfd_energy_terms first, in the same pass */
+/* v += half_dt a and sfd_energy_terms first, in the same pass */
 int sfd_kick_reduce_state(const float* pos, const double* x64, float* vel, const float* acc, const float* mas,
                           const float* pot, float half_dt, float* ken, float* pen, const float* u, unsigned int N,
                           double G, double eps, double* red, hipStream_t s);
+/* the same with the exact policy's roundings; the blocks' partials alone, for
+   sfd_energy_sums_exact */
+int sfd_kick_reduce_exact(const float* pos, float* vel, const float* acc, const float* mas, const float* pot,
+                          float half_dt, float* ken, float* pen, const float* u, unsigned int N, double G,
+                          double eps, double* red, hipStream_t s);
 
 #ifdef __cplusplus
 }
