@@ -44,12 +44,12 @@ DT = 1.0e-3
 SEED = 11
 PEAK_FP32_TFLOPS = 157.3
 FLOPS_PER_INTERACTION = 20
-# HBM bytes of one k_pp_fast dispatch at N = 262144 (8 block slices of FP64
-# partials): rocprofv3 FETCH_SIZE 18330 KiB x 2.0 + WRITE_SIZE 65536 KiB x 1.0,
-# the factors from a 1 GiB copy read under the same counters
-# (profiles/pp_fast_n262144.md).  The writes are the slice partials; the
-# kernel is VALU-bound.
-PP_FAST_TRAFFIC_BYTES = (18330 * 2 + 65536) * 1024
+# HBM bytes of one k_pp_sym dispatch at N = 262144 (128 planes of j sums, 512 MiB,
+# and the planes of i sums): rocprofv3 FETCH_SIZE 164600 KiB x 2.0 + WRITE_SIZE
+# 821700 KiB x 1.0, the factors from a 1 GiB copy read under the same counters
+# (profiles/pp_sym_n262144.md).  The writes are the planes; the kernel is
+# VALU-bound.
+PP_FAST_TRAFFIC_BYTES = (164600 * 2 + 821700) * 1024
 
 
 def hip_sync():
@@ -851,7 +851,7 @@ def main():
                    "N": N_PP, "epsilon": EPS, "dt": DT, "parallelism": "single GPU"},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": PP_FAST_TRAFFIC_BYTES,
-                     "kernel": "k_pp_fast", "kernel_ms": pp_avg_s * 1e3,
+                     "kernel": "k_pp_sym", "kernel_ms": pp_avg_s * 1e3,
                      "peak_source": "MI355X FP32 157.3 TFLOP/s; the kernel is FP32 VALU work (rsqrt and FMA, no MFMA)",
                      "flops_per_launch": FLOPS_PER_INTERACTION * inter},
         "energy_check": {"K": st["K"], "W": st["W"], "T_ken": st["T"]},

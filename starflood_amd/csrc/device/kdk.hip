@@ -3,7 +3,7 @@
 //
 // Exact policy: FP32 elementwise updates in the reference's operation order
 // (file compiled with -ffp-contract=off); T and V are exact_sum.hip's.
-// Fast policy: kick and FP64 drift fused in one pass over the state, and
+// Fast policy: kick and FP64 drift fused in one pass over the state.  Both:
 // tree-shaped FP64 block reductions with a fixed grid, which are
 // deterministic and more accurate than a sequential sum.
 #include <hip/hip_runtime.h>

@@ -7,8 +7,9 @@
 //  2. 63-bit Morton codes: q = floor((x - lo) * (2^21 / extent)) in FP64,
 //     clamped to [0, 2^21), bits interleaved x-y-z from the top.  Exactly
 //     reproducible by a CPU restatement.
-//  3. Stable LSD radix sort of (code, index), 8 passes of 8-bit digits, with
-//     per-tile histograms, one scan, and a ballot-based stable local rank.
+//  3. Stable LSD radix sort of (code, index), 8 passes of 8-bit digits, one
+//     launch each: a ballot-based stable local rank, and the tiles' offsets
+//     by looking back.
 //  4. Binary radix tree from the sorted codes (Karras 2012): internal node i
 //     covers a contiguous range of the sorted particles; equal codes are
 //     separated by their sorted position.

@@ -8,8 +8,8 @@
 
 #include "sf_host.h"
 
-/* j slices of the one-sided kernels (the force VJP below 10240 bodies, the SPH
-   all-pairs passes): enough blocks to give every CU several waves */
+/* j slices of the cubic SPH all-pairs passes: enough blocks to give every CU
+   several waves */
 static unsigned int pp_slices(unsigned int n_pad) {
 	/* one j range per wavefront of 64 i; about 128k wavefronts, while each
 	   range keeps at least 256 j */

@@ -14,9 +14,8 @@ int sf_solve_gravity_pp(sf_ctx* c);
 /* gravity.c: a whole step of the fast policy with PP gravity and no SPH:
    kick and drift, force, closing kick and energy terms, in three launches */
 int sf_step_gravity_pp(sf_ctx* c);
-/* gravity.c: j ranges of the fast PP kernel (and of the SPH all-pairs and
-   VJP passes) for n_pad particles, the bytes of slice partials the fast PP
-   kernel writes, the fast PP force of packed bodies ended by *epi, and the
+/* gravity.c: j ranges of the cubic SPH all-pairs passes for n_pad particles, the
+   bytes of partial sums the fast PP kernels write, the fast PP force of packed bodies ended by *epi, and the
    one of caller arrays (body: n_pad float4, part: part_bytes >=
    sf_pp_part_bytes(n_pad), pot may be NULL) */
 unsigned int sf_pp_slice_count(unsigned int n_pad);
