@@ -52,6 +52,7 @@ constexpr unsigned kMaxLevels = 17;           // depths 0..16: tree_depth_max is
 constexpr unsigned kFirstBatch = 6, kNextBatch = 3;   // levels queued per host synchronisation
 constexpr unsigned kPer = 4;                  // particles per thread of a tile
 constexpr unsigned kTileP = kBlock * kPer;    // consecutive particles per block
+static_assert(kBlock / 64u == 4u, "k_level_particles: two octants per wavefront of the block");
 
 enum Status { RUNNING = 0, DONE = 1, FALLBACK = 2 };
 // A level: its slots, the level-major id of the first, splits of the shallower
