@@ -54,9 +54,12 @@ __device__ __forceinline__ void kahan(float& s, float& c, float x) {
 	s = t;
 }
 
-template <unsigned I, class M>
+// WAVES: the block's wavefronts, where a launch runs models of different sizes;
+// those that this one does not need wait.
+template <unsigned I, unsigned WAVES = 0, class M>
 __device__ __forceinline__ void run(const M& md, unsigned N) {
 	constexpr unsigned kC = M::kComps, kChainWaves = chain_waves<I, kC>();
+	static_assert(WAVES == 0 || WAVES >= kChainWaves + kMakers, "the model's wavefronts");
 	constexpr unsigned kPer = 64u / I;           // bodies a wavefront takes at once
 	constexpr unsigned kLane = kRun / kPer;      // bodies of a run per lane
 	__shared__ float s_term[2][kC][kJ][I];
@@ -64,6 +67,10 @@ __device__ __forceinline__ void run(const M& md, unsigned N) {
 	const unsigned part = I == 64u ? 0u : lane / I, il = lane % I;
 	const unsigned i = blockIdx.x * I + il;
 	const unsigned tiles = (N + kJ - 1u) / kJ;
+	if (WAVES && wv >= kChainWaves + kMakers) {
+		for (unsigned t = 0; t <= tiles; ++t) __syncthreads();
+		return;
+	}
 	if (wv >= kChainWaves) {
 		const typename M::Self me = md.self(min(i, N - 1u));
 		const unsigned first = (wv - kChainWaves) * kRun;

@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
+#include "exact_pp.h"
 #include "order_chain.h"
 
 namespace {
@@ -140,6 +141,41 @@ __global__ __launch_bounds__((chain::block_size<I, 1>())) void k_rho_ref(const f
 	chain::run<I>(RhoRef<KAHAN>{ra, rh, rho}, N);
 }
 
+// The density (blockIdx.y 0) beside the gravity that the force is added to
+// (blockIdx.y 1), which do not need each other.  Up to 4096 particles their
+// blocks fit one to a CU and overlap; a CU with one of each takes as long as
+// one after the other.  Solve, apart -> together (us): 512 particles 50.7 ->
+// 42.6, 2000 120 -> 95, 4096 214 -> 166, 4100 216 -> 207, 4600 239 -> 229, 5200
+// 267 both, 6000 303 -> 305, 8192 403 -> 408.  Hence kTogetherN.
+constexpr unsigned kTogetherN = 5120;
+static_assert(kTogetherN <= chain::kFewN, "32 particles a block");
+
+template <bool KAHAN_ACC, bool KAHAN_POT, bool PHYS>
+__global__ __launch_bounds__((chain::block_size<32, 4>())) void k_rho_pp_ref(
+    const float4* __restrict__ ra, const float4* __restrict__ rh, float* __restrict__ rho, const float* __restrict__ pos,
+    const float* __restrict__ mas, unsigned N, float eps2, float negG, float* __restrict__ acc, float* __restrict__ pot) {
+	constexpr unsigned kWaves = chain::block_size<32, 4>() / 64u;
+	if (blockIdx.y == 0u) chain::run<32, kWaves>(RhoRef<KAHAN_ACC>{ra, rh, rho}, N);
+	else chain::run<32>(chain::ExactPP<KAHAN_ACC, KAHAN_POT, PHYS>{pos, mas, eps2, negG, acc, pot}, N);
+}
+
+void launch_rho_pp(const sf_exact_pp* g, const float4* ra, const float4* rh, float* rho, const float* pos,
+                   const float* mas, unsigned N, float* acc, hipStream_t s) {
+	auto k = k_rho_pp_ref<true, true, true>;
+	switch ((g->kahan_acc ? 4 : 0) | (g->kahan_pot ? 2 : 0) | (g->acc_phys ? 1 : 0)) {
+	case 0: k = k_rho_pp_ref<false, false, false>; break;
+	case 1: k = k_rho_pp_ref<false, false, true>; break;
+	case 2: k = k_rho_pp_ref<false, true, false>; break;
+	case 3: k = k_rho_pp_ref<false, true, true>; break;
+	case 4: k = k_rho_pp_ref<true, false, false>; break;
+	case 5: k = k_rho_pp_ref<true, false, true>; break;
+	case 6: k = k_rho_pp_ref<true, true, false>; break;
+	default: break;
+	}
+	hipLaunchKernelGGL(k, dim3((N + 31u) / 32u, 2), dim3(chain::block_size<32, 4>()), 0, s, ra, rh, rho, pos, mas, N,
+	                   g->eps2, g->neg_g, acc, g->pot);
+}
+
 // P = (K rho)^(1/n + 1) with K = 0.1, n = 1 (src/sph.c:147-157), and the
 // momentum-equation factor P / rho^2 (src/sph.c:189-192, :225-226), which
 // takes the mass's place in the record
@@ -213,10 +249,11 @@ __global__ __launch_bounds__((chain::block_size<I, 3>())) void k_force_ref(const
 }
 
 template <unsigned I, bool KAHAN>
-void launch_ref(const float4* ra, const float4* rh, const float4* rd, const float* mas, unsigned N, float* rho,
-                float* prs, float4* ra_con, float* acc, hipStream_t s) {
+void launch_ref(const sf_exact_pp* gravity, const float4* ra, const float4* rh, const float4* rd, const float* pos,
+                const float* mas, unsigned N, float* rho, float* prs, float4* ra_con, float* acc, hipStream_t s) {
 	const dim3 g((N + I - 1u) / I);
-	hipLaunchKernelGGL((k_rho_ref<I, KAHAN>), g, dim3(chain::block_size<I, 1>()), 0, s, ra, rh, N, rho);
+	if (gravity) launch_rho_pp(gravity, ra, rh, rho, pos, mas, N, acc, s);
+	else hipLaunchKernelGGL((k_rho_ref<I, KAHAN>), g, dim3(chain::block_size<I, 1>()), 0, s, ra, rh, N, rho);
 	hipLaunchKernelGGL(k_eos_ref, dim3((N + kBlock - 1u) / kBlock), dim3(kBlock), 0, s, rho, N, prs, ra_con);
 	hipLaunchKernelGGL((k_force_ref<I, KAHAN>), g, dim3(chain::block_size<I, 3>()), 0, s, ra, rd, mas, N, acc);
 }
@@ -386,16 +423,22 @@ extern "C" {
 
 size_t sfd_sph_tmp_floats(unsigned n_pad) { return 12u * (size_t)n_pad + 16u; }
 
-int sfd_sph_ref(const float* pos, const float* mas, const float* rad, unsigned N, int kahan, float* rho, float* prs,
-                float* acc, float* tmp, hipStream_t s) {
+int sfd_sph_ref(const float* pos, const float* mas, const float* rad, unsigned N, int kahan, const sf_exact_pp* gravity,
+                float* rho, float* prs, float* acc, float* tmp, hipStream_t s) {
 	if (N == 0) return 0;
+	if (gravity && N > kTogetherN) {
+		if (sfd_pp_exact(pos, mas, N, gravity->eps2, gravity->neg_g, gravity->acc_phys, gravity->kahan_acc,
+		                 gravity->kahan_pot, acc, gravity->pot, s))
+			return -1;
+		gravity = nullptr;
+	}
 	float4* ra = reinterpret_cast<float4*>(tmp);
 	float4* rh = ra + N;
 	float4* rd = ra + 2u * (size_t)N;
 	hipLaunchKernelGGL(k_tables_ref, grid(N), dim3(kBlock), 0, s, pos, mas, rad, N, ra, rh, rd);
 	auto go = N <= chain::kFewN ? (kahan ? launch_ref<32, true> : launch_ref<32, false>)
 	                            : (kahan ? launch_ref<64, true> : launch_ref<64, false>);
-	go(ra, rh, rd, mas, N, rho, prs, ra, acc, s);
+	go(gravity, ra, rh, rd, pos, mas, N, rho, prs, ra, acc, s);
 	return sf_hip_check(hipGetLastError(), "solve_sph", "launch");
 }
 

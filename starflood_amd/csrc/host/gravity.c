@@ -50,14 +50,21 @@ int sf_pp_force_arrays(const sf_params_t* p, unsigned int N, unsigned int n_pad,
 	return force(p, N, n_pad, pos, mas, body, part, part_bytes, &epi, s);
 }
 
+sf_exact_pp sf_exact_pp_params(sf_ctx* c) {
+	const sf_params_t* p = sf_params();
+	return (sf_exact_pp){.eps2 = eps2_f32(p->epsilon), .neg_g = (float)(-p->G),
+	                     .acc_phys = p->acc_mode == SF_ACC_PHYSICAL, .kahan_acc = p->kahan_solver,
+	                     .kahan_pot = p->kahan_energy, .pot = sf_blk(c->d_mem, c->N, SF_E_POT)};
+}
+
 int sf_solve_gravity_pp(sf_ctx* c) {
 	const sf_params_t* p = sf_params();
 	const unsigned int N = c->N;
 	const float *pos = sf_blk(c->d_mem, N, SF_E_POS), *mas = sf_blk(c->d_mem, N, SF_E_MAS);
 	float *acc = sf_blk(c->d_mem, N, SF_E_ACC), *pot = sf_blk(c->d_mem, N, SF_E_POT);
 	if (p->precision == SF_PRECISION_EXACT) {
-		return sfd_pp_exact(pos, mas, N, eps2_f32(p->epsilon), (float)(-p->G), p->acc_mode == SF_ACC_PHYSICAL,
-		                    p->kahan_solver, p->kahan_energy, acc, pot, c->stream);
+		const sf_exact_pp e = sf_exact_pp_params(c);
+		return sfd_pp_exact(pos, mas, N, e.eps2, e.neg_g, e.acc_phys, e.kahan_acc, e.kahan_pot, acc, pot, c->stream);
 	}
 	if (sf_ctx_reserve_part(c, sf_pp_part_bytes(c->n_pad))) return -1;
 	return sf_pp_force_arrays(p, N, c->n_pad, pos, mas, c->d_body, c->d_part, c->part_bytes, acc, pot, c->stream);

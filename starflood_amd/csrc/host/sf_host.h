@@ -11,6 +11,8 @@
 
 /* gravity.c: PP gravity from d_mem pos/mas into d_mem acc/pot */
 int sf_solve_gravity_pp(sf_ctx* c);
+/* the exact policy's parameters for it */
+sf_exact_pp sf_exact_pp_params(sf_ctx* c);
 /* gravity.c: a whole step of the fast policy with PP gravity and no SPH:
    kick and drift, force, closing kick and energy terms, in three launches */
 int sf_step_gravity_pp(sf_ctx* c);
@@ -33,9 +35,10 @@ int sf_solve_gravity_tree(sf_ctx* c, tree_t* tree, unsigned int step_number, int
 int sf_tree_check(tree_t* tree, hipStream_t s, const char* fn);
 /* sph.c: density, EOS and pressure force, added into acc.  For the cubic
    model sf_sph_prepare packs the particle records first, while acc still
-   holds the previous forces: velocities and u are predicted pred_dt ahead. */
+   holds the previous forces: velocities and u are predicted pred_dt ahead.
+   gravity (reference model, may be NULL): the exact PP gravity, made first. */
 int sf_sph_prepare(sf_ctx* c, float pred_dt);
-int sf_solve_sph(sf_ctx* c);
+int sf_solve_sph(sf_ctx* c, const sf_exact_pp* gravity);
 /* simulation.c: sim_solv and sim_step, whichever prototype form the library
    exports (SOLVER_VIS or not) */
 int sf_sim_solv(sim_t* SF_RESTRICT sim_ptr);

@@ -164,13 +164,19 @@ int sf_solve_all(sf_ctx* c, tree_t* tree, unsigned int step_number, float sph_pr
 	int rc = 0;
 	if (c->N == 0) return 0;   /* no particles: no forces, no densities */
 	if (p->enable_sph && sf_sph_prepare(c, sph_pred_dt)) return -1;
+	if (p->enable_sph && !p->enable_tree && p->precision == SF_PRECISION_EXACT &&
+	    p->sph_model == SF_SPH_REFERENCE) {
+		/* gravity and density do not need each other: one launch */
+		const sf_exact_pp gravity = sf_exact_pp_params(c);
+		return sf_solve_sph(c, &gravity) ? -1 : 0;
+	}
 	if (p->enable_tree) {
 		if (sf_solve_gravity_tree(c, tree, step_number, prev_acc)) rc = -1;
 	} else {
 		if (sf_solve_gravity_pp(c)) rc = -1;
 	}
 	if (p->enable_sph) {
-		if (sf_solve_sph(c)) rc = -1;
+		if (sf_solve_sph(c, NULL)) rc = -1;
 	}
 	return rc;
 }

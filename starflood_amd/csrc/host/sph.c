@@ -13,8 +13,8 @@
 
 /* kernels in device/sph.hip */
 size_t sfd_sph_tmp_floats(unsigned int n_pad);
-int sfd_sph_ref(const float* pos, const float* mas, const float* rad, unsigned int N, int kahan, float* rho, float* prs,
-                float* acc, float* tmp, hipStream_t s);
+int sfd_sph_ref(const float* pos, const float* mas, const float* rad, unsigned int N, int kahan,
+                const sf_exact_pp* gravity, float* rho, float* prs, float* acc, float* tmp, hipStream_t s);
 int sfd_sph_cubic_pack(const float* pos, const float* vel, const float* acc, const float* mas, const float* rad,
                        const float* u, const float* dudt, unsigned int N, unsigned int n_pad, float pred_dt, float* tmp,
                        hipStream_t s);
@@ -42,7 +42,7 @@ int sf_sph_prepare(sf_ctx* c, float pred_dt) {
 	                          c->stream);
 }
 
-int sf_solve_sph(sf_ctx* c) {
+int sf_solve_sph(sf_ctx* c, const sf_exact_pp* gravity) {
 	const sf_params_t* p = sf_params();
 	const unsigned int N = c->N;
 	if (N == 0) return 0;
@@ -66,7 +66,7 @@ int sf_solve_sph(sf_ctx* c) {
 	}
 	const int tok = sf_prof_begin("sph_ref", c->stream);
 	const int rc = sfd_sph_ref(sf_blk(c->d_mem, N, SF_E_POS), sf_blk(c->d_mem, N, SF_E_MAS),
-	                           sf_blk(c->d_mem, N, SF_E_RAD), N, p->kahan_solver, rho, prs, acc, c->d_sph_tmp,
+	                           sf_blk(c->d_mem, N, SF_E_RAD), N, p->kahan_solver, gravity, rho, prs, acc, c->d_sph_tmp,
 	                           c->stream);
 	sf_prof_end(tok, c->stream);
 	return rc;
@@ -85,7 +85,7 @@ int solve_sph(const sim_t* SF_RESTRICT sim_ptr) {
 	/* pos, vel, acc, mas, then rad */
 	if (sf_upload_blocks(c, SF_SPANS({SF_E_POS, 10u}, {SF_E_RAD, 1u}))) return STARFLOOD_FAILURE;
 	int rc = sf_sph_prepare(c, 0.0f);
-	if (!rc) rc = sf_solve_sph(c);
+	if (!rc) rc = sf_solve_sph(c, NULL);
 	if (sf_download_blocks(c, SF_SPANS({SF_E_ACC, 3u}, {SF_E_RHO, 2u}), NULL)) rc = -1;
 	if (sf_finish(c, "solve_sph")) rc = -1;
 	return rc ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;

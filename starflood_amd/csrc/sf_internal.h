@@ -122,6 +122,12 @@ int sfd_kick_drift_pack(float* vel, const float* acc, double* x64, float* pos, c
 /* Reference-order PP gravity (src/gravity.c:693-812). */
 int sfd_pp_exact(const float* pos, const float* mas, unsigned int N, float eps2, float negG,
                  int acc_phys, int kahan_acc, int kahan_pot, float* acc, float* pot, hipStream_t s);
+/* its parameters, for a launch that makes it beside other sums */
+typedef struct sf_exact_pp {
+	float eps2, neg_g;
+	int acc_phys, kahan_acc, kahan_pot;   /* kahan_acc: that of the other sums too */
+	float* pot;
+} sf_exact_pp;
 
 /* What the fast force's combine does with each acceleration
    (device/force_epi.h): SF_EPI_STORE writes acc and (unless NULL) pot;
