@@ -18,6 +18,11 @@
 // the nine row partials are added in fixed row order, so results do not
 // depend on scheduling.  The pair arithmetic is the all-pairs kernels'
 // (device/sph.hip); only the order of each particle's sum differs.
+//
+// Small systems are bound by the step's launches: with the largest h, the cell
+// size, the table's clearing and its runs in launches of their own (four more)
+// a step of 2000 particles took 100 us, now 92 (three systems in turn 68 and
+// 57.5 each); 65536, mostly gravity, 1051 and 1036.
 #include <hip/hip_runtime.h>
 
 #include "../sf_internal.h"
@@ -65,70 +70,69 @@ __device__ __forceinline__ float cubic_dw(float q, float inv_h) {
 	return q <= 0.5f ? k * inner : (q <= 1.0f ? k * -6.0f * t * t : 0.0f);
 }
 
-// hm[0] = bits of max |h| (non-negative floats order as integers)
-__global__ __launch_bounds__(kBlock) void k_hmax(const float* __restrict__ rad, unsigned N, unsigned* __restrict__ hm) {
-	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-	float h = i < N ? fabsf(rad[i]) : 0.0f;
-	if (!(h <= 3.0e38f)) h = 0.0f;   // NaN and inf take no part in the search radius
-	unsigned v = __float_as_uint(h);
+// The largest of a wavefront's values, then of the block's, in every thread.
+__device__ __forceinline__ unsigned block_max(unsigned v) {
+	__shared__ unsigned sh[kBlock / 64];
 	for (int o = 32; o > 0; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o));
-	if ((threadIdx.x & 63u) == 0u) atomicMax(hm, v);
+	if ((threadIdx.x & 63u) == 0u) sh[threadIdx.x >> 6] = v;
+	__syncthreads();
+	for (unsigned w = 0; w < kBlock / 64; ++w) v = max(v, sh[w]);
+	return v;
 }
 
-// 1 / c with c = h_max (1 + 2^-10), the margin covering the FP32 rounding of
-// the pair test; unit cells when every h is zero
-__global__ void k_cell_scale(const unsigned* __restrict__ hm, double* __restrict__ inv_c) {
-	if (blockIdx.x != 0 || threadIdx.x != 0) return;
-	const double h = (double)__uint_as_float(hm[0]);
-	inv_c[0] = h > 0.0 ? 1.0 / (h * (1.0 + 1.0 / 1024.0)) : 1.0;
+// Each block's bits of max |h| (non-negative floats order as integers).  One
+// word for all by atomics took 12.8 us at N = 65536, its clearing and the cell
+// size after it a launch each; k_grid_keys takes the blocks' values instead.
+constexpr unsigned kHmaxBlocks = kBlock;
+__global__ __launch_bounds__(kBlock) void k_hmax(const float* __restrict__ rad, unsigned N, unsigned* __restrict__ hm) {
+	unsigned v = 0u;
+	for (unsigned i = blockIdx.x * kBlock + threadIdx.x; i < N; i += gridDim.x * kBlock) {
+		const float h = fabsf(rad[i]);
+		if (h <= 3.0e38f) v = max(v, __float_as_uint(h));   // NaN and inf take no part in the search radius
+	}
+	v = block_max(v);
+	if (threadIdx.x == 0u) hm[blockIdx.x] = v;
 }
 
-__global__ void k_zero_u32(unsigned* __restrict__ x) {
-	if (blockIdx.x == 0 && threadIdx.x == 0) x[0] = 0u;
-}
-
-// key = bucket of the particle's cell, val = index; padding keys kNone
+// key = bucket of the particle's cell, val = index; padding keys kNone.  The
+// cells' inverse side is 1 / c with c = h_max (1 + 2^-10), the margin covering
+// the FP32 rounding of the pair test; unit cells when every h is zero.  Every
+// block finds it from k_hmax's n_hm values.  Clears the bucket table.
 __global__ __launch_bounds__(kBlock) void k_grid_keys(const float4* __restrict__ q0, unsigned N, unsigned n_sort,
-                                                      const double* __restrict__ inv_c, unsigned mask,
-                                                      unsigned long long* __restrict__ key,
+                                                      const unsigned* __restrict__ hm, unsigned n_hm,
+                                                      double* __restrict__ inv_c, unsigned T,
+                                                      uint2* __restrict__ bucket, unsigned long long* __restrict__ key,
                                                       unsigned* __restrict__ val) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+	const double h = (double)__uint_as_float(block_max(threadIdx.x < n_hm ? hm[threadIdx.x] : 0u));
+	const double ic = h > 0.0 ? 1.0 / (h * (1.0 + 1.0 / 1024.0)) : 1.0;
+	if (i == 0u) inv_c[0] = ic;
+	for (unsigned b = i; b < T; b += gridDim.x * kBlock) bucket[b] = make_uint2(0u, 0u);
 	if (i >= n_sort) return;
 	unsigned long long k = kNone;
 	if (i < N) {
 		const float4 a = q0[i];
-		const double ic = inv_c[0];
-		k = cell_hash(cell_coord(a.x, ic), cell_coord(a.y, ic), cell_coord(a.z, ic), mask);
+		k = cell_hash(cell_coord(a.x, ic), cell_coord(a.y, ic), cell_coord(a.z, ic), T - 1u);
 	}
 	key[i] = k;
 	val[i] = i;
 }
 
-__global__ __launch_bounds__(kBlock) void k_bucket_clear(uint2* __restrict__ bucket, unsigned T) {
-	const unsigned b = blockIdx.x * kBlock + threadIdx.x;
-	if (b < T) bucket[b] = make_uint2(0u, 0u);
-}
-
-// [first, end) of each bucket's run of sorted keys
-__global__ __launch_bounds__(kBlock) void k_bucket_mark(const unsigned long long* __restrict__ key, unsigned N,
-                                                        uint2* __restrict__ bucket) {
-	const unsigned p = blockIdx.x * kBlock + threadIdx.x;
-	if (p >= N) return;
-	const unsigned long long k = key[p];
-	const unsigned b = (unsigned)k;
-	if (p == 0u || key[p - 1u] != k) bucket[b].x = p;
-	if (p + 1u == N || key[p + 1u] != k) bucket[b].y = p + 1u;
-}
-
-// packed records and cell codes in bucket order
+// [first, end) of each bucket's run of sorted keys; packed records and cell
+// codes in bucket order
 __global__ __launch_bounds__(kBlock) void k_grid_gather(const float4* __restrict__ q0, const float4* __restrict__ q1,
-                                                        const float4* __restrict__ q2, const unsigned* __restrict__ val,
-                                                        unsigned N, const double* __restrict__ inv_c,
+                                                        const float4* __restrict__ q2,
+                                                        const unsigned long long* __restrict__ key,
+                                                        const unsigned* __restrict__ val, unsigned N,
+                                                        const double* __restrict__ inv_c, uint2* __restrict__ bucket,
                                                         float4* __restrict__ s0, float4* __restrict__ s1,
                                                         float4* __restrict__ s2,
                                                         unsigned long long* __restrict__ scode) {
 	const unsigned p = blockIdx.x * kBlock + threadIdx.x;
 	if (p >= N) return;
+	const unsigned long long k = key[p];
+	if (p == 0u || key[p - 1u] != k) bucket[(unsigned)k].x = p;
+	if (p + 1u == N || key[p + 1u] != k) bucket[(unsigned)k].y = p + 1u;
 	const unsigned i = val[p];
 	const float4 a = q0[i];
 	s0[p] = a;
@@ -286,7 +290,7 @@ Layout layout(unsigned N) {
 	sz[S0] = sz[S1] = sz[S2] = 16u * (size_t)N;
 	sz[SCODE] = 8u * (size_t)N;
 	sz[PART] = 16u * (size_t)kRows * N;
-	sz[HM] = 4u;
+	sz[HM] = 4u * kHmaxBlocks;
 	sz[INVC] = 8u;
 	size_t o = 0;
 	for (int k = 0; k < kPlanes; ++k) {
@@ -337,18 +341,15 @@ int sfd_sph_cubic_grid(const float* rad, unsigned N, unsigned n_pad, float gamma
 	while (passes < 8u && (unsigned long long)mask >= (1ull << (8u * passes)) - 1ull) ++passes;
 
 	const int tok = sf_prof_begin("sph_grid_sort", s);
-	hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, hm);
-	hipLaunchKernelGGL(k_hmax, dim3(blocks(N)), dim3(kBlock), 0, s, rad, N, hm);
-	hipLaunchKernelGGL(k_cell_scale, dim3(1), dim3(64), 0, s, hm, inv_c);
-	hipLaunchKernelGGL(k_grid_keys, dim3(blocks(L.n_sort)), dim3(kBlock), 0, s, q0, N, L.n_sort, inv_c, mask, key0,
-	                   val0);
+	const unsigned n_hm = blocks(N) < kHmaxBlocks ? blocks(N) : kHmaxBlocks;
+	hipLaunchKernelGGL(k_hmax, dim3(n_hm), dim3(kBlock), 0, s, rad, N, hm);
+	hipLaunchKernelGGL(k_grid_keys, dim3(blocks(L.n_sort)), dim3(kBlock), 0, s, q0, N, L.n_sort, hm, n_hm, inv_c, L.T,
+	                   bucket, key0, val0);
 	if (sfd_radix_sort_passes(key0, val0, key1, val1, L.n_sort, hist, passes, s)) return -1;
 	unsigned long long* key = (passes & 1u) ? key1 : key0;
 	unsigned* val = (passes & 1u) ? val1 : val0;
-	hipLaunchKernelGGL(k_bucket_clear, dim3(blocks(L.T)), dim3(kBlock), 0, s, bucket, L.T);
-	hipLaunchKernelGGL(k_bucket_mark, dim3(blocks(N)), dim3(kBlock), 0, s, key, N, bucket);
-	hipLaunchKernelGGL(k_grid_gather, dim3(blocks(N)), dim3(kBlock), 0, s, q0, q1, q2, val, N, inv_c, s0, s1, s2,
-	                   scode);
+	hipLaunchKernelGGL(k_grid_gather, dim3(blocks(N)), dim3(kBlock), 0, s, q0, q1, q2, key, val, N, inv_c, bucket, s0, s1,
+	                   s2, scode);
 	sf_prof_end(tok, s);
 	const int tok1 = sf_prof_begin("sph_rho_grid", s);
 	hipLaunchKernelGGL(k_rho_grid, dim3(blocks((size_t)kRows * N)), dim3(kBlock), 0, s, s0, s1, scode, bucket, N,
