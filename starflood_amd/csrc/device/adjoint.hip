@@ -483,7 +483,7 @@ extern "C" {
 // bytes of part for sfd_force_vjp: k_vjp_sym's planes, or below kVjpSymMin
 // bodies k_vjp's
 size_t sfd_vjp_part_bytes(unsigned n_pad) {
-	return n_pad >= kVjpSymMin ? sym_part_bytes(n_pad, false) : (size_t)few_geometry(n_pad).bslices * n_pad * 32u;
+	return n_pad >= kVjpSymMin ? sym_part_bytes(n_pad, false, kVjpRecord) : (size_t)few_geometry(n_pad).bslices * n_pad * 32u;
 }
 
 int sfd_pack_nu(const float* mu, const float* mas, unsigned N, unsigned n_pad, float coef, int acc_phys, float* nu,
@@ -506,7 +506,7 @@ int sfd_force_vjp(const float* body, const float* nu, unsigned N, unsigned n_pad
 	float4* p4 = reinterpret_cast<float4*>(part);
 	const dim3 cgrid((N + kCombI - 1) / kCombI);
 	if (n_pad >= kVjpSymMin) {
-		const SymGeometry q = sym_geometry(n_pad, false);
+		const SymGeometry q = sym_geometry(n_pad, false, kVjpRecord);
 		double4* run = reinterpret_cast<double4*>(p4 + ((size_t)q.chunks + q.dchunks + q.per_launch) * n_pad);
 		for (unsigned d0 = 0; d0 < q.offsets; d0 += q.per_launch) {
 			const unsigned ch = d0 + q.per_launch < q.offsets ? q.per_launch : q.offsets - d0;

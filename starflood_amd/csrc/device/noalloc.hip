@@ -5,7 +5,7 @@
 // loops).  No counterpart in the reference.
 //
 // scratch holds the force kernels' partial sums.  It is sized for every N up to
-// SF_NOALLOC_MAX_N: 16.3 MiB (65 planes of one float4 per body at the largest
+// SF_NOALLOC_MAX_N: 32.5 MiB (65 planes of one double4 per body at the largest
 // n_pad).  Each device holds its own copy; its address comes from
 // hipGetSymbolAddress, once per device, on the first call with that device
 // current.

@@ -11,7 +11,8 @@
 // A block takes one set of i against a run of 64-body tiles of j.  It
 // writes the sums of its i to an i plane (one plane per run) and those of
 // each tile's j to the j plane of the offset: a body gets one contribution
-// per offset.  Planes hold one float4 per body.
+// per offset.  Planes hold one record per body, in FP64 (pp_sym.hip) or one
+// float4 (adjoint.hip).
 //
 // Two layouts.  Narrow: a set is 256 bodies, held by each of the block's
 // four wavefronts, which take a tile each.  Wide: a set is 1024 bodies, 256
@@ -26,15 +27,21 @@
 constexpr unsigned kSymTile = 64;                      // j per tile
 constexpr unsigned kSymNarrow = 256, kSymWide = 1024;  // bodies per set
 // Below kSymMin bodies the one-sided kernel (k_pp_few).  A force with its combine
-// and the wait for it, general masses: 9216 bodies one-sided 47.6 us, each pair
-// once 52.6; 10240 56.4 and 56.2; 11264 61.8 and 55.7; 12288 71.6 and 62.6.
+// and the wait for it, general masses: 10240 bodies one-sided 53.5 us, each pair
+// once 53.4; 11264 58.7 and 54.4; 12288 68.7 and 62.0 (with float4 planes 9216
+// 47.6 and 52.6).
 constexpr unsigned kSymMin = 10240;
 // The same line for the force VJP (k_vjp, k_vjp_sym).
 constexpr unsigned kVjpSymMin = 10240;
-// The wide layout from here: at 16384 bodies it takes 75.5 us and the narrow
-// one 73.9, at 24576 146 and 140, at 32768 226 and 230, at 65536 832 and 845.
+// The wide layout from here.  The line was drawn where the two met with float4
+// planes and packed bodies (kernels alone: 24576 bodies wide 146 us, narrow 140;
+// 32768 226 and 230).  With FP64 planes they meet higher: a step with equal masses
+// 26624 195 and 184, 32768 274 and 257, 49152 519 and 518, 57344 681 and 711, 65536
+// 875 and 920; general masses 32768 300 and 288, 65536 1046 and 1054.
 constexpr unsigned kSymWideMin = 25600;
 constexpr size_t kSymPlaneBytes = (size_t)512 << 20;   // j planes of one launch, at most
+constexpr unsigned kPpRecord = 32;                     // bytes of a body in a plane: the force's
+constexpr unsigned kVjpRecord = 16;                    // and its VJP's
 
 struct SymGeometry {
 	unsigned set;          // bodies per set
@@ -55,15 +62,15 @@ constexpr unsigned sym_items(unsigned S, unsigned offsets, unsigned tiles) {
 // Wide layout: the fewest tiles per block that leave at most ~4500 blocks,
 // four to five times what is resident (1024), up to 32.  Fewer, longer
 // blocks leave compute units idle at the end; more of them write and read
-// more i planes.  Measured, tiles: microseconds -- 32768 bodies 1: 247, 2:
+// more i planes.  Measured with float4 planes, tiles: microseconds -- 32768 bodies 1: 247, 2:
 // 226, 4: 233; 65536 2: 885, 8: 882, 16: 939; 131072 8: 3438, 32: 3410, 64:
 // 3592; 262144 16: 13619, 32: 13429, 64: 13630.
-constexpr SymGeometry sym_geometry(unsigned n_pad, bool wide) {
+constexpr SymGeometry sym_geometry(unsigned n_pad, bool wide, unsigned record) {
 	SymGeometry g{};
 	g.set = wide ? kSymWide : kSymNarrow;
 	g.blocks = n_pad / g.set;
 	g.offsets = g.blocks / 2u;
-	size_t fit = kSymPlaneBytes / ((size_t)n_pad * 16u);
+	size_t fit = kSymPlaneBytes / ((size_t)n_pad * record);
 	if (fit < 1u) fit = 1u;
 	g.per_launch = fit < g.offsets ? (unsigned)fit : g.offsets;
 	g.tiles = 1u;
@@ -82,10 +89,10 @@ constexpr SymGeometry sym_geometry(unsigned n_pad, bool wide) {
 
 // Bytes of all planes, and of the FP64 running sums (one double4 per body)
 // that several launches need.
-constexpr size_t sym_part_bytes(unsigned n_pad, bool wide) {
-	const SymGeometry g = sym_geometry(n_pad, wide);
+constexpr size_t sym_part_bytes(unsigned n_pad, bool wide, unsigned record) {
+	const SymGeometry g = sym_geometry(n_pad, wide, record);
 	const size_t planes = (size_t)g.chunks + g.dchunks + g.per_launch;
-	return planes * n_pad * 16u + (g.per_launch < g.offsets ? (size_t)n_pad * 32u : 0u);
+	return planes * n_pad * record + (g.per_launch < g.offsets ? (size_t)n_pad * 32u : 0u);
 }
 
 // the layout of the force kernel
@@ -106,7 +113,7 @@ constexpr FewGeometry few_geometry(unsigned n_pad) {
 }
 // bytes of partial sums of the fast PP force
 constexpr size_t pp_part_bytes(unsigned n_pad) {
-	return n_pad == 0u ? 0u : (n_pad >= kSymMin ? sym_part_bytes(n_pad, sym_pp_wide(n_pad))
+	return n_pad == 0u ? 0u : (n_pad >= kSymMin ? sym_part_bytes(n_pad, sym_pp_wide(n_pad), kPpRecord)
 	                                            : (size_t)few_geometry(n_pad).bslices * n_pad * 32u);
 }
 

@@ -3,8 +3,15 @@
 // The distance, 1/s and 1/s^3 of a pair serve both of its bodies: with equal
 // masses 16 VALU operations and one v_rsq_f32 for two interactions, where the
 // one-sided kernel (pp.hip) takes 24 and two (general masses: 19 and one
-// against 26 and two).  Every term has the one-sided kernel's bits; only the
-// order of each body's sum differs.
+// against 26 and two).  Every term has the one-sided kernel's bits.
+//
+// A body's sum.  In FP32 are added, plainly, its terms with the j of two tiles
+// (128, the one-sided kernel's two), which Kahan's steps then collect, and as j
+// its terms with a wavefront's 256 i: 64 sums of four at most, 67 roundings in a
+// row.  Everything further is FP64: the wavefronts' sums, the planes, the
+// combine.  With float4 planes a body's sum was rounded to 24 bits once per plane
+// (193 of them at N = 262144); the FP64 ones cost 1 % there (12.71 -> 12.85 ms a
+// step), 2.5 % at 65536, and 57 -> 60 us at 10007.
 //
 // What bounds it.  Measured on gfx950 with two or more wavefronts per SIMD:
 // a wave64 FP32 operation on VGPRs issues every 0.95-1.05 ns (1.17 for the
@@ -22,9 +29,10 @@
 //  * a step's j record is read one step ahead: 12.9 -> 12.7 ms, and 8 % at
 //    N = 10007, where fewer wavefronts hide the LDS latency.
 //
-// Kernel and combine, one-sided -> this, same box: N = 262144 17.3 -> 13.4 ms
-// (another box 17.0 -> 12.7; general masses 18.0 -> 15.6), N = 65536 1085 ->
-// 863 us, N = 16384 80 -> 67 us (general masses 83 -> 76), N = 10007 42 -> 35.
+// Kernel and combine, one-sided -> this, same box, with float4 planes (FP64 ones:
+// above): N = 262144 17.3 -> 13.4 ms (another box 17.0 -> 12.7; general masses
+// 18.0 -> 15.6), N = 65536 1085 -> 863 us, N = 16384 80 -> 67 us (general masses
+// 83 -> 76), N = 10007 42 -> 35.
 // The rest of its time at N = 16384 (54 us at the large-N rate) is the last
 // wavefronts of 2112 blocks on 1024 slots, and the combine.
 #include <hip/hip_runtime.h>
@@ -143,8 +151,8 @@ __device__ __forceinline__ void sym_tile(const float4* __restrict__ sj, float4* 
 template <bool POT>
 __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__ body, unsigned n_pad, unsigned S,
                                                       unsigned d0, unsigned d1, unsigned tiles, unsigned chunks,
-                                                      unsigned dchunks, float eps2, float4* __restrict__ part_i,
-                                                      float* __restrict__ part_j) {
+                                                      unsigned dchunks, float eps2, double4* __restrict__ part_i,
+                                                      double* __restrict__ part_j) {
 	__shared__ float4 s_j[2][2u * kSymTile];
 	__shared__ float4 s_acc[2][kWaves][2u * kSymTile];
 	const unsigned t = threadIdx.x, lane = t & 63u;
@@ -229,7 +237,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 			}
 			// the j side of m w (r_j - r_i) has the opposite sign
 			const double sc = uni ? (double)mu : 1.0;
-			part_j[((size_t)(tt / kSymWide) * n_pad + j) * 4u + t] = (float)(comp < 3u ? -sc * s : sc * s);
+			part_j[((size_t)(tt / kSymWide) * n_pad + j) * 4u + t] = comp < 3u ? -sc * s : sc * s;
 		}
 		// fold the i sums after two tiles of one kind
 		pending = !pending;
@@ -241,9 +249,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 	const unsigned plane = sym ? c : chunks + c;
 #pragma unroll
 	for (int k = 0; k < kPer; ++k)   // Kahan's compensation holds the negated lost low part
-		part_i[(size_t)plane * n_pad + i0 + 64u * k] = make_float4(
-		    (float)((double)sum[k][0] - (double)com[k][0]), (float)((double)sum[k][1] - (double)com[k][1]),
-		    (float)((double)sum[k][2] - (double)com[k][2]), (float)((double)sum[k][3] - (double)com[k][3]));
+		part_i[(size_t)plane * n_pad + i0 + 64u * k] =
+		    make_double4((double)sum[k][0] - (double)com[k][0], (double)sum[k][1] - (double)com[k][1],
+		                 (double)sum[k][2] - (double)com[k][2], (double)sum[k][3] - (double)com[k][3]);
 }
 
 // Narrow layout.  The block's four wavefronts hold the same 256 i and take
@@ -256,8 +264,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_pp_sym(const float4* __restrict__
 template <bool POT, class L>
 __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const L bodies, unsigned n_pad, unsigned S,
                                                              unsigned d0, unsigned chunks, unsigned dchunks,
-                                                             float eps2, float4* __restrict__ part_i,
-                                                             float4* __restrict__ part_j) {
+                                                             float eps2, double4* __restrict__ part_i,
+                                                             double4* __restrict__ part_j) {
 	__shared__ float4 s_mem[kWaves][4u * kSymTile];   // a wavefront's j and j sums, then its i sums
 	static_assert(kSet == 4u * kSymTile, "the i sums take the place of j and the j sums");
 	const unsigned t = threadIdx.x, lane = t & 63u;
@@ -268,7 +276,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const L bodies, uns
 	const unsigned nd = S / 2u - (((S & 1u) || ib < S / 2u) ? 0u : 1u);
 	const size_t out = (size_t)c * n_pad + ib * kSymNarrow + t;
 	if (sym && d0 + c >= nd) {
-		part_i[out] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+		part_i[out] = make_double4(0.0, 0.0, 0.0, 0.0);
 		return;
 	}
 	unsigned jb = sym ? ib + 1u + d0 + c : ib;
@@ -290,8 +298,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const L bodies, uns
 		const float4 p = acc[lane], q = acc[lane + kSymTile];
 		const double sc = uni ? (double)mu : 1.0;
 		part_j[(size_t)c * n_pad + j + lane] =
-		    make_float4((float)(-sc * ((double)p.x + (double)q.x)), (float)(-sc * ((double)p.y + (double)q.y)),
-		                (float)(-sc * ((double)p.z + (double)q.z)), (float)(sc * ((double)p.w + (double)q.w)));
+		    make_double4(-sc * ((double)p.x + (double)q.x), -sc * ((double)p.y + (double)q.y),
+		                 -sc * ((double)p.z + (double)q.z), sc * ((double)p.w + (double)q.w));
 	} else {
 		if (uni) sym_tile<POT, true, false>(sj, acc, lane, eps2, a);
 		else sym_tile<POT, false, false>(sj, acc, lane, eps2, a);
@@ -312,7 +320,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const L bodies, uns
 		sz += (double)p.z;
 		sp += (double)p.w;
 	}
-	part_i[out] = make_float4((float)sx, (float)sy, (float)sz, (float)sp);
+	part_i[out] = make_double4(sx, sy, sz, sp);
 }
 
 // Fixed-order FP64 sum of a launch's planes (the i planes, then the j
@@ -321,7 +329,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_pp_sym_narrow(const L bodies, uns
 // 64 particles; its wavefronts take every fourth plane each.
 constexpr unsigned kCombI = 64;
 template <class E, class L>
-__global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict__ part, unsigned n_pad,
+__global__ __launch_bounds__(kBlock) void k_sym_combine(const double4* __restrict__ part, unsigned n_pad,
                                                         unsigned planes, unsigned S, int last_offset, int first,
                                                         int last, double4* __restrict__ run, const L bodies,
                                                         float4* body, unsigned N, double G, int acc_phys, E epi) {
@@ -333,11 +341,11 @@ __global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict
 	double sx = 0.0, sy = 0.0, sz = 0.0, sp = 0.0;
 #pragma unroll 4
 	for (unsigned s = g; s < planes; s += kWaves) {
-		const float4 a = part[(size_t)s * n_pad + i];
-		sx += (double)a.x;
-		sy += (double)a.y;
-		sz += (double)a.z;
-		sp += (double)a.w;
+		const double4 a = part[(size_t)s * n_pad + i];
+		sx += a.x;
+		sy += a.y;
+		sz += a.z;
+		sp += a.w;
 	}
 	red[g][0][il] = sx;
 	red[g][1][il] = sy;
@@ -367,7 +375,7 @@ __global__ __launch_bounds__(kBlock) void k_sym_combine(const float4* __restrict
 }
 
 struct CombineArgs {
-	const float4* part;
+	const double4* part;
 	unsigned n_pad, planes, S;
 	int first, last;
 	double4* run;
@@ -386,7 +394,7 @@ void launch_combine(const CombineArgs& c, const L& bodies, const sf_force_epi& e
 
 // The force of n_pad bodies (a multiple of 1024, at least 2048), ended by *epi:
 // of the caller's arrays where pos is set (the narrow layout only), else of the
-// packed bodies; part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad)).
+// packed bodies; part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad), kPpRecord).
 extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsigned N, unsigned n_pad, float eps2,
                           double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
@@ -395,26 +403,26 @@ extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsig
 		sf_error("sfd_pp_sym", "n_pad %u does not fit N = %u", n_pad, N);
 		return -1;
 	}
-	const SymGeometry g = sym_geometry(n_pad, wide);
+	const SymGeometry g = sym_geometry(n_pad, wide, kPpRecord);
 	float4* b4 = reinterpret_cast<float4*>(body);
 	const PackedBodies packed{b4};
 	const ArrayBodies arrays{pos, mas, N};
 	const bool pot = epi->kind == SF_EPI_KICK || (epi->kind == SF_EPI_STORE && epi->pot);
-	float4* p4 = reinterpret_cast<float4*>(part);
-	double4* run = reinterpret_cast<double4*>(p4 + ((size_t)g.chunks + g.dchunks + g.per_launch) * n_pad);
+	double4* p4 = reinterpret_cast<double4*>(part);
+	double4* run = p4 + ((size_t)g.chunks + g.dchunks + g.per_launch) * n_pad;
 	for (unsigned d0 = 0; d0 < g.offsets; d0 += g.per_launch) {
 		const unsigned d1 = d0 + g.per_launch < g.offsets ? d0 + g.per_launch : g.offsets;
 		const int first = d0 == 0u, last = d1 == g.offsets;
 		const unsigned ch = wide ? g.chunks : d1 - d0;
 		const unsigned dch = first ? g.dchunks : 0u;   // the sets themselves go with the first launch
 		const unsigned pi = ch + dch;
-		float4* pj = p4 + (size_t)pi * n_pad;
+		double4* pj = p4 + (size_t)pi * n_pad;
 		const dim3 grid(g.blocks * pi);
 		const int tok = sf_prof_begin("pp_fast", s);
 		if (wide) {
 			auto k = pot ? k_pp_sym<true> : k_pp_sym<false>;
 			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, b4, n_pad, g.blocks, d0, d1, g.tiles, ch, dch, eps2, p4,
-			                   reinterpret_cast<float*>(pj));
+			                   reinterpret_cast<double*>(pj));
 		} else if (pos) {
 			auto k = pot ? k_pp_sym_narrow<true, ArrayBodies> : k_pp_sym_narrow<false, ArrayBodies>;
 			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, arrays, n_pad, g.blocks, d0, ch, dch, eps2, p4, pj);

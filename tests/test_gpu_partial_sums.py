@@ -1,0 +1,49 @@
+"""The partial sums of the kernels that split a body's sum over blocks, on
+states whose terms are whole numbers: everything that is added in FP32 stays
+below 2^24 and is exact; what a block hands to the combine may be odd and
+larger, and is exact only if it is held in more than 24 bits.  The result is
+then the rounded exact sum, bit for bit.
+
+Bodies of even index are sources at (1, 0, 0), those of odd index massless
+targets at the origin: s^2 rounds to 1 and a term is the source's mass, a
+number of 18 bits.  The sources of every second set (of 256 or 1024 bodies)
+lie at (-1, 0, 0) instead, so that the sums of the sets cancel.  Checked are
+the targets at the middle of a tile, whose j sums take half of their terms
+from each of the two copies."""
+import numpy as np
+import pytest
+import torch
+
+from starflood_amd import _lib as L
+from starflood_amd.sim import Simulation
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -20
+
+
+def sources(N, set_size):
+    """index, sign and value of the sources, and the targets that are checked"""
+    i = np.arange(N)
+    src = i % 2 == 0
+    sign = np.where((i // set_size) % 2 == 0, 1.0, -1.0)
+    value = np.random.default_rng(N).integers(2 ** 17, 2 ** 18, N).astype(np.float64)
+    rows = np.flatnonzero(~src & (abs(i % 64 - 31) <= 2))
+    return src, sign, value, rows
+
+
+@pytest.mark.parametrize("N,set_size", [(12200, 256), (26500, 1024), (67500, 1024), (300950, 1024)])
+def test_force_of_whole_numbers_is_exact(N, set_size):
+    print(f"whole-number force N={N}", flush=True)
+    src, sign, value, rows = sources(N, set_size)
+    with Simulation(N, enable_tree=0, logging=0, epsilon=EPS, precision=L.SF_PRECISION_FAST,
+                    acc_mode=L.SF_ACC_PHYSICAL) as s:
+        s.pos[:] = 0
+        s.pos[src, 0] = sign[src]
+        s.mas[:] = np.where(src, value, 0.0)
+        s.solve_gravity_pp()
+        got = s.acc[rows].copy()
+    L.set_params()
+    want = np.float32((sign * value)[src].sum())
+    assert abs(want) < 2 ** 25
+    assert np.all(got[:, 0] == want), np.unique(got[:, 0] - want)
+    assert np.all(got[:, 1:] == 0)
