@@ -128,9 +128,17 @@ __global__ __launch_bounds__(kBlock) void k_vjp(const float4* __restrict__ body,
 // wavefront, 43 ns at N = 65536 (the model of pp_sym.hip says 38).  One-sided
 // -> this, with the combine, us: N = 10007 75 -> 57, 16384 137 -> 110 (general
 // masses 160 -> 125), 65536 1884 -> 1422; at 8192 the one-sided kernel's 49 is
-// not beaten.
+// not beaten.  (With float4 planes.  A VJP call with general masses, float4
+// planes -> FP64 ones: 10007 76.3 -> 77.7, 16384 137.8 -> 139.5, 65536 1610 ->
+// 1647.)
 constexpr int kPer = 4;
 constexpr unsigned kWaves = kBlock / 64;
+
+// a body's sums in a plane
+struct Sum3 {
+	double x, y, z;
+};
+static_assert(sizeof(Sum3) == kVjpRecord, "the planes' bytes");
 
 struct KSet {
 	float x[kPer], y[kPer], z[kPer], m[kPer], nx[kPer], ny[kPer], nz[kPer];
@@ -188,8 +196,8 @@ __device__ __forceinline__ void vjp_sym_tile(const float4* __restrict__ sb, cons
 
 __global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict__ body, const float4* __restrict__ nu,
                                                        unsigned n_pad, unsigned S, unsigned d0, unsigned chunks,
-                                                       unsigned dchunks, float eps2, float4* __restrict__ part_i,
-                                                       float4* __restrict__ part_j) {
+                                                       unsigned dchunks, float eps2, Sum3* __restrict__ part_i,
+                                                       Sum3* __restrict__ part_j) {
 	__shared__ float4 s_mem[kWaves][6u * kSymTile];   // a wavefront's bodies, nu and j sums, then its k sums
 	const unsigned t = threadIdx.x, lane = t & 63u;
 	const unsigned wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -200,7 +208,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict_
 	const size_t out = (size_t)c * n_pad + ib * kSymNarrow + t;
 	const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	if (sym && d0 + c >= nd) {
-		part_i[out] = zero;
+		part_i[out] = {0.0, 0.0, 0.0};
 		return;
 	}
 	unsigned jb = sym ? ib + 1u + d0 + c : ib;
@@ -237,9 +245,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict_
 		else vjp_sym_tile<false, true>(sb, sn, acc, lane, eps2, a);
 		const float4 p = acc[lane], q = acc[lane + kSymTile];
 		const double sc = uni ? -(double)mu : -1.0;
-		part_j[(size_t)c * n_pad + j + lane] =
-		    make_float4((float)(sc * ((double)p.x + (double)q.x)), (float)(sc * ((double)p.y + (double)q.y)),
-		                (float)(sc * ((double)p.z + (double)q.z)), 0.0f);
+		part_j[(size_t)c * n_pad + j + lane] = {sc * ((double)p.x + (double)q.x), sc * ((double)p.y + (double)q.y),
+		                                        sc * ((double)p.z + (double)q.z)};
 	} else {
 		if (uni) vjp_sym_tile<true, false>(sb, sn, acc, lane, eps2, a);
 		else vjp_sym_tile<false, false>(sb, sn, acc, lane, eps2, a);
@@ -258,7 +265,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_vjp_sym(const float4* __restrict_
 		sy += (double)p.y;
 		sz += (double)p.z;
 	}
-	part_i[out] = make_float4((float)sx, (float)sy, (float)sz, 0.0f);
+	part_i[out] = {sx, sy, sz};
 }
 
 // What a combine does with g_k: store it, or take the adjoint one step
@@ -343,11 +350,11 @@ __global__ __launch_bounds__(kBlock) void k_vjp_combine(const double4* __restric
 	epi(k, (float)(G * sx), (float)(G * sy), (float)(G * sz));
 }
 
-// The same for a launch's planes of k_vjp_sym (one float4 per body and plane,
+// The same for a launch's planes of k_vjp_sym (one Sum3 per body and plane,
 // the k planes, then the j planes), added to the sums of the launches before
 // it (run, when !first), which all but the last keep there.
 template <class E>
-__global__ __launch_bounds__(kBlock) void k_vjp_sym_combine(const float4* __restrict__ part, unsigned n_pad,
+__global__ __launch_bounds__(kBlock) void k_vjp_sym_combine(const Sum3* __restrict__ part, unsigned n_pad,
                                                             unsigned planes, int first, int last,
                                                             double4* __restrict__ run, unsigned N, double G, E epi) {
 	__shared__ double red[kCombG][3][kCombI];
@@ -358,10 +365,10 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_combine(const float4* __rest
 	double sx = 0.0, sy = 0.0, sz = 0.0;
 #pragma unroll 4
 	for (unsigned s = w; s < planes; s += kCombG) {
-		const float4 a = part[(size_t)s * n_pad + k];
-		sx += (double)a.x;
-		sy += (double)a.y;
-		sz += (double)a.z;
+		const Sum3 a = part[(size_t)s * n_pad + k];
+		sx += a.x;
+		sy += a.y;
+		sz += a.z;
 	}
 	red[w][0][kl] = sx;
 	red[w][1][kl] = sy;
@@ -503,24 +510,24 @@ int sfd_force_vjp(const float* body, const float* nu, unsigned N, unsigned n_pad
 	if (n_pad == 0 || n_pad % 1024u != 0) return -1;
 	const float4* b4 = reinterpret_cast<const float4*>(body);
 	const float4* nu4 = reinterpret_cast<const float4*>(nu);
-	float4* p4 = reinterpret_cast<float4*>(part);
 	const dim3 cgrid((N + kCombI - 1) / kCombI);
 	if (n_pad >= kVjpSymMin) {
 		const SymGeometry q = sym_geometry(n_pad, false, kVjpRecord);
-		double4* run = reinterpret_cast<double4*>(p4 + ((size_t)q.chunks + q.dchunks + q.per_launch) * n_pad);
+		Sum3* planes = reinterpret_cast<Sum3*>(part);
+		double4* run = reinterpret_cast<double4*>(planes + ((size_t)q.chunks + q.dchunks + q.per_launch) * n_pad);
 		for (unsigned d0 = 0; d0 < q.offsets; d0 += q.per_launch) {
 			const unsigned ch = d0 + q.per_launch < q.offsets ? q.per_launch : q.offsets - d0;
 			const int first = d0 == 0u, last = d0 + ch == q.offsets;
 			const unsigned pi = ch + (first ? q.dchunks : 0u);
 			const int tok = sf_prof_begin("force_vjp", s);
 			hipLaunchKernelGGL(k_vjp_sym, dim3(q.blocks * pi), dim3(kBlock), 0, s, b4, nu4, n_pad, q.blocks, d0, ch,
-			                   pi - ch, eps2, p4, p4 + (size_t)pi * n_pad);
+			                   pi - ch, eps2, planes, planes + (size_t)pi * n_pad);
 			sf_prof_end(tok, s);
 			if (epi->step)
-				hipLaunchKernelGGL(k_vjp_sym_combine<VjpStep>, cgrid, dim3(kBlock), 0, s, p4, n_pad, pi + ch, first,
+				hipLaunchKernelGGL(k_vjp_sym_combine<VjpStep>, cgrid, dim3(kBlock), 0, s, planes, n_pad, pi + ch, first,
 				                   last, run, N, G, VjpStep(*epi));
 			else
-				hipLaunchKernelGGL(k_vjp_sym_combine<VjpStore>, cgrid, dim3(kBlock), 0, s, p4, n_pad, pi + ch, first,
+				hipLaunchKernelGGL(k_vjp_sym_combine<VjpStore>, cgrid, dim3(kBlock), 0, s, planes, n_pad, pi + ch, first,
 				                   last, run, N, G, VjpStore(*epi));
 		}
 		return sf_hip_check(hipGetLastError(), "sfd_force_vjp", "launch");

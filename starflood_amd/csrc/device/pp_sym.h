@@ -11,8 +11,8 @@
 // A block takes one set of i against a run of 64-body tiles of j.  It
 // writes the sums of its i to an i plane (one plane per run) and those of
 // each tile's j to the j plane of the offset: a body gets one contribution
-// per offset.  Planes hold one record per body, in FP64 (pp_sym.hip) or one
-// float4 (adjoint.hip).
+// per offset.  Planes hold one record per body, in FP64: nothing is rounded
+// between a block and the combine.
 //
 // Two layouts.  Narrow: a set is 256 bodies, held by each of the block's
 // four wavefronts, which take a tile each.  Wide: a set is 1024 bodies, 256
@@ -41,7 +41,7 @@ constexpr unsigned kVjpSymMin = 10240;
 constexpr unsigned kSymWideMin = 25600;
 constexpr size_t kSymPlaneBytes = (size_t)512 << 20;   // j planes of one launch, at most
 constexpr unsigned kPpRecord = 32;                     // bytes of a body in a plane: the force's
-constexpr unsigned kVjpRecord = 16;                    // and its VJP's
+constexpr unsigned kVjpRecord = 24;                    // and its VJP's
 
 struct SymGeometry {
 	unsigned set;          // bodies per set

@@ -47,3 +47,30 @@ def test_force_of_whole_numbers_is_exact(N, set_size):
     assert abs(want) < 2 ** 25
     assert np.all(got[:, 0] == want), np.unique(got[:, 0] - want)
     assert np.all(got[:, 1:] == 0)
+
+
+@pytest.mark.parametrize("masses", ["equal", "general"])
+@pytest.mark.parametrize("N", [12200, 140200])
+def test_vjp_of_whole_numbers_is_exact(N, masses):
+    """The weights take the masses' place: nu_j along y, across the distance,
+    so that a term of g is m_k nu_j - m_j nu_k = nu_j."""
+    print(f"whole-number VJP N={N} masses={masses}", flush=True)
+    src, sign, value, rows = sources(N, 256)
+    pos, mu = np.zeros((2, N, 3), np.float32)
+    pos[src, 0] = 1
+    mu[src, 1] = (sign * value)[src]
+    mas = np.ones(N, np.float32)
+    if masses == "general":
+        mas[src] = np.random.default_rng(N + 1).uniform(0.5, 1.5, N)[src].astype(np.float32)
+    lib = L.load()
+    L.set_params(epsilon=EPS, acc_mode=L.SF_ACC_PHYSICAL)
+    x, m, u = (torch.from_numpy(a).cuda() for a in (pos, mas, mu))
+    g = torch.empty_like(x)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.sf_force_vjp_dev(N, x.data_ptr(), m.data_ptr(), u.data_ptr(), g.data_ptr(), stream) == 0
+    got = g.cpu().numpy()[rows]
+    L.set_params()
+    want = np.float32((sign * value)[src].sum())
+    assert abs(want) < 2 ** 25
+    assert np.all(got[:, 1] == want), np.unique(got[:, 1] - want)
+    assert np.all(got[:, [0, 2]] == 0)
