@@ -91,37 +91,33 @@ __device__ __forceinline__ float wave_max(float v) {
 // p + 48 of the group, as many of these slots as the group fills.
 constexpr int kWays = 4;
 
-__device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
-	const float y = x - c;
-	const float t = s + y;
-	c = (t - s) - y;
-	s = t;
-}
-
 struct Slots {
 	float x[kWays], y[kWays], z[kWays];
 	float t[kWays][4];   // plain sums of at most 64 terms
-	float s[4], c[4];    // running Kahan sums of particle `lane`
+	double s[4];         // running sums of particle `lane`
 	int terms;           // in t, per lane
 };
 
 // a of the upper 32 lanes with b of the lower ones, and the same for odd and even rows
-__device__ __forceinline__ float swap_add32(float a, float b) {
+__device__ __forceinline__ double swap_add32(float a, float b) {
 	const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-	return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+	return (double)__uint_as_float(v[0]) + (double)__uint_as_float(v[1]);
 }
-__device__ __forceinline__ float swap_add16(float a, float b) {
-	const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-	return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+__device__ __forceinline__ double swap_add16(double a, double b) {
+	const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+	const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+	return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
 }
 
 // Adds t over the rows, slot r's sum to row r: lane l then holds particle l's.
+// In FP64: added plainly in FP32 the rows would make one sum of up to 256 terms
+// before the running sum sees it (the 1M step 1753 -> 1761 us).
 __device__ __forceinline__ void fold(Slots& a) {
 #pragma unroll
 	for (int u = 0; u < 4; ++u) {
-		const float lo = swap_add32(a.t[0][u], a.t[2][u]);   // lower half: slot 0, upper: slot 2
-		const float hi = swap_add32(a.t[1][u], a.t[3][u]);
-		kahan_add(a.s[u], a.c[u], swap_add16(lo, hi));
+		const double lo = swap_add32(a.t[0][u], a.t[2][u]);   // lower half: slot 0, upper: slot 2
+		const double hi = swap_add32(a.t[1][u], a.t[3][u]);
+		a.s[u] += swap_add16(lo, hi);
 #pragma unroll
 		for (int j = 0; j < kWays; ++j) a.t[j][u] = 0.0f;
 	}
@@ -307,7 +303,7 @@ __global__ __launch_bounds__(kBlock, QUAD ? 4 : 5) void k_walk(const float4* __r
 			for (int u = 0; u < 4; ++u) a.t[j][u] = 0.0f;
 		}
 #pragma unroll
-		for (int u = 0; u < 4; ++u) a.s[u] = a.c[u] = 0.0f;
+		for (int u = 0; u < 4; ++u) a.s[u] = 0.0;
 		a.terms = 0;
 		gx0 = wave_min(gx0);
 		gy0 = wave_min(gy0);
@@ -504,13 +500,11 @@ __global__ __launch_bounds__(kBlock, QUAD ? 4 : 5) void k_walk(const float4* __r
 		fold(a);
 		if (live) {
 			const unsigned i = order[p];
-			const double sx = (double)a.s[0] - (double)a.c[0], sy = (double)a.s[1] - (double)a.c[1],
-			             sz = (double)a.s[2] - (double)a.c[2], sp2 = (double)a.s[3] - (double)a.c[3];
 			const double f = acc_phys ? G : G * (double)body[p].w;
-			acc[3u * i + 0u] = (float)(f * sx);
-			acc[3u * i + 1u] = (float)(f * sy);
-			acc[3u * i + 2u] = (float)(f * sz);
-			pot[i] = (float)(-G * sp2);
+			acc[3u * i + 0u] = (float)(f * a.s[0]);
+			acc[3u * i + 1u] = (float)(f * a.s[1]);
+			acc[3u * i + 2u] = (float)(f * a.s[2]);
+			pot[i] = (float)(-G * a.s[3]);
 		}
 		n_cell_tot += (n_cell + n_mono) * (unsigned long long)cnt;
 		n_part_tot += (n_part - n_mono) * (unsigned long long)cnt;

@@ -74,3 +74,24 @@ def test_vjp_of_whole_numbers_is_exact(N, masses):
     assert abs(want) < 2 ** 25
     assert np.all(got[:, 1] == want), np.unique(got[:, 1] - want)
     assert np.all(got[:, [0, 2]] == 0)
+
+
+@pytest.mark.parametrize("seed", range(8))
+def test_walk_of_whole_numbers_is_exact(seed):
+    """The LBVH walk's sums over list entries: 40 targets at the origin, 256
+    sources at distance 1 (to the last bit of s^2) that a tiny theta opens, so
+    that a target's potential is the rounded sum of the sources' masses."""
+    print(f"whole-number walk seed={seed}", flush=True)
+    k = np.arange(256)
+    value = np.random.default_rng(seed).integers(2 ** 16, 2 ** 17, 256) * 2 + 1
+    with Simulation(296, logging=0, epsilon=EPS, theta=1e-9, precision=L.SF_PRECISION_FAST, tree_mode=L.SF_TREE_LBVH,
+                    acc_mode=L.SF_ACC_PHYSICAL) as s:
+        s.pos[:] = 0
+        s.pos[40:] = np.stack([np.ones(256), (k % 16) * 2.0 ** -20, (k // 16) * 2.0 ** -20], 1)
+        s.mas[:40] = 0
+        s.mas[40:] = value
+        s.solve()
+        got = s.pot[:40].copy()
+    L.set_params()
+    want = np.float32(-value.sum())
+    assert np.all(got == want), np.unique(got - want)
