@@ -322,9 +322,9 @@ extern "C" int sfd_energy_sums_exact(const float* ken, const float* pen, unsigne
 	const unsigned np = N ? (N + kChunk - 1u) / kChunk : 1u;
 	Partial* p = static_cast<Partial*>(part);
 	const int tok = sf_prof_begin("energy_sum_seq", s);
-	hipLaunchKernelGGL(k_exact_chunks, dim3(np, red ? 3 : 2), dim3(kBlock), 0, s, ken, pen, N, p, out, red,
+	hipLaunchKernelGGL(k_exact_chunks, dim3(np, pen ? (red ? 3 : 2) : 1), dim3(kBlock), 0, s, ken, pen, N, p, out, red,
 	                   fold::blocks(N));
-	if (np > 1u) hipLaunchKernelGGL(k_exact_finish, dim3(2), dim3(kBlock), 0, s, ken, pen, N, p, np, out);
+	if (np > 1u) hipLaunchKernelGGL(k_exact_finish, dim3(pen ? 2 : 1), dim3(kBlock), 0, s, ken, pen, N, p, np, out);
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_energy_sums_exact", "launch");
 }

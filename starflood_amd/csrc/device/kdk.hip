@@ -47,14 +47,25 @@ __global__ __launch_bounds__(kBlock) void k_drift_exact(float* __restrict__ pos,
 	if (k < n3) pos[k] = pos[k] + dt * vel[k];
 }
 
-// ken_i = (0.5 m_i) * ((vx^2 + vy^2) + vz^2); pen_i = m_i pot_i  (src/simulation.c:434-451)
-__global__ __launch_bounds__(kBlock) void k_energy_terms(const float* __restrict__ vel, const float* __restrict__ mas,
+// ken_i = (0.5 m_i) * ((vx^2 + vy^2) + vz^2); pen_i = m_i pot_i  (src/simulation.c:434-451).
+// KICK: the fast policy's closing kick first, for the step times log.
+template <bool KICK>
+__global__ __launch_bounds__(kBlock) void k_energy_terms(float* __restrict__ vel, const float* __restrict__ acc,
+                                                         float half_dt, const float* __restrict__ mas,
                                                          const float* __restrict__ pot, unsigned N,
                                                          float* __restrict__ ken, float* __restrict__ pen) {
 	const unsigned i = blockIdx.x * kBlock + threadIdx.x;
 	if (i >= N) return;
 	const float m = mas[i];
-	const float vx = vel[3u * i], vy = vel[3u * i + 1u], vz = vel[3u * i + 2u];
+	float vx = vel[3u * i], vy = vel[3u * i + 1u], vz = vel[3u * i + 2u];
+	if (KICK) {
+		vx = __builtin_fmaf(half_dt, acc[3u * i], vx);
+		vy = __builtin_fmaf(half_dt, acc[3u * i + 1u], vy);
+		vz = __builtin_fmaf(half_dt, acc[3u * i + 2u], vz);
+		vel[3u * i] = vx;
+		vel[3u * i + 1u] = vy;
+		vel[3u * i + 2u] = vz;
+	}
 	const float v2 = (vx * vx + vy * vy) + vz * vz;
 	ken[i] = 0.5f * m * v2;
 	pen[i] = m * pot[i];
@@ -193,9 +204,20 @@ extern "C" int sfd_energy_terms(const float* vel, const float* mas, const float*
                                 float* pen, hipStream_t s) {
 	if (!N) return 0;
 	const int tok = sf_prof_begin("energy_terms", s);
-	hipLaunchKernelGGL(k_energy_terms, dim3(grid_for(N)), dim3(kBlock), 0, s, vel, mas, pot, N, ken, pen);
+	hipLaunchKernelGGL(k_energy_terms<false>, dim3(grid_for(N)), dim3(kBlock), 0, s, const_cast<float*>(vel), nullptr,
+	                   0.0f, mas, pot, N, ken, pen);   // vel is not written without the kick
 	sf_prof_end(tok, s);
 	return sf_hip_check(hipGetLastError(), "sfd_energy_terms", "launch");
+}
+
+extern "C" int sfd_kick_energy_fast(float* vel, const float* acc, const float* mas, const float* pot, unsigned N,
+                                    float half_dt, float* ken, float* pen, hipStream_t s) {
+	if (!N) return 0;
+	const int tok = sf_prof_begin("kick", s);
+	hipLaunchKernelGGL(k_energy_terms<true>, dim3(grid_for(N)), dim3(kBlock), 0, s, vel, acc, half_dt, mas, pot, N, ken,
+	                   pen);
+	sf_prof_end(tok, s);
+	return sf_hip_check(hipGetLastError(), "sfd_kick_energy_fast", "launch");
 }
 
 extern "C" int sfd_x64_refresh(const float* pos, double* x64, unsigned n3, hipStream_t s) {

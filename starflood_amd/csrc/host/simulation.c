@@ -265,20 +265,25 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 
 	double* red_out = c->d_red + (size_t)(sfd_reduce_scratch_doubles(N) - SF_RED_VALUES);
 	const float* u = c->have_u ? c->d_u : NULL;
-	const int apart = exact && timing;
-	if (apart) {
+	/* the step times log has its columns apart */
+	if (timing && exact) {
 		if (sfd_kick_exact(vel, acc, n3, half_dt, s)) return STARFLOOD_FAILURE;    /* kick_1 */
 		tev_record(4, s);
 		if (sfd_energy_terms(vel, mas, pot, N, ken, pen, s)) return STARFLOOD_FAILURE;
-		/* ken_sum and pen_sum in one pass (its time is logged as ken_sum's) */
-		if (sfd_energy_sums_exact(ken, pen, N, red_out + SF_RED_VALUES, red_out + 12, NULL, s)) return STARFLOOD_FAILURE;
+		if (sfd_energy_sums_exact(ken, NULL, N, red_out + SF_RED_VALUES, red_out + 12, NULL, s))
+			return STARFLOOD_FAILURE;   /* ken_sum */
 		tev_record(5, s);
+		if (sfd_energy_sums_exact(pen, NULL, N, red_out + SF_RED_VALUES, red_out + 13, NULL, s))
+			return STARFLOOD_FAILURE;   /* pen_sum */
 		tev_record(6, s);
+	} else if (timing) {
+		/* kick_1 with the energy terms; the sums below are logged as ken_sum */
+		if (sfd_kick_energy_fast(vel, acc, mas, pot, N, half_dt, ken, pen, s)) return STARFLOOD_FAILURE;
+		tev_record(4, s);
 	}
 	/* FP64 W, P, L (and T, V in the fast policy), with kick_1 and the energy
-	   terms in the same pass: the fast policy's time is logged as kick_1's, the
-	   exact policy's log has them apart */
-	if (apart || fused) {
+	   terms in the same pass */
+	if (timing || fused) {
 		if (sfd_reduce_state(pos, exact ? NULL : c->d_x64, vel, mas, pot, ken, pen, u, N, p->G, p->epsilon, c->d_red, s))
 			return STARFLOOD_FAILURE;
 	} else if (exact) {
@@ -290,7 +295,6 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 		return STARFLOOD_FAILURE;
 	}
 	if (!exact && timing) {
-		tev_record(4, s);
 		tev_record(5, s);
 		tev_record(6, s);
 	}

@@ -184,10 +184,14 @@ int sfd_kick_drift_exact(float* vel, const float* acc, float* pos, unsigned int 
 /* ken_i = (0.5 m_i) |v_i|^2, pen_i = m_i pot_i */
 int sfd_energy_terms(const float* vel, const float* mas, const float* pot, unsigned int N,
                      float* ken, float* pen, hipStream_t s);
+/* v += half_dt a (the fast policy's rounding) first, in the same pass */
+int sfd_kick_energy_fast(float* vel, const float* acc, const float* mas, const float* pot, unsigned int N,
+                         float half_dt, float* ken, float* pen, hipStream_t s);
 /* exact_sum.hip: the sequential FP64 Kahan sums of ken and pen in index order
    (src/simulation.c:455-497), bit for bit, into out[0] and out[1]; part is
-   scratch of sfd_energy_scratch_bytes(N).  red (may be NULL): partials that
-   sfd_kick_reduce_exact left, folded in the same launch. */
+   scratch of sfd_energy_scratch_bytes(N).  pen NULL: the first sum alone.  red
+   (may be NULL, with pen only): partials that sfd_kick_reduce_exact left, folded
+   in the same launch. */
 size_t sfd_energy_scratch_bytes(unsigned int N);
 int sfd_energy_sums_exact(const float* ken, const float* pen, unsigned int N, void* part, double* out, double* red,
                           hipStream_t s);
