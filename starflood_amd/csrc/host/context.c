@@ -15,8 +15,6 @@
 #include "../sf_internal.h"
 #include "sf_host.h"
 
-#define SF_MAX_CTX 16
-
 static sf_ctx* g_ctx[SF_MAX_CTX];
 static hipStream_t g_default_stream = NULL;
 static int g_default_stream_ready = 0;
@@ -42,6 +40,11 @@ sf_ctx* sf_ctx_lookup(const void* host_mem, const char* func) {
 	}
 	sf_error(func, "sim.mem %p was not allocated by sim_init()", host_mem);
 	return NULL;
+}
+
+void sf_ctx_each(void (*f)(const sf_ctx*)) {
+	for (int k = 0; k < SF_MAX_CTX; ++k)
+		if (g_ctx[k]) f(g_ctx[k]);
 }
 
 static size_t round_up(size_t v, size_t m) { return (v + m - 1u) / m * m; }

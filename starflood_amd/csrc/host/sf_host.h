@@ -9,6 +9,11 @@
 
 #include "../sf_internal.h"
 
+/* context.c: at most SF_MAX_CTX live simulations; f of each */
+#define SF_MAX_CTX 16
+void sf_ctx_each(void (*f)(const sf_ctx*));
+/* fork.c: forked children find sim.mem where it is page-locked too */
+void sf_keep_in_children(void);
 /* gravity.c: PP gravity from d_mem pos/mas into d_mem acc/pot */
 int sf_solve_gravity_pp(sf_ctx* c);
 /* the exact policy's parameters for it */

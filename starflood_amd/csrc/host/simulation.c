@@ -102,6 +102,7 @@ int sim_init(sim_t* SF_RESTRICT sim_ptr, unsigned int N) {
 		return STARFLOOD_FAILURE;
 	}
 	c->host_pinned_base = pinned;
+	if (pinned) sf_keep_in_children();
 	if (pinned && hipHostGetDevicePointer((void**)&c->host_dev, mem, 0) != hipSuccess) {
 		(void)hipGetLastError();
 		c->host_dev = NULL;
