@@ -178,6 +178,10 @@ typedef struct {
 /* Statistics of the current device state (the T, V of the last sim_step
    are the values it logged). */
 int sf_get_stats(const sim_t* sim_ptr, sf_stats_t* out);
+/* The same of the last sim_step, as its own passes left them on the host
+   (STARFLOOD_FAILURE where they did not: no step yet, or one in RESIDENT mode
+   without logging or verbose). */
+int sf_step_stats(const sim_t* sim_ptr, sf_stats_t* out);
 
 /* --- initial conditions (synthetic, seeded, FP64 on the host) ---
    Each generator writes host sim.mem (pos, vel, mas; rad is left to the

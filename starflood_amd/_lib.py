@@ -116,6 +116,7 @@ _SIG = [
     ("sf_device_ext", C.c_void_p, [C.POINTER(SimT), C.c_int]),
     ("sf_ext_copy", C.c_int, [C.POINTER(SimT), C.c_int, C.c_void_p, C.c_int]),
     ("sf_get_stats", C.c_int, [C.POINTER(SimT), C.POINTER(Stats)]),
+    ("sf_step_stats", C.c_int, [C.POINTER(SimT), C.POINTER(Stats)]),
     ("sf_ic_uniform_ball", C.c_int, [C.POINTER(SimT), C.c_uint32, C.c_double, C.c_double, C.c_double]),
     ("sf_ic_plummer", C.c_int, [C.POINTER(SimT), C.c_uint32, C.c_uint, C.c_uint, C.c_double, C.c_double,
                                 C.POINTER(C.c_double), C.POINTER(C.c_double)]),

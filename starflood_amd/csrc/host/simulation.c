@@ -229,6 +229,7 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 	   launches (the same operations; the log's timings need them apart) */
 	const int fused = N && !exact && !timing && !p->enable_tree && !p->enable_sph;
 	int rc = 0;
+	c->have_stats = 0;
 
 	if (timing && !g_tev_ready) {
 		g_tev_ready = 1;
@@ -320,6 +321,7 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 			st->L[k] = r[7 + k];
 		}
 		st->K = r[10];
+		c->have_stats = 1;
 		if (p->logging && g_log_statistics) {
 			fprintf(g_log_statistics, "%u,%.015f,%.015f,%.015f\n", sim.step_number, st->V + st->T, st->V, st->T);
 			fflush(g_log_statistics);
@@ -341,6 +343,18 @@ int sf_sim_step(sim_t* SF_RESTRICT sim_ptr) {
 	sim.tree = sim_ptr->tree;
 	*sim_ptr = sim;
 	return rc ? STARFLOOD_FAILURE : STARFLOOD_SUCCESS;
+}
+
+int sf_step_stats(const sim_t* sim_ptr, sf_stats_t* out) {
+	if (!sim_ptr || !out) return STARFLOOD_FAILURE;
+	sf_ctx* c = sf_ctx_lookup(sim_ptr->mem, "sf_step_stats");
+	if (!c) return STARFLOOD_FAILURE;
+	if (!c->have_stats) {
+		sf_error("sf_step_stats", "the last sim_step left no statistics on the host");
+		return STARFLOOD_FAILURE;
+	}
+	*out = c->stats;
+	return STARFLOOD_SUCCESS;
 }
 
 int sf_get_stats(const sim_t* sim_ptr, sf_stats_t* out) {

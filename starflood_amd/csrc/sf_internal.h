@@ -53,7 +53,8 @@ typedef struct sf_ctx {
 	float* d_sph_tmp;        /* SPH scratch (packed records, 12 n_pad floats) */
 	void* d_sph_grid;        /* cell-grid pair search scratch (cubic model) */
 	hipStream_t stream;
-	sf_stats_t stats;        /* statistics of the last sim_step */
+	sf_stats_t stats;        /* statistics of the last sim_step, */
+	int have_stats;          /* where it left them on the host */
 	int have_u;
 } sf_ctx;
 

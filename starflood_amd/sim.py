@@ -142,8 +142,14 @@ class Simulation:
         return self._get_ext(L.SF_EXT_DUDT)
 
     def stats(self) -> dict:
+        return self._stats("sf_get_stats")
+
+    def step_stats(self) -> dict:
+        return self._stats("sf_step_stats")
+
+    def _stats(self, call: str) -> dict:
         s = L.Stats()
-        L.check(self.lib.sf_get_stats(C.byref(self.sim), C.byref(s)), "sf_get_stats")
+        L.check(getattr(self.lib, call)(C.byref(self.sim), C.byref(s)), call)
         return {"T": s.T, "V": s.V, "E": s.E, "W": s.W, "U": s.U, "P": list(s.P), "L": list(s.L), "K": s.K}
 
     def ic_uniform_ball(self, seed: int, radius: float = 1.0, total_mass: float = 1.0, v_hubble: float = 0.0):
