@@ -311,8 +311,8 @@ extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsig
 extern "C" int sfd_pp_fast(const float* pos, const float* mas, float* body, unsigned N, unsigned n_pad, float eps2,
                            double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
-	if (n_pad % 1024u != 0 || N > n_pad || (pos && epi->kind != SF_EPI_STORE)) {
-		sf_error("sfd_pp_fast", "n_pad %u does not fit N = %u", n_pad, N);
+	if (n_pad % 1024u != 0 || N > n_pad || (pos != nullptr) != (epi->kind == SF_EPI_STORE)) {
+		sf_error("sfd_pp_fast", "n_pad %u does not fit N = %u, or the bodies what they are for", n_pad, N);
 		return -1;
 	}
 	// part holds sfd_pp_part_bytes(n_pad)
@@ -347,12 +347,9 @@ extern "C" int sfd_pp_fast(const float* pos, const float* mas, float* body, unsi
 	else if (epi->kind == SF_EPI_KDK)
 		hipLaunchKernelGGL((k_pp_combine<EpiKdk, PackedBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, packed,
 		                   b4, N, G, acc_phys, EpiKdk(*epi));
-	else if (pos)
+	else
 		hipLaunchKernelGGL((k_pp_combine<EpiStore, ArrayBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices, arrays,
 		                   b4, N, G, acc_phys, EpiStore(*epi));
-	else
-		hipLaunchKernelGGL((k_pp_combine<EpiStore, PackedBodies>), cgrid, dim3(kBlock), 0, s, p4, n_pad, g.bslices,
-		                   packed, b4, N, G, acc_phys, EpiStore(*epi));
 	sf_prof_end(tok2, s);
 	return sf_hip_check(hipGetLastError(), "sfd_pp_fast", "k_pp_combine launch");
 }

@@ -393,14 +393,15 @@ void launch_combine(const CombineArgs& c, const L& bodies, const sf_force_epi& e
 }  // namespace
 
 // The force of n_pad bodies (a multiple of 1024, at least 2048), ended by *epi:
-// of the caller's arrays where pos is set (the narrow layout only), else of the
-// packed bodies; part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad), kPpRecord).
+// in the narrow layout SF_EPI_STORE's of the caller's arrays, else of the packed
+// bodies (pos NULL); part holds sym_part_bytes(n_pad, sym_pp_wide(n_pad), kPpRecord).
 extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsigned N, unsigned n_pad, float eps2,
                           double G, int acc_phys, float* part, const sf_force_epi* epi, hipStream_t s) {
 	if (N == 0) return 0;
 	const bool wide = sym_pp_wide(n_pad);
-	if (n_pad % kSymWide != 0 || n_pad < 2u * kSymWide || N > n_pad || (pos && (wide || epi->kind != SF_EPI_STORE))) {
-		sf_error("sfd_pp_sym", "n_pad %u does not fit N = %u", n_pad, N);
+	if (n_pad % kSymWide != 0 || n_pad < 2u * kSymWide || N > n_pad ||
+	    (pos != nullptr) != (!wide && epi->kind == SF_EPI_STORE)) {
+		sf_error("sfd_pp_sym", "n_pad %u does not fit N = %u, or the bodies what they are for", n_pad, N);
 		return -1;
 	}
 	const SymGeometry g = sym_geometry(n_pad, wide, kPpRecord);
@@ -423,7 +424,7 @@ extern "C" int sfd_pp_sym(const float* pos, const float* mas, float* body, unsig
 			auto k = pot ? k_pp_sym<true> : k_pp_sym<false>;
 			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, b4, n_pad, g.blocks, d0, d1, g.tiles, ch, dch, eps2, p4,
 			                   reinterpret_cast<double*>(pj));
-		} else if (pos) {
+		} else if (epi->kind == SF_EPI_STORE) {
 			auto k = pot ? k_pp_sym_narrow<true, ArrayBodies> : k_pp_sym_narrow<false, ArrayBodies>;
 			hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, arrays, n_pad, g.blocks, d0, ch, dch, eps2, p4, pj);
 		} else {

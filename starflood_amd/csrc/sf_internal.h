@@ -164,8 +164,8 @@ typedef struct {
 	float *gx0, *gv0;
 } sf_vjp_epi;
 
-/* Fast PP gravity of the n_pad packed bodies (a multiple of 1024), or of pos
-   and mas where pos is set (SF_EPI_STORE only; body is then scratch): partial
+/* Fast PP gravity of pos and mas (SF_EPI_STORE; body is then scratch) or of the
+   n_pad packed bodies (a multiple of 1024; pos NULL, the other epilogues): partial
    sums into part (sfd_pp_part_bytes), then a fixed-order FP64 combine that ends
    with *epi (only SF_EPI_KDK writes body).  From kSymMin bodies each pair is
    evaluated once (device/pp_sym.hip); below, every i against every j. */
