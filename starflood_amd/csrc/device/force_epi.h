@@ -24,8 +24,8 @@ struct EpiStore {
 	}
 };
 
-// sim_step: the closing kick and the particle's energies as well, with
-// k_kick_energy_fast's operations
+// sim_step: the closing kick and the particle's energies as well, with the
+// operations of kdk.hip's k_reduce_state<kFastKick> and k_energy_terms<true>
 struct EpiKick {
 	float *acc, *pot, *vel, *ken, *pen;
 	float h;

@@ -386,8 +386,9 @@ __global__ __launch_bounds__(kBlock) void k_karras(const unsigned long long* __r
 
 // ---- FP64 inclusive prefix sums over the sorted particles of (m, m x, m y,
 // m z) and, for quadrupoles, of m x' x'^T (x' = x - ref, six components).
-// Fixed shape: 16 consecutive elements per thread, a Hillis-Steele scan of
-// the 256 thread sums per block, one block scanning the block sums.
+// Fixed shape: spans of 1024 elements, summed by a wavefront each, 64 consecutive
+// elements at a time; tiles of four spans, whose sums one block scans; then
+// every span scanned in 64s from what lies before it.
 struct d4 {
 	double m, x, y, z;
 	__device__ static d4 zero() { return {0.0, 0.0, 0.0, 0.0}; }
@@ -399,7 +400,6 @@ struct d4 {
 	__device__ d4 shfl_up(unsigned o) const {
 		return {__shfl_up(m, o), __shfl_up(x, o), __shfl_up(y, o), __shfl_up(z, o)};
 	}
-	__device__ d4 shfl(int src) const { return {__shfl(m, src), __shfl(x, src), __shfl(y, src), __shfl(z, src)}; }
 };
 struct d6 {   // xx, xy, xz, yy, yz, zz
 	double v[6];
@@ -416,11 +416,6 @@ struct d6 {   // xx, xy, xz, yy, yz, zz
 	__device__ d6 shfl_up(unsigned o) const {
 		d6 r;
 		for (int k = 0; k < 6; ++k) r.v[k] = __shfl_up(v[k], o);
-		return r;
-	}
-	__device__ d6 shfl(int src) const {
-		d6 r;
-		for (int k = 0; k < 6; ++k) r.v[k] = __shfl(v[k], src);
 		return r;
 	}
 };

@@ -148,12 +148,12 @@ __device__ __forceinline__ bool opens(const float* bmin, const float* bmax, cons
 	return theta <= ratio;
 }
 
-// The node as one monopole, less particle i when the node's box holds it and
-// other bodies (holds; src/gravity.c:380-640), added into the (Kahan) sums.
 __device__ __forceinline__ bool in_box(const float* b, const float* ri) {   // b: the lower corner, then the upper
 	return b[0] <= ri[0] && ri[0] <= b[3] && b[1] <= ri[1] && ri[1] <= b[4] && b[2] <= ri[2] && ri[2] <= b[5];
 }
 
+// The node as one monopole, less particle i when the node's box holds it and
+// other bodies (holds; src/gravity.c:380-640), added into the (Kahan) sums.
 template <bool KAHAN_ACC, bool KAHAN_POT>
 __device__ __forceinline__ void add_monopole(const float* params, bool holds, const float* ri, float mi, float eps2,
                                              float* sum, float* com) {

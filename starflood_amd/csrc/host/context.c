@@ -120,10 +120,11 @@ int sf_ctx_reserve_part(sf_ctx* c, size_t bytes) {
 }
 
 /* Transfers of up to this many bytes go by kernel: it starts and ends in stream
-   order, while the copy engine's signals cost about 10 us a copy.  With larger
-   ones the engine's rate wins: 0.26 to 0.85 MB are faster by kernel (a step of
-   16384 bodies 371 us instead of 402), 1.6 MB slower (a frame of 65536 bodies
-   816 us instead of 805). */
+   order, while the copy engine's signals cost about 10 us a copy.  Then the
+   engine's rate catches up.  A Barnes-Hut step in mirror mode, kernel and engine:
+   0.33 MB up and 0.43 down 264 and 281 us, 1.04 and 1.35 334 and 348, 1.31 and 1.70
+   357 and 369, 1.64 and 2.13 383 and 393, 2.62 and 3.41 474 and 475; a frame of
+   65536 bodies, with 1.57 up and the frame's own transfers, 816 and 805. */
 #define SF_KERNEL_COPY_MAX 1310720u
 
 static int move_blocks(sf_ctx* c, const sf_blocks* span, unsigned int spans, int to_device, const double* red) {

@@ -144,10 +144,9 @@ static int is_device_pointer(const void* p) {
 	return attr.type == hipMemoryTypeDevice;
 }
 
-/* Reference-mode build from device pos/mas into d->d_node; reports the
-   reference's errors (src/tree.c:180-189) after a synchronisation. */
-/* Queues the reference build on s; d->order_n = N when the parallel build made
-   the tree (d->par.ev[0] marks its end on s). */
+/* Queues the reference-mode build from device pos/mas into d->d_node on s;
+   d->order_n = N when the parallel build made the tree (d->par.ev[0] marks its
+   end on s). */
 static int build_ref(sf_tree_dev* d, unsigned int N, const float* pos, const float* mas, hipStream_t s) {
 	const sf_params_t* p = sf_params();
 	/* 0: serial build only (also for no particles: the root alone) */
@@ -191,7 +190,8 @@ static int build_ref(sf_tree_dev* d, unsigned int N, const float* pos, const flo
 	return 0;
 }
 
-/* num_nodes, the host's nodes (mirror mode) and the build's result.  After a
+/* num_nodes, the host's nodes (mirror mode) and the build's result, with the
+   reference's errors (src/tree.c:180-189), after a synchronisation.  After a
    parallel build the copies run on its side stream, beside what s does next
    (the walk). */
 static int finish_ref(sf_tree_dev* d, tree_t* t, hipStream_t s) {
