@@ -44,12 +44,12 @@ DT = 1.0e-3
 SEED = 11
 PEAK_FP32_TFLOPS = 157.3
 FLOPS_PER_INTERACTION = 20
-# HBM bytes of one k_pp_sym dispatch at N = 262144 (128 planes of j sums, 512 MiB,
-# and the planes of i sums): rocprofv3 FETCH_SIZE 164600 KiB x 2.0 + WRITE_SIZE
-# 821700 KiB x 1.0, the factors from a 1 GiB copy read under the same counters
-# (profiles/pp_sym_n262144.md).  The writes are the planes; the kernel is
-# VALU-bound.
-PP_FAST_TRAFFIC_BYTES = (164600 * 2 + 821700) * 1024
+# HBM bytes of one of the two k_pp_sym dispatches of a force at N = 262144 (64
+# planes of j sums, 512 MiB, and the planes of i sums): rocprofv3 FETCH_SIZE 90540
+# KiB x 2.0 + WRITE_SIZE 805120 KiB x 1.0, the factors from a 1 GiB copy read under
+# the same counters (profiles/pp_sym_n262144.md).  The writes are the planes; the
+# kernel is VALU-bound.
+PP_FAST_TRAFFIC_BYTES = (90540 * 2 + 805120) * 1024
 
 
 def hip_sync():
@@ -832,7 +832,9 @@ def main():
     inter = float(N_PP) * N_PP
     value = inter * args.steps / elapsed / 1e9
     pp_avg_s = pp_ms / max(pp_n, 1) / 1e3
-    achieved = FLOPS_PER_INTERACTION * inter / pp_avg_s / 1e12
+    # a force takes one launch or more (pp_n of them over the steps)
+    flops_per_launch = FLOPS_PER_INTERACTION * inter * args.steps / max(pp_n, 1)
+    achieved = flops_per_launch / pp_avg_s / 1e12
     out = {
         "metric": METRIC,
         "value": value,
@@ -853,7 +855,7 @@ def main():
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": PP_FAST_TRAFFIC_BYTES,
                      "kernel": "k_pp_sym", "kernel_ms": pp_avg_s * 1e3,
                      "peak_source": "MI355X FP32 157.3 TFLOP/s; the kernel is FP32 VALU work (rsqrt and FMA, no MFMA)",
-                     "flops_per_launch": FLOPS_PER_INTERACTION * inter},
+                     "flops_per_launch": flops_per_launch},
         "energy_check": {"K": st["K"], "W": st["W"], "T_ken": st["T"]},
     }
     if not args.no_extra:

@@ -3,8 +3,8 @@
 // A launch of its own for each of these passes costs 4 to 5 us on the
 // stream, as much as a force of 2000 bodies: with these passes in the combine
 // a step of the adjoint forward is two launches instead of five, its backward
-// two instead of five, and 40 steps forward and back of 16384 bodies take
-// 8.3 ms instead of 9.1.
+// two instead of five, and 40 steps forward and back of 16384 bodies took
+// 8.3 ms instead of 9.1 (8.4 since the planes are FP64).
 #ifndef SF_FORCE_EPI_H
 #define SF_FORCE_EPI_H
 
